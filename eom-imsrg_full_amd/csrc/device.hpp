@@ -231,9 +231,8 @@ void launch_ob_partial(hipStream_t s, const DevLayout &L, const double *Lop, con
 void launch_ob_final(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop, const double *part,
                      double *RES, int hres, unsigned mask, const int *act, int nact, double *acc = nullptr,
                      double coef = 0.0, const double *coefp = nullptr, double *npart = nullptr);
-// sqrt of the sum of the nmirror + nob partials into out[inst * kScal]
-void launch_norm_from_parts(hipStream_t s, const DevLayout &L, const double *npart, double *out, const int *act,
-                            int nact);
+// sqrt of the sum of the n partials of each instance into out[inst * kScal]
+void launch_norm_from_parts(hipStream_t s, int n, const double *npart, double *out, const int *act, int nact);
 // E0 = 110 + 220 into RES[inst * rstride]
 void launch_e0(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop, double *RES,
                int hL, int hR, unsigned mask, double *partials, const int *act, int nact, long long rstride);
@@ -270,8 +269,42 @@ void launch_hf_2b(hipStream_t s, const DevLayout &L, const double *D, double *op
 void launch_hf_2b_window(hipStream_t s, const DevLayout &L, const double *D, double *op, double *W, int herm,
                          int r0, int nrows, long long wofs);
 
-void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, int mode, double coef, int store,
-                        int test, double conv, double tiny, int *live);
+struct GateArgs {
+  int mode;          // 0 BCH, 1 Magnus
+  double coef;
+  int store, test;   // Magnus: the advals slot to write (-1 none) and the one to test
+  double conv, tiny;
+  int seq;           // this gate's number: live[k] = seq << 1 | goes on
+  int *live;         // host memory, one entry per position
+};
+void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, const GateArgs &G);
+// launch_norm_from_parts (n partials per instance) and the gate after it in one launch
+void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
+                      const GateArgs &G);
+
+// A whole FP64 commutator (every one- and two-body term) in three launches,
+// for small bases (k_small_a, _b, _c).
+struct PhRow {      // per global pair row: what its upper elements' ph sums share
+  long long dbase;  // ph_desc index of column 0 (the row's first descriptor minus its column)
+  long long tbase;  // the row's first J' term
+  int b0, half;     // its 6j list in ap6_val; 1 when the pair is (i,i)
+};
+struct SmallArgs {
+  const double *Lop, *Rop;
+  double *RES, *acc;
+  double *ccL, *ccR, *Z, *wpp, *partials, *npart;
+  int hL, hR, hres, prepL;  // prepL: ccL is still to be made from L
+  unsigned mask;
+  double coef;
+  const double *coefp;
+  const SegProb *pp_probs, *ph_probs;
+  const int4 *pp_tiles, *ph_tiles, *tiles16;
+  int n_pp, n_ph, n16, n_diff, nsplit;
+  const int *diff_ob;       // one-body outputs whose orbits differ in (l, j, tz)
+  const PhRow *phrow;
+  const int *act;
+};
+void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallArgs A, int nact);
 
 // ---- adjoint commutator (adjoint.hip): Ybar += d<C,[P,Y]>/dY term by term
 void launch_adj_e0(hipStream_t s, const DevLayout &L, const double *P, const double *C, double *Y, int hP, int hY,

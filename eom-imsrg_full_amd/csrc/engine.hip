@@ -258,6 +258,37 @@ static int scratch_setup(imsrg_ctx_s *c) {
 }
 
 // ---------------------------------------------------------------- context
+// Tables of the three-launch commutator (launch_small), for bases that may use it.
+static constexpr long long kSmallElems = 1000000;  // two-body elements times instances (the rule at use_small)
+static int small_setup(imsrg_ctx_s *c, const std::vector<int> &same_ob) {
+  const Layout &Ly = c->lay;
+  const DevLayout &D = c->dl;
+  if (Ly.vsize > kSmallElems || D.n122_frows > 0 || D.n122_items == 0 || D.nccol == 0 || D.nphterm == 0 || D.nob == 0)
+    return 0;
+  std::vector<int4> t16;
+  for (int q = 0; q < Ly.nblocks; q++) {
+    const int nt = (Ly.bdim[q] + 15) / 16;
+    for (int a = 0; a < nt; a++)
+      for (int b = a; b < nt; b++) t16.push_back(make_int4(q, a, b, 0));
+  }
+  std::vector<PhRow> pr(Ly.npairs);
+  for (int r = 0; r < Ly.npairs; r++) {
+    const int q = Ly.pair_q[r], i = Ly.pair_a[r], j = Ly.pair_b[r];
+    const int key = ((Ly.jj[i] >> 1) * Ly.nhalf + (Ly.jj[j] >> 1)) * Ly.nJ + (Ly.bJ[q] >> 1);
+    pr[r] = PhRow{Ly.ph_ubase[r] - (r - Ly.pbase[q]), Ly.ph_tbase[r], Ly.ap6_base[key], i == j};
+  }
+  std::vector<int> diff;
+  for (int t = 0; t < D.nob; t++)
+    if (!std::binary_search(same_ob.begin(), same_ob.end(), t)) diff.push_back(t);
+  int rc = upload_table(c, t16, &c->tiles16);
+  if (!rc) rc = upload_table(c, pr, &c->phrow);
+  if (!rc) rc = upload_table(c, diff, &c->diff_ob);
+  if (rc) return rc;
+  c->n_tiles16 = (int)t16.size();
+  c->n_diff_ob = (int)diff.size();
+  c->small = true;
+  return 0;
+}
 int imsrg_ctx_create(int nsp, const int *n, const int *l, const int *jj, const int *tz, const int *con,
                      int device, imsrg_ctx *out) {
   return imsrg_ctx_create_batch(nsp, n, l, jj, tz, con, device, 1, out);
@@ -390,7 +421,13 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   UP(Ly.ccrow, ccrow); UP(Ly.ccrbase, ccrbase); UP(Ly.ccrow_a, ccrow_a); UP(Ly.ccrow_b, ccrow_b);
   UP(Ly.cccbase, cccbase); UP(Ly.cccol_p, cccol_p); UP(Ly.cccol_h, cccol_h); UP(cccol_q, cccol_q);
   UP(Ly.sixj, sixj);
-  UP(Ly.ap6_val, ap6_val); UP(Ly.ap6_base, ap6_base);
+  {
+    // 64 zeros past the end: an absent J' sum is read with weight 0 up to 62 entries past its row's list
+    std::vector<double> v6(Ly.ap6_val);
+    v6.resize(v6.size() + 64, 0.0);
+    UP(v6, ap6_val);
+  }
+  UP(Ly.ap6_base, ap6_base);
   D.ap6_max = Ly.ap6_max;
   UP(Ly.ph_quads, ph_quads);
   D.nquad = (long long)Ly.ph_quads.size();
@@ -453,6 +490,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   }
   D.nmirror = (int)mtiles.size();
   UP(mtiles, mirror_tiles);
+  if (!rc) rc = small_setup(c, same_ob);
 #undef UP
   const size_t B = (size_t)nbatch;
   if (!rc) rc = dalloc(c, (size_t)Ly.vsize * B, &c->wpp);
@@ -463,7 +501,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   if (!rc) rc = dalloc(c, Ly.ph_terms.size() * B, &c->tph);
   if (!rc) rc = dalloc(c, kPartials * B, &c->partials);
   if (!rc) rc = dalloc(c, (size_t)std::max(D.nsame, 1) * D.ob_nchunk * B, &c->obpart);
-  if (!rc) rc = dalloc(c, (size_t)(D.nmirror + D.nob) * B, &c->npart);
+  if (!rc) rc = dalloc(c, (size_t)(std::max(D.nmirror, c->n_tiles16) + D.nob) * B, &c->npart);
   if (!rc) rc = dalloc(c, kScal * B, &c->scal);
   if (!rc) rc = dalloc(c, 1, &c->coef_d);
   if (!rc) rc = dalloc(c, (size_t)Ly.nsp * Ly.nsp * B, &c->mono);
@@ -574,6 +612,10 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
     if (!rc) rc = upload_table(c, tp, (const int4 **)&c->adj_pp_tiles);
     if (!rc) rc = upload_table(c, ph, (const GemmProb **)&c->adj_ph_probs);
     if (!rc) rc = upload_table(c, th, (const int4 **)&c->adj_ph_tiles);
+  }
+  if (!rc && c->small) {
+    const std::vector<DevLayout> dl(1, c->dl);
+    rc = upload_table(c, dl, &c->dl_d);
   }
   if (!rc) launch_fill(c->stream, c->wpp, Ly.vsize * B, 0.0);
   if (!rc && Ly.cwsize > 0) launch_fill(c->stream, c->wph, Ly.cwsize * B, 0.0);
@@ -1102,6 +1144,8 @@ struct CommEpi {
   double coef = 0.0;
   const double *coefp = nullptr;  // coef in device memory (graph replays)
   bool norm = false;
+  int *gate_act = nullptr;        // series table of the gate that follows (nullptr: none)
+  GateArgs gate{};
 };
 // cc_ready bits: kLPrepped -- cc[0] already holds the Pandya matrices of L,
 // and with int8 slices the slices of L too (prep_L; drivers reuse them across
@@ -1112,6 +1156,21 @@ struct CommEpi {
 enum { kLPrepped = 1, kLPandya = 2, kRPandya = 4 };
 static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                          int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi());
+
+// The three-launch form (launch_small) of a whole FP64 commutator: while the
+// two-body part of all instances holds at most 10^6 elements, issuing the
+// separate kernels costs more than they run.  Per commutator of a BCH series,
+// separate / three launches, in us: emax 2 82 / 39, emax 4 91 / 52, emax 5
+// 124 / 83, emax 6 (9.6e5 elements) 151 / 146, 4 x emax 5 (1.15e6) 163 / 175,
+// 16 x emax 4 (1.16e6) 187 / 222, emax 7 323 / 349, emax 8 640 / 912: past the
+// line the ph sums straight from Z cost more than the J' terms made once.
+// Masks with terms left out, profiling, tile shapes set to 128 x 64 and bases
+// with 122 sets past 32 rows keep the separate kernels.
+static bool use_small(imsrg_ctx_s *c, unsigned mask, int cc_ready, int na) {
+  const unsigned all = T111 | T121 | T122 | T221 | T222PPHH | T222PH;
+  return c->small && c->prec == IMSRG_PREC_FP64 && !c->prof_on && (mask & all) == all &&
+         !(cc_ready & (kLPandya | kRPandya)) && c->shape_pp != 1 && c->shape_ph != 1 && c->lay.vsize * na <= kSmallElems;
+}
 
 // Tile-shape autotuner: on the first FP64 commutator of a context, each 222
 // GEMM is timed (HIP events, best of 3) in both FP64 tile shapes on the
@@ -1172,16 +1231,19 @@ static int autotune(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R) {
 // addresses, so a replay is the same work as the eager sequence.
 static int comm_impl(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                      int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi()) {
-  if (c->prec == IMSRG_PREC_FP64 && c->shape_pp < 0 && a.n() > 0 && (mask & (T222PPHH | T221 | T222PH))) {
+  if (c->prec == IMSRG_PREC_FP64 && c->shape_pp < 0 && a.n() > 0 && (mask & (T222PPHH | T221 | T222PH)) &&
+      !use_small(c, mask, cc_ready, a.g())) {
     c->fork_mark = nullptr;  // the tuning launches follow the mark on the stream
     int rc = autotune(c, L, R);
     if (rc) return rc;
   }
   if (!c->graphs || c->prof_on || a.n() == 0) return comm_launches(c, L, R, RES, mask, cc_ready, a, epi);
+  // the gate's arguments change with every term: it stays outside the graph
   c->fork_mark = nullptr;  // a replayed graph runs on one stream
   // the series coefficient goes through device memory, written before the
   // replay, so the terms of a series share one graph
   CommEpi ge = epi;
+  ge.gate_act = nullptr;
   if (ge.acc) {
     launch_fill(c->stream, c->coef_d, 1, epi.coef);
     ge.coef = 0.0;
@@ -1211,6 +1273,7 @@ static int comm_impl(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *R
   }
   HIPCHK(hipGraphLaunch(it->second, c->stream));
   c->graph_launches++;
+  if (epi.gate_act) launch_series_gate(c->stream, epi.gate_act, a.g(), c->scal, epi.gate);
   return 0;
 }
 
@@ -1224,6 +1287,24 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
   const long long OS = D.op_size;
   if (na == 0) {
     c->fork_mark = nullptr;
+    return 0;
+  }
+  if (use_small(c, mask, cc_ready, na)) {
+    SmallArgs A{};
+    A.Lop = L->d; A.Rop = R->d; A.RES = RES->d; A.acc = epi.acc;
+    A.ccL = c->cc[0]; A.ccR = c->cc[1]; A.Z = c->wph; A.wpp = c->wpp; A.partials = c->partials;
+    A.npart = epi.norm ? c->npart : nullptr;
+    A.hL = hL; A.hR = hR; A.hres = hres; A.prepL = !lcc;
+    A.mask = mask; A.coef = epi.coef; A.coefp = epi.coefp;
+    A.pp_probs = c->pp_probs; A.ph_probs = c->ph_probs;
+    A.pp_tiles = c->pp_tiles; A.ph_tiles = c->ph_tiles; A.tiles16 = c->tiles16;
+    A.n_pp = c->n_pp_tiles; A.n_ph = c->n_ph_tiles; A.n16 = c->n_tiles16; A.n_diff = c->n_diff_ob;
+    A.diff_ob = c->diff_ob; A.phrow = c->phrow; A.act = ad;
+    launch_small(s, D, c->dl_d, A, na);
+    c->fork_mark = nullptr;
+    if (epi.gate_act) launch_norm_gate(s, c->npart, c->n_tiles16 + D.nob, epi.gate_act, na, c->scal, epi.gate);
+    else if (epi.norm) launch_norm_from_parts(s, c->n_tiles16 + D.nob, c->npart, c->scal, ad, na);
+    HIPCHK(hipGetLastError());
     return 0;
   }
   // The pp/hh chain (122 or clear, pp/hh GEMM, one-body partials) and the
@@ -1300,7 +1381,11 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
   PROF(c, IMSRG_PROF_MIRROR, launch_sym_mirror(s, D, RES->d, hres, ad, na, epi.acc, epi.coef, epi.coefp, np));
   PROF(c, IMSRG_PROF_ONEBODY,
        launch_ob_final(s, D, L->d, R->d, c->obpart, RES->d, hres, mask, ad, na, epi.acc, epi.coef, epi.coefp, np));
-  if (epi.norm) PROF(c, IMSRG_PROF_NORM, launch_norm_from_parts(s, D, c->npart, c->scal, ad, na));
+  if (epi.gate_act)
+    PROF(c, IMSRG_PROF_NORM,
+         launch_norm_gate(s, c->npart, D.nmirror + D.nob, epi.gate_act, na, c->scal, epi.gate));
+  else if (epi.norm)
+    PROF(c, IMSRG_PROF_NORM, launch_norm_from_parts(s, D.nmirror + D.nob, c->npart, c->scal, ad, na));
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1508,24 +1593,41 @@ static void prep_L(imsrg_ctx_s *c, imsrg_op_s *G, const ActSet &set) {
     launch_slice_cc(c->stream, c->dl, c->i8, ns, c->cc[0], c->i8pm, c->i8c[0], c->i8cs[0], set.d, set.n());
   }
 }
-// The series gate after nested commutator n: the test on the device, its
-// live flags into ring slot n % kGateRing, marked by an event.
-static int series_gate(imsrg_ctx_s *c, int slot, const ActSet &set, int n, int mode, double coef, int store,
-                       int test) {
-  const int r = n % imsrg_ctx_s::kGateRing;
-  launch_series_gate(c->stream, c->act_d[slot], set.g(), c->scal, mode, coef, store, test, kConv, kTiny,
-                     c->live_d + (size_t)r * c->nbatch);
-  HIPCHK(hipEventRecord(c->ev_gate[r], c->stream));
-  return 0;
+// The series gate after nested commutator n: the test on the device, its live
+// flags into ring slot n % kGateRing under the gate's sequence number.
+static GateArgs gate_args(imsrg_ctx_s *c, int n, int mode, double coef, int store, int test) {
+  c->gate_seq = c->gate_seq == (1 << 30) - 1 ? 1 : c->gate_seq + 1;
+  return GateArgs{mode, coef, store, test, kConv, kTiny, c->gate_seq,
+                  c->live_d + (size_t)(n % imsrg_ctx_s::kGateRing) * c->nbatch};
 }
-// Waits for the live flags of gate n; live[k] = 1 for positions that go on.
-static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, std::vector<int> &live, int &nlive) {
-  const int r = n % imsrg_ctx_s::kGateRing;
-  HIPCHK(hipEventSynchronize(c->ev_gate[r]));
-  const volatile int *f = c->live_h + (size_t)r * c->nbatch;
+// marks gate n on the stream: the second stream of the next commutator forks
+// from there (nullptr when that commutator runs on one stream)
+static hipEvent_t gate_mark(imsrg_ctx_s *c, int n, const ActSet &set) {
+  if (!c->dual || c->graphs || use_small(c, IMSRG_TALL, kLPrepped, set.g())) return nullptr;
+  hipEvent_t e = c->ev_gate[n % imsrg_ctx_s::kGateRing];
+  return hipEventRecord(e, c->stream) == hipSuccess ? e : nullptr;
+}
+// Waits for the live flags of gate n (sequence number seq), read from the
+// pinned ring as the kernel writes them (an event costs a record and a wake-up
+// per commutator); live[k] = 1 for positions that go on.  The stream is asked
+// now and then, so a failed launch ends the wait.
+static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, int seq, std::vector<int> &live, int &nlive) {
+  const volatile int *f = c->live_h + (size_t)(n % imsrg_ctx_s::kGateRing) * c->nbatch;
   live.assign(set.n(), 0);
   nlive = 0;
-  for (int k = 0; k < set.n(); k++) nlive += (live[k] = f[k] ? 1 : 0);
+  for (int k = 0; k < set.n(); k++) {
+    int v = f[k];
+    for (long long spin = 1; (v >> 1) != seq; v = f[k], spin++) {
+      if (spin % 4096) continue;
+      const hipError_t e = hipStreamQuery(c->stream);
+      if (e == hipErrorNotReady) continue;
+      v = f[k];
+      if (e != hipSuccess || (v >> 1) != seq)
+        return fail(IMSRG_EDEVICE, std::string("series gate: ") + hipGetErrorString(e));
+      break;
+    }
+    nlive += (live[k] = v & 1);
+  }
   return 0;
 }
 
@@ -1552,7 +1654,8 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
   const ActSet cur = series_set(c, 1, a);
   prep_L(c, G, cur);
   std::vector<int> live(a.n(), 1);  // positions in the series for nested commutator iw
-  int nlive = a.n();
+  int nlive = a.n(), seq = 0;
+  hipEvent_t mark = nullptr;
   double coef = 1.0;
   for (int iw = 2; iw <= 40; iw++) {
     coef = coef / (iw - 1.0);
@@ -1561,11 +1664,14 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
     epi.acc = HS->d;
     epi.coef = coef;
     epi.norm = true;
+    epi.gate_act = c->act_d[1];
+    epi.gate = gate_args(c, iw, 0, coef, -1, 0);
     // nothing was enqueued since the last gate: the second stream can fork from its event
-    c->fork_mark = iw > 2 ? c->ev_gate[(iw - 1) % imsrg_ctx_s::kGateRing] : nullptr;
+    c->fork_mark = mark;
     int rc = comm_impl(c, G, AD, INT2, IMSRG_TALL, kLPrepped, cur, epi);
-    if (!rc) rc = series_gate(c, 1, cur, iw, 0, coef, -1, 0);
-    if (!rc && iw > 2) rc = series_live(c, cur, iw - 1, live, nlive);
+    mark = gate_mark(c, iw, cur);
+    if (!rc && iw > 2) rc = series_live(c, cur, iw - 1, seq, live, nlive);
+    seq = epi.gate.seq;
     if (rc) return rc;
     if (nlive == 0) return 0;  // the test after iw-1 stopped every instance
     for (int k = 0; k < cur.n(); k++) nterms[k] += live[k];
@@ -1573,7 +1679,7 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
     AD = c->tmp[0];
     INT2 = c->tmp[1];
   }
-  int rc = series_live(c, cur, 40, live, nlive);
+  int rc = series_live(c, cur, 40, seq, live, nlive);
   if (rc) return rc;
   if (nlive > 0) return fail(IMSRG_ECLIP, "clipping BCH");
   return 0;
@@ -1636,11 +1742,12 @@ static int magexp_impl(imsrg_ctx_s *c, imsrg_op_s *DG, imsrg_op_s *G, const ActS
        launch_sumsq(c->stream, c->dl, cur->d, c->partials, c->scal + kAdvSlot, set.d, set.n()));
   PROF(c, IMSRG_PROF_NORM,
        launch_sumsq(c->stream, c->dl, G->d, c->partials, c->scal + kFullSlot, set.d, set.n()));
-  int rc = series_gate(c, 2, set, 1, 1, 0.0, -1, 0);
-  if (rc) return rc;
+  GateArgs g = gate_args(c, 1, 1, 0.0, -1, 0);
+  launch_series_gate(c->stream, c->act_d[2], set.g(), c->scal, g);
   prep_L(c, G, set);
   std::vector<int> live;
-  int nlive = 0;
+  int nlive = 0, seq = g.seq, rc = 0;
+  hipEvent_t mark = nullptr;  // prep_L follows the first gate on the stream
   for (int i = 2; i <= 7; i++) {
     // q of the early exit before nested commutator i+1 (advals(i+1-q) is tested)
     const int q = (std::fabs(cof[i - 1]) > kConv) ? 1 : 2;
@@ -1649,11 +1756,15 @@ static int magexp_impl(imsrg_ctx_s *c, imsrg_op_s *DG, imsrg_op_s *G, const ActS
     epi.acc = DG->d;
     epi.coef = cof[i - 1];
     epi.norm = true;
-    c->fork_mark = i > 2 ? c->ev_gate[(i - 1) % imsrg_ctx_s::kGateRing] : nullptr;
+    if (i < 7) {  // advals(i) = ||oth|| |cof(i)|, then the test for commutator i+1
+      epi.gate_act = c->act_d[2];
+      epi.gate = gate_args(c, i, 1, std::fabs(cof[i - 1]), i - 1, i - q);
+    }
+    c->fork_mark = mark;
     rc = comm_impl(c, G, cur, oth, IMSRG_TALL & ~(T110 | T220), kLPrepped, set, epi);
-    // advals(i) = ||oth|| |cof(i)|, then the test for commutator i+1
-    if (!rc && i < 7) rc = series_gate(c, 2, set, i, 1, std::fabs(cof[i - 1]), i - 1, i - q);
-    if (!rc) rc = series_live(c, set, i - 1, live, nlive);
+    mark = i < 7 ? gate_mark(c, i, set) : nullptr;
+    if (!rc) rc = series_live(c, set, i - 1, seq, live, nlive);
+    seq = epi.gate.seq;
     if (rc) return rc;
     if (nlive == 0) break;
     for (int k = 0; k < set.n(); k++) nterms[k] += live[k];

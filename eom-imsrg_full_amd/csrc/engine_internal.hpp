@@ -48,11 +48,13 @@ struct imsrg_ctx_s {
   hipEvent_t fork_mark = nullptr;
   bool dual = true;        // use stream2 (imsrg_ctx_set_concurrency)
   // BCH / Magnus series: the gate kernel after nested commutator n writes one
-  // live flag per series position into ring slot n % kGateRing of pinned host
-  // memory and ev_gate marks it; the host reads slot n-1 while commutator n runs
+  // live flag per series position, under the gate's sequence number, into ring
+  // slot n % kGateRing of pinned host memory; the host reads slot n-1 while
+  // commutator n runs.  ev_gate marks the gate for the second stream's fork.
   static constexpr int kGateRing = 4;
   int *live_h = nullptr, *live_d = nullptr;  // host and device views, kGateRing * nbatch
   hipEvent_t ev_gate[kGateRing] = {};
+  int gate_seq = 0;        // number of the last series gate (GateArgs::seq)
   bool capturing = false;  // graph capture records one stream only
   std::vector<void *> dallocs;
   int nbatch = 1;           // independent instances per operator
@@ -78,6 +80,14 @@ struct imsrg_ctx_s {
   int n_pp_tiles = 0, n_ph_tiles = 0;
   int4 *pp_tiles_w = nullptr, *ph_tiles_w = nullptr;    // 128 x 64 tiles (FP64 path)
   int n_pp_tiles_w = 0, n_ph_tiles_w = 0;
+  // the three-launch commutator of small bases (launch_small): tables, and the
+  // layout's view in device memory; small = false when the basis is not taken
+  bool small = false;
+  const DevLayout *dl_d = nullptr;
+  const int4 *tiles16 = nullptr;
+  const PhRow *phrow = nullptr;
+  const int *diff_ob = nullptr;
+  int n_tiles16 = 0, n_diff_ob = 0;
   // FP64 tile shape per GEMM, chosen by timing both on the first FP64
   // commutator of the context: -1 not yet tuned, 0 64x64, 1 128x64
   int shape_pp = -1, shape_ph = -1;

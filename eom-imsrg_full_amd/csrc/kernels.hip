@@ -512,25 +512,12 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
   }
 }
 
+// one workgroup's tile `tl` (operands of the instance)
 template <bool A_KMAJOR, int MODE, int EPI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 4 : 1))) void k_seg_gemm(const SegProb *__restrict__ probs,
-                                                  const int4 *__restrict__ tiles, int ntiles,
-                                                  const double *__restrict__ X0,
-                                                  const double *__restrict__ X1, double g0, double g1,
-                                                  double *__restrict__ C, double *__restrict__ W,
-                                                  double sigma, const int *act, long long sx,
-                                                  long long sc, long long sw) {
-  const int t = blockIdx.x;
-  if (t >= ntiles) return;
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    X0 += inst * sx;
-    X1 += inst * sx;
-    if (C) C += inst * sc;
-    if (W) W += inst * sw;
-  }
-  const int4 tl = tiles[t];
+__device__ __forceinline__ void seg_block(const SegProb *__restrict__ probs, const int4 tl,
+                                          const double *__restrict__ X0, const double *__restrict__ X1, double g0,
+                                          double g1, double *__restrict__ C, double *__restrict__ W, double sigma,
+                                          GemmSmem &S) {
   if (tl.x < 0) return;  // padding slot of the XCD-balanced schedule
   const SegProb &p = probs[tl.x];
   const int m0 = tl.y * GT, n0 = tl.z * GT, M = p.M;
@@ -545,12 +532,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
       if (r16 < M && c16 < M && !(diag && r16 > c16)) need |= 1u << (2 * ti + tj);
     }
   need = __builtin_amdgcn_readfirstlane(need);  // uniform per wavefront
-  __shared__ GemmSmem S;
   // workgroup-uniform choice: an off-diagonal tile inside the block needs every sub-tile
   if (MODE == 0 && !diag && m0 + GT <= M && n0 + GT <= M)
     seg_tile<A_KMAJOR, MODE, EPI, true>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
   else
     seg_tile<A_KMAJOR, MODE, EPI, false>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
+}
+template <bool A_KMAJOR, int MODE, int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 4 : 1))) void k_seg_gemm(const SegProb *__restrict__ probs,
+                                                  const int4 *__restrict__ tiles, int ntiles,
+                                                  const double *__restrict__ X0,
+                                                  const double *__restrict__ X1, double g0, double g1,
+                                                  double *__restrict__ C, double *__restrict__ W,
+                                                  double sigma, const int *act, long long sx,
+                                                  long long sc, long long sw) {
+  const int t = blockIdx.x;
+  if (t >= ntiles) return;
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  __shared__ GemmSmem S;
+  seg_block<A_KMAJOR, MODE, EPI>(probs, tiles[t], X0 + inst * sx, X1 + inst * sx, g0, g1, C ? C + inst * sc : nullptr,
+                                 W ? W + inst * sw : nullptr, sigma, S);
 }
 
 // ---- FP64 path on 128 x 64 tiles: 4 wavefronts, each 32 rows x 64 columns
@@ -834,17 +836,8 @@ void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4
 // LDS once per column: the 6j slice {jp jh JC; ja jb J'}, the pair positions
 // of (h,a) and (p,b) in every J' block, block offsets and sizes, and the
 // orbit quantum numbers, so each J' term does a single global load.
-__global__ __launch_bounds__(256) void k_pandya(DevLayout L, const double *__restrict__ op,
-                                                double *__restrict__ cc, const int *act) {
-  extern __shared__ double pan_lds[];
-  const int col = blockIdx.x;
-  if (col >= L.nccol) return;
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    op += inst * L.op_size;
-    cc += inst * L.ccsize;
-  }
+__device__ __forceinline__ void pandya_col(const DevLayout &L, const double *__restrict__ op,
+                                           double *__restrict__ cc, int col, double *pan_lds) {
   const int q1 = L.cccol_q[col];
   const int c = col - L.cccbase[q1];
   const int p = L.cccol_p[col], h = L.cccol_h[col];
@@ -964,6 +957,13 @@ __global__ __launch_bounds__(256) void k_pandya(DevLayout L, const double *__res
     out[r] = val;
   }
 }
+__global__ __launch_bounds__(256) void k_pandya(DevLayout L, const double *__restrict__ op,
+                                                double *__restrict__ cc, const int *act) {
+  extern __shared__ double pan_lds[];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  pandya_col(L, op + inst * L.op_size, cc + inst * L.ccsize, blockIdx.x, pan_lds);
+}
 size_t pandya_lds_bytes(const DevLayout &L) {
   return sizeof(double) * L.nhalf * L.nhalf * L.nJ + sizeof(long long) * L.nblocks +
          sizeof(int) * (L.nblocks + L.nsp) + sizeof(short) * 2 * L.nJ * L.nsp;
@@ -1076,9 +1076,28 @@ __global__ __launch_bounds__(256) void k_122w(DevLayout L, const double *__restr
 // columns 2(lane%16), +1 of a half as one 16-byte access: its even and odd
 // columns are two 16-column tiles.  The block's last chunk, when shorter,
 // runs as four 16-column tiles with clamped columns.  Sets past 16 rows run
-// as two 16-row output tiles over two 16-row halves of the rows read.
-template <int NK, int TU, bool FULL>
-__device__ __forceinline__ void s122_wave(const int *__restrict__ RL, const double *__restrict__ Wt, int n, int dim,
+// as two 16-row output tiles over two 16-row halves of the rows read.  The
+// weights come from k_122w's table (TabW) or from the slot entries themselves
+// (SlotW, the small bases' form: one launch less, two more reads a weight).
+struct TabW {
+  const double *Wt;
+  __device__ __forceinline__ double operator()(int m, int j, int n) const { return Wt[m * 2 * n + j]; }
+};
+struct SlotW {
+  const int2 *sx;
+  const dpair_t *sc;
+  const double *FL, *FR;
+  __device__ __forceinline__ double operator()(int m, int j, int n) const {
+    const int i = m * n + (j >> 1);
+    const int2 x = sx[i];
+    const dpair_t c = sc[i];
+    const double *F = (j & 1) ? FR : FL;
+    const double w = c.x * F[x.x] + c.y * F[x.y];
+    return (j & 1) ? -w : w;
+  }
+};
+template <int NK, int TU, bool FULL, class WT>
+__device__ __forceinline__ void s122_wave(const int *__restrict__ RL, const WT &Wt, int n, int dim,
                                           const double *src, int c0, double hres, double *OV, int nhalf) {
   const int lane = threadIdx.x & 63, cc = lane & 15, g = lane >> 4, n2 = 2 * n;
   for (int mt = 0; mt < nhalf; mt++) {
@@ -1093,7 +1112,7 @@ __device__ __forceinline__ void s122_wave(const int *__restrict__ RL, const doub
         const int r0 = RL[min(16 * kh + 2 * kq, n - 1)], r1 = RL[min(16 * kh + 2 * kq + 1, n - 1)];
         pr[kq] = (g >> 1) ? r1 : r0;
         const int m = 16 * mt + cc, j = 32 * kh + 4 * kq + g;
-        const double w = Wt[min(m, n - 1) * n2 + min(j, n2 - 1)];
+        const double w = Wt(min(m, n - 1), min(j, n2 - 1), n);
         a[kq] = (m < n && j < n2) ? w : 0.0;
       }
       if (FULL) {
@@ -1156,18 +1175,16 @@ __device__ __forceinline__ void s122_wave(const int *__restrict__ RL, const doub
   }
 }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_122s(
-    DevLayout L, const double *__restrict__ Lop, const double *__restrict__ Rop, double *__restrict__ RES,
-    const double *__restrict__ W, double hres, const int *act) {
-  const int2 it = L.s122_items[blockIdx.x];
-  const long long inst = inst_id(act);
-  if (inst < 0) return;
-  const long long o = inst * L.op_size;
+// the work item `it` of one wavefront: operands of the instance, W(set) its weights
+template <class MakeW>
+__device__ __forceinline__ void s122_item(const DevLayout &L, const int2 it, const double *__restrict__ Lop,
+                                          const double *__restrict__ Rop, double *__restrict__ RES, double hres,
+                                          const MakeW &W) {
   const Set122 S = L.s122_sets[it.x];
   const int n = S.n, dim = S.dim, c0 = 64 * it.y;
-  const long long bo = o + L.v_off + S.bo;
+  const long long bo = L.v_off + S.bo;
   const int *RL = L.s122_rowl + S.rs;
-  const double *Wt = W + inst * 2 * (long long)L.n122_slots + S.ab;
+  const auto Wt = W(S.ab);
   // k = 4kq + lane/16: odd k read L
   const double *src = ((threadIdx.x >> 4) & 1) ? Lop + bo : Rop + bo;
   double *OV = RES + bo;
@@ -1182,6 +1199,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     else if (n <= 8) s122_wave<4, 2, false>(RL, Wt, n, dim, src, c0, hres, OV, 1);
     else s122_wave<8, 1, false>(RL, Wt, n, dim, src, c0, hres, OV, n > 16 ? 2 : 1);
   }
+}
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_122s(
+    DevLayout L, const double *__restrict__ Lop, const double *__restrict__ Rop, double *__restrict__ RES,
+    const double *__restrict__ W, double hres, const int *act) {
+  const int2 it = L.s122_items[blockIdx.x];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  const long long o = inst * L.op_size;
+  const double *Wi = W + inst * 2 * (long long)L.n122_slots;
+  s122_item(L, it, Lop + o, Rop + o, RES + o, hres, [&](long long ab) { return TabW{Wi + ab}; });
 }
 
 void launch_122(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop, double *RES,
@@ -1570,27 +1597,14 @@ __device__ __forceinline__ double w221(const DevLayout &L, const double *Wpp, co
 // 256, one workgroup per chunk, each writing its (2J+1)-weighted partial sum;
 // k_ob_final adds the partials in chunk order, so results do not depend on
 // scheduling.
-__global__ __launch_bounds__(256) void k_ob_partial(DevLayout L, const double *__restrict__ Lop,
-                                                    const double *__restrict__ Rop,
-                                                    const double *__restrict__ Wpp, double *__restrict__ part,
-                                                    int hL, int hR, unsigned mask, const int *act) {
-  __shared__ double red[4];
-  const int sp = blockIdx.x / L.ob_nchunk, ch = blockIdx.x - sp * L.ob_nchunk;
-  if (sp >= L.nsame) return;
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    Lop += inst * L.op_size;
-    Rop += inst * L.op_size;
-    Wpp += inst * L.vsize;
-    part += inst * (long long)L.nsame * L.ob_nchunk;
-  }
-  const int tid = threadIdx.x, t = L.same_ob[sp];
+// term `it` (of the chunks' numbering) of the 121 + 221 sums of one-body output t
+__device__ __forceinline__ double ob_term(const DevLayout &L, const double *__restrict__ Lop,
+                                          const double *__restrict__ Rop, const double *__restrict__ Wpp, int t,
+                                          int it, int hL, int hR, unsigned mask) {
   const int p = L.ob_p[t], qo = L.ob_q[t], N = L.nsp, MJ = L.nJ;
   const double *FL = Lop + L.f_off, *FR = Rop + L.f_off;
   const double *VL = Lop + L.v_off, *VR = Rop + L.v_off;
   const int n121 = (mask & T121) ? L.nphp * MJ : 0, n221 = (mask & T221) ? N * MJ : 0;
-  const int it = ch * 256 + tid;
   double v = 0.0;
   if (it < n121) {
     const int e = it / MJ, m = it - e * MJ;
@@ -1610,10 +1624,39 @@ __global__ __launch_bounds__(256) void k_ob_partial(DevLayout L, const double *_
     const int jc = L.jj[c], ji = L.jj[p], JT = abs(jc - ji) + 2 * m;
     if (JT <= jc + ji) v = w221(L, Wpp, VL, VR, c, p, qo, JT, (double)(hL * hR)) * (JT + 1);
   }
+  return v;
+}
+__global__ __launch_bounds__(256) void k_ob_partial(DevLayout L, const double *__restrict__ Lop,
+                                                    const double *__restrict__ Rop,
+                                                    const double *__restrict__ Wpp, double *__restrict__ part,
+                                                    int hL, int hR, unsigned mask, const int *act) {
+  __shared__ double red[4];
+  const int sp = blockIdx.x / L.ob_nchunk, ch = blockIdx.x - sp * L.ob_nchunk;
+  if (sp >= L.nsame) return;
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  const int tid = threadIdx.x;
+  double v = ob_term(L, Lop + inst * L.op_size, Rop + inst * L.op_size, Wpp + inst * L.vsize, L.same_ob[sp],
+                     ch * 256 + tid, hL, hR, mask);
   v = wave_sum(v);
   if ((tid & 63) == 0) red[tid >> 6] = v;
   __syncthreads();
-  if (tid == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  if (tid == 0) part[inst * (long long)L.nsame * L.ob_nchunk + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+// writes one-body output (p,q) and its mirror, adds coef times both to AF when
+// there is one, and returns the output's sum of squares
+__device__ __forceinline__ double ob_write(const DevLayout &L, double *F, double *AF, int p, int qo, double val,
+                                           int hres, double coef) {
+  const int N = L.nsp;
+  const double vt = (p != qo) ? hres * val : 0.0;  // F(q,p)
+  if (p == qo && hres == -1) val = 0.0;
+  F[p * N + qo] = val;
+  if (p != qo) F[qo * N + p] = vt;
+  if (AF) {
+    AF[p * N + qo] = AF[p * N + qo] + coef * val;
+    if (p != qo) AF[qo * N + p] = AF[qo * N + p] + coef * vt;
+  }
+  return val * val + vt * vt;
 }
 // one wavefront per one-body output (p,q): 111 (full F products), plus the
 // 121 + 221 partials / (2j_p + 1); writes F(p,q) and F(q,p) = herm F(p,q)
@@ -1643,19 +1686,10 @@ __global__ __launch_bounds__(64) void k_ob_final(DevLayout L, const double *__re
       for (int c = 0; c < L.ob_nchunk; c++) sm += part[(long long)sp * L.ob_nchunk + c];
       val += sm / (L.jj[p] + 1.0);
     }
-    double *F = RES + L.f_off;
-    const double vt = (p != qo) ? hres * val : 0.0;  // F(q,p)
-    if (p == qo && hres == -1) val = 0.0;
-    F[p * N + qo] = val;
-    if (p != qo) F[qo * N + p] = vt;
-    if (acc) {
-      double *A = acc + inst * L.op_size;
-      double *AF = A + L.f_off;
-      AF[p * N + qo] = AF[p * N + qo] + coef * val;
-      if (p != qo) AF[qo * N + p] = AF[qo * N + p] + coef * vt;
-      if (t == 0) A[0] = A[0] + coef * RES[0];  // E0 (as add_sq_op)
-    }
-    if (npart) npart[inst * (long long)(L.nmirror + L.nob) + L.nmirror + t] = val * val + vt * vt;
+    double *A = acc ? acc + inst * L.op_size : nullptr;
+    const double sq = ob_write(L, RES + L.f_off, A ? A + L.f_off : nullptr, p, qo, val, hres, coef);
+    if (A && t == 0) A[0] = A[0] + coef * RES[0];  // E0 (as add_sq_op)
+    if (npart) npart[inst * (long long)(L.nmirror + L.nob) + L.nmirror + t] = sq;
   }
 }
 void launch_ob_partial(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop,
@@ -1676,17 +1710,8 @@ void launch_ob_final(hipStream_t s, const DevLayout &L, const double *Lop, const
 
 // 220 per block (commutators.f90:399-432) into partials[q * nsplit + split]; 110 into
 // partials[nblocks * nsplit] (nsplit workgroups per block, as many as kPartials allows, at most kE0Split)
-__global__ __launch_bounds__(256) void k_e0_partial(DevLayout L, const double *Lop, const double *Rop,
-                                                     int hL, int hR, double *partials, const int *act, int nsplit) {
-  __shared__ double sh[256];
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    Lop += inst * L.op_size;
-    Rop += inst * L.op_size;
-    partials += inst * kPartials;
-  }
-  const int b = blockIdx.x;
+__device__ __forceinline__ void e0_part(const DevLayout &L, const double *Lop, const double *Rop, int hL, int hR,
+                                        double *partials, int b, int nsplit, double *sh) {
   if (b < L.nblocks * nsplit) {
     // nsplit workgroups per block, each a strided share of its pphh elements
     const int q = b / nsplit, sp = b - q * nsplit;
@@ -1714,6 +1739,14 @@ __global__ __launch_bounds__(256) void k_e0_partial(DevLayout L, const double *L
     if (threadIdx.x == 0) partials[b] = s;
   }
 }
+__global__ __launch_bounds__(256) void k_e0_partial(DevLayout L, const double *Lop, const double *Rop,
+                                                     int hL, int hR, double *partials, const int *act, int nsplit) {
+  __shared__ double sh[256];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  e0_part(L, Lop + inst * L.op_size, Rop + inst * L.op_size, hL, hR, partials + inst * kPartials, blockIdx.x, nsplit,
+          sh);
+}
 __global__ __launch_bounds__(256) void k_e0_final(int nparts, const double *partials, double *RES,
                                                    int use110, int use220, const int *act, long long rstride) {
   __shared__ double sh[256];
@@ -1733,10 +1766,13 @@ __global__ __launch_bounds__(256) void k_e0_final(int nparts, const double *part
     RES[0] = e;
   }
 }
+static int e0_nsplit(const DevLayout &L) {
+  return std::max(1, std::min(kE0Split, (kPartials - 1) / std::max(L.nblocks, 1)));
+}
 void launch_e0(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop, double *RES,
                int hL, int hR, unsigned mask, double *partials, const int *act, int nact, long long rstride) {
   if (nact <= 0) return;
-  const int nsplit = std::max(1, std::min(kE0Split, (kPartials - 1) / std::max(L.nblocks, 1)));
+  const int nsplit = e0_nsplit(L);
   hipLaunchKernelGGL(k_e0_partial, dim3(L.nblocks * nsplit + 1, nact), dim3(256), 0, s, L, Lop, Rop, hL, hR,
                      partials, act, nsplit);
   const int use220 = (mask & T220) && (hL * hR == -1);
@@ -1801,12 +1837,10 @@ void launch_sumsq(hipStream_t s, const DevLayout &L, const double *op, double *p
 }
 
 // the Frobenius norm from the partial sums of squares that k_sym_mirror and
-// k_ob_final wrote (nmirror + nob per instance), into out[inst * kScal]
-void launch_norm_from_parts(hipStream_t s, const DevLayout &L, const double *npart, double *out, const int *act,
-                            int nact) {
+// k_ob_final wrote (n per instance), into out[inst * kScal]
+void launch_norm_from_parts(hipStream_t s, int n, const double *npart, double *out, const int *act, int nact) {
   if (nact <= 0) return;
-  hipLaunchKernelGGL(k_final_sum, dim3(1, nact), dim3(256), 0, s, npart, L.nmirror + L.nob, out, 1, act,
-                     (long long)(L.nmirror + L.nob));
+  hipLaunchKernelGGL(k_final_sum, dim3(1, nact), dim3(256), 0, s, npart, n, out, 1, act, (long long)n);
 }
 
 // mbpt2 (basic_IMSRG.f90:4030-4064): one workgroup per block
@@ -2017,30 +2051,323 @@ void launch_gather_e0(hipStream_t s, const double *op, long long stride, double 
 //   |cof|; advals in scalar slots kAdvSlot.., ||Omega|| in kFullSlot), then goes
 //   on while !(fullnorm < tiny) and !(|advals[test] / fullnorm| < conv).
 // ||ad^n|| is scalar slot 0.  live[k] (host memory) gets 1 or 0 per position.
-__global__ void k_series_gate(int *act, int nact, double *scal, int mode, double coef, int store, int test,
-                              double conv, double tiny, int *live) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nact) return;
+// live[k] carries the gate's sequence number above its flag, so that the host
+// can wait for this gate's answer by reading the flag itself.
+__device__ __forceinline__ void gate_position(int *act, int k, double *scal, const GateArgs &G) {
   const int inst = act[k];
   int on = 0;
   if (inst >= 0) {
     double *sc = scal + (long long)inst * kScal;
-    if (mode == 0) {
-      on = !(sc[0] * coef < conv);
+    if (G.mode == 0) {
+      on = !(sc[0] * G.coef < G.conv);
     } else {
-      if (store >= 0) sc[kAdvSlot + store] = sc[0] * coef;
+      if (G.store >= 0) sc[kAdvSlot + G.store] = sc[0] * G.coef;
       const double full = sc[kFullSlot];
-      on = !(full < tiny) && !(fabs(sc[kAdvSlot + test] / full) < conv);
+      on = !(full < G.tiny) && !(fabs(sc[kAdvSlot + G.test] / full) < G.conv);
     }
     if (!on) act[k] = -1;
   }
-  live[k] = on;
+  G.live[k] = (G.seq << 1) | on;
   __threadfence_system();
 }
-void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, int mode, double coef, int store,
-                        int test, double conv, double tiny, int *live) {
+__global__ void k_series_gate(int *act, int nact, double *scal, GateArgs G) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < nact) gate_position(act, k, scal, G);
+}
+void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, const GateArgs &G) {
   if (nact <= 0) return;
-  hipLaunchKernelGGL(k_series_gate, dim3((nact + 63) / 64), dim3(64), 0, s, act, nact, scal, mode, coef, store,
-                     test, conv, tiny, live);
+  hipLaunchKernelGGL(k_series_gate, dim3((nact + 63) / 64), dim3(64), 0, s, act, nact, scal, G);
+}
+
+// The norm of a nested commutator (k_final_sum over its partial sums of
+// squares, the same order) and the series gate in one launch: one workgroup
+// per position of the series table, whose first thread then makes the test.
+__global__ __launch_bounds__(256) void k_norm_gate(const double *npart, int n, int *act, double *scal, GateArgs G) {
+  __shared__ double sh[256];
+  const int inst = act[blockIdx.y];
+  double s = 0.0;
+  if (inst >= 0) {
+    const double *p = npart + (long long)inst * n;
+    for (int i0 = threadIdx.x; i0 < n; i0 += 8 * 256) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = p[min(i0 + 256 * u, n - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (i0 + 256 * u < n) s += v[u];
+    }
+  }
+  s = block_sum256(s, sh);
+  if (threadIdx.x == 0) {
+    if (inst >= 0) scal[(long long)inst * kScal] = sqrt(s);
+    gate_position(act, blockIdx.y, scal, G);
+  }
+}
+void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
+                      const GateArgs &G) {
+  if (nact > 0) hipLaunchKernelGGL(k_norm_gate, dim3(1, nact), dim3(256), 0, s, npart, n, act, scal, G);
+}
+
+// ------------------------------------------------------------------ small bases: a commutator in three launches
+// In bases up to about emax = 5 a commutator's thirteen kernels run 2-8 us
+// each and issuing them costs the host more (5 us a launch, and as much for
+// each event between the two streams).  The same work in three launches: every
+// kernel below is a list of workgroups of different kinds that only need what
+// the launch before left behind.
+//   k_small_a  Pandya columns, 122 sets (weights formed in place), E0 partials
+//   k_small_b  the pp/hh product (onto the 122 rows) and the Pandya product
+//   k_small_c  per 16 x 16 tile pair: the ph terms and their 6j-weighted sums
+//              straight from Z, then symmetrise + mirror; one-body outputs; E0
+// The arithmetic and its order are those of the separate kernels, so results
+// are the same bits (the norm's partial sums are per 16 x 16 tile here).
+// Measured, whole flows (per commutator): see the rule in comm_launches.
+__global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ Lp, SmallArgs A) {
+  extern __shared__ double lds[];
+  const DevLayout &L = *Lp;
+  const long long inst = inst_id(A.act);
+  if (inst < 0) return;
+  const long long o = inst * L.op_size;
+  const double *Lop = A.Lop + o, *Rop = A.Rop + o;
+  int b = blockIdx.x;
+  if (b < L.nccol) {
+    pandya_col(L, Rop, A.ccR + inst * L.ccsize, b, lds);
+    return;
+  }
+  b -= L.nccol;
+  if (A.prepL) {
+    if (b < L.nccol) {
+      pandya_col(L, Lop, A.ccL + inst * L.ccsize, b, lds);
+      return;
+    }
+    b -= L.nccol;
+  }
+  const int nw = (L.n122_items + 3) / 4;
+  if (b < nw) {
+    const int i = 4 * b + (int)(threadIdx.x >> 6);
+    if (i >= L.n122_items) return;
+    const SlotW w0{L.s122_sx, reinterpret_cast<const dpair_t *>(L.s122_sc), Lop + L.f_off, Rop + L.f_off};
+    s122_item(L, L.s122_items[i], Lop, Rop, A.RES + o, (double)A.hres, [&](long long ab) {
+      return SlotW{w0.sx + (ab >> 1), w0.sc + (ab >> 1), w0.FL, w0.FR};
+    });
+    return;
+  }
+  e0_part(L, Lop, Rop, A.hL, A.hR, A.partials + inst * kPartials, b - nw, A.nsplit, lds);
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_small_b(
+    const DevLayout *__restrict__ Lp, SmallArgs A) {
+  __shared__ GemmSmem S;
+  const DevLayout &L = *Lp;
+  const long long inst = inst_id(A.act);
+  if (inst < 0) return;
+  const int b = blockIdx.x;
+  if (b < A.n_pp) {
+    const long long o = inst * L.op_size + L.v_off;
+    seg_block<false, 0, 0>(A.pp_probs, A.pp_tiles[b], A.Lop + o, A.Rop + o, 1.0, 1.0, A.RES + o,
+                           A.wpp + inst * L.vsize, 0.0, S);
+  } else {
+    const long long o = inst * L.ccsize;
+    const double hL = A.hL, hR = A.hR;
+    seg_block<true, 0, 1>(A.ph_probs, A.ph_tiles[b - A.n_pp], A.ccL + o, A.ccR + o, hL, -hR, A.Z + inst * L.cwsize,
+                          nullptr, -hL * hR, S);
+  }
+}
+
+// Upper element (r, c) of a block: the row header gives where its terms and
+// 6j runs start, its descriptor the rest (ph_decode).  Four lanes sum an
+// element's terms in k_ph_apply's order, each lane two terms at a time; the
+// term itself is made from its two Z elements as k_ph_terms makes it.
+__device__ __forceinline__ void small_tile(const DevLayout &L, const SmallArgs &A, long long inst, int bt, double *sh) {
+  __shared__ double U[16][17], W[16][17];
+  const int4 t = A.tiles16[bt];
+  const int q = t.x, dim = L.bdim[q], base = L.pbase[q], r0 = t.y * 16, c0 = t.z * 16;
+  const bool diag = t.y == t.z;
+  double *OV = A.RES + inst * L.op_size + L.v_off + L.boff[q];
+  double *AV = A.acc ? A.acc + inst * L.op_size + L.v_off + L.boff[q] : nullptr;
+  const double2 *Z2 = reinterpret_cast<const double2 *>(A.Z + inst * L.cwsize);
+  const double sigma = -(double)A.hL * (double)A.hR;
+  const int tid = threadIdx.x, g = tid >> 2, sub = tid & 3;
+  // this thread's elements of the mirror pass: loaded first, off any branch
+  const int tx = tid & 15, ty = tid >> 4;
+  const bool in1 = r0 + ty < dim && c0 + tx < dim, in2 = c0 + ty < dim && r0 + tx < dim;
+  const long long o1 = in1 ? (long long)(r0 + ty) * dim + c0 + tx : 0;
+  const long long o2 = in2 ? (long long)(c0 + ty) * dim + r0 + tx : 0;
+  const double y = OV[o2], au = (AV ? AV : OV)[o1], al = (AV ? AV : OV)[o2];
+  // outputs g, g + 64, g + 128, g + 192 of the tile: headers, then descriptors
+  // and old values, then term addresses, then the Z halves of two outputs at a time
+  PhRow h[4];
+  bool on[4];
+  unsigned long long d[4];
+  double old[4];
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + (g >> 4) + 4 * u, c = c0 + (g & 15);
+    on[u] = r < dim && c < dim && r <= c;
+    h[u] = A.phrow[base + min(r, dim - 1)];
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + (g >> 4) + 4 * u, c = c0 + (g & 15);
+    d[u] = L.ph_desc[on[u] ? h[u].dbase + c : 0];
+    old[u] = OV[on[u] ? (long long)r * dim + c : 0];
+    if (!on[u]) d[u] = 0ull;
+  }
+  const int m0 = 2 * sub;
+#pragma unroll
+  for (int v = 0; v < 4; v += 2) {
+    uint2 blk[2][2];
+    unsigned sel[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      const int u = v + x;
+      const int n = (int)((d[u] >> 23) & 31) + (int)((d[u] >> 28) & 31);
+      const long long t0 = n > 0 ? h[u].tbase + (long long)(d[u] & 0x7FFFFFull) : 0;
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        const long long e = t0 + (m0 + 8 * w < n ? m0 + 8 * w : 0);
+        blk[x][w] = *reinterpret_cast<const uint2 *>(L.ph_zblk + e);
+        sel[x][w] = *reinterpret_cast<const unsigned short *>(L.ph_zsel + e);
+      }
+    }
+    double2 z[2][2][4];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        z[x][w][0] = Z2[blk[x][w].x];
+        z[x][w][1] = Z2[blk[x][w].x ^ 1u];
+        z[x][w][2] = Z2[blk[x][w].y];
+        z[x][w][3] = Z2[blk[x][w].y ^ 1u];
+      }
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+      const int u = v + x;
+      int toff, n1, n, f1, f2;
+      double g1, g2, pre2;
+      ph_decode(d[u], toff, n1, n, f1, f2, g1, g2, pre2);
+      const double *S6 = L.ap6_val + h[u].b0;
+      double acc = 0.0;
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        const int m = m0 + 8 * w;
+        if (m < n) {
+          const double ta = ph_term(sel[x][w] & 255u, z[x][w][0], z[x][w][1], sigma);
+          const double tb = ph_term(sel[x][w] >> 8, z[x][w][2], z[x][w][3], sigma);
+          acc += ph_coef(S6, m, n, n1, f1, f2, g1, g2) * ta + ph_coef(S6, m + 1, n, n1, f1, f2, g1, g2) * tb;
+        }
+      }
+      for (int m = m0 + 16; m < n; m += 8) {
+        const long long e = h[u].tbase + toff + m;
+        const uint2 bk = *reinterpret_cast<const uint2 *>(L.ph_zblk + e);
+        const unsigned sl = *reinterpret_cast<const unsigned short *>(L.ph_zsel + e);
+        const double ta = ph_term(sl & 255u, Z2[bk.x], Z2[bk.x ^ 1u], sigma);
+        const double tb = ph_term(sl >> 8, Z2[bk.y], Z2[bk.y ^ 1u], sigma);
+        acc += ph_coef(S6, m, n, n1, f1, f2, g1, g2) * ta + ph_coef(S6, m + 1, n, n1, f1, f2, g1, g2) * tb;
+      }
+      acc += __shfl_xor(acc, 1, 64);
+      acc += __shfl_xor(acc, 2, 64);
+      const double pre = h[u].half ? .70710678118 : 1.0;
+      if (sub == 0) U[(g >> 4) + 4 * u][g & 15] = on[u] ? old[u] + acc * pre2 * pre : 0.0;
+    }
+  }
+  W[ty][tx] = in2 ? y : 0.0;
+  __syncthreads();
+  // k_sym_mirror's last pass on a 16 x 16 tile pair
+  const double hh = (double)A.hres;
+  double sq = 0.0;
+  if (in1 && (!diag || ty <= tx)) {
+    double v = U[ty][tx];
+    if (!diag || ty < tx) v += hh * W[tx][ty];
+    else if (A.hres == -1) v = 0.0;
+    OV[o1] = v;
+    sq += v * v;
+    if (AV) AV[o1] = au + A.coef * v;
+  }
+  if (in2 && (!diag || tx < ty)) {
+    const double v = hh * (U[tx][ty] + hh * W[ty][tx]);
+    OV[o2] = v;
+    sq += v * v;
+    if (AV) AV[o2] = al + A.coef * v;
+  }
+  if (A.npart) {
+    sq = block_sum256(sq, sh);
+    if (tid == 0) A.npart[inst * (A.n16 + L.nob) + bt] = sq;
+  }
+}
+__global__ __launch_bounds__(256) void k_small_c(const DevLayout *__restrict__ Lp, SmallArgs A) {
+  __shared__ double sh[256];
+  const DevLayout &L = *Lp;
+  const long long inst = inst_id(A.act);
+  if (inst < 0) return;
+  if (A.coefp) A.coef = *A.coefp;
+  int b = blockIdx.x;
+  if (b < A.n16) {
+    small_tile(L, A, inst, b, sh);
+    return;
+  }
+  b -= A.n16;
+  const long long o = inst * L.op_size;
+  const double *Lop = A.Lop + o, *Rop = A.Rop + o;
+  double *RES = A.RES + o, *acc = A.acc ? A.acc + o : nullptr;
+  const double *FL = Lop + L.f_off, *FR = Rop + L.f_off;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, N = L.nsp;
+  auto f111 = [&](int p, int qo) {
+    double val = 0.0;
+    for (int k = lane; k < N; k += 64) val += FL[p * N + k] * FR[k * N + qo] - FR[p * N + k] * FL[k * N + qo];
+    return wave_sum(val);
+  };
+  auto put = [&](int t, int p, int qo, double val) {
+    const double sq = ob_write(L, RES + L.f_off, acc ? acc + L.f_off : nullptr, p, qo, val, A.hres, A.coef);
+    if (A.npart) A.npart[inst * (A.n16 + L.nob) + A.n16 + t] = sq;
+  };
+  if (b < L.nsame) {  // 111 + 121 + 221 of one output, the chunks of k_ob_partial one after another
+    const int t = L.same_ob[b], p = L.ob_p[t], qo = L.ob_q[t];
+    double val = f111(p, qo), sm = 0.0;
+    for (int ch = 0; ch < L.ob_nchunk; ch++) {
+      const double v = wave_sum(ob_term(L, Lop, Rop, A.wpp + inst * L.vsize, t, ch * 256 + tid, A.hL, A.hR, A.mask));
+      __syncthreads();
+      if (lane == 0) sh[wave] = v;
+      __syncthreads();
+      sm += sh[0] + sh[1] + sh[2] + sh[3];
+    }
+    val += sm / (L.jj[p] + 1.0);
+    if (tid == 0) put(t, p, qo, val);
+    return;
+  }
+  b -= L.nsame;
+  const int nd = (A.n_diff + 3) / 4;
+  if (b < nd) {  // the other outputs: 111 alone, one wavefront each
+    const int i = 4 * b + wave;
+    if (i >= A.n_diff) return;
+    const int t = A.diff_ob[i], p = L.ob_p[t], qo = L.ob_q[t];
+    const double val = f111(p, qo);
+    if (lane == 0) put(t, p, qo, val);
+    return;
+  }
+  // E0: k_e0_final's sum, and its share of the series accumulator
+  if (A.mask & (T110 | T220)) {
+    const double *part = A.partials + inst * kPartials;
+    const int n = L.nblocks * A.nsplit;
+    double s = 0.0;
+    for (int i = tid; i < n; i += 256) s += part[i];
+    s = block_sum256(s, sh);
+    if (tid == 0) {
+      double e = 0.0;
+      if (A.mask & T110) e = part[n];
+      if ((A.mask & T220) && A.hL * A.hR == -1) e = e + s * 2.0;
+      RES[0] = e;
+    }
+  }
+  if (tid == 0 && acc) acc[0] = acc[0] + A.coef * RES[0];
+}
+void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallArgs A, int nact) {
+  if (nact <= 0) return;
+  A.nsplit = e0_nsplit(L);
+  const int ne0 = (A.mask & (T110 | T220)) ? L.nblocks * A.nsplit + 1 : 0;
+  const int na = L.nccol * (A.prepL ? 2 : 1) + (L.n122_items + 3) / 4 + ne0;
+  const size_t lds = std::max(pandya_lds_bytes(L), 256 * sizeof(double));
+  hipLaunchKernelGGL(k_small_a, dim3(na, nact), dim3(256), lds, s, Ld, A);
+  hipLaunchKernelGGL(k_small_b, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
+  hipLaunchKernelGGL(k_small_c, dim3(A.n16 + L.nsame + (A.n_diff + 3) / 4 + 1, nact), dim3(256), 0, s, Ld, A);
 }
 }  // namespace imsrg
