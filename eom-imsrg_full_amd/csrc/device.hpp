@@ -243,8 +243,18 @@ void launch_mbpt2(hipStream_t s, const DevLayout &L, const double *op, double *p
                   const int *act, int nact);
 void launch_monopole(hipStream_t s, const DevLayout &L, const double *H, double *mono, const int *act,
                      int nact);
-void launch_eta(hipStream_t s, const DevLayout &L, const double *Hden, const double *Hnum,
-                const double *mono, double *ETA, int kind, const int *act, int nact);
+// What a flow step reports of its Hamiltonian, in pinned host memory (one per instance)
+struct StepReport {
+  double mbpt2, e0;
+  int seq, pad;  // the step's number, written last
+};
+// White (kind 0) or atan (1) generator ETA (cleared first) from the denominators
+// of Hden and the numerators of Hnum; with rep, MBPT2 and E0 of Hden go there
+void launch_generator(hipStream_t s, const DevLayout &L, const double *Hden, const double *Hnum, double *mono,
+                      double *ETA, int kind, double *partials, const int *act, int nact, StepReport *rep, int seq);
+// A copied to C1 (and C2, may be null) on the instances of act, and act to own
+void launch_series_begin(hipStream_t s, long long n, const double *A, double *C1, double *C2, const int *act, int *own,
+                         int nact, long long stride);
 void launch_normal_order(hipStream_t s, const DevLayout &L, const double *T, double *H, const int *act,
                          int nact);
 void launch_gather_e0(hipStream_t s, const double *op, long long stride, double *out, const int *act, int nact);
@@ -281,6 +291,11 @@ void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, const G
 // launch_norm_from_parts (n partials per instance) and the gate after it in one launch
 void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
                       const GateArgs &G);
+
+// ||DG|| and ||Om|| into the Magnus scalar slots and the series' first gate;
+// partials: 2 * kPartials * nbatch
+void launch_magnus_gate(hipStream_t s, const DevLayout &L, const double *DG, const double *Om, double *partials,
+                        int nbatch, int *act, int nact, double *scal, const GateArgs &G);
 
 // A whole FP64 commutator (every one- and two-body term) in three launches,
 // for small bases (k_small_a, _b, _c).

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -170,7 +171,7 @@ static ActSet all_set(imsrg_ctx_s *c) {
 // Writes `list` into table `slot` (an asynchronous copy on the context
 // stream).  Drivers rewrite a slot only after a stream synchronization, so
 // the pinned source is never overwritten while a copy from it is pending.
-// Slots 1 and 2 are the BCH and Magnus series tables (series_set).
+// Slots 1 and 2 are the BCH and Magnus series tables (series_begin).
 // With pad > list size the table is padded with -1 entries to pad entries.
 static ActSet make_set(imsrg_ctx_s *c, int slot, const std::vector<int> &list, int pad = 0) {
   ActSet a;
@@ -190,13 +191,29 @@ static int op_new(imsrg_ctx_s *c, int herm, imsrg_op_s **out) {
   imsrg_op_s *op = new imsrg_op_s;
   op->ctx = c;
   op->herm = herm;
-  if (hipMalloc(&op->d, sizeof(double) * c->lay.op_size * c->nbatch) != hipSuccess) {
+  const size_t bytes = sizeof(double) * c->lay.op_size * c->nbatch;
+  if (!c->op_pool.empty()) {
+    op->d = c->op_pool.back();
+    c->op_pool.pop_back();
+  } else if (dev_malloc(c, (void **)&op->d, bytes) != hipSuccess) {
     delete op;
     return fail(IMSRG_ENOMEM, "hipMalloc operator failed");
   }
   launch_fill(c->stream, op->d, c->lay.op_size * c->nbatch, 0.0);
   *out = op;
   return 0;
+}
+// gives an operator's buffer back: to the context's pool, or to the device
+static void op_release(imsrg_op_s *op) {
+  imsrg_ctx_s *c = op->ctx;
+  const size_t bytes = sizeof(double) * c->lay.op_size * c->nbatch;
+  if (c->op_pool.size() < imsrg_ctx_s::kOpPool && (c->op_pool.size() + 1) * bytes <= imsrg_ctx_s::kOpPoolBytes) {
+    c->op_pool.push_back(op->d);
+  } else {
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(op->d);
+  }
+  delete op;
 }
 static imsrg_op_s *tmp_op(imsrg_ctx_s *c, int slot, int herm) {
   if (!c->tmp[slot]) {
@@ -499,7 +516,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   if (!rc) rc = dalloc(c, Ly.cwsize * B, &c->wph);
   if (!rc) rc = dalloc(c, Ly.s122_sx.size() * B, &c->w122);
   if (!rc) rc = dalloc(c, Ly.ph_terms.size() * B, &c->tph);
-  if (!rc) rc = dalloc(c, kPartials * B, &c->partials);
+  if (!rc) rc = dalloc(c, 2 * kPartials * B, &c->partials);  // two sets (launch_magnus_gate)
   if (!rc) rc = dalloc(c, (size_t)std::max(D.nsame, 1) * D.ob_nchunk * B, &c->obpart);
   if (!rc) rc = dalloc(c, (size_t)(std::max(D.nmirror, c->n_tiles16) + D.nob) * B, &c->npart);
   if (!rc) rc = dalloc(c, kScal * B, &c->scal);
@@ -528,6 +545,12 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
                             hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
               hipHostGetDevicePointer((void **)&c->live_d, c->live_h, 0) != hipSuccess))
     rc = fail(IMSRG_ENOMEM, "hipHostMalloc series gate ring failed");
+  if (!rc && (hipHostMalloc((void **)&c->rep_h, B * sizeof(StepReport), hipHostMallocMapped | hipHostMallocCoherent) !=
+                  hipSuccess ||
+              hipHostGetDevicePointer((void **)&c->rep_d, c->rep_h, 0) != hipSuccess))
+    rc = fail(IMSRG_ENOMEM, "hipHostMalloc step report failed");
+  if (!rc) std::memset(c->rep_h, 0, B * sizeof(StepReport));
+  if (!rc) std::memset(c->live_h, 0, imsrg_ctx_s::kGateRing * B * sizeof(int));
   if (!rc &&
       hipHostMalloc((void **)&c->hstage, std::max<size_t>(Ly.op_size * B, Ly.ccsize) * sizeof(double),
                     hipHostMallocDefault) != hipSuccess)
@@ -637,6 +660,7 @@ int imsrg_ctx_destroy(imsrg_ctx c) {
       (void)hipFree(t->d);
       delete t;
     }
+  for (double *p : c->op_pool) (void)hipFree(p);
   for (auto &kv : c->gexec) (void)hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : c->evpool) (void)hipEventDestroy(e);
   for (void *p : c->dallocs) (void)hipFree(p);
@@ -649,6 +673,7 @@ int imsrg_ctx_destroy(imsrg_ctx c) {
   for (hipEvent_t e : c->ev_gate)
     if (e) (void)hipEventDestroy(e);
   if (c->live_h) (void)hipHostFree(c->live_h);
+  if (c->rep_h) (void)hipHostFree(c->rep_h);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -771,11 +796,11 @@ static int i8_setup(imsrg_ctx_s *c) {
   for (int k = 0; k < 2 && !rc; k++) {
     void *p = nullptr;
     const size_t vb = (size_t)c->i8.v_bytes * B, cb = (size_t)c->i8.c_bytes * B;
-    if (hipMalloc(&p, std::max<size_t>(vb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
+    if (dev_malloc(c, &p, std::max<size_t>(vb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
     c->dallocs.push_back(p);
     c->i8v[k] = (signed char *)p;
     HIPCHK(hipMemset(p, 0, std::max<size_t>(vb, 256)));
-    if (hipMalloc(&p, std::max<size_t>(cb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
+    if (dev_malloc(c, &p, std::max<size_t>(cb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
     c->dallocs.push_back(p);
     c->i8c[k] = (signed char *)p;
     HIPCHK(hipMemset(p, 0, std::max<size_t>(cb, 256)));
@@ -854,10 +879,11 @@ static void drop_graphs_of(imsrg_ctx_s *c, const void *d) {
 }
 int imsrg_op_destroy(imsrg_op op) {
   if (!op) return 0;
-  (void)hipStreamSynchronize(op->ctx->stream);
-  drop_graphs_of(op->ctx, op->d);
-  (void)hipFree(op->d);
-  delete op;
+  if (!op->ctx->gexec.empty()) {  // a graph that names the buffer may still be running
+    (void)hipStreamSynchronize(op->ctx->stream);
+    drop_graphs_of(op->ctx, op->d);
+  }
+  op_release(op);
   return 0;
 }
 int imsrg_op_set_herm(imsrg_op op, int herm) {
@@ -1527,24 +1553,22 @@ int imsrg_commutator_adjoint(imsrg_ctx c, imsrg_op P, imsrg_op Cbar, imsrg_op Yb
 }
 
 // ---------------------------------------------------------------- generators
+// rep: the device view of the step reports when Hden's MBPT2 and E0 are wanted (seq their number)
 static void gen_simple(imsrg_ctx_s *c, imsrg_op_s *Hden, imsrg_op_s *Hnum, imsrg_op_s *ETA, int kind,
-                       const ActSet &a) {
-  hipStream_t s = c->stream;
-  PROF(c, IMSRG_PROF_GENERATOR, {
-    launch_fill(s, ETA->d + c->lay.f_off, c->lay.op_size - c->lay.f_off, 0.0, a.d, a.n(), c->lay.op_size);
-    launch_monopole(s, c->dl, Hden->d, c->mono, a.d, a.n());
-    launch_eta(s, c->dl, Hden->d, Hnum->d, c->mono, ETA->d, kind, a.d, a.n());
-  });
+                       const ActSet &a, StepReport *rep = nullptr, int seq = 0) {
+  PROF(c, IMSRG_PROF_GENERATOR, launch_generator(c->stream, c->dl, Hden->d, Hnum->d, c->mono, ETA->d, kind, c->partials,
+                                                 a.d, a.n(), rep, seq));
   ETA->herm = -1;
 }
-static int gen_impl(imsrg_ctx_s *c, int kind, imsrg_op_s *H, imsrg_op_s *ETA, const ActSet &a) {
+static int gen_impl(imsrg_ctx_s *c, int kind, imsrg_op_s *H, imsrg_op_s *ETA, const ActSet &a,
+                    StepReport *rep = nullptr, int seq = 0) {
   if (kind == IMSRG_GEN_WHITE || kind == IMSRG_GEN_ATAN) {
-    gen_simple(c, H, H, ETA, kind == IMSRG_GEN_WHITE ? 0 : 1, a);
+    gen_simple(c, H, H, ETA, kind == IMSRG_GEN_WHITE ? 0 : 1, a, rep, seq);
   } else if (kind == IMSRG_GEN_W2) {
     // build_gs_w2 (generators.f90:109-160)
     imsrg_op_s *E1 = tmp_op(c, 2, -1), *H2 = tmp_op(c, 3, 1), *E2 = tmp_op(c, 4, -1);
     if (!E1 || !H2 || !E2) return IMSRG_ENOMEM;
-    gen_simple(c, H, H, E1, 1, a);
+    gen_simple(c, H, H, E1, 1, a, rep, seq);
     int rc = comm_impl(c, E1, H, H2, IMSRG_TALL, 0, a);
     if (rc) return rc;
     gen_simple(c, H, H2, E2, 1, a);
@@ -1554,6 +1578,19 @@ static int gen_impl(imsrg_ctx_s *c, int kind, imsrg_op_s *H, imsrg_op_s *ETA, co
     return fail(IMSRG_EINVAL, "unknown generator kind");
   }
   HIPCHK(hipGetLastError());
+  return 0;
+}
+// Spins on a number that a kernel writes to pinned host memory; the stream is
+// asked now and then, so a failed launch ends the wait.
+template <class Read>
+static int wait_seq(imsrg_ctx_s *c, int seq, const char *what, Read &&read) {
+  for (long long spin = 1; read() != seq; spin++) {
+    if (spin % 4096) continue;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e == hipSuccess && read() == seq) break;
+    return fail(IMSRG_EDEVICE, std::string(what) + ": " + hipGetErrorString(e));
+  }
   return 0;
 }
 int imsrg_generator(imsrg_ctx c, int kind, imsrg_op H, imsrg_op ETA) {
@@ -1574,13 +1611,17 @@ static const double kTiny = (double)1e-9f;   // fullnorm < 1e-9 (default-real li
 // A BCH or Magnus series works on its own copy of the caller's instance
 // table (slot `slot`), which the gate kernels edit: an instance that stops
 // gets -1 there and every later kernel of the series skips it.  The copy is
-// made on the stream, behind the launches that read the slot before.
-static ActSet series_set(imsrg_ctx_s *c, int slot, const ActSet &a) {
+// made on the stream, behind the launches that read the slot before, by the
+// launch that copies the series' first operand A to C1 (and C2).
+static ActSet series_begin(imsrg_ctx_s *c, int slot, const ActSet &a, imsrg_op_s *A, imsrg_op_s *C1, imsrg_op_s *C2) {
   ActSet s;
   s.d = c->act_d[slot];
   s.h = a.h;
   s.ng = a.ng;
-  (void)hipMemcpyAsync(c->act_d[slot], a.d, a.g() * sizeof(int), hipMemcpyDeviceToDevice, c->stream);
+  launch_series_begin(c->stream, c->lay.op_size, A->d, C1->d, C2 ? C2->d : nullptr, a.d, c->act_d[slot], a.g(),
+                      c->lay.op_size);
+  C1->herm = A->herm;
+  if (C2) C2->herm = A->herm;
   return s;
 }
 // The operand L = Omega of every nested commutator of a series, prepared once:
@@ -1609,24 +1650,15 @@ static hipEvent_t gate_mark(imsrg_ctx_s *c, int n, const ActSet &set) {
 }
 // Waits for the live flags of gate n (sequence number seq), read from the
 // pinned ring as the kernel writes them (an event costs a record and a wake-up
-// per commutator); live[k] = 1 for positions that go on.  The stream is asked
-// now and then, so a failed launch ends the wait.
+// per commutator); live[k] = 1 for positions that go on.
 static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, int seq, std::vector<int> &live, int &nlive) {
   const volatile int *f = c->live_h + (size_t)(n % imsrg_ctx_s::kGateRing) * c->nbatch;
   live.assign(set.n(), 0);
   nlive = 0;
   for (int k = 0; k < set.n(); k++) {
-    int v = f[k];
-    for (long long spin = 1; (v >> 1) != seq; v = f[k], spin++) {
-      if (spin % 4096) continue;
-      const hipError_t e = hipStreamQuery(c->stream);
-      if (e == hipErrorNotReady) continue;
-      v = f[k];
-      if (e != hipSuccess || (v >> 1) != seq)
-        return fail(IMSRG_EDEVICE, std::string("series gate: ") + hipGetErrorString(e));
-      break;
-    }
-    nlive += (live[k] = v & 1);
+    const int rc = wait_seq(c, seq, "series gate", [&] { return f[k] >> 1; });
+    if (rc) return rc;
+    nlive += (live[k] = f[k] & 1);
   }
   return 0;
 }
@@ -1642,16 +1674,14 @@ static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, int seq, std::v
 // of nested commutators instance a.h[k] used.
 static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H, const ActSet &a,
                     std::vector<int> &nterms) {
-  imsrg_op_s *AD = tmp_op(c, 0, 1), *INT2 = tmp_op(c, 1, 1);
-  if (!AD || !INT2) return IMSRG_ENOMEM;
+  imsrg_op_s *T[2] = {tmp_op(c, 0, 1), tmp_op(c, 1, 1)};
+  if (!T[0] || !T[1]) return IMSRG_ENOMEM;
   nterms.assign(a.n(), 0);
   if (a.n() == 0) return 0;
-  op_copy(H, HS, a);
-  op_copy(H, AD, a);  // AD_1 = H
-  // [G, X] with G anti-hermitian keeps the hermiticity of X
-  AD->herm = H->herm;
-  INT2->herm = H->herm;
-  const ActSet cur = series_set(c, 1, a);
+  const ActSet cur = series_begin(c, 1, a, H, HS, nullptr);
+  // AD_1 = H itself; [G, X] with G anti-hermitian keeps the hermiticity of X
+  imsrg_op_s *AD = H, *INT2 = T[0];
+  T[0]->herm = T[1]->herm = H->herm;
   prep_L(c, G, cur);
   std::vector<int> live(a.n(), 1);  // positions in the series for nested commutator iw
   int nlive = a.n(), seq = 0;
@@ -1675,9 +1705,8 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
     if (rc) return rc;
     if (nlive == 0) return 0;  // the test after iw-1 stopped every instance
     for (int k = 0; k < cur.n(); k++) nterms[k] += live[k];
-    std::swap(c->tmp[0], c->tmp[1]);
-    AD = c->tmp[0];
-    INT2 = c->tmp[1];
+    AD = INT2;
+    INT2 = T[AD == T[0] ? 1 : 0];
   }
   int rc = series_live(c, cur, 40, seq, live, nlive);
   if (rc) return rc;
@@ -1733,17 +1762,12 @@ static int magexp_impl(imsrg_ctx_s *c, imsrg_op_s *DG, imsrg_op_s *G, const ActS
   if (a.n() == 0) return 0;
   imsrg_op_s *cur = tmp_op(c, 0, DG->herm), *oth = tmp_op(c, 1, DG->herm);
   if (!cur || !oth) return IMSRG_ENOMEM;
-  op_copy(DG, cur, a);
-  op_copy(DG, oth, a);
-  const ActSet set = series_set(c, 2, a);
-  // advals(1) = ||DG|| and fullnorm = ||G|| into the series scalar slots; the
-  // first gate: fullnorm < 1e-9 returns, then the test on advals(1)
+  const ActSet set = series_begin(c, 2, a, DG, cur, oth);
+  // advals(1) = ||DG|| and fullnorm = ||G||; the first gate: fullnorm < 1e-9
+  // returns, then the test on advals(1)
+  const GateArgs g = gate_args(c, 1, 1, 0.0, -1, 0);
   PROF(c, IMSRG_PROF_NORM,
-       launch_sumsq(c->stream, c->dl, cur->d, c->partials, c->scal + kAdvSlot, set.d, set.n()));
-  PROF(c, IMSRG_PROF_NORM,
-       launch_sumsq(c->stream, c->dl, G->d, c->partials, c->scal + kFullSlot, set.d, set.n()));
-  GateArgs g = gate_args(c, 1, 1, 0.0, -1, 0);
-  launch_series_gate(c->stream, c->act_d[2], set.g(), c->scal, g);
+       launch_magnus_gate(c->stream, c->dl, DG->d, G->d, c->partials, c->nbatch, c->act_d[2], set.g(), c->scal, g));
   prep_L(c, G, set);
   std::vector<int> live;
   int nlive = 0, seq = g.seq, rc = 0;
@@ -1789,7 +1813,7 @@ struct imsrg_flow_s {
   imsrg_op_s *HS = nullptr, *G = nullptr, *H0 = nullptr, *DG = nullptr;
   int gen_kind = 0;
   double ds = 0.5;
-  std::vector<double> s, crit, emp2;
+  std::vector<double> s, crit, emp2, e0;
   std::vector<int> steps;
 };
 
@@ -1805,7 +1829,7 @@ static int flow_setup(imsrg_ctx c, imsrg_op HS, imsrg_op G, int gen_kind, double
   imsrg_flow_s *f = new imsrg_flow_s;
   f->ctx = c; f->HS = HS; f->G = G; f->gen_kind = gen_kind; f->ds = ds;
   const int B = c->nbatch;
-  f->s.assign(B, restart ? s0 : 0.0); f->crit.assign(B, 0.0); f->emp2.assign(B, 0.0);
+  f->s.assign(B, restart ? s0 : 0.0); f->crit.assign(B, 0.0); f->emp2.assign(B, 0.0); f->e0.assign(B, 0.0);
   f->steps.assign(B, restart ? (int)std::lround(s0 / ds) : 0);
   const ActSet all = all_set(c);
   int rc = op_new(c, 1, &f->H0);
@@ -1936,7 +1960,6 @@ int imsrg_flow_step(imsrg_flow f, double *rec) {
   for (int k = 0; k < B; k++)
     if (f->crit[k] > kConv) live.push_back(k);
   std::vector<int> nm(B, 0), nb(B, 0);
-  std::vector<double> e0(B, 0.0);
   int rc = 0;
   if (!live.empty()) {
     const ActSet a = ((int)live.size() == B) ? all_set(c) : make_set(c, 3, live, c->graphs ? B : 0);
@@ -1948,28 +1971,35 @@ int imsrg_flow_step(imsrg_flow f, double *rec) {
                       c->lay.op_size));  // euler_step :756-766
     rc = bch_impl(c, f->HS, f->G, f->H0, a, tb);
     if (rc) return rc;
-    rc = gen_impl(c, f->gen_kind, f->HS, f->DG, a);
-    if (rc) return rc;
-    std::vector<double> mp;
-    rc = mbpt2_set(f->HS, a, mp);
+    const int seq = c->rep_seq = c->rep_seq == INT_MAX ? 1 : c->rep_seq + 1;
+    rc = gen_impl(c, f->gen_kind, f->HS, f->DG, a, c->rep_d, seq);
     if (rc) return rc;
     for (int m = 0; m < a.n(); m++) {
       const int k = a.h[m];
+      const StepReport *r = c->rep_h + k;
+      rc = wait_seq(c, seq, "flow step", [&] { return __atomic_load_n(&r->seq, __ATOMIC_ACQUIRE); });
+      if (rc) return rc;
       f->s[k] += f->ds;
-      f->emp2[k] = mp[m];
-      f->crit[k] = std::fabs(mp[m]);
+      f->emp2[k] = r->mbpt2;
+      f->e0[k] = r->e0;
+      f->crit[k] = std::fabs(r->mbpt2);
       f->steps[k]++;
       nm[k] = tm[m];
       nb[k] = tb[m];
     }
   }
   if (rec) {
-    rc = imsrg_op_e0_batch(f->HS, e0.data());
-    if (rc) return rc;
     std::vector<char> stepped(B, 0);
     for (int k : live) stepped[k] = 1;
+    if ((int)live.size() < B) {  // instances that did not step: E0 as HS holds it
+      std::vector<double> e0(B, 0.0);
+      rc = imsrg_op_e0_batch(f->HS, e0.data());
+      if (rc) return rc;
+      for (int k = 0; k < B; k++)
+        if (!stepped[k]) f->e0[k] = e0[k];
+    }
     for (int k = 0; k < B; k++) {
-      const double r[8] = {f->s[k], e0[k], e0[k] + f->emp2[k], f->crit[k], (double)nm[k], (double)nb[k],
+      const double r[8] = {f->s[k], f->e0[k], f->e0[k] + f->emp2[k], f->crit[k], (double)nm[k], (double)nb[k],
                            (double)f->steps[k], stepped[k] ? 1.0 : 0.0};
       std::memcpy(rec + 8 * (size_t)k, r, sizeof(r));
     }

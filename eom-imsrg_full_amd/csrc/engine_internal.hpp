@@ -54,6 +54,14 @@ struct imsrg_ctx_s {
   static constexpr int kGateRing = 4;
   int *live_h = nullptr, *live_d = nullptr;  // host and device views, kGateRing * nbatch
   hipEvent_t ev_gate[kGateRing] = {};
+  StepReport *rep_h = nullptr, *rep_d = nullptr;  // flow step reports (pinned), one per instance
+  // operator buffers given back (imsrg_op_destroy, drivers' temporaries), reused
+  // by the next op_new of this context: its work is all ordered by its streams.
+  // At most kOpPool of them and kOpPoolBytes; freed with the context, or when
+  // an allocation fails.
+  static constexpr size_t kOpPool = 64, kOpPoolBytes = (size_t)4 << 30;
+  std::vector<double *> op_pool;
+  int rep_seq = 0;         // number of the last flow step report
   int gate_seq = 0;        // number of the last series gate (GateArgs::seq)
   bool capturing = false;  // graph capture records one stream only
   std::vector<void *> dallocs;
@@ -149,11 +157,22 @@ struct imsrg_op_s {
 inline int i8_planes(int prec) {
   return prec == IMSRG_PREC_INT8X5 ? 5 : prec == IMSRG_PREC_INT8X4 ? 4 : 0;
 }
+// hipMalloc for a context; when it fails, the context's pool of operator
+// buffers goes back to the device and the call is made again
+inline hipError_t dev_malloc(imsrg_ctx_s *c, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess || c->op_pool.empty()) return e;
+  (void)hipGetLastError();
+  (void)hipStreamSynchronize(c->stream);
+  for (double *q : c->op_pool) (void)hipFree(q);
+  c->op_pool.clear();
+  return hipMalloc(p, bytes);
+}
 template <class T>
 inline int upload_table(imsrg_ctx_s *c, const std::vector<T> &v, const T **out) {
   size_t bytes = std::max<size_t>(v.size(), 1) * sizeof(T);
   void *p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc table failed");
+  if (dev_malloc(c, &p, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc table failed");
   c->dallocs.push_back(p);
   if (!v.empty()) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   *out = (const T *)p;
@@ -161,7 +180,7 @@ inline int upload_table(imsrg_ctx_s *c, const std::vector<T> &v, const T **out) 
 }
 inline int dalloc(imsrg_ctx_s *c, size_t ndouble, double **out) {
   void *p = nullptr;
-  if (hipMalloc(&p, std::max<size_t>(ndouble, 1) * sizeof(double)) != hipSuccess)
+  if (dev_malloc(c, &p, std::max<size_t>(ndouble, 1) * sizeof(double)) != hipSuccess)
     return fail(IMSRG_ENOMEM, "hipMalloc workspace failed (" + std::to_string(ndouble * 8) + " bytes)");
   c->dallocs.push_back(p);
   *out = (double *)p;

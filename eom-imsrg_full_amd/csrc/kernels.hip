@@ -73,6 +73,34 @@ void launch_copy(hipStream_t s, long long n, const double *A, double *C, const i
   hipLaunchKernelGGL(k_copy, dim3(grid, nact), dim3(256), 0, s, n, A, C, act, stride);
 }
 
+// The start of a BCH or Magnus series in one launch: op A copied to C1 (and
+// C2), and the caller's instance table to the series' own (workgroup 0 of each
+// position).
+__global__ void k_series_begin(long long n, const double *A, double *C1, double *C2, const int *act, int *own,
+                               long long stride) {
+  const int id = act[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x == 0) own[blockIdx.y] = id;
+  if (id < 0) return;
+  const long long o = id * stride;
+  A += o;
+  C1 += o;
+  if (C2) C2 += o;
+  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long st = (long long)gridDim.x * blockDim.x;
+  for (; i < n; i += st) {
+    const double v = A[i];
+    C1[i] = v;
+    if (C2) C2[i] = v;
+  }
+}
+void launch_series_begin(hipStream_t s, long long n, const double *A, double *C1, double *C2, const int *act, int *own,
+                         int nact, long long stride) {
+  if (n <= 0 || nact <= 0) return;
+  const long long nb = (n + 255) / 256;
+  hipLaunchKernelGGL(k_series_begin, dim3((unsigned)(nb < 8192 ? nb : 8192), nact), dim3(256), 0, s, n, A, C1, C2,
+                     act, own, stride);
+}
+
 // ------------------------------------------------------------------ segmented grouped GEMM
 // Every output block C (M x M) is a signed sum of K segments,
 //   C = sum_s sign_s * A_s * B_s,
@@ -1781,14 +1809,17 @@ void launch_e0(hipStream_t s, const DevLayout &L, const double *Lop, const doubl
 }
 
 // sum of squares of F and V = mat_frob_norm^2 (basic_IMSRG.f90:3921-3952)
-__global__ __launch_bounds__(256) void k_sumsq_partial(const double *x, long long n, double *partials,
-                                                        const int *act, long long stride) {
+// (blockIdx.z: the operator, x or x2, and its set of partials, pstride apart)
+__global__ __launch_bounds__(256) void k_sumsq_partial(const double *x, const double *x2, long long n,
+                                                        double *partials, long long pstride, const int *act,
+                                                        long long stride) {
   __shared__ double sh[256];
+  if (blockIdx.z) x = x2;
   {
     const long long inst = inst_id(act);
     if (inst < 0) return;
     x += inst * stride;
-    partials += inst * kPartials;
+    partials += inst * kPartials + blockIdx.z * pstride;
   }
   // eight strided elements per round, read off any branch (clamped to the
   // last element, discarded past it): the same summation order as one at a time
@@ -1805,6 +1836,20 @@ __global__ __launch_bounds__(256) void k_sumsq_partial(const double *x, long lon
   s = block_sum256(s, sh);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
+// sum of n values by one workgroup: eight per round off any branch, in the
+// one-at-a-time order
+__device__ __forceinline__ double sum256(const double *p, int n, double *sh) {
+  double s = 0.0;
+  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * 256) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = p[min(i0 + 256 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (i0 + 256 * u < n) s += v[u];
+  }
+  return block_sum256(s, sh);
+}
 __global__ __launch_bounds__(256) void k_final_sum(const double *partials, int n, double *out, int do_sqrt,
                                                     const int *act, long long pstride) {
   __shared__ double sh[256];
@@ -1814,24 +1859,15 @@ __global__ __launch_bounds__(256) void k_final_sum(const double *partials, int n
     partials += inst * pstride;
     out += inst * kScal;
   }
-  double s = 0.0;  // eight partials per round off any branch, in the one-at-a-time order
-  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * 256) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) v[u] = partials[min(i0 + 256 * u, n - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; u++)
-      if (i0 + 256 * u < n) s += v[u];
-  }
-  s = block_sum256(s, sh);
+  const double s = sum256(partials, n, sh);
   if (threadIdx.x == 0) out[0] = do_sqrt ? sqrt(s) : s;
 }
 void launch_sumsq(hipStream_t s, const DevLayout &L, const double *op, double *partials, double *out,
                   const int *act, int nact) {
   if (nact <= 0) return;
   const long long n = L.op_size - L.f_off;
-  hipLaunchKernelGGL(k_sumsq_partial, dim3(kPartials, nact), dim3(256), 0, s, op + L.f_off, n, partials, act,
-                     L.op_size);
+  hipLaunchKernelGGL(k_sumsq_partial, dim3(kPartials, nact), dim3(256), 0, s, op + L.f_off, nullptr, n, partials,
+                     0LL, act, L.op_size);
   hipLaunchKernelGGL(k_final_sum, dim3(1, nact), dim3(256), 0, s, partials, kPartials, out, 1, act,
                      (long long)kPartials);
 }
@@ -1844,16 +1880,8 @@ void launch_norm_from_parts(hipStream_t s, int n, const double *npart, double *o
 }
 
 // mbpt2 (basic_IMSRG.f90:4030-4064): one workgroup per block
-__global__ __launch_bounds__(256) void k_mbpt2_partial(DevLayout L, const double *H, double *partials,
-                                                        const int *act) {
-  __shared__ double sh[256];
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    H += inst * L.op_size;
-    partials += inst * kPartials;
-  }
-  const int q = blockIdx.x;
+__device__ __forceinline__ void mbpt2_block(const DevLayout &L, const double *H, double *partials, int q,
+                                            double *sh) {
   const int np = L.bnp[q], nb = L.bnb[q], nh = L.bnh[q], dim = L.bdim[q], base = L.pbase[q], N = L.nsp;
   const double *V = H + L.v_off + L.boff[q];
   const double *F = H + L.f_off;
@@ -1869,6 +1897,13 @@ __global__ __launch_bounds__(256) void k_mbpt2_partial(DevLayout L, const double
   s = block_sum256(s, sh);
   if (threadIdx.x == 0) partials[q] = (L.bJ[q] + 1.0) * s;
 }
+__global__ __launch_bounds__(256) void k_mbpt2_partial(DevLayout L, const double *H, double *partials,
+                                                        const int *act) {
+  __shared__ double sh[256];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  mbpt2_block(L, H + inst * L.op_size, partials + inst * kPartials, blockIdx.x, sh);
+}
 void launch_mbpt2(hipStream_t s, const DevLayout &L, const double *op, double *partials, double *out,
                   const int *act, int nact) {
   if (nact <= 0) return;
@@ -1879,14 +1914,7 @@ void launch_mbpt2(hipStream_t s, const DevLayout &L, const double *op, double *p
 
 // ------------------------------------------------------------------ generators
 // twobody_monopole (basic_IMSRG.f90:2031-2046) for every orbit pair
-__global__ void k_monopole(DevLayout L, const double *H, double *mono, const int *act) {
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    H += inst * L.op_size;
-    mono += inst * L.nsp * L.nsp;
-  }
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void monopole_at(const DevLayout &L, const double *H, double *mono, int t) {
   const int N = L.nsp;
   if (t >= N * N) return;
   const int a = t / N, b = t % N, ja = L.jj[a], jb = L.jj[b];
@@ -1894,6 +1922,11 @@ __global__ void k_monopole(DevLayout L, const double *H, double *mono, const int
   double sm = 0.0;
   for (int JT = abs(ja - jb); JT <= ja + jb; JT += 2) sm = sm + (JT + 1) * dv(L, V, a, b, a, b, JT);
   mono[t] = sm / (ja + 1.0) / (jb + 1.0);
+}
+__global__ void k_monopole(DevLayout L, const double *H, double *mono, const int *act) {
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  monopole_at(L, H + inst * L.op_size, mono + inst * L.nsp * L.nsp, blockIdx.x * blockDim.x + threadIdx.x);
 }
 void launch_monopole(hipStream_t s, const DevLayout &L, const double *H, double *mono, const int *act,
                      int nact) {
@@ -1904,18 +1937,8 @@ void launch_monopole(hipStream_t s, const DevLayout &L, const double *H, double 
 
 // build_gs_white / build_gs_atan / build_gs_atanxx (generators.f90:4-374):
 // ETA must be zero on entry; kind 0 = H/Eden, 1 = atan(2H/Eden)/2
-__global__ void k_eta_onebody(DevLayout L, const double *Hden, const double *Hnum, double *ETA, int kind,
-                              const int *act) {
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    const long long o = inst * L.op_size;
-    Hden += o;
-    Hnum += o;
-    ETA += o;
-  }
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= L.nphp) return;
+__device__ __forceinline__ void eta_onebody(const DevLayout &L, const double *Hden, const double *Hnum, double *ETA,
+                                            int kind, int e) {
   const int a = L.php_a[e], i = L.php_i[e], N = L.nsp, ji = L.jj[i];
   const double *V = Hden + L.v_off, *Fd = Hden + L.f_off;
   double Eden = 0.0;
@@ -1927,22 +1950,14 @@ __global__ void k_eta_onebody(DevLayout L, const double *Hden, const double *Hnu
   ETA[L.f_off + a * N + i] = eta;
   ETA[L.f_off + i * N + a] = -eta;
 }
-__global__ __launch_bounds__(256) void k_eta_twobody(DevLayout L, const double *Hden, const double *Hnum,
-                                                      const double *mono, double *ETA, int kind, const int *act) {
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    Hden += inst * L.op_size;
-    Hnum += inst * L.op_size;
-    ETA += inst * L.op_size;
-    mono += inst * L.nsp * L.nsp;
-  }
-  const int q = blockIdx.x;
+// (elements e0, e0 + st, ... of block q)
+__device__ __forceinline__ void eta_twobody(const DevLayout &L, const double *Hden, const double *Hnum,
+                                            const double *mono, double *ETA, int kind, int q, int e0, int st) {
   const int np = L.bnp[q], nb = L.bnb[q], nh = L.bnh[q], dim = L.bdim[q], base = L.pbase[q], N = L.nsp;
   const double *Fd = Hden + L.f_off;
   const double *Vn = Hnum + L.v_off + L.boff[q];
   double *Ve = ETA + L.v_off + L.boff[q];
-  for (int e = threadIdx.x; e < np * nh; e += 256) {
+  for (int e = e0; e < np * nh; e += st) {
     const int ix = e / nh, jx = e % nh;
     const int a = L.pair_a[base + ix], b = L.pair_b[base + ix];
     const int i = L.pair_a[base + np + nb + jx], j = L.pair_b[base + np + nb + jx];
@@ -1961,14 +1976,70 @@ __global__ __launch_bounds__(256) void k_eta_twobody(DevLayout L, const double *
     Ve[(long long)(np + nb + jx) * dim + ix] = -eta;
   }
 }
-void launch_eta(hipStream_t s, const DevLayout &L, const double *Hden, const double *Hnum,
-                const double *mono, double *ETA, int kind, const int *act, int nact) {
+// A generator in two launches.  k_gen_a: ETA cleared, the monopoles of Hden
+// and, for a flow step's report, its MBPT2 sums per block.  k_gen_b: the
+// one- and two-body elements, and the report: MBPT2 and E0 of Hden to pinned
+// host memory under a sequence number.  (They were four launches, and the
+// report two more, two copies and two stream waits.)
+constexpr int kEtaSplit = 4;  // workgroups per channel block (a block's elements are few)
+__global__ __launch_bounds__(256) void k_gen_a(DevLayout L, const double *Hden, double *mono, double *ETA,
+                                               double *partials, const int *act, int nmono, int nmb, int nfill) {
+  __shared__ double sh[256];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  const long long o = inst * L.op_size;
+  int b = blockIdx.x;
+  if (b < nmono) {
+    monopole_at(L, Hden + o, mono + inst * L.nsp * L.nsp, b * 256 + (int)threadIdx.x);
+    return;
+  }
+  b -= nmono;
+  if (b < nmb) {
+    mbpt2_block(L, Hden + o, partials + inst * kPartials, b, sh);
+    return;
+  }
+  b -= nmb;
+  const long long n = L.op_size - L.f_off, st = 256LL * nfill;
+  double *p = ETA + o + L.f_off;
+  for (long long i = 256LL * b + threadIdx.x; i < n; i += st) p[i] = 0.0;
+}
+__global__ __launch_bounds__(256) void k_gen_b(DevLayout L, const double *Hden, const double *Hnum, const double *mono,
+                                               double *ETA, int kind, const double *partials, const int *act, int n1,
+                                               StepReport *rep, int seq) {
+  __shared__ double sh[256];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  const long long o = inst * L.op_size;
+  int b = blockIdx.x;
+  if (b < n1) {
+    const int e = b * 256 + (int)threadIdx.x;
+    if (e < L.nphp) eta_onebody(L, Hden + o, Hnum + o, ETA + o, kind, e);
+    return;
+  }
+  b -= n1;
+  if (b < L.nblocks * kEtaSplit) {
+    eta_twobody(L, Hden + o, Hnum + o, mono + inst * L.nsp * L.nsp, ETA + o, kind, b / kEtaSplit,
+                256 * (b % kEtaSplit) + (int)threadIdx.x, 256 * kEtaSplit);
+    return;
+  }
+  const double s = sum256(partials + inst * kPartials, L.nblocks, sh);
+  if (threadIdx.x == 0) {
+    StepReport *r = rep + inst;
+    r->mbpt2 = s;
+    r->e0 = Hden[o];
+    __threadfence_system();
+    __hip_atomic_store(&r->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+void launch_generator(hipStream_t s, const DevLayout &L, const double *Hden, const double *Hnum, double *mono,
+                      double *ETA, int kind, double *partials, const int *act, int nact, StepReport *rep, int seq) {
   if (nact <= 0) return;
-  if (L.nphp > 0)
-    hipLaunchKernelGGL(k_eta_onebody, dim3((L.nphp + 63) / 64, nact), dim3(64), 0, s, L, Hden, Hnum, ETA, kind,
-                       act);
-  hipLaunchKernelGGL(k_eta_twobody, dim3(L.nblocks, nact), dim3(256), 0, s, L, Hden, Hnum, mono, ETA, kind,
-                     act);
+  const int nmono = (L.nsp * L.nsp + 255) / 256, nmb = rep ? L.nblocks : 0, n1 = (L.nphp + 255) / 256;
+  const int nfill = (int)std::min<long long>(8192, (L.op_size - L.f_off + 255) / 256);
+  hipLaunchKernelGGL(k_gen_a, dim3(nmono + nmb + nfill, nact), dim3(256), 0, s, L, Hden, mono, ETA, partials, act,
+                     nmono, nmb, nfill);
+  hipLaunchKernelGGL(k_gen_b, dim3(n1 + L.nblocks * kEtaSplit + (rep ? 1 : 0), nact), dim3(256), 0, s, L, Hden, Hnum,
+                     (const double *)mono, ETA, kind, (const double *)partials, act, n1, rep, seq);
 }
 
 // ------------------------------------------------------------------ normal ordering
@@ -2085,27 +2156,40 @@ void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, const G
 __global__ __launch_bounds__(256) void k_norm_gate(const double *npart, int n, int *act, double *scal, GateArgs G) {
   __shared__ double sh[256];
   const int inst = act[blockIdx.y];
-  double s = 0.0;
   if (inst >= 0) {
-    const double *p = npart + (long long)inst * n;
-    for (int i0 = threadIdx.x; i0 < n; i0 += 8 * 256) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = p[min(i0 + 256 * u, n - 1)];
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (i0 + 256 * u < n) s += v[u];
-    }
+    const double s = sum256(npart + (long long)inst * n, n, sh);
+    if (threadIdx.x == 0) scal[(long long)inst * kScal] = sqrt(s);
   }
-  s = block_sum256(s, sh);
-  if (threadIdx.x == 0) {
-    if (inst >= 0) scal[(long long)inst * kScal] = sqrt(s);
-    gate_position(act, blockIdx.y, scal, G);
-  }
+  if (threadIdx.x == 0) gate_position(act, blockIdx.y, scal, G);
 }
 void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
                       const GateArgs &G) {
   if (nact > 0) hipLaunchKernelGGL(k_norm_gate, dim3(1, nact), dim3(256), 0, s, npart, n, act, scal, G);
+}
+// The start of a Magnus series: advals(1) = ||DG|| and ||Omega|| into their
+// scalar slots, and the first gate (partials: one set of kPartials * nbatch
+// per operator).
+__global__ __launch_bounds__(256) void k_magnus_gate(const double *partials, long long pstride, int *act,
+                                                     double *scal, GateArgs G) {
+  __shared__ double sh[256];
+  const int inst = act[blockIdx.y];
+  if (inst >= 0) {
+    const double *p = partials + (long long)inst * kPartials;
+    const double d = sum256(p, kPartials, sh), o = sum256(p + pstride, kPartials, sh);
+    if (threadIdx.x == 0) {
+      scal[(long long)inst * kScal + kAdvSlot] = sqrt(d);
+      scal[(long long)inst * kScal + kFullSlot] = sqrt(o);
+    }
+  }
+  if (threadIdx.x == 0) gate_position(act, blockIdx.y, scal, G);
+}
+void launch_magnus_gate(hipStream_t s, const DevLayout &L, const double *DG, const double *Om, double *partials,
+                        int nbatch, int *act, int nact, double *scal, const GateArgs &G) {
+  if (nact <= 0) return;
+  const long long n = L.op_size - L.f_off, ps = (long long)kPartials * nbatch;
+  hipLaunchKernelGGL(k_sumsq_partial, dim3(kPartials, nact, 2), dim3(256), 0, s, DG + L.f_off, Om + L.f_off, n,
+                     partials, ps, act, L.op_size);
+  hipLaunchKernelGGL(k_magnus_gate, dim3(1, nact), dim3(256), 0, s, partials, ps, act, scal, G);
 }
 
 // ------------------------------------------------------------------ small bases: a commutator in three launches
