@@ -190,8 +190,10 @@ void launch_axpby(hipStream_t s, long long n, double a, const double *A, double 
                   const int *act, int nact, long long stride);
 void launch_copy(hipStream_t s, long long n, const double *A, double *C, const int *act, int nact,
                  long long stride);
-// mode: 0 FP64 MFMA (64 x 64 tiles), 1 split-FP32 (3 FP32-MFMA products), 2 split-BF16
-// (6 BF16-MFMA products), 3 FP64 MFMA on 128 x 64 tiles (tile list built for that shape).
+// mode: 0 FP64 MFMA (pp/hh: 32 x 32 tiles, K split over a workgroup's wavefronts; Pandya
+// product: 64 x 64 tiles), 1 split-FP32 (3 FP32-MFMA products), 2 split-BF16 (6 BF16-MFMA
+// products), 3 FP64 MFMA on 128 x 64 tiles, 4 the Pandya product as pp/hh in mode 0
+// (tile lists built for those shapes; modes 1 and 2: 64 x 64).
 // 222_pp_hh: RES(upper) += L*D*R - R*D*L per channel block; with W, the pp part
 // (W1 - pm*W1^T) is also stored to W (upper triangle) for commutator_221.
 void launch_seg_gemm_pphh(hipStream_t s, int mode, const SegProb *probs, const int4 *tiles, int ntiles,
@@ -314,7 +316,7 @@ struct SmallArgs {
   const double *coefp;
   const SegProb *pp_probs, *ph_probs;
   const int4 *pp_tiles, *ph_tiles, *tiles16;
-  int n_pp, n_ph, n16, n_diff, nsplit;
+  int n_pp, n_ph, n16, n_diff, nsplit, split;
   const int *diff_ob;       // one-body outputs whose orbits differ in (l, j, tz)
   const PhRow *phrow;
   const int *act;

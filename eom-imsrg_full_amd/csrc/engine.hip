@@ -191,7 +191,8 @@ static int op_new(imsrg_ctx_s *c, int herm, imsrg_op_s **out) {
   imsrg_op_s *op = new imsrg_op_s;
   op->ctx = c;
   op->herm = herm;
-  const size_t bytes = sizeof(double) * c->lay.op_size * c->nbatch;
+  // (the FP64 products' 16-byte reads may take one element past the last block)
+  const size_t bytes = sizeof(double) * (c->lay.op_size * c->nbatch + 8);
   if (!c->op_pool.empty()) {
     op->d = c->op_pool.back();
     c->op_pool.pop_back();
@@ -276,6 +277,7 @@ static int scratch_setup(imsrg_ctx_s *c) {
 
 // ---------------------------------------------------------------- context
 // Tables of the three-launch commutator (launch_small), for bases that may use it.
+static constexpr long long kSplitElems = 300000;  // two-body elements (the rule at wave_pair)
 static constexpr long long kSmallElems = 1000000;  // two-body elements times instances (the rule at use_small)
 static int small_setup(imsrg_ctx_s *c, const std::vector<int> &same_ob) {
   const Layout &Ly = c->lay;
@@ -582,7 +584,11 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
     build_seg_tiles(pp, tw, 128, 64);
     c->n_pp_tiles = (int)tiles.size();
     c->n_pp_tiles_w = (int)tw.size();
-    rc = upload_table(c, pp, (const SegProb **)&c->pp_probs);
+    std::vector<int4> ts;
+    build_seg_tiles(pp, ts, 32, 32);
+    c->n_pp_tiles_s = (int)ts.size();
+    rc = upload_table(c, ts, (const int4 **)&c->pp_tiles_s);
+    if (!rc) rc = upload_table(c, pp, (const SegProb **)&c->pp_probs);
     if (!rc) rc = upload_table(c, tiles, (const int4 **)&c->pp_tiles);
     if (!rc) rc = upload_table(c, tw, (const int4 **)&c->pp_tiles_w);
   }
@@ -605,7 +611,14 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
     build_seg_tiles(ph, tw, 128, 64);
     c->n_ph_tiles = (int)tiles.size();
     c->n_ph_tiles_w = (int)tw.size();
-    rc = upload_table(c, ph, (const SegProb **)&c->ph_probs);
+    c->split = Ly.vsize <= kSplitElems;
+    if (c->split) {
+      std::vector<int4> ts;
+      build_seg_tiles(ph, ts, 32, 32);
+      c->n_ph_tiles_s = (int)ts.size();
+      rc = upload_table(c, ts, (const int4 **)&c->ph_tiles_s);
+    }
+    if (!rc) rc = upload_table(c, ph, (const SegProb **)&c->ph_probs);
     if (!rc) rc = upload_table(c, tiles, (const int4 **)&c->ph_tiles);
     if (!rc) rc = upload_table(c, tw, (const int4 **)&c->ph_tiles_w);
   }
@@ -1226,8 +1239,9 @@ static int autotune(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R) {
     return best;
   };
   const double *X0 = L->d + D.v_off, *X1 = R->d + D.v_off;
+  const bool sp = c->split;
   c->tune_ms[0] = timed([&] {
-    launch_seg_gemm_pphh(s, 0, c->pp_probs, c->pp_tiles, c->n_pp_tiles, X0, X1, nullptr, nullptr, a.d, a.n(), D.op_size,
+    launch_seg_gemm_pphh(s, 0, c->pp_probs, c->pp_tiles_s, c->n_pp_tiles_s, X0, X1, nullptr, nullptr, a.d, a.n(), D.op_size,
                          D.vsize);
   });
   c->tune_ms[1] = timed([&] {
@@ -1237,7 +1251,8 @@ static int autotune(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R) {
   launch_pandya(s, D, L->d, c->cc[0], a.d, a.n());
   launch_pandya(s, D, R->d, c->cc[1], a.d, a.n());
   c->tune_ms[2] = timed([&] {
-    launch_seg_gemm_z(s, 0, c->ph_probs, c->ph_tiles, c->n_ph_tiles, c->cc[0], c->cc[1], c->wph, (double)L->herm,
+    launch_seg_gemm_z(s, sp ? 4 : 0, c->ph_probs, sp ? c->ph_tiles_s : c->ph_tiles,
+                      sp ? c->n_ph_tiles_s : c->n_ph_tiles, c->cc[0], c->cc[1], c->wph, (double)L->herm,
                       (double)R->herm, a.d, a.n(), D.ccsize, D.cwsize);
   });
   c->tune_ms[3] = timed([&] {
@@ -1323,8 +1338,10 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     A.hL = hL; A.hR = hR; A.hres = hres; A.prepL = !lcc;
     A.mask = mask; A.coef = epi.coef; A.coefp = epi.coefp;
     A.pp_probs = c->pp_probs; A.ph_probs = c->ph_probs;
-    A.pp_tiles = c->pp_tiles; A.ph_tiles = c->ph_tiles; A.tiles16 = c->tiles16;
-    A.n_pp = c->n_pp_tiles; A.n_ph = c->n_ph_tiles; A.n16 = c->n_tiles16; A.n_diff = c->n_diff_ob;
+    A.split = c->split;
+    A.pp_tiles = c->pp_tiles_s; A.ph_tiles = c->split ? c->ph_tiles_s : c->ph_tiles;
+    A.n_pp = c->n_pp_tiles_s; A.n_ph = c->split ? c->n_ph_tiles_s : c->n_ph_tiles;
+    A.tiles16 = c->tiles16; A.n16 = c->n_tiles16; A.n_diff = c->n_diff_ob;
     A.diff_ob = c->diff_ob; A.phrow = c->phrow; A.act = ad;
     launch_small(s, D, c->dl_d, A, na);
     c->fork_mark = nullptr;
@@ -1366,10 +1383,11 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
                              c->i8vs[1], (double)hR, (double)hL, (mask & T222PPHH) ? RES->d + D.v_off : nullptr,
                              (mask & T221) ? c->wpp : nullptr, ad, na, c->i8.v_bytes, c->i8.v_sr, OS, D.vsize));
   } else if (mask & (T222PPHH | T221)) {
-    const bool w = c->prec == IMSRG_PREC_FP64 && c->shape_pp == 1;
+    const bool w = c->prec == IMSRG_PREC_FP64 && c->shape_pp == 1, sp = c->prec == IMSRG_PREC_FP64 && !w;
     PROFK(c, IMSRG_PROF_GEMM_PPHH,
-          launch_seg_gemm_pphh(s2, w ? 3 : c->prec, c->pp_probs, w ? c->pp_tiles_w : c->pp_tiles,
-                               w ? c->n_pp_tiles_w : c->n_pp_tiles, L->d + D.v_off, R->d + D.v_off,
+          launch_seg_gemm_pphh(s2, w ? 3 : c->prec, c->pp_probs,
+                               w ? c->pp_tiles_w : sp ? c->pp_tiles_s : c->pp_tiles,
+                               w ? c->n_pp_tiles_w : sp ? c->n_pp_tiles_s : c->n_pp_tiles, L->d + D.v_off, R->d + D.v_off,
                                (mask & T222PPHH) ? RES->d + D.v_off : nullptr, (mask & T221) ? c->wpp : nullptr,
                                ad, na, OS, D.vsize));
   }
@@ -1388,10 +1406,11 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
                             c->i8cs[1], (double)hL, -(double)hR, c->wph, -(double)hL * (double)hR, ad, na,
                             c->i8.c_bytes, c->i8.c_sr, D.cwsize));
     } else {
-      const bool w = c->prec == IMSRG_PREC_FP64 && c->shape_ph == 1;
+      const bool w = c->prec == IMSRG_PREC_FP64 && c->shape_ph == 1, sp = c->prec == IMSRG_PREC_FP64 && !w && c->split;
       PROFK(c, IMSRG_PROF_GEMM_PH,
-            launch_seg_gemm_z(s, w ? 3 : c->prec, c->ph_probs, w ? c->ph_tiles_w : c->ph_tiles,
-                             w ? c->n_ph_tiles_w : c->n_ph_tiles, c->cc[0], c->cc[1], c->wph, (double)hL,
+            launch_seg_gemm_z(s, w ? 3 : sp ? 4 : c->prec, c->ph_probs,
+                             w ? c->ph_tiles_w : sp ? c->ph_tiles_s : c->ph_tiles,
+                             w ? c->n_ph_tiles_w : sp ? c->n_ph_tiles_s : c->n_ph_tiles, c->cc[0], c->cc[1], c->wph, (double)hL,
                              (double)hR, ad, na, D.ccsize, D.cwsize));
     }
     PROF(c, IMSRG_PROF_PH_TERMS, launch_ph_terms(s, D, c->wph, c->tph, (double)hL, (double)hR, ad, na));

@@ -96,6 +96,10 @@ struct imsrg_ctx_s {
   const PhRow *phrow = nullptr;
   const int *diff_ob = nullptr;
   int n_tiles16 = 0, n_diff_ob = 0;
+  // 32 x 32 tile lists of the K-split FP64 products; split: the Pandya product uses them too
+  int4 *pp_tiles_s = nullptr, *ph_tiles_s = nullptr;
+  int n_pp_tiles_s = 0, n_ph_tiles_s = 0;
+  bool split = false;
   // FP64 tile shape per GEMM, chosen by timing both on the first FP64
   // commutator of the context: -1 not yet tuned, 0 64x64, 1 128x64
   int shape_pp = -1, shape_ph = -1;

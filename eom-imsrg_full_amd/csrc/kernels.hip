@@ -106,196 +106,22 @@ void launch_series_begin(hipStream_t s, long long n, const double *A, double *C1
 //   C = sum_s sign_s * A_s * B_s,
 // where segment s takes A from X[src] and B from X[1-src] (X0, X1 = the two
 // operands of the commutator, or their Pandya matrices).  A_s is M x K_s,
-// row-major (element (m,k) at m*lda + k) or, with A_KMAJOR, K-major (k*lda + m);
-// B_s is K_s x M with element (k,n) at k*ldb + n.  The outputs are
-// herm-symmetric, so only tiles tm <= tn are launched: one 64x64 tile per
-// workgroup, 4 wavefronts with 32x32 quadrants of 2x2 v_mfma_f64_16x16x4
-// tiles; in a diagonal tile the strictly-lower quadrant does no MFMA work.
-// K is staged through double-buffered LDS slabs of 16 (one barrier per slab,
-// the next slab's global loads in flight during the current slab's MFMAs).
-#ifndef IMSRG_GEMM_BK
-#define IMSRG_GEMM_BK 16
-#endif
-#ifndef IMSRG_GEMM_PF
-#define IMSRG_GEMM_PF 2  // K slabs of global loads in flight ahead of the MFMAs (1 or 2)
-#endif
-constexpr int GT = 64, GK = IMSRG_GEMM_BK, GP = 1, GJ = GK / 4;
-static_assert(GK == 16 || GK == 32, "K slab of 16 or 32");
+// row-major (element (m,k) at m*lda + k) or, for the Pandya product, K-major
+// (k*lda + m); B_s is K_s x M with element (k,n) at k*ldb + n.  The outputs are
+// herm-symmetric, so only tiles with an element on or above the diagonal are
+// launched.
+constexpr int GT = 64;
 
-struct GemmSmem {
-  double A[2][GK][GT + GP];
-  double B[2][GK][GT + GP];
-};
-static_assert(sizeof(GemmSmem) >= sizeof(double) * GT * (GT + GP), "transpose buffer must fit");
-
-// `need` bit (2*ti + tj): the 16x16 sub-tile holds outputs that are used
-// (inside the block and not strictly below the diagonal); others do no MFMA.
-// `need` is wave-uniform (an SGPR).  Off-diagonal tiles inside their block
-// run the FULL instantiation (straight-line MFMAs); the kernel picks it once
-// per workgroup, so neither path carries the other's registers through the
-// K loop.
-template <bool FULL>
-__device__ __forceinline__ void slab_mfma(const GemmSmem &S, int buf, double4_t acc[2][2], unsigned need) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-#pragma unroll
-  for (int kq = 0; kq < GK / 4; kq++) {
-    const int k = kq * 4 + (lane >> 4);
-    const double a0 = S.A[buf][k][wm * 32 + (lane & 15)];
-    const double a1 = S.A[buf][k][wm * 32 + 16 + (lane & 15)];
-    const double b0 = S.B[buf][k][wn * 32 + (lane & 15)];
-    const double b1 = S.B[buf][k][wn * 32 + 16 + (lane & 15)];
-    if (FULL || (need & 1)) acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-    if (FULL || (need & 2)) acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-    if (FULL || (need & 4)) acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-    if (FULL || (need & 8)) acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-  }
-}
-
-// acc += sgn * A * B over one segment, FP64 MFMA.  Each thread owns 4 A and
-// 4 B elements of every slab at fixed (row, k-in-slab) positions, kept as
-// 32-bit offsets from the segment base that advance by one slab per step.
-// Loads are issued unconditionally (an out-of-range element reads offset 0,
-// the segment's first element) and the in-range flags are applied, with the
-// sign, only when the slab is written to LDS after the current slab's MFMAs,
-// so the next slab's loads stay in flight meanwhile.
-template <bool A_KMAJOR, bool FULL>
-__device__ void seg_f64(const SegDesc &sgd, double sgn, int M, const double *__restrict__ A,
-                        const double *__restrict__ B, int m0, int n0, GemmSmem &S, double4_t acc[2][2],
-                        unsigned need) {
-  const int K = sgd.K, lda = sgd.lda, ldb = sgd.ldb;
-  const int nk = (K + GK - 1) / GK;
-  if (nk == 0) return;
-  const int tid = threadIdx.x;
-  int aoff[GJ], boff[GJ], akk[GJ], bkk[GJ];
-  unsigned rowok = 0;  // bits 0..GJ-1: A rows in range, bits 16..: B columns in range
-  if (A_KMAJOR) {
-    const int m = m0 + (tid & 63);
-    const bool mv = m < M;
-#pragma unroll
-    for (int j = 0; j < GJ; j++) {
-      akk[j] = (tid >> 6) + 4 * j;
-      aoff[j] = akk[j] * lda + (mv ? m : 0);
-      rowok |= (unsigned)mv << j;
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < GJ; j++) {
-      const int m = m0 + tid / GK + (256 / GK) * j;
-      const bool mv = m < M;
-      akk[j] = tid % GK;
-      aoff[j] = (mv ? m : 0) * lda + akk[j];
-      rowok |= (unsigned)mv << j;
-    }
-  }
-  {
-    const int n = n0 + (tid & 63);
-    const bool nv = n < M;
-#pragma unroll
-    for (int j = 0; j < GJ; j++) {
-      bkk[j] = (tid >> 6) + 4 * j;
-      boff[j] = bkk[j] * ldb + (nv ? n : 0);
-      rowok |= (unsigned)nv << (16 + j);
-    }
-  }
-  const int ainc = A_KMAJOR ? GK * lda : GK, binc = GK * ldb;
-  // two register sets: the loads of slab kt+2 are issued while slab kt is
-  // multiplied, so each load has two slabs of MFMA work to arrive in
-  double ra0[GJ], rb0[GJ], ra1[GJ], rb1[GJ];
-  unsigned ok0 = 0, ok1 = 0;
-  // FULL tiles have every row and column in range, so a slab that lies
-  // wholly inside K (all but a partial last one) is loaded and stored
-  // without checks; the test is on scalars, one branch per slab.
-  auto load = [&](int k0, double (&ra)[GJ], double (&rb)[GJ], unsigned &ok) {
-    if (FULL && k0 + GK <= K) {
-#pragma unroll
-      for (int j = 0; j < GJ; j++) {
-        ra[j] = A[aoff[j]];
-        rb[j] = B[boff[j]];
-        aoff[j] += ainc;
-        boff[j] += binc;
-      }
-      return;
-    }
-    ok = 0;
-#pragma unroll
-    for (int j = 0; j < GJ; j++) {
-      const bool ga = ((rowok >> j) & 1) && (k0 + akk[j] < K);
-      const bool gb = ((rowok >> (16 + j)) & 1) && (k0 + bkk[j] < K);
-      ra[j] = A[ga ? aoff[j] : 0];
-      rb[j] = B[gb ? boff[j] : 0];
-      ok |= ((unsigned)ga << j) | ((unsigned)gb << (16 + j));
-      aoff[j] += ainc;
-      boff[j] += binc;
-    }
-  };
-  auto store = [&](int buf, const double (&ra)[GJ], const double (&rb)[GJ], unsigned ok, int k0) {
-    if (FULL && k0 + GK <= K) {
-#pragma unroll
-      for (int j = 0; j < GJ; j++) {
-        if (A_KMAJOR) S.A[buf][(tid >> 6) + 4 * j][tid & 63] = ra[j];
-        else S.A[buf][tid % GK][tid / GK + (256 / GK) * j] = ra[j];
-        S.B[buf][(tid >> 6) + 4 * j][tid & 63] = sgn * rb[j];
-      }
-      return;
-    }
-#pragma unroll
-    for (int j = 0; j < GJ; j++) {
-      const double a = ((ok >> j) & 1) ? ra[j] : 0.0;
-      const double b = ((ok >> (16 + j)) & 1) ? sgn * rb[j] : 0.0;
-      if (A_KMAJOR) S.A[buf][(tid >> 6) + 4 * j][tid & 63] = a;
-      else S.A[buf][tid % GK][tid / GK + (256 / GK) * j] = a;
-      S.B[buf][(tid >> 6) + 4 * j][tid & 63] = b;
-    }
-  };
-#if IMSRG_GEMM_PF == 2
-  load(0, ra0, rb0, ok0);
-  store(0, ra0, rb0, ok0, 0);
-  if (nk > 1) load(GK, ra1, rb1, ok1);
-  __syncthreads();
-  for (int kt = 0; kt < nk; kt += 2) {
-    // slab kt in LDS 0, slab kt+1 in registers 1, registers 0 free
-    if (kt + 2 < nk) load((kt + 2) * GK, ra0, rb0, ok0);
-    if (need) slab_mfma<FULL>(S, 0, acc, need);
-    if (kt + 1 < nk) store(1, ra1, rb1, ok1, (kt + 1) * GK);
-    __syncthreads();
-    if (kt + 1 >= nk) break;
-    // slab kt+1 in LDS 1, slab kt+2 in registers 0, registers 1 free
-    if (kt + 3 < nk) load((kt + 3) * GK, ra1, rb1, ok1);
-    if (need) slab_mfma<FULL>(S, 1, acc, need);
-    if (kt + 2 < nk) store(0, ra0, rb0, ok0, (kt + 2) * GK);
-    __syncthreads();
-  }
-#else
-  (void)ra1;
-  (void)rb1;
-  (void)ok1;
-  load(0, ra0, rb0, ok0);
-  store(0, ra0, rb0, ok0, 0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; kt++) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < nk;
-    if (more) load((kt + 1) * GK, ra0, rb0, ok0);
-    if (need) slab_mfma<FULL>(S, cur, acc, need);
-    if (more) store(cur ^ 1, ra0, rb0, ok0, (kt + 1) * GK);
-    __syncthreads();
-  }
-#endif
-}
-
-// local (row, col) of accumulator element (ti, tj, v) of this lane.
-// D[i][j] has j = lane%16 and, for v_mfma_f64_16x16x4, i = lane/16 + 4v; for
-// v_mfma_f32_16x16x4f32 and v_mfma_f32_16x16x32_bf16, i = 4*(lane/16) + v.
-template <int MODE>
+// local (row, col) of accumulator element (ti, tj, v) of this lane in a 64 x 64
+// tile of 32 x 32 quadrants: D[i][j] of v_mfma_f32_16x16x4f32 and
+// v_mfma_f32_16x16x32_bf16 has i = 4*(lane/16) + v, j = lane%16.
 __device__ __forceinline__ int acc_row(int ti, int v) {
   const int g = (threadIdx.x & 63) >> 4;
-  return ((threadIdx.x >> 6) >> 1) * 32 + ti * 16 + (MODE == 0 ? g + 4 * v : 4 * g + v);
+  return ((threadIdx.x >> 6) >> 1) * 32 + ti * 16 + 4 * g + v;
 }
 __device__ __forceinline__ int acc_col(int tj) {
   return ((threadIdx.x >> 6) & 1) * 32 + tj * 16 + (threadIdx.x & 15);
 }
-
 
 // ---- split-precision segments: the same 64x64 tile and 2x2 quadrant layout;
 // products accumulate in FP32 inside one K slab and in FP64 across slabs.
@@ -448,17 +274,16 @@ __device__ void seg_bf16(const SegDesc &sg, double sgn, int M, const double *__r
   }
 }
 
-template <bool A_KMAJOR, int MODE, bool FULL>
+template <bool A_KMAJOR, int MODE>
 __device__ __forceinline__ void run_segments(const SegProb &p, int s0, int s1, const double *X0,
                                              const double *X1, double g0, double g1, int m0, int n0,
-                                             GemmSmem &S, double4_t acc[2][2], unsigned need) {
+                                             double4_t acc[2][2], unsigned need) {
   for (int s = s0; s < s1; s++) {
     const SegDesc &sg = p.seg[s];
     const double *A = (sg.src ? X1 : X0) + sg.a_off;
     const double *B = (sg.src ? X0 : X1) + sg.b_off;
     const double sgn = sg.sign * (sg.src ? g1 : g0);
-    if constexpr (MODE == 0) seg_f64<A_KMAJOR, FULL>(sg, sgn, p.M, A, B, m0, n0, S, acc, need);
-    else if constexpr (MODE == 1) seg_s32<A_KMAJOR>(sg, sgn, p.M, A, B, m0, n0, acc, need);
+    if constexpr (MODE == 1) seg_s32<A_KMAJOR>(sg, sgn, p.M, A, B, m0, n0, acc, need);
     else seg_bf16<A_KMAJOR>(sg, sgn, p.M, A, B, m0, n0, acc, need);
   }
 }
@@ -467,10 +292,10 @@ __device__ __forceinline__ void run_segments(const SegProb &p, int s0, int s1, c
 //   after the first nmid segments is also stored to W (upper triangle).
 // EPI 1 (Pandya product): Z = acc on the whole tile and sigma * acc^T on the
 //   mirrored tile, both written row-contiguously through an LDS transpose.
-template <bool A_KMAJOR, int MODE, int EPI, bool FULL>
+template <bool A_KMAJOR, int MODE, int EPI>
 __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const double *X0, const double *X1,
                                          double g0, double g1, double *C, double *W, double sigma,
-                                         unsigned need, GemmSmem &S) {
+                                         unsigned need) {
   const int M = p.M;
   const bool active = need != 0;
   double4_t acc[2][2];
@@ -479,7 +304,7 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = (double4_t){0.0, 0.0, 0.0, 0.0};
   if (EPI == 0) {
-    run_segments<A_KMAJOR, MODE, FULL>(p, 0, p.nmid, X0, X1, g0, g1, m0, n0, S, acc, need);
+    run_segments<A_KMAJOR, MODE>(p, 0, p.nmid, X0, X1, g0, g1, m0, n0, acc, need);
     if (W && active) {
       double *Wp = W + p.w_off;
 #pragma unroll
@@ -488,11 +313,11 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
         for (int tj = 0; tj < 2; tj++)
 #pragma unroll
           for (int v = 0; v < 4; v++) {
-            const int row = m0 + acc_row<MODE>(ti, v), col = n0 + acc_col(tj);
+            const int row = m0 + acc_row(ti, v), col = n0 + acc_col(tj);
             if (row < M && col < M && row <= col) Wp[(long long)row * M + col] = acc[ti][tj][v];
           }
     }
-    run_segments<A_KMAJOR, MODE, FULL>(p, p.nmid, p.nseg, X0, X1, g0, g1, m0, n0, S, acc, need);
+    run_segments<A_KMAJOR, MODE>(p, p.nmid, p.nseg, X0, X1, g0, g1, m0, n0, acc, need);
     if (C && active) {
       // every old value of C first (element 0 outside the upper triangle),
       // so the loads are in flight together, then the stores
@@ -504,7 +329,7 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
         for (int tj = 0; tj < 2; tj++)
 #pragma unroll
           for (int v = 0; v < 4; v++) {
-            const int row = m0 + acc_row<MODE>(ti, v), col = n0 + acc_col(tj);
+            const int row = m0 + acc_row(ti, v), col = n0 + acc_col(tj);
             old[ti][tj][v] = Cp[(row < M && col < M && row <= col) ? (long long)row * M + col : 0];
           }
 #pragma unroll
@@ -513,12 +338,12 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
         for (int tj = 0; tj < 2; tj++)
 #pragma unroll
           for (int v = 0; v < 4; v++) {
-            const int row = m0 + acc_row<MODE>(ti, v), col = n0 + acc_col(tj);
+            const int row = m0 + acc_row(ti, v), col = n0 + acc_col(tj);
             if (row < M && col < M && row <= col) Cp[(long long)row * M + col] = old[ti][tj][v] + acc[ti][tj][v];
           }
     }
   } else {
-    run_segments<A_KMAJOR, MODE, FULL>(p, 0, p.nseg, X0, X1, g0, g1, m0, n0, S, acc, need);
+    run_segments<A_KMAJOR, MODE>(p, 0, p.nseg, X0, X1, g0, g1, m0, n0, acc, need);
     // Z in 2x2 blocks, upper blocks only: every computed element on or above
     // the diagonal directly, and the strictly lower element of a diagonal block
     // as sigma * its mirror
@@ -530,7 +355,7 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
         for (int tj = 0; tj < 2; tj++)
 #pragma unroll
           for (int v = 0; v < 4; v++) {
-            const int row = m0 + acc_row<MODE>(ti, v), col = n0 + acc_col(tj);
+            const int row = m0 + acc_row(ti, v), col = n0 + acc_col(tj);
             if (row < M && col < M && row <= col) {
               Zp[zidx(row, col, M)] = acc[ti][tj][v];
               if (row < col && (row >> 1) == (col >> 1)) Zp[zidx(col, row, M)] = sigma * acc[ti][tj][v];
@@ -540,17 +365,31 @@ __device__ __forceinline__ void seg_tile(const SegProb &p, int m0, int n0, const
   }
 }
 
-// one workgroup's tile `tl` (operands of the instance)
 template <bool A_KMAJOR, int MODE, int EPI>
-__device__ __forceinline__ void seg_block(const SegProb *__restrict__ probs, const int4 tl,
-                                          const double *__restrict__ X0, const double *__restrict__ X1, double g0,
-                                          double g1, double *__restrict__ C, double *__restrict__ W, double sigma,
-                                          GemmSmem &S) {
+__global__ __launch_bounds__(256) void k_seg_gemm(const SegProb *__restrict__ probs, const int4 *__restrict__ tiles,
+                                                  int ntiles, const double *__restrict__ X0,
+                                                  const double *__restrict__ X1, double g0, double g1,
+                                                  double *__restrict__ C, double *__restrict__ W,
+                                                  double sigma, const int *act, long long sx,
+                                                  long long sc, long long sw) {
+  const int t = blockIdx.x;
+  if (t >= ntiles) return;
+  {
+    const long long inst = inst_id(act);
+    if (inst < 0) return;
+    X0 += inst * sx;
+    X1 += inst * sx;
+    if (C) C += inst * sc;
+    if (W) W += inst * sw;
+  }
+  const int4 tl = tiles[t];
   if (tl.x < 0) return;  // padding slot of the XCD-balanced schedule
   const SegProb &p = probs[tl.x];
   const int m0 = tl.y * GT, n0 = tl.z * GT, M = p.M;
   const bool diag = tl.y == tl.z;
   const int wave = threadIdx.x >> 6;
+  // `need` bit (2*ti + tj): the 16x16 sub-tile holds outputs that are used
+  // (inside the block and not strictly below the diagonal)
   unsigned need = 0;
 #pragma unroll
   for (int ti = 0; ti < 2; ti++)
@@ -560,27 +399,7 @@ __device__ __forceinline__ void seg_block(const SegProb *__restrict__ probs, con
       if (r16 < M && c16 < M && !(diag && r16 > c16)) need |= 1u << (2 * ti + tj);
     }
   need = __builtin_amdgcn_readfirstlane(need);  // uniform per wavefront
-  // workgroup-uniform choice: an off-diagonal tile inside the block needs every sub-tile
-  if (MODE == 0 && !diag && m0 + GT <= M && n0 + GT <= M)
-    seg_tile<A_KMAJOR, MODE, EPI, true>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
-  else
-    seg_tile<A_KMAJOR, MODE, EPI, false>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
-}
-template <bool A_KMAJOR, int MODE, int EPI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ? 4 : 1))) void k_seg_gemm(const SegProb *__restrict__ probs,
-                                                  const int4 *__restrict__ tiles, int ntiles,
-                                                  const double *__restrict__ X0,
-                                                  const double *__restrict__ X1, double g0, double g1,
-                                                  double *__restrict__ C, double *__restrict__ W,
-                                                  double sigma, const int *act, long long sx,
-                                                  long long sc, long long sw) {
-  const int t = blockIdx.x;
-  if (t >= ntiles) return;
-  const long long inst = inst_id(act);
-  if (inst < 0) return;
-  __shared__ GemmSmem S;
-  seg_block<A_KMAJOR, MODE, EPI>(probs, tiles[t], X0 + inst * sx, X1 + inst * sx, g0, g1, C ? C + inst * sc : nullptr,
-                                 W ? W + inst * sw : nullptr, sigma, S);
+  seg_tile<A_KMAJOR, MODE, EPI>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need);
 }
 
 // ---- FP64 path on 128 x 64 tiles: 4 wavefronts, each 32 rows x 64 columns
@@ -590,12 +409,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 ?
 // above the diagonal are not launched.  Writes: direct for row <= col, and
 // (EPI 1) mirrored sigma * value for row < col, which covers every element of
 // Z exactly once whatever the tile shape.
-constexpr int WM = 128, WN = 64;
+constexpr int WM = 128, WN = 64, GK = 16, GP = 1;
 struct GemmSmemW {
   double A[2][GK][WM + GP];
   double B[2][GK][WN + GP];
 };
-static_assert(sizeof(GemmSmemW) >= sizeof(double) * 64 * (64 + GP), "transpose buffer must fit");
 
 template <bool FULL>
 __device__ __forceinline__ void slab_mfma_w(const GemmSmemW &S, int buf, double4_t acc[2][4], unsigned need) {
@@ -815,6 +633,257 @@ __global__ __launch_bounds__(256) void k_seg_gemm_w(const SegProb *__restrict__ 
     seg_tile_w<A_KMAJOR, EPI, false>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
 }
 
+// ---- FP64 products, one 32 x 32 output tile per wavefront, operands straight
+// from L1/L2 into registers: no LDS staging, no barriers.  The segments come in
+// pairs over one K range, X0 X1 and X1 X0; a K chunk of 8 of a pair is eight
+// 16-byte loads a lane and 16 v_mfma_f64_16x16x4 (1024 matrix-core cycles).
+// The loop body is straight-line (every load made, clamped past the range), so
+// the next chunk's loads stay in flight under this chunk's products, and four
+// wavefronts share a SIMD.  A lane's 16 bytes are two neighbours of a K row of
+// B (and of A when A is K-major): the tile's even and odd columns (rows) are
+// its two 16-wide sub-tiles; or, for a row-major A, two neighbouring k of one
+// row, with the K rows of B taken in the same order (k = 2 g + t in step t).
+// Rows and columns past M are read clamped and never stored; k past the range
+// is zeroed on both sides.  M is the leading dimension of every operand.
+// NW = 4: the four wavefronts of a workgroup share one tile, each taking every
+// fourth K chunk, and add their sums through LDS: a tile's K chain is a quarter
+// as long, which is the time in small bases and the tail of the schedule in
+// large ones.  Measured alone, in us (64 x 64 tiles of LDS slabs, the form
+// before / a quadrant a wavefront / four wavefronts a tile): pp/hh emax 4 17 / - / 7,
+// emax 6 43 / 25 / 20, 16 x emax 6 233 / 263 / 240, emax 7 73 / 55 / 47, emax 8
+// 168 / 162 / 149 (36 TF/s); Pandya product emax 4 9.6 / 7.5 / 5.0, emax 6
+// 20.5 / 15.9 / 18.0, 16 x emax 6 202 / 162 / 221, emax 8 177 / 147 (44 TF/s) / 165.
+// Hence pp/hh always shares, the Pandya product while the basis' two-body part
+// holds at most 3e5 elements (emax 5); the choice is the basis', so a batch has
+// its instances' bits.
+struct WFrag {
+  dpair_t a[2][2], b[2][2];  // [segment of the pair][A: sub-tile or step, B: step]
+};
+template <bool Z, int NW>
+__device__ __forceinline__ void wave_pair(const SegDesc &d0, const SegDesc &d1, int M, const double *__restrict__ X0,
+                                          const double *__restrict__ X1, double g0, double g1, int m0, int n0, int w,
+                                          double4_t acc[2][2]) {
+  const int K = d0.K, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  if (8 * w >= K) return;
+  const double sg0 = d0.sign * g0, sg1 = d1.sign * g1;
+  const double *A0 = X0 + d0.a_off, *B0 = X1 + d0.b_off, *A1 = X1 + d1.a_off, *B1 = X0 + d1.b_off;
+  // columns 2c, 2c + 1 of the tile (an odd M's last column is read with the
+  // element after it, which the block's padding or next row holds)
+  const int nc = n0 + 2 * c < M ? n0 + 2 * c : 0;
+  const int mc = Z ? (m0 + 2 * c < M ? m0 + 2 * c : 0) : 0;
+  const int r0 = Z ? 0 : min(m0 + c, M - 1) * M, r1 = Z ? 0 : min(m0 + 16 + c, M - 1) * M;
+  auto fetch = [&](WFrag &f, int k) {
+    if (Z) {
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        const int o = min(k + 4 * t + g, K - 1) * M;
+        f.a[0][t] = *(const dpair_t *)(A0 + (o + mc));
+        f.b[0][t] = *(const dpair_t *)(B0 + (o + nc));
+        f.a[1][t] = *(const dpair_t *)(A1 + (o + mc));
+        f.b[1][t] = *(const dpair_t *)(B1 + (o + nc));
+      }
+    } else {
+      // (a pair whose second k is past the range reads the element after it)
+      const int kp = min(k + 2 * g, K - 1);
+      f.a[0][0] = *(const dpair_t *)(A0 + (r0 + kp));
+      f.a[0][1] = *(const dpair_t *)(A0 + (r1 + kp));
+      f.a[1][0] = *(const dpair_t *)(A1 + (r0 + kp));
+      f.a[1][1] = *(const dpair_t *)(A1 + (r1 + kp));
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        const int o = min(k + 2 * g + t, K - 1) * M + nc;
+        f.b[0][t] = *(const dpair_t *)(B0 + o);
+        f.b[1][t] = *(const dpair_t *)(B1 + o);
+      }
+    }
+  };
+  auto product = [&](WFrag &f, int k) {
+    if (K - k < 8) {
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+        if (k + (Z ? 4 * t + g : 2 * g + t) >= K) {
+#pragma unroll
+          for (int q = 0; q < 2; q++) {
+            f.b[q][t] = (dpair_t){0.0, 0.0};
+            if (Z) f.a[q][t] = (dpair_t){0.0, 0.0};
+            else f.a[q][0][t] = f.a[q][1][t] = 0.0;
+          }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      f.a[q][0] *= q ? sg1 : sg0;
+      f.a[q][1] *= q ? sg1 : sg0;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int ti = 0; ti < 2; ti++)
+#pragma unroll
+          for (int tj = 0; tj < 2; tj++)
+            acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(Z ? f.a[q][t][ti] : f.a[q][ti][t], f.b[q][t][tj],
+                                                               acc[ti][tj], 0, 0, 0);
+    }
+  };
+  constexpr int S = 8 * NW;
+  WFrag f0, f1;
+  fetch(f0, 8 * w);
+  for (int k = 8 * w; k < K; k += 2 * S) {
+    fetch(f1, k + S);
+    product(f0, k);
+    if (k + S >= K) break;
+    fetch(f0, k + 2 * S);
+    product(f1, k + S);
+  }
+}
+// segments [s0, s1) of a problem, which are pairs
+template <bool Z, int NW>
+__device__ __forceinline__ void wave_segments(const SegProb &p, int s0, int s1, const double *__restrict__ X0,
+                                              const double *__restrict__ X1, double g0, double g1, int m0, int n0,
+                                              int w, double4_t acc[2][2]) {
+  for (int s = s0; s < s1; s += 2)
+    wave_pair<Z, NW>(p.seg[s], p.seg[s + 1], p.M, X0, X1, g0, g1, m0, n0, w, acc);
+}
+// Z tile: a lane's four sums of one v are one 2x2 block (32 bytes), upper blocks
+// only; the strictly lower element of a diagonal block is sigma * its mirror
+__device__ __forceinline__ void z_block(double *__restrict__ Zp, int M, int u, int w, double z00, double z01,
+                                        double z10, double z11, double sigma) {
+  if (2 * u >= M || 2 * w >= M || u > w) return;
+  double *q = Zp + ((long long)u * (M >> 1) + w) * 4;
+  if (u == w) z10 = sigma * z01;
+  *(double2 *)q = make_double2(z00, z11);
+  *(double2 *)(q + 2) = make_double2(z01, z10);
+}
+// The Pandya product on a 64 x 64 tile list, a 32 x 32 quadrant per wavefront
+// (accumulator element (ti, tj, v): row 2 (lane/16 + 4 v) + ti, column 2 (lane%16) + tj)
+__device__ __forceinline__ void wave_tile_z(const SegProb *__restrict__ probs, const int4 tl,
+                                            const double *__restrict__ X0, const double *__restrict__ X1, double g0,
+                                            double g1, double *__restrict__ C, double sigma) {
+  if (tl.x < 0) return;  // padding slot of the XCD-balanced schedule
+  const SegProb &p = probs[tl.x];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), M = p.M;
+  const int m0 = tl.y * 64 + 32 * (wave >> 1), n0 = tl.z * 64 + 32 * (wave & 1);
+  if (m0 >= M || n0 >= M || m0 > n0) return;
+  double4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  wave_segments<true, 1>(p, 0, p.nseg, X0, X1, g0, g1, m0, n0, 0, acc);
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    z_block(C + p.c_off, M, (m0 >> 1) + (lane >> 4) + 4 * v, (n0 >> 1) + (lane & 15), acc[0][0][v], acc[0][1][v],
+            acc[1][0][v], acc[1][1][v], sigma);
+}
+// Either product on a 32 x 32 tile list, four wavefronts to a tile (row-major A:
+// element (ti, tj, v) at row 16 ti + lane/16 + 4 v).  The partial sums lie in LDS as [wavefront][row][column]; thread t adds and writes the 2x2
+// block (t/16, t%16).
+struct SplitSmem {
+  double s[4][32][34];
+};
+template <bool Z>
+__device__ __forceinline__ void split_tile(const SegProb *__restrict__ probs, const int4 tl,
+                                           const double *__restrict__ X0, const double *__restrict__ X1, double g0,
+                                           double g1, double *__restrict__ C, double *__restrict__ W, double sigma,
+                                           SplitSmem &S) {
+  if (tl.x < 0) return;
+  const SegProb &p = probs[tl.x];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), M = p.M, lane = threadIdx.x & 63;
+  const int m0 = tl.y * 32, n0 = tl.z * 32, u = threadIdx.x >> 4, w = threadIdx.x & 15;
+  double4_t acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  double z[2][2];
+  auto reduce = [&]() {
+    __syncthreads();
+#pragma unroll
+    for (int ti = 0; ti < 2; ti++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int i = (lane >> 4) + 4 * v;
+        *(double2 *)&S.s[wave][Z ? 2 * i + ti : 16 * ti + i][2 * (lane & 15)] =
+            make_double2(acc[ti][0][v], acc[ti][1][v]);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      double2 x = *(const double2 *)&S.s[0][2 * u + i][2 * w];
+#pragma unroll
+      for (int k = 1; k < 4; k++) {
+        const double2 y = *(const double2 *)&S.s[k][2 * u + i][2 * w];
+        x.x += y.x;
+        x.y += y.y;
+      }
+      z[i][0] = x.x;
+      z[i][1] = x.y;
+    }
+  };
+  const int row = m0 + 2 * u, col = n0 + 2 * w;
+  if (Z) {
+    wave_segments<true, 4>(p, 0, p.nseg, X0, X1, g0, g1, m0, n0, wave, acc);
+    reduce();
+    z_block(C + p.c_off, M, row >> 1, col >> 1, z[0][0], z[0][1], z[1][0], z[1][1], sigma);
+    return;
+  }
+  double old[2][2];
+  if (C) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        old[i][j] = C[p.c_off + (row + i < M && col + j < M && row + i <= col + j ? (long long)(row + i) * M + col + j : 0)];
+  }
+  wave_segments<false, 4>(p, 0, p.nmid, X0, X1, g0, g1, m0, n0, wave, acc);
+  if (W) {
+    reduce();
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        if (row + i < M && col + j < M && row + i <= col + j) W[p.w_off + (long long)(row + i) * M + col + j] = z[i][j];
+  }
+  wave_segments<false, 4>(p, p.nmid, p.nseg, X0, X1, g0, g1, m0, n0, wave, acc);
+  if (C) {
+    reduce();
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        if (row + i < M && col + j < M && row + i <= col + j)
+          C[p.c_off + (long long)(row + i) * M + col + j] = old[i][j] + z[i][j];
+  }
+}
+// SPLIT: 32 x 32 tiles, four wavefronts each; else 64 x 64 tiles, a quadrant a wavefront
+template <bool Z, bool SPLIT>
+__device__ __forceinline__ void gemm_tile(const SegProb *__restrict__ probs, const int4 tl,
+                                          const double *__restrict__ X0, const double *__restrict__ X1, double g0,
+                                          double g1, double *__restrict__ C, double *__restrict__ W, double sigma,
+                                          SplitSmem *S) {
+  if constexpr (SPLIT) {
+    split_tile<Z>(probs, tl, X0, X1, g0, g1, C, W, sigma, *S);
+  } else {
+    static_assert(Z, "64 x 64 tiles: the Pandya product");
+    wave_tile_z(probs, tl, X0, X1, g0, g1, C, sigma);
+  }
+}
+template <bool Z, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_wave_gemm(
+    const SegProb *__restrict__ probs, const int4 *__restrict__ tiles, const double *__restrict__ X0,
+    const double *__restrict__ X1, double g0, double g1, double *__restrict__ C, double *__restrict__ W, double sigma,
+    const int *act, long long sx, long long sc, long long sw) {
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  const int4 tl = tiles[blockIdx.x];
+  X0 += inst * sx;
+  X1 += inst * sx;
+  if (C) C += inst * sc;
+  if (W) W += inst * sw;
+  __shared__ __align__(16) double sm[SPLIT ? sizeof(SplitSmem) / sizeof(double) : 1];
+  gemm_tile<Z, SPLIT>(probs, tl, X0, X1, g0, g1, C, W, sigma, reinterpret_cast<SplitSmem *>(sm));
+}
+
 void launch_seg_gemm_pphh(hipStream_t s, int mode, const SegProb *probs, const int4 *tiles, int ntiles,
                           const double *X0, const double *X1, double *C, double *W, const int *act, int nact,
                           long long sop, long long sw) {
@@ -832,8 +901,7 @@ void launch_seg_gemm_pphh(hipStream_t s, int mode, const SegProb *probs, const i
     launch_k(k_seg_gemm<false, 2, 0>, g, b, 0, s, probs, tiles, ntiles, X0, X1, 1.0, 1.0, C, W, 0.0,
                        act, sop, sop, sw);
   else
-    launch_k(k_seg_gemm<false, 0, 0>, g, b, 0, s, probs, tiles, ntiles, X0, X1, 1.0, 1.0, C, W, 0.0,
-                       act, sop, sop, sw);
+    launch_k(k_wave_gemm<false, true>, g, b, 0, s, probs, tiles, X0, X1, 1.0, 1.0, C, W, 0.0, act, sop, sop, sw);
 }
 void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4 *tiles, int ntiles,
                        const double *LCC, const double *RCC, double *Z, double hL, double hR, const int *act,
@@ -846,6 +914,10 @@ void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4
                        act, scc, sz, 0LL);
     return;
   }
+  if (mode == 4) {
+    launch_k(k_wave_gemm<true, true>, g, b, 0, s, probs, tiles, LCC, RCC, g0, g1, Z, nullptr, sigma, act, scc, sz, 0LL);
+    return;
+  }
   if (mode == 1)
     launch_k(k_seg_gemm<true, 1, 1>, g, b, 0, s, probs, tiles, ntiles, LCC, RCC, g0, g1, Z, nullptr,
                        sigma, act, scc, sz, 0LL);
@@ -853,8 +925,7 @@ void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4
     launch_k(k_seg_gemm<true, 2, 1>, g, b, 0, s, probs, tiles, ntiles, LCC, RCC, g0, g1, Z, nullptr,
                        sigma, act, scc, sz, 0LL);
   else
-    launch_k(k_seg_gemm<true, 0, 1>, g, b, 0, s, probs, tiles, ntiles, LCC, RCC, g0, g1, Z, nullptr,
-                       sigma, act, scc, sz, 0LL);
+    launch_k(k_wave_gemm<true, false>, g, b, 0, s, probs, tiles, LCC, RCC, g0, g1, Z, nullptr, sigma, act, scc, sz, 0LL);
 }
 
 // ------------------------------------------------------------------ Pandya transform
@@ -2238,22 +2309,23 @@ __global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ L
   e0_part(L, Lop, Rop, A.hL, A.hR, A.partials + inst * kPartials, b - nw, A.nsplit, lds);
 }
 
+template <bool SPLIT>  // of the Pandya product
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_small_b(
     const DevLayout *__restrict__ Lp, SmallArgs A) {
-  __shared__ GemmSmem S;
+  __shared__ SplitSmem S;
   const DevLayout &L = *Lp;
   const long long inst = inst_id(A.act);
   if (inst < 0) return;
   const int b = blockIdx.x;
   if (b < A.n_pp) {
     const long long o = inst * L.op_size + L.v_off;
-    seg_block<false, 0, 0>(A.pp_probs, A.pp_tiles[b], A.Lop + o, A.Rop + o, 1.0, 1.0, A.RES + o,
-                           A.wpp + inst * L.vsize, 0.0, S);
+    split_tile<false>(A.pp_probs, A.pp_tiles[b], A.Lop + o, A.Rop + o, 1.0, 1.0, A.RES + o, A.wpp + inst * L.vsize,
+                      0.0, S);
   } else {
     const long long o = inst * L.ccsize;
     const double hL = A.hL, hR = A.hR;
-    seg_block<true, 0, 1>(A.ph_probs, A.ph_tiles[b - A.n_pp], A.ccL + o, A.ccR + o, hL, -hR, A.Z + inst * L.cwsize,
-                          nullptr, -hL * hR, S);
+    gemm_tile<true, SPLIT>(A.ph_probs, A.ph_tiles[b - A.n_pp], A.ccL + o, A.ccR + o, hL, -hR, A.Z + inst * L.cwsize,
+                           nullptr, -hL * hR, &S);
   }
 }
 
@@ -2451,7 +2523,8 @@ void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallA
   const int na = L.nccol * (A.prepL ? 2 : 1) + (L.n122_items + 3) / 4 + ne0;
   const size_t lds = std::max(pandya_lds_bytes(L), 256 * sizeof(double));
   hipLaunchKernelGGL(k_small_a, dim3(na, nact), dim3(256), lds, s, Ld, A);
-  hipLaunchKernelGGL(k_small_b, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
+  if (A.split) hipLaunchKernelGGL(k_small_b<true>, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
+  else hipLaunchKernelGGL(k_small_b<false>, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
   hipLaunchKernelGGL(k_small_c, dim3(A.n16 + L.nsame + (A.n_diff + 3) / 4 + 1, nact), dim3(256), 0, s, Ld, A);
 }
 }  // namespace imsrg
