@@ -84,7 +84,8 @@ struct PhChunk {
   long long dbase;  // ph_desc index of the first output
   int n;            // outputs, 1..64
   int b0, len;      // the row key's packed 6j list (ap6_val) start and length
-  int half;         // 1 when i == j (the outputs carry 1/sqrt 2)
+  short half;       // 1 when i == j (the outputs carry 1/sqrt 2)
+  short diag;       // 1 when the first output is the row's diagonal element
   long long tbase;  // the row's first J' term: descriptors hold term offsets relative to it
 };
 
@@ -206,6 +207,7 @@ void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4
 void launch_pandya(hipStream_t s, const DevLayout &L, const double *op, double *cc, const int *act, int nact);
 size_t pandya_lds_bytes(const DevLayout &L);  // per-workgroup LDS of the Pandya kernel
 hipError_t pandya_allow_lds(size_t bytes);
+hipError_t adjoint_allow_lds(size_t bytes);
 // 122: M = A_L R - A_R L over whole channel blocks (diagonal symmetrised);
 // launch_sym_mirror later forms RES = M + herm*M^T
 void launch_122(hipStream_t s, const DevLayout &L, const double *Lop, const double *Rop, double *RES,
@@ -324,20 +326,21 @@ struct SmallArgs {
 void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallArgs A, int nact);
 
 // ---- adjoint commutator (adjoint.hip): Ybar += d<C,[P,Y]>/dY term by term
-void launch_adj_e0(hipStream_t s, const DevLayout &L, const double *P, const double *C, double *Y, int hP, int hY,
-                   unsigned mask);
-void launch_adj_onebody(hipStream_t s, const DevLayout &L, const double *P, const double *C, double *Y, int hP,
-                        int hY, int hC, unsigned mask);
-void launch_adj_122(hipStream_t s, const DevLayout &L, const double *P, const double *C, double *Y, int hC);
-void launch_adj_pphh(hipStream_t s, const DevLayout &L, const double *Q, double *Y, int hP, int hC);
-void launch_adj_ph_apply(hipStream_t s, const DevLayout &L, const double *C, double *Tbar, int hC);
-void launch_adj_ph_terms(hipStream_t s, const DevLayout &L, const double *Tbar, double *Zbar, double sigma);
-void launch_adj_ph_sbt(hipStream_t s, const DevLayout &L, const int *ccrlen_host, double *Z, int hP, int hY);
-void launch_adj_pandya(hipStream_t s, const DevLayout &L, const double *ccb, double *Y);
+// Ybar (herm hY, projected) of one commutator's terms in mask, from P and the cotangent Cin
+struct AdjArgs {
+  const double *P, *Cin;
+  double *C, *Y;                // projected copy of Cin; result
+  double *ccP, *ccY, *Q, *T, *Z;  // Pandya of P and of Y, P C, cotangents of the J' terms and of Z
+  int hP, hY, hC;
+  unsigned mask;
+  const GemmProb *pp_probs, *ph_probs;
+  const int4 *pp_tiles, *ph_tiles, *sbt_tiles;
+  int n_pp, n_ph, n_sbt, n_chunks;
+  int ph, n_ob, n_122, n_ap, n_111, nfill;  // (launch_adjoint's)
+};
+void launch_adjoint(hipStream_t s, const DevLayout &L, AdjArgs A);
 // X <- (X + h X^T)/2 on the one-body part and every channel block; E0 <- 0 unless keep_e0
 void launch_project(hipStream_t s, const DevLayout &L, double *X, int h, int keep_e0);
-void launch_gemm_plain(hipStream_t s, const GemmProb *probs, const int4 *tiles, int ntiles, const double *A,
-                       const double *B, double *C);
 // transpose of the White (kind 0) / atan (kind 1) generator at H (mono = its
 // monopoles): Hb += d<Eb, eta(H)>/dH; mbar: nsp*nsp scratch
 void launch_adj_generator(hipStream_t s, const DevLayout &L, const double *H, const double *mono,

@@ -381,7 +381,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
       return fail(IMSRG_EINVAL, "basis too large: the Pandya kernel stages " + std::to_string(need) +
                                     " bytes of tables per workgroup (device limit " + std::to_string(lds_max) + ")");
     }
-    if (need > 65536 && pandya_allow_lds(need) != hipSuccess) {
+    if (need > 65536 && (pandya_allow_lds(need) != hipSuccess || adjoint_allow_lds(need) != hipSuccess)) {
       imsrg_ctx_destroy(c);
       return fail(IMSRG_EDEVICE, "the Pandya kernel cannot take " + std::to_string(need) + " bytes of LDS");
     }
@@ -493,11 +493,13 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
         h.b0 = Ly.ap6_base[key];
         h.len = Ly.ap6_base[key + 1] - Ly.ap6_base[key];
         h.half = i == j;
+        h.diag = s0 == rl;
         h.tbase = Ly.ph_tbase[r];
         chunks.push_back(h);
         wa.push_back(16.0 + h.n);
       }
     }
+    c->n_ph_chunks = (int)chunks.size();
     D.xs_apply = make_split(wa);
     UP(chunks, ph_chunks);
   }
@@ -631,20 +633,25 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
       if (dim == 0) continue;
       const int id = (int)pp.size();
       pp.push_back(GemmProb{dim, dim, dim, dim, dim, dim, Ly.boff[q], Ly.boff[q], Ly.boff[q]});
-      for (int i = 0; i < (dim + 63) / 64; i++)
-        for (int j = 0; j < (dim + 63) / 64; j++) tp.push_back(make_int4(id, i, j, 0));
+      for (int i = 0; i < (dim + 31) / 32; i++)
+        for (int j = 0; j < (dim + 31) / 32; j++) tp.push_back(make_int4(id, i, j, 0));
     }
+    std::vector<int4> ts;
     for (int q = 0; q < Ly.ncc; q++) {
       const int r = Ly.ccrlen[q], nbq = Ly.ccnph[q];
       if (r == 0 || nbq == 0) continue;
       const int id = (int)ph.size();
       ph.push_back(GemmProb{nbq, r, r, r, r, r, Ly.ccoff[q], Ly.cwoff[q], Ly.ccoff[q]});
-      for (int i = 0; i < (nbq + 63) / 64; i++)
-        for (int j = 0; j < (r + 63) / 64; j++) th.push_back(make_int4(id, i, j, 0));
+      for (int i = 0; i < (nbq + 31) / 32; i++)
+        for (int j = 0; j < (r + 31) / 32; j++) th.push_back(make_int4(id, i, j, 0));
+      for (int i = 0; i < (r + 31) / 32; i++)
+        for (int j = i; j < (r + 31) / 32; j++) ts.push_back(make_int4(q, i, j, 0));
     }
+    c->n_adj_sbt_tiles = (int)ts.size();
+    rc = upload_table(c, ts, (const int4 **)&c->adj_sbt_tiles);
     c->n_adj_pp_tiles = (int)tp.size();
     c->n_adj_ph_tiles = (int)th.size();
-    rc = upload_table(c, pp, (const GemmProb **)&c->adj_pp_probs);
+    if (!rc) rc = upload_table(c, pp, (const GemmProb **)&c->adj_pp_probs);
     if (!rc) rc = upload_table(c, tp, (const int4 **)&c->adj_pp_tiles);
     if (!rc) rc = upload_table(c, ph, (const GemmProb **)&c->adj_ph_probs);
     if (!rc) rc = upload_table(c, th, (const int4 **)&c->adj_ph_tiles);
@@ -1528,36 +1535,18 @@ int imsrg_commutator_222_ph_cc(imsrg_ctx c, const double *lcc, int hL, const dou
 // not depend on E0 of its operands).  <,> is the Frobenius product over the
 // full device layout.  Single-instance contexts only.
 static int adjoint_impl(imsrg_ctx_s *c, imsrg_op_s *P, imsrg_op_s *Cin, imsrg_op_s *Ybar, int hY, unsigned mask) {
-  hipStream_t s = c->stream;
-  const DevLayout &D = c->dl;
-  const Layout &Ly = c->lay;
   const int hP = P->herm, hC = -hP * hY;
   if (Cin->herm != hC) return fail(IMSRG_EINVAL, "cotangent herm must be -herm(P)*hY");
-  const ActSet all = all_set(c);
   imsrg_op_s *Ct = tmp_op(c, 5, hC);
   if (!Ct) return IMSRG_ENOMEM;
-  op_copy(Cin, Ct, all);
-  launch_project(s, D, Ct->d, hC, 1);
-  launch_fill(s, Ybar->d, Ly.op_size, 0.0);
-  if (mask & (T110 | T220)) launch_adj_e0(s, D, P->d, Ct->d, Ybar->d, hP, hY, mask);
-  launch_adj_onebody(s, D, P->d, Ct->d, Ybar->d, hP, hY, hC, mask);
-  if (mask & T122) launch_adj_122(s, D, P->d, Ct->d, Ybar->d, hC);
-  if (mask & T222PPHH) {
-    launch_gemm_plain(s, c->adj_pp_probs, c->adj_pp_tiles, c->n_adj_pp_tiles, P->d + D.v_off, Ct->d + D.v_off,
-                      c->wpp);
-    launch_adj_pphh(s, D, c->wpp, Ybar->d, hP, hC);
-  }
-  if (mask & T222PH) {
-    launch_pandya(s, D, P->d, c->cc[0], all.d, all.n());
-    launch_fill(s, c->tph, (long long)Ly.ph_terms.size(), 0.0);
-    launch_adj_ph_apply(s, D, Ct->d, c->tph, hC);
-    launch_fill(s, c->wph, Ly.cwsize, 0.0);
-    launch_adj_ph_terms(s, D, c->tph, c->wph, (double)(-hP * hY));
-    launch_adj_ph_sbt(s, D, Ly.ccrlen.data(), c->wph, hP, hY);
-    launch_gemm_plain(s, c->adj_ph_probs, c->adj_ph_tiles, c->n_adj_ph_tiles, c->cc[0], c->wph, c->cc[1]);
-    launch_adj_pandya(s, D, c->cc[1], Ybar->d);
-  }
-  launch_project(s, D, Ybar->d, hY, 0);
+  AdjArgs A{};
+  A.P = P->d; A.Cin = Cin->d; A.C = Ct->d; A.Y = Ybar->d;
+  A.ccP = c->cc[0]; A.ccY = c->cc[1]; A.Q = c->wpp; A.T = c->tph; A.Z = c->wph;
+  A.hP = hP; A.hY = hY; A.hC = hC; A.mask = mask;
+  A.pp_probs = c->adj_pp_probs; A.ph_probs = c->adj_ph_probs;
+  A.pp_tiles = c->adj_pp_tiles; A.ph_tiles = c->adj_ph_tiles; A.sbt_tiles = c->adj_sbt_tiles;
+  A.n_pp = c->n_adj_pp_tiles; A.n_ph = c->n_adj_ph_tiles; A.n_sbt = c->n_adj_sbt_tiles; A.n_chunks = c->n_ph_chunks;
+  launch_adjoint(c->stream, c->dl, A);
   Ybar->herm = hY;
   HIPCHK(hipGetLastError());
   return 0;

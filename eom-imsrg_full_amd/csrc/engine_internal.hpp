@@ -83,7 +83,9 @@ struct imsrg_ctx_s {
   SegProb *pp_probs = nullptr, *ph_probs = nullptr;
   GemmProb *adj_pp_probs = nullptr, *adj_ph_probs = nullptr;  // adjoint products
   int4 *adj_pp_tiles = nullptr, *adj_ph_tiles = nullptr;
-  int n_adj_pp_tiles = 0, n_adj_ph_tiles = 0;
+  int n_adj_pp_tiles = 0, n_adj_ph_tiles = 0;                 // 32 x 32 tiles
+  int4 *adj_sbt_tiles = nullptr;                              // 32 x 32 tile pairs of the Pandya blocks
+  int n_adj_sbt_tiles = 0, n_ph_chunks = 0;
   int4 *pp_tiles = nullptr, *ph_tiles = nullptr;        // 64 x 64 tiles
   int n_pp_tiles = 0, n_ph_tiles = 0;
   int4 *pp_tiles_w = nullptr, *ph_tiles_w = nullptr;    // 128 x 64 tiles (FP64 path)

@@ -13,7 +13,7 @@
 #include <cmath>
 
 #include "device.hpp"
-#include "devfun.hpp"
+#include "comm_dev.hpp"
 
 namespace imsrg {
 
@@ -633,116 +633,6 @@ __global__ __launch_bounds__(256) void k_seg_gemm_w(const SegProb *__restrict__ 
     seg_tile_w<A_KMAJOR, EPI, false>(p, m0, n0, X0, X1, g0, g1, C, W, sigma, need, S);
 }
 
-// ---- FP64 products, one 32 x 32 output tile per wavefront, operands straight
-// from L1/L2 into registers: no LDS staging, no barriers.  The segments come in
-// pairs over one K range, X0 X1 and X1 X0; a K chunk of 8 of a pair is eight
-// 16-byte loads a lane and 16 v_mfma_f64_16x16x4 (1024 matrix-core cycles).
-// The loop body is straight-line (every load made, clamped past the range), so
-// the next chunk's loads stay in flight under this chunk's products, and four
-// wavefronts share a SIMD.  A lane's 16 bytes are two neighbours of a K row of
-// B (and of A when A is K-major): the tile's even and odd columns (rows) are
-// its two 16-wide sub-tiles; or, for a row-major A, two neighbouring k of one
-// row, with the K rows of B taken in the same order (k = 2 g + t in step t).
-// Rows and columns past M are read clamped and never stored; k past the range
-// is zeroed on both sides.  M is the leading dimension of every operand.
-// NW = 4: the four wavefronts of a workgroup share one tile, each taking every
-// fourth K chunk, and add their sums through LDS: a tile's K chain is a quarter
-// as long, which is the time in small bases and the tail of the schedule in
-// large ones.  Measured alone, in us (64 x 64 tiles of LDS slabs, the form
-// before / a quadrant a wavefront / four wavefronts a tile): pp/hh emax 4 17 / - / 7,
-// emax 6 43 / 25 / 20, 16 x emax 6 233 / 263 / 240, emax 7 73 / 55 / 47, emax 8
-// 168 / 162 / 149 (36 TF/s); Pandya product emax 4 9.6 / 7.5 / 5.0, emax 6
-// 20.5 / 15.9 / 18.0, 16 x emax 6 202 / 162 / 221, emax 8 177 / 147 (44 TF/s) / 165.
-// Hence pp/hh always shares, the Pandya product while the basis' two-body part
-// holds at most 3e5 elements (emax 5); the choice is the basis', so a batch has
-// its instances' bits.
-struct WFrag {
-  dpair_t a[2][2], b[2][2];  // [segment of the pair][A: sub-tile or step, B: step]
-};
-template <bool Z, int NW>
-__device__ __forceinline__ void wave_pair(const SegDesc &d0, const SegDesc &d1, int M, const double *__restrict__ X0,
-                                          const double *__restrict__ X1, double g0, double g1, int m0, int n0, int w,
-                                          double4_t acc[2][2]) {
-  const int K = d0.K, lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  if (8 * w >= K) return;
-  const double sg0 = d0.sign * g0, sg1 = d1.sign * g1;
-  const double *A0 = X0 + d0.a_off, *B0 = X1 + d0.b_off, *A1 = X1 + d1.a_off, *B1 = X0 + d1.b_off;
-  // columns 2c, 2c + 1 of the tile (an odd M's last column is read with the
-  // element after it, which the block's padding or next row holds)
-  const int nc = n0 + 2 * c < M ? n0 + 2 * c : 0;
-  const int mc = Z ? (m0 + 2 * c < M ? m0 + 2 * c : 0) : 0;
-  const int r0 = Z ? 0 : min(m0 + c, M - 1) * M, r1 = Z ? 0 : min(m0 + 16 + c, M - 1) * M;
-  auto fetch = [&](WFrag &f, int k) {
-    if (Z) {
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const int o = min(k + 4 * t + g, K - 1) * M;
-        f.a[0][t] = *(const dpair_t *)(A0 + (o + mc));
-        f.b[0][t] = *(const dpair_t *)(B0 + (o + nc));
-        f.a[1][t] = *(const dpair_t *)(A1 + (o + mc));
-        f.b[1][t] = *(const dpair_t *)(B1 + (o + nc));
-      }
-    } else {
-      // (a pair whose second k is past the range reads the element after it)
-      const int kp = min(k + 2 * g, K - 1);
-      f.a[0][0] = *(const dpair_t *)(A0 + (r0 + kp));
-      f.a[0][1] = *(const dpair_t *)(A0 + (r1 + kp));
-      f.a[1][0] = *(const dpair_t *)(A1 + (r0 + kp));
-      f.a[1][1] = *(const dpair_t *)(A1 + (r1 + kp));
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        const int o = min(k + 2 * g + t, K - 1) * M + nc;
-        f.b[0][t] = *(const dpair_t *)(B0 + o);
-        f.b[1][t] = *(const dpair_t *)(B1 + o);
-      }
-    }
-  };
-  auto product = [&](WFrag &f, int k) {
-    if (K - k < 8) {
-#pragma unroll
-      for (int t = 0; t < 2; t++)
-        if (k + (Z ? 4 * t + g : 2 * g + t) >= K) {
-#pragma unroll
-          for (int q = 0; q < 2; q++) {
-            f.b[q][t] = (dpair_t){0.0, 0.0};
-            if (Z) f.a[q][t] = (dpair_t){0.0, 0.0};
-            else f.a[q][0][t] = f.a[q][1][t] = 0.0;
-          }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      f.a[q][0] *= q ? sg1 : sg0;
-      f.a[q][1] *= q ? sg1 : sg0;
-#pragma unroll
-      for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int ti = 0; ti < 2; ti++)
-#pragma unroll
-          for (int tj = 0; tj < 2; tj++)
-            acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(Z ? f.a[q][t][ti] : f.a[q][ti][t], f.b[q][t][tj],
-                                                               acc[ti][tj], 0, 0, 0);
-    }
-  };
-  constexpr int S = 8 * NW;
-  WFrag f0, f1;
-  fetch(f0, 8 * w);
-  for (int k = 8 * w; k < K; k += 2 * S) {
-    fetch(f1, k + S);
-    product(f0, k);
-    if (k + S >= K) break;
-    fetch(f0, k + 2 * S);
-    product(f1, k + S);
-  }
-}
-// segments [s0, s1) of a problem, which are pairs
-template <bool Z, int NW>
-__device__ __forceinline__ void wave_segments(const SegProb &p, int s0, int s1, const double *__restrict__ X0,
-                                              const double *__restrict__ X1, double g0, double g1, int m0, int n0,
-                                              int w, double4_t acc[2][2]) {
-  for (int s = s0; s < s1; s += 2)
-    wave_pair<Z, NW>(p.seg[s], p.seg[s + 1], p.M, X0, X1, g0, g1, m0, n0, w, acc);
-}
 // Z tile: a lane's four sums of one v are one 2x2 block (32 bytes), upper blocks
 // only; the strictly lower element of a diagonal block is sigma * its mirror
 __device__ __forceinline__ void z_block(double *__restrict__ Zp, int M, int u, int w, double z00, double z01,
@@ -778,9 +668,6 @@ __device__ __forceinline__ void wave_tile_z(const SegProb *__restrict__ probs, c
 // Either product on a 32 x 32 tile list, four wavefronts to a tile (row-major A:
 // element (ti, tj, v) at row 16 ti + lane/16 + 4 v).  The partial sums lie in LDS as [wavefront][row][column]; thread t adds and writes the 2x2
 // block (t/16, t%16).
-struct SplitSmem {
-  double s[4][32][34];
-};
 template <bool Z>
 __device__ __forceinline__ void split_tile(const SegProb *__restrict__ probs, const int4 tl,
                                            const double *__restrict__ X0, const double *__restrict__ X1, double g0,
@@ -929,139 +816,12 @@ void launch_seg_gemm_z(hipStream_t s, int mode, const SegProb *probs, const int4
 }
 
 // ------------------------------------------------------------------ Pandya transform
-// calculate_cross_coupled (cross_coupled.f90:1190-1300): one workgroup per
-// Pandya column (p,h), threads over rows (a,b); output column-major per block.
-// Everything a term needs except the operator element itself is staged in
-// LDS once per column: the 6j slice {jp jh JC; ja jb J'}, the pair positions
-// of (h,a) and (p,b) in every J' block, block offsets and sizes, and the
-// orbit quantum numbers, so each J' term does a single global load.
-__device__ __forceinline__ void pandya_col(const DevLayout &L, const double *__restrict__ op,
-                                           double *__restrict__ cc, int col, double *pan_lds) {
-  const int q1 = L.cccol_q[col];
-  const int c = col - L.cccbase[q1];
-  const int p = L.cccol_p[col], h = L.cccol_h[col];
-  const int JC = L.ccJ[q1], rlen = L.ccrlen[q1];
-  const int jp = L.jj[p], jh = L.jj[h], lp = L.l[p], lh = L.l[h], tp = L.tz[p], th = L.tz[h];
-  const double *V = op + L.v_off;
-  double *out = cc + L.ccoff[q1] + (long long)c * rlen;
-  const double sq = sqrt(JC + 1.0);
-  const int N = L.nsp, h6 = L.nhalf, nJ = L.nJ, nsl = h6 * h6 * nJ, NB = L.nblocks;
-  const size_t NN = (size_t)N * N;
-  double *S6 = pan_lds;
-  long long *BO = reinterpret_cast<long long *>(S6 + nsl);
-  int *BD = reinterpret_cast<int *>(BO + NB);
-  int *OQ = BD + NB;                           // jj | l << 8 | (2tz + 1) << 16
-  // [J'/2][a]: position of pair (h,a) in block J'; [J'/2][b]: of pair (p,b)
-  // (16 bits: positions below 2^15, -1 absent; the smaller list lets eight
-  // wavefronts per SIMD stay resident)
-  short *PR = reinterpret_cast<short *>(OQ + N);
-  short *PS = PR + nJ * N;
-  {
-    // every staging load of a batch is issued before the first LDS store, so
-    // a thread waits for one memory latency per batch, not one per element
-    const double *six0 = L.sixj + (((size_t)(jp >> 1) * h6 + (jh >> 1)) * nJ + (JC >> 1)) * (size_t)nsl;
-    for (int e0 = 0; e0 < nsl; e0 += 256 * 8) {
-      double v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = six0[min(e0 + (int)threadIdx.x + 256 * u, nsl - 1)];  // off any branch
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int e = e0 + (int)threadIdx.x + 256 * u;
-        if (e < nsl) S6[e] = v[u];
-      }
-    }
-    for (int e = threadIdx.x; e < NB; e += 256) {
-      BO[e] = L.boff[e];
-      BD[e] = L.bdim[e];
-    }
-    for (int e0 = 0; e0 < nJ * N; e0 += 256 * 8) {
-      int vr[8], vs[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int e = min(e0 + (int)threadIdx.x + 256 * u, nJ * N - 1);  // off any branch
-        const int J2 = e / N, x = e - J2 * N;
-        const int *pj = L.pidx + (size_t)J2 * NN;
-        vr[u] = pj[h > x ? x * N + h : h * N + x];
-        vs[u] = pj[p > x ? x * N + p : p * N + x];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int e = e0 + (int)threadIdx.x + 256 * u;
-        if (e < nJ * N) {
-          PR[e] = (short)vr[u];
-          PS[e] = (short)vs[u];
-        }
-      }
-    }
-    for (int e = threadIdx.x; e < N; e += 256) OQ[e] = L.jj[e] | (L.l[e] << 8) | ((L.tz[e] + 1) << 16);
-  }
-  __syncthreads();
-  // the next row's orbits are loaded while the current row's terms are summed
-  const int *rowa = L.ccrow_a + L.ccrbase[q1], *rowb = L.ccrow_b + L.ccrbase[q1];
-  int a_next = -1, b_next = -1;
-  if ((int)threadIdx.x < rlen) {
-    a_next = rowa[threadIdx.x];
-    b_next = rowb[threadIdx.x];
-  }
-  for (int r = threadIdx.x; r < rlen; r += blockDim.x) {
-    const int a = a_next, b = b_next;
-    if (r + (int)blockDim.x < rlen) {
-      a_next = rowa[r + blockDim.x];
-      b_next = rowb[r + blockDim.x];
-    }
-    if (a < 0) {  // zero row that makes the row count even
-      out[r] = 0.0;
-      continue;
-    }
-    const int qa = OQ[a], qbb = OQ[b];
-    const int ja = qa & 255, jb = qbb & 255, la = (qa >> 8) & 255, lb = (qbb >> 8) & 255;
-    const int ta = (qa >> 16) - 1, tb = (qbb >> 16) - 1;
-    double val = 0.0;
-    if ((((la + lh) & 1) == ((lb + lp) & 1)) && (ta + th == tb + tp)) {
-      const int Jmin = max(abs(jp - jb), abs(ja - jh));
-      const int Jmax = min(jp + jb, ja + jh);
-      // v_elem(h,a,p,b;J'): bra pair (h,a), ket pair (p,b), block (J', T2, P)
-      const int qb = 2 * ((th + ta) / 2 + 1) + ((lh + la) & 1);
-      const bool sw1 = h > a, sw2 = p > b;
-      const double *six = S6 + ((ja >> 1) * h6 + (jb >> 1)) * nJ;
-      double sm = 0.0;
-      // eight J' terms a batch; the element offsets and weights first (a J'
-      // past Jmax, or an element the block does not hold, reads element 0
-      // with weight 0), then the eight gathers, none of them on a branch, so
-      // they are in flight together
-      for (int J0 = Jmin; J0 <= Jmax; J0 += 16) {
-        long long off[8];
-        double w[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int JT = min(J0 + 2 * u, Jmax);
-          const int rr = PR[(JT >> 1) * N + a], ss = PS[(JT >> 1) * N + b], q = 3 * JT + qb;
-          double pre = 1.0;
-          if (sw1) pre = sgnp(1 + ((jh + ja - JT) >> 1));
-          else if (h == a) pre = pre * M_SQRT2;
-          if (sw2) pre = pre * sgnp(1 + ((jp + jb - JT) >> 1));
-          else if (p == b) pre = pre * M_SQRT2;
-          const bool ok = J0 + 2 * u <= Jmax && (rr | ss) >= 0;
-          off[u] = ok ? BO[q] + (long long)rr * BD[q] + ss : 0;
-          w[u] = ok ? pre * (double)(sgnp(JT >> 1) * (JT + 1)) * six[JT >> 1] : 0.0;
-        }
-        double vv[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) vv[u] = V[off[u]];
-#pragma unroll
-        for (int u = 0; u < 8; u++) sm = sm + w[u] * vv[u];
-      }
-      val = sm * sgnp((jh + jb + JC) >> 1) * sq;
-    }
-    out[r] = val;
-  }
-}
 __global__ __launch_bounds__(256) void k_pandya(DevLayout L, const double *__restrict__ op,
                                                 double *__restrict__ cc, const int *act) {
   extern __shared__ double pan_lds[];
   const long long inst = inst_id(act);
   if (inst < 0) return;
-  pandya_col(L, op + inst * L.op_size, cc + inst * L.ccsize, blockIdx.x, pan_lds);
+  pandya_col<false>(L, op + inst * L.op_size, cc + inst * L.ccsize, blockIdx.x, pan_lds);
 }
 size_t pandya_lds_bytes(const DevLayout &L) {
   return sizeof(double) * L.nhalf * L.nhalf * L.nJ + sizeof(long long) * L.nblocks +
@@ -1437,24 +1197,6 @@ void launch_ph_terms(hipStream_t s, const DevLayout &L, const double *Z, double 
 // wavefront covers its 64 outputs as four groups of 16, with every group's
 // descriptor, old value and first two loads issued before any is used, and
 // two lane exchanges add each output's four partial sums.
-__device__ __forceinline__ void ph_decode(unsigned long long d, int &toff, int &n1, int &n, int &o1, int &o2,
-                                          double &g1, double &g2, double &pre2) {
-  toff = (int)(d & 0x7FFFFFull);
-  n1 = (int)((d >> 23) & 31);
-  n = n1 + (int)((d >> 28) & 31);
-  o1 = (int)((d >> 33) & 4095);
-  o2 = (int)((d >> 45) & 4095) - n1;
-  g1 = ((d >> 57) & 1) ? (((d >> 58) & 1) ? -1.0 : 1.0) : 0.0;
-  g2 = ((d >> 59) & 1) ? 1.0 : 0.0;
-  pre2 = ((d >> 60) & 1) ? .70710678118 : 1.0;
-}
-// 6j weight of term m of an output (0 past its run); index 0 when unused
-__device__ __forceinline__ double ph_coef(const double *S6, int m, int n, int n1, int o1, int o2, double g1,
-                                          double g2) {
-  const bool s1 = m < n1, in = m < n;
-  const int e = in ? (s1 ? o1 + m : o2 + m) : 0;
-  return (in ? (s1 ? g1 : g2) : 0.0) * S6[e];
-}
 __global__ __launch_bounds__(64) void k_ph_apply(DevLayout L, const double *__restrict__ Tbuf,
                                                  double *__restrict__ RES, const int *act) {
   extern __shared__ double S6[];  // max(ap6_max, 64) doubles
@@ -2285,13 +2027,13 @@ __global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ L
   const double *Lop = A.Lop + o, *Rop = A.Rop + o;
   int b = blockIdx.x;
   if (b < L.nccol) {
-    pandya_col(L, Rop, A.ccR + inst * L.ccsize, b, lds);
+    pandya_col<false>(L, Rop, A.ccR + inst * L.ccsize, b, lds);
     return;
   }
   b -= L.nccol;
   if (A.prepL) {
     if (b < L.nccol) {
-      pandya_col(L, Lop, A.ccL + inst * L.ccsize, b, lds);
+      pandya_col<false>(L, Lop, A.ccL + inst * L.ccsize, b, lds);
       return;
     }
     b -= L.nccol;
