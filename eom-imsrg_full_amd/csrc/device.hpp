@@ -95,6 +95,21 @@ struct GemmProb {
   long long a_off, b_off, c_off;
 };
 
+// A sub-block of a host stream: element (row j, column i), j < nr, i < nc, at
+// src + j ld + i of the operator and, column by column (rows j >= i only when
+// tri), from dst of the stream; mir: its mirror image's sub-block, or -1.
+struct PackSeg {
+  long long src, dst, mir;
+  int nr, nc, ld, tri;
+};
+struct PackTables {
+  const PackSeg *segs;
+  const int4 *tiles;          // (segment, 32-row tile, 32-column tile)
+  int ntiles, nhead;
+  const int *head, *head_mir; // operator offsets of the first nhead entries, and of their mirrors (-1 none)
+  const double *head_sgn;     // the mirrors' sign beside the hermiticity
+};
+
 // One K segment of a segmented GEMM: sign * A * B with A taken from operand
 // `src` and B from the other one (offsets in doubles from the operand base).
 struct SegDesc {
@@ -189,6 +204,11 @@ void launch_fill(hipStream_t s, double *p, long long n, double v, const int *act
                  long long stride = 0);
 void launch_axpby(hipStream_t s, long long n, double a, const double *A, double b, const double *B, double *C,
                   const int *act, int nact, long long stride);
+// operator(s) <-> host stream order in device memory (nbatch instances)
+void launch_pack(hipStream_t s, const PackTables &P, const double *op, long long sop, double *vec, long long svec,
+                 int nbatch);
+void launch_unpack(hipStream_t s, const PackTables &P, const double *vec, long long svec, double *op, long long sop,
+                   double herm, int nbatch);
 void launch_copy(hipStream_t s, long long n, const double *A, double *C, const int *act, int nact,
                  long long stride);
 // mode: 0 FP64 MFMA (pp/hh: 32 x 32 tiles, K split over a workgroup's wavefronts; Pandya

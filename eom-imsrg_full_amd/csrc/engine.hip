@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -10,6 +11,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <tuple>
 #include <vector>
 
@@ -688,6 +690,9 @@ int imsrg_ctx_destroy(imsrg_ctx c) {
   for (int k = 0; k < imsrg_ctx_s::kSlots; k++)
     if (c->act_h[k]) (void)hipHostFree(c->act_h[k]);
   if (c->hstage) (void)hipHostFree(c->hstage);
+  if (c->ring) (void)hipHostFree(c->ring);
+  for (hipEvent_t e : c->ev_ring)
+    if (e) (void)hipEventDestroy(e);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   for (hipEvent_t e : c->ev_gate)
@@ -916,29 +921,186 @@ int imsrg_op_get_herm(imsrg_op op, int *herm) {
   *herm = op->herm;
   return 0;
 }
+// ---- host streams
+int pack_tables(imsrg_ctx_s *c, const std::vector<PackSeg> &segs, const std::vector<int> &head,
+                const std::vector<int> &mir, const std::vector<double> &sgn, PackTables *out) {
+  std::vector<int4> tiles;
+  for (size_t k = 0; k < segs.size(); k++)
+    for (int j = 0; j < (segs[k].nr + 31) / 32; j++)
+      for (int i = 0; i < (segs[k].nc + 31) / 32; i++)
+        if (!segs[k].tri || j >= i) tiles.push_back(make_int4((int)k, j, i, 0));
+  PackTables P{};
+  P.ntiles = (int)tiles.size();
+  P.nhead = (int)head.size();
+  int rc = upload_table(c, segs, &P.segs);
+  if (!rc) rc = upload_table(c, tiles, &P.tiles);
+  if (!rc) rc = upload_table(c, head, &P.head);
+  if (!rc) rc = upload_table(c, mir, &P.head_mir);
+  if (!rc) rc = upload_table(c, sgn, &P.head_sgn);
+  if (!rc) *out = P;
+  return rc;
+}
+// the order of Layout::pack_vec / unpack_vec
+static int pack_setup(imsrg_ctx_s *c) {
+  if (c->pack_d) return 0;
+  const Layout &Ly = c->lay;
+  std::vector<int> head(1, 0), mir(1, -1);
+  const int n = Ly.nsp, f = (int)Ly.f_off;
+  for (int i : Ly.holes)
+    for (int j : Ly.holes) head.push_back(f + j * n + i), mir.push_back(-1);
+  for (int i : Ly.parts)
+    for (int j : Ly.parts) head.push_back(f + j * n + i), mir.push_back(-1);
+  for (int i : Ly.holes)
+    for (int j : Ly.parts) head.push_back(f + j * n + i), mir.push_back(f + i * n + j);
+  std::vector<PackSeg> segs;
+  long long k = (long long)head.size();
+  static const int row[6] = {0, 0, 0, 1, 2, 1}, col[6] = {0, 1, 2, 1, 2, 2};  // classes of gam1..gam6
+  for (int q = 0; q < Ly.nblocks; q++) {
+    const int dim = Ly.bdim[q], off[4] = {0, Ly.bnp[q], Ly.bnp[q] + Ly.bnb[q], dim};
+    for (int g = 0; g < 6; g++) {
+      const int r0 = off[row[g]], c0 = off[col[g]], nr = off[row[g] + 1] - r0, nc = off[col[g] + 1] - c0;
+      const int tri = row[g] == col[g];
+      if (nr == 0 || nc == 0) continue;
+      const long long M = Ly.v_off + Ly.boff[q];
+      segs.push_back(PackSeg{M + (long long)r0 * dim + c0, k, M + (long long)c0 * dim + r0, nr, nc, dim, tri});
+      k += tri ? (long long)nr * (nr + 1) / 2 : (long long)nr * nc;
+    }
+  }
+  if (k != Ly.neq) return fail(IMSRG_EINVAL, "stream tables do not cover the stream");
+  int rc = pack_tables(c, segs, head, mir, std::vector<double>(head.size(), 1.0), &c->pack);
+  if (!rc) rc = dalloc(c, (size_t)Ly.neq * c->nbatch, &c->pack_d);
+  return rc;
+}
+// Copies shorter than this go through hstage in one piece (the threads and
+// events of the ring cost about 0.1 ms).
+static constexpr int64_t kLongCopy = (int64_t)1 << 20;  // bytes
+static int copy_threads(int64_t bytes) {
+  const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
+  return std::max(1, std::min({8, hw, (int)(bytes / (int64_t)imsrg_ctx_s::kRingBytes)}));
+}
+// Runs f(0) .. f(nt - 1), one thread each (f(0) on the caller's).
+template <class F>
+static void on_threads(int nt, F &&f) {
+  std::vector<std::thread> th;
+  int made = 1;
+  try {
+    for (; made < nt; made++) th.emplace_back([&f, made] { f(made); });
+  } catch (...) {  // no more threads: the caller does the rest
+  }
+  f(0);
+  for (int k = made; k < nt; k++) f(k);
+  for (auto &t : th) t.join();
+}
+int stream_to_host(imsrg_ctx_s *c, const double *dev, int64_t n, double *host) {
+  const int64_t bytes = n * (int64_t)sizeof(double);
+  if (bytes <= kLongCopy && n <= std::max<int64_t>(c->lay.op_size * c->nbatch, c->lay.ccsize)) {
+    HIPCHK(hipMemcpyAsync(c->hstage, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(host, c->hstage, bytes);
+    return 0;
+  }
+  // chunk k goes through ring slot k % kRing to pinned memory, from where the
+  // next free thread copies it out (the user's pages are often touched for the
+  // first time here, which costs more than the copy): 29 MB in about 1 ms where
+  // one pageable copy takes 2.4
+  constexpr int R = imsrg_ctx_s::kRing;
+  const int64_t cb = (int64_t)imsrg_ctx_s::kRingBytes;
+  if (!c->ring) {
+    for (auto &e : c->ev_ring) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (hipHostMalloc((void **)&c->ring, R * cb, hipHostMallocDefault) != hipSuccess)
+      return fail(IMSRG_ENOMEM, "hipHostMalloc copy ring failed");
+  }
+  const int nk = (int)((bytes + cb - 1) / cb), nt = copy_threads(bytes);
+  std::vector<std::atomic<int>> state(nk);  // 0 not issued, 1 in flight, 2 copied out
+  for (auto &x : state) x.store(0);
+  std::atomic<int> bad{0};
+  auto issue = [&](int k) {
+    const int64_t o = k * cb;
+    if (hipMemcpyAsync(c->ring + (k % R) * cb, (const char *)dev + o, std::min(cb, bytes - o), hipMemcpyDeviceToHost,
+                       c->stream) != hipSuccess ||
+        hipEventRecord(c->ev_ring[k % R], c->stream) != hipSuccess)
+      bad.store(1);
+    state[k].store(1);
+  };
+  for (int k = 0; k < std::min(R, nk); k++) issue(k);
+  std::atomic<int> next{R}, take{0};  // chunks from R on are issued by whoever frees their slot
+  std::mutex mu;
+  on_threads(nt, [&](int) {
+    (void)hipSetDevice(c->device);
+    for (int k = take++; k < nk; k = take++) {
+      while (state[k].load() == 0 && !bad.load()) std::this_thread::yield();
+      if (bad.load() || hipEventSynchronize(c->ev_ring[k % R]) != hipSuccess) {
+        bad.store(1);
+        return;
+      }
+      const int64_t o = k * cb;
+      std::memcpy((char *)host + o, c->ring + (k % R) * cb, std::min(cb, bytes - o));
+      state[k].store(2);
+      std::lock_guard<std::mutex> lock(mu);
+      while (next.load() < nk && state[next.load() - R].load() == 2) issue(next++);
+    }
+  });
+  HIPCHK(hipStreamSynchronize(c->stream));
+  return bad.load() ? fail(IMSRG_EDEVICE, "copy to the host failed") : 0;
+}
+int stream_to_dev(imsrg_ctx_s *c, const double *host, int64_t n, double *dev) {
+  HIPCHK(hipStreamSynchronize(c->stream));  // hstage may still be read
+  const int64_t cap = std::max<int64_t>(c->lay.op_size * c->nbatch, c->lay.ccsize);
+  for (int64_t o = 0; o < n; o += cap) {
+    const int64_t m = std::min(cap, n - o);
+    const int nt = copy_threads(m * (int64_t)sizeof(double));
+    on_threads(nt, [&](int t) {
+      const int64_t a = m * t / nt, b = m * (t + 1) / nt;
+      std::memcpy(c->hstage + a, host + o + a, sizeof(double) * (b - a));
+    });
+    HIPCHK(hipMemcpyAsync(dev + o, c->hstage, sizeof(double) * m, hipMemcpyHostToDevice, c->stream));
+    if (o + m < n) HIPCHK(hipStreamSynchronize(c->stream));
+  }
+  return 0;
+}
+// Operators up to 64 KiB (emax 2: 22 KiB) are packed on the host: the pack
+// kernel's launch costs more (upload 12 / 30 us, download 12 / 19 us host /
+// device at emax 2; at emax 4, 0.6 MiB, 37 / 35 and 68 / 38 us; at emax 8
+// 6.7 / 0.8 and 4.4 / 1.2 ms).
+static bool pack_on_host(const imsrg_ctx_s *c) {
+  return sizeof(double) * c->lay.op_size * c->nbatch <= (size_t)64 << 10;
+}
+
 // vec holds nbatch vectorize-order vectors back to back
 int imsrg_op_upload(imsrg_op op, const double *vec, int64_t n) {
   if (!op || !vec) return fail(IMSRG_EINVAL, "null argument");
   imsrg_ctx_s *c = op->ctx;
-  if (n != c->lay.neq * c->nbatch) return fail(IMSRG_EINVAL, "length must be neq * nbatch");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  for (int k = 0; k < c->nbatch; k++)
-    c->lay.unpack_vec(vec + (size_t)k * c->lay.neq, op->herm, c->hstage + (size_t)k * c->lay.op_size);
-  HIPCHK(hipMemcpyAsync(op->d, c->hstage, sizeof(double) * c->lay.op_size * c->nbatch, hipMemcpyHostToDevice,
-                        c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  const Layout &Ly = c->lay;
+  if (n != Ly.neq * c->nbatch) return fail(IMSRG_EINVAL, "length must be neq * nbatch");
+  if (pack_on_host(c)) {
+    HIPCHK(hipStreamSynchronize(c->stream));  // hstage may still be read
+    for (int k = 0; k < c->nbatch; k++)
+      Ly.unpack_vec(vec + (size_t)k * Ly.neq, op->herm, c->hstage + (size_t)k * Ly.op_size);
+    HIPCHK(hipMemcpyAsync(op->d, c->hstage, sizeof(double) * Ly.op_size * c->nbatch, hipMemcpyHostToDevice, c->stream));
+    return 0;
+  }
+  if (int rc = pack_setup(c)) return rc;
+  if (int rc = stream_to_dev(c, vec, n, c->pack_d)) return rc;
+  launch_unpack(c->stream, c->pack, c->pack_d, Ly.neq, op->d, Ly.op_size, (double)op->herm, c->nbatch);
+  HIPCHK(hipGetLastError());
   return 0;
 }
 int imsrg_op_download(imsrg_op op, double *vec, int64_t n) {
   if (!op || !vec) return fail(IMSRG_EINVAL, "null argument");
   imsrg_ctx_s *c = op->ctx;
-  if (n != c->lay.neq * c->nbatch) return fail(IMSRG_EINVAL, "length must be neq * nbatch");
-  HIPCHK(hipMemcpyAsync(c->hstage, op->d, sizeof(double) * c->lay.op_size * c->nbatch, hipMemcpyDeviceToHost,
-                        c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  for (int k = 0; k < c->nbatch; k++)
-    c->lay.pack_vec(c->hstage + (size_t)k * c->lay.op_size, vec + (size_t)k * c->lay.neq);
-  return 0;
+  const Layout &Ly = c->lay;
+  if (n != Ly.neq * c->nbatch) return fail(IMSRG_EINVAL, "length must be neq * nbatch");
+  if (pack_on_host(c)) {
+    HIPCHK(hipMemcpyAsync(c->hstage, op->d, sizeof(double) * Ly.op_size * c->nbatch, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int k = 0; k < c->nbatch; k++)
+      Ly.pack_vec(c->hstage + (size_t)k * Ly.op_size, vec + (size_t)k * Ly.neq);
+    return 0;
+  }
+  if (int rc = pack_setup(c)) return rc;
+  launch_pack(c->stream, c->pack, op->d, Ly.op_size, c->pack_d, Ly.neq, c->nbatch);
+  HIPCHK(hipGetLastError());
+  return stream_to_host(c, c->pack_d, n, vec);
 }
 int imsrg_op_copy(imsrg_op src, imsrg_op dst) {
   if (!src || !dst || src->ctx != dst->ctx) return fail(IMSRG_EINVAL, "bad operands");
@@ -1507,6 +1669,7 @@ int imsrg_commutator_222_ph_cc(imsrg_ctx c, const double *lcc, int hL, const dou
   if (n != imsrg_cross_coupled_size(c)) return fail(IMSRG_EINVAL, "Pandya stream size mismatch");
   const Layout &Ly = c->lay;
   const double *src[2] = {lcc, rcc};
+  HIPCHK(hipStreamSynchronize(c->stream));  // hstage may still be read
   for (int k = 0; k < 2; k++) {
     std::memset(c->hstage, 0, sizeof(double) * Ly.ccsize);
     int64_t o = 0;

@@ -77,6 +77,14 @@ struct imsrg_ctx_s {
   double *scal = nullptr;   // device scalars, kScal per instance
   double *coef_d = nullptr; // series coefficient of the next graph replay
   double *hscal = nullptr;  // pinned host mirror of scal
+  // host streams: the pack tables and their device buffer (neq * nbatch), made
+  // on first use, and a pinned ring for long copies
+  PackTables pack{};
+  double *pack_d = nullptr;
+  static constexpr int kRing = 8;
+  static constexpr size_t kRingBytes = (size_t)4 << 20;
+  char *ring = nullptr;
+  hipEvent_t ev_ring[kRing] = {};
   double *mono = nullptr;
   double *mbar = nullptr;   // generator-transpose scratch (nsp * nsp)
   double *hstage = nullptr; // pinned staging: max(op_size * nbatch, ccsize) doubles
@@ -163,6 +171,13 @@ struct imsrg_op_s {
 inline int i8_planes(int prec) {
   return prec == IMSRG_PREC_INT8X5 ? 5 : prec == IMSRG_PREC_INT8X4 ? 4 : 0;
 }
+// PackTables from host lists; a segment's tiles are added here
+int pack_tables(imsrg_ctx_s *c, const std::vector<PackSeg> &segs, const std::vector<int> &head,
+                const std::vector<int> &mir, const std::vector<double> &sgn, PackTables *out);
+// n doubles of device memory to / from the host (any memory), behind the
+// context's stream; the call returns when they are there
+int stream_to_host(imsrg_ctx_s *c, const double *dev, int64_t n, double *host);
+int stream_to_dev(imsrg_ctx_s *c, const double *host, int64_t n, double *dev);
 // hipMalloc for a context; when it fails, the context's pool of operator
 // buffers goes back to the device and the call is made again
 inline hipError_t dev_malloc(imsrg_ctx_s *c, void **p, size_t bytes) {

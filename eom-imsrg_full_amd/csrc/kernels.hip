@@ -101,6 +101,87 @@ void launch_series_begin(hipStream_t s, long long n, const double *A, double *C1
                      act, own, stride);
 }
 
+// ------------------------------------------------------------------ host streams
+// Between an operator and its host stream (vectorize / repackage order, or a
+// tensor's sub-blocks): the head (E0 and one-body entries) through an index
+// table, the two-body sub-blocks as 32 x 32 tiles transposed in LDS, since the
+// stream is column-major.  Only the stream crosses PCIe (half of the full
+// blocks), already in order: packing emax 8 on the host took 2.4 ms.
+__global__ __launch_bounds__(256) void k_pack(PackTables P, const double *op, long long sop, double *vec,
+                                              long long svec) {
+  __shared__ double U[32][33];
+  op += blockIdx.y * sop;
+  vec += blockIdx.y * svec;
+  const int nh = (P.nhead + 255) / 256;
+  if ((int)blockIdx.x < nh) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < P.nhead) vec[k] = op[P.head[k]];
+    return;
+  }
+  const int4 t = P.tiles[blockIdx.x - nh];
+  const PackSeg s = P.segs[t.x];
+  const int j0 = t.y * 32, i0 = t.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const int j = j0 + ty + k, i = i0 + tx;
+    if (j < s.nr && i < s.nc) U[ty + k][tx] = op[s.src + (long long)j * s.ld + i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const int j = j0 + tx, i = i0 + ty + k;
+    if (j >= s.nr || i >= s.nc || (s.tri && j < i)) continue;
+    vec[s.dst + (long long)i * s.nr + j - (s.tri ? (long long)i * (i + 1) / 2 : 0)] = U[tx][ty + k];
+  }
+}
+void launch_pack(hipStream_t s, const PackTables &P, const double *op, long long sop, double *vec, long long svec,
+                 int nbatch) {
+  hipLaunchKernelGGL(k_pack, dim3((P.nhead + 255) / 256 + P.ntiles, nbatch), dim3(256), 0, s, P, op, sop, vec, svec);
+}
+// The way back, into an operator whose entries outside the stream are zero.
+// Sub-blocks with a mirror (mir: offset of the transposed sub-block, ld
+// the same) get herm times their transpose there; of a square one the diagonal
+// is written last as herm * x, as repackage does.
+__global__ __launch_bounds__(256) void k_unpack(PackTables P, const double *vec, long long svec, double *op,
+                                                long long sop, double herm) {
+  __shared__ double U[32][33];
+  op += blockIdx.y * sop;
+  vec += blockIdx.y * svec;
+  const int nh = (P.nhead + 255) / 256;
+  if ((int)blockIdx.x < nh) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < P.nhead) {
+      const double x = vec[k];
+      op[P.head[k]] = x;
+      if (P.head_mir[k] >= 0) op[P.head_mir[k]] = herm * P.head_sgn[k] * x;
+    }
+    return;
+  }
+  const int4 t = P.tiles[blockIdx.x - nh];
+  const PackSeg s = P.segs[t.x];
+  const int j0 = t.y * 32, i0 = t.z * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const int j = j0 + tx, i = i0 + ty + k;
+    if (j >= s.nr || i >= s.nc || (s.tri && j < i)) continue;
+    const double x = vec[s.dst + (long long)i * s.nr + j - (s.tri ? (long long)i * (i + 1) / 2 : 0)];
+    U[tx][ty + k] = x;
+    if (s.mir >= 0) op[s.mir + (long long)i * s.ld + j] = herm * x;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k += 8) {
+    const int j = j0 + ty + k, i = i0 + tx;
+    if (j >= s.nr || i >= s.nc || (s.tri && j <= i)) continue;
+    op[s.src + (long long)j * s.ld + i] = U[ty + k][tx];
+  }
+}
+void launch_unpack(hipStream_t s, const PackTables &P, const double *vec, long long svec, double *op, long long sop,
+                   double herm, int nbatch) {
+  hipLaunchKernelGGL(k_unpack, dim3((P.nhead + 255) / 256 + P.ntiles, nbatch), dim3(256), 0, s, P, vec, svec, op, sop,
+                     herm);
+}
+
 // ------------------------------------------------------------------ segmented grouped GEMM
 // Every output block C (M x M) is a signed sum of K segments,
 //   C = sum_s sign_s * A_s * B_s,

@@ -973,6 +973,8 @@ struct TensorSpace {
   long long xsize = 0, rsize = 0, wsize = 0;
   std::vector<double> x6, s6;
   long long n9size = 0;
+  PackTables pack{};
+  double *pack_d = nullptr;
   DevTensor dt{};
   double *gcc = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
   double *w1 = nullptr, *w2 = nullptr, *part = nullptr, *hpart = nullptr;
@@ -1360,89 +1362,68 @@ int imsrg_tensor_get_herm(imsrg_tensor t, int *herm) {
   return 0;
 }
 
-// stream <-> device image (see the header for the stream order)
-static void stream_to_image(const Layout &Ly, const TensorSpace &S, int herm, const double *v, double *img) {
-  std::fill(img, img + S.op_size, 0.0);
-  const int A = Ly.nhole, P = Ly.npart, n = Ly.nsp;
-  long long k = 0;
-  img[0] = v[k++];
-  double *F = img + Ly.f_off;
-  for (int j = 0; j < A; j++)
-    for (int i = 0; i < A; i++) F[(size_t)Ly.holes[i] * n + Ly.holes[j]] = v[k + i + (long long)j * A];
-  k += (long long)A * A;
-  for (int j = 0; j < P; j++)
-    for (int i = 0; i < P; i++) F[(size_t)Ly.parts[i] * n + Ly.parts[j]] = v[k + i + (long long)j * P];
-  k += (long long)P * P;
-  for (int j = 0; j < A; j++)
-    for (int i = 0; i < P; i++) {
-      const int p = Ly.parts[i], h = Ly.holes[j];
-      const double x = v[k + i + (long long)j * P];
-      F[(size_t)p * n + h] = x;
-      F[(size_t)h * n + p] = x * herm * (((Ly.jj[h] - Ly.jj[p]) / 2) & 1 ? -1.0 : 1.0);
-    }
-  k += (long long)P * A;
-  double *V = img + S.v_off;
+// stream <-> device (see the header for the stream order): the pack tables and
+// their device buffer, made on first use
+static int tpack_setup(imsrg_ctx_s *c, TensorSpace &S) {
+  if (S.pack_d) return 0;
+  const Layout &Ly = c->lay;
+  std::vector<int> head(1, 0), mir(1, -1);
+  std::vector<double> sgn(1, 1.0);
+  const int n = Ly.nsp, f = (int)Ly.f_off;
+  auto put = [&](int i, int j, bool m) {
+    head.push_back(f + i * n + j);
+    mir.push_back(m ? f + j * n + i : -1);
+    sgn.push_back(((Ly.jj[j] - Ly.jj[i]) / 2) & 1 ? -1.0 : 1.0);
+  };
+  for (int j : Ly.holes)
+    for (int i : Ly.holes) put(i, j, false);
+  for (int j : Ly.parts)
+    for (int i : Ly.parts) put(i, j, false);
+  for (int j : Ly.holes)
+    for (int i : Ly.parts) put(i, j, true);
+  std::vector<PackSeg> segs;
+  long long k = (long long)head.size();
+  static const int sea1[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2}, sea2[9] = {0, 1, 2, 1, 2, 2, 0, 0, 1};
   for (int q = 0; q < S.nblk; q++) {
     const int m1 = S.n1[q], m2 = S.n2[q];
     if (m1 == 0 || m2 == 0) continue;
     const int b1 = S.q1[q], b2 = S.q2[q];
     const int s1[4] = {0, Ly.bnp[b1], Ly.bnp[b1] + Ly.bnb[b1], m1};
     const int s2[4] = {0, Ly.bnp[b2], Ly.bnp[b2] + Ly.bnb[b2], m2};
-    static const int sea1[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2}, sea2[9] = {0, 1, 2, 1, 2, 2, 0, 0, 1};
     for (int g = 0; g < 9; g++) {
       const int r0 = s1[sea1[g]], nr = s1[sea1[g] + 1] - r0, c0 = s2[sea2[g]], nc = s2[sea2[g] + 1] - c0;
-      for (int jc = 0; jc < nc; jc++)
-        for (int ir = 0; ir < nr; ir++) V[S.off[q] + (long long)(r0 + ir) * m2 + c0 + jc] = v[k++];
+      if (nr == 0 || nc == 0) continue;
+      segs.push_back(PackSeg{S.v_off + S.off[q] + (long long)r0 * m2 + c0, k, -1, nr, nc, m2, 0});
+      k += (long long)nr * nc;
     }
   }
-}
-static void image_to_stream(const Layout &Ly, const TensorSpace &S, const double *img, double *v) {
-  const int A = Ly.nhole, P = Ly.npart, n = Ly.nsp;
-  long long k = 0;
-  v[k++] = img[0];
-  const double *F = img + Ly.f_off;
-  for (int j = 0; j < A; j++)
-    for (int i = 0; i < A; i++) v[k++] = F[(size_t)Ly.holes[i] * n + Ly.holes[j]];
-  for (int j = 0; j < P; j++)
-    for (int i = 0; i < P; i++) v[k++] = F[(size_t)Ly.parts[i] * n + Ly.parts[j]];
-  for (int j = 0; j < A; j++)
-    for (int i = 0; i < P; i++) v[k++] = F[(size_t)Ly.parts[i] * n + Ly.holes[j]];
-  const double *V = img + S.v_off;
-  for (int q = 0; q < S.nblk; q++) {
-    const int m1 = S.n1[q], m2 = S.n2[q];
-    if (m1 == 0 || m2 == 0) continue;
-    const int b1 = S.q1[q], b2 = S.q2[q];
-    const int s1[4] = {0, Ly.bnp[b1], Ly.bnp[b1] + Ly.bnb[b1], m1};
-    const int s2[4] = {0, Ly.bnp[b2], Ly.bnp[b2] + Ly.bnb[b2], m2};
-    static const int sea1[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2}, sea2[9] = {0, 1, 2, 1, 2, 2, 0, 0, 1};
-    for (int g = 0; g < 9; g++) {
-      const int r0 = s1[sea1[g]], nr = s1[sea1[g] + 1] - r0, c0 = s2[sea2[g]], nc = s2[sea2[g] + 1] - c0;
-      for (int jc = 0; jc < nc; jc++)
-        for (int ir = 0; ir < nr; ir++) v[k++] = V[S.off[q] + (long long)(r0 + ir) * m2 + c0 + jc];
-    }
-  }
+  if (k != S.neq) return fail(IMSRG_EINVAL, "tensor stream tables do not cover the stream");
+  int rc = pack_tables(c, segs, head, mir, sgn, &S.pack);
+  if (!rc) rc = dalloc(c, S.neq, &S.pack_d);
+  return rc;
 }
 
 int imsrg_tensor_upload(imsrg_tensor t, const double *vec, int64_t n) {
   if (!t || !vec) return fail(IMSRG_EINVAL, "null argument");
-  const TensorSpace &S = *t->ts;
+  TensorSpace &S = *t->ts;
+  imsrg_ctx_s *c = t->ctx;
   if (n != S.neq) return fail(IMSRG_EINVAL, "tensor stream length " + std::to_string(n) + " != " + std::to_string(S.neq));
-  std::vector<double> img(S.op_size);
-  stream_to_image(t->ctx->lay, S, t->herm, vec, img.data());
-  HIPCHK(hipMemcpyAsync(t->d, img.data(), sizeof(double) * S.op_size, hipMemcpyHostToDevice, t->ctx->stream));
-  HIPCHK(hipStreamSynchronize(t->ctx->stream));
+  if (int rc = tpack_setup(c, S)) return rc;
+  if (int rc = stream_to_dev(c, vec, n, S.pack_d)) return rc;
+  launch_unpack(c->stream, S.pack, S.pack_d, 0, t->d, 0, (double)t->herm, 1);
+  HIPCHK(hipGetLastError());
   return 0;
 }
 
 int imsrg_tensor_download(imsrg_tensor t, double *vec, int64_t n) {
   if (!t || !vec) return fail(IMSRG_EINVAL, "null argument");
-  const TensorSpace &S = *t->ts;
+  TensorSpace &S = *t->ts;
+  imsrg_ctx_s *c = t->ctx;
   if (n != S.neq) return fail(IMSRG_EINVAL, "tensor stream length " + std::to_string(n) + " != " + std::to_string(S.neq));
-  std::vector<double> img(S.op_size);
-  HIPCHK(hipMemcpyAsync(img.data(), t->d, sizeof(double) * S.op_size, hipMemcpyDeviceToHost, t->ctx->stream));
-  HIPCHK(hipStreamSynchronize(t->ctx->stream));
-  image_to_stream(t->ctx->lay, S, img.data(), vec);
-  return 0;
+  if (int rc = tpack_setup(c, S)) return rc;
+  launch_pack(c->stream, S.pack, t->d, 0, S.pack_d, 0, 1);
+  HIPCHK(hipGetLastError());
+  return stream_to_host(c, S.pack_d, n, vec);
 }
 
 static int same_space(imsrg_tensor a, imsrg_tensor b) {
