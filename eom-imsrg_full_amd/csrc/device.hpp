@@ -279,8 +279,7 @@ void launch_generator(hipStream_t s, const DevLayout &L, const double *Hden, con
 // A copied to C1 (and C2, may be null) on the instances of act, and act to own
 void launch_series_begin(hipStream_t s, long long n, const double *A, double *C1, double *C2, const int *act, int *own,
                          int nact, long long stride);
-void launch_normal_order(hipStream_t s, const DevLayout &L, const double *T, double *H, const int *act,
-                         int nact);
+void launch_normal_order(hipStream_t s, const DevLayout &L, double *H, const int *act, int nact);
 void launch_gather_e0(hipStream_t s, const double *op, long long stride, double *out, const int *act, int nact);
 // truncation test of a BCH (mode 0) or Magnus (mode 1) series after a nested
 // commutator: instances that stop get -1 in the series table `act`; live[k]
@@ -290,19 +289,24 @@ constexpr int kHFMaxGroup = 16;
 void launch_hf_init(hipStream_t s, const DevLayout &L, const double *op, double *D, double *Tm, double *eig,
                     int reset);
 // one self-consistency iteration; state = {converged, iterations}: every kernel
-// returns at once when converged, the last one counts and tests crit > conv
-void launch_hf_iteration(hipStream_t s, const DevLayout &L, const double *op, double *D, double *rho,
-                         const double *Tm, double *Vg, double *Fm, double *eig, double *cpart, double *crit,
-                         double *state, double conv);
+// returns at once when converged.  An iteration's test crit > conv is made at
+// the start of the next one (first = 0), or by launch_hf_test after the last.
+void launch_hf_iteration(hipStream_t s, const DevLayout &L, const double *op, double *D, const double *Tm, double *Vg,
+                         double *Fm, double *eig, double *cpart, double *crit, double *state, double conv, int first);
+void launch_hf_test(hipStream_t s, const DevLayout &L, const double *cpart, double *crit, double *state, double conv);
 void launch_hf_finish_1b(hipStream_t s, const DevLayout &L, double *D, const double *M, double *op, int herm,
                          const double *Tm, const double *Vg, double *tv, double *ehf);
-void launch_hf_2b(hipStream_t s, const DevLayout &L, const double *D, double *op, double *W, int herm);
-// the same transform for the pair rows [r0, r0 + nrows), which must cover whole
+// two-body transform with the coefficients D: the weights U once (one double per
+// hf_nb entry), then the pair rows [r0, r0 + nrows), which must cover whole
 // channel blocks: W holds only their blocks, W[0] = element v_off + wofs of a
-// full operator layout (wofs = the first block's offset inside V)
-void launch_hf_2b_window(hipStream_t s, const DevLayout &L, const double *D, double *op, double *W, int herm,
-                         int r0, int nrows, long long wofs);
+// full operator layout (wofs = the first block's offset inside V); items: those
+// rows in runs of hf_col_rows(maxdim) of one block (first row, rows)
+int hf_col_rows(int maxdim);
+void launch_hf_u(hipStream_t s, const DevLayout &L, const double *D, double *U);
+void launch_hf_2b(hipStream_t s, const DevLayout &L, const double *U, double *op, double *W, int herm, int r0,
+                  int nrows, long long wofs, const int2 *items, int nitems, int maxdim);
 
+// the number a series gate writes, and what it tests
 struct GateArgs {
   int mode;          // 0 BCH, 1 Magnus
   double coef;

@@ -514,6 +514,18 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   D.nmirror = (int)mtiles.size();
   UP(mtiles, mirror_tiles);
   if (!rc) rc = small_setup(c, same_ob);
+  if (!rc) {
+    for (int d : Ly.bdim) c->hf_maxdim = std::max(c->hf_maxdim, d);
+    const int R = hf_col_rows(c->hf_maxdim);
+    std::vector<int2> items;
+    for (int q = 0; q < Ly.nblocks; q++) {
+      c->hf_item0.push_back((int)items.size());
+      for (int r = 0; r < Ly.bdim[q]; r += R) items.push_back(make_int2(Ly.pbase[q] + r, std::min(R, Ly.bdim[q] - r)));
+    }
+    c->hf_item0.push_back((int)items.size());
+    rc = upload_table(c, items, &c->hf_items);
+    if (!rc) rc = dalloc(c, Ly.hf_nb.size(), &c->hf_U);
+  }
 #undef UP
   const size_t B = (size_t)nbatch;
   if (!rc) rc = dalloc(c, (size_t)Ly.vsize * B, &c->wpp);
@@ -1180,23 +1192,46 @@ int imsrg_mbpt2(imsrg_op H, double *out) {
 int imsrg_normal_order(imsrg_op H) {
   if (!H) return fail(IMSRG_EINVAL, "null operand");
   imsrg_ctx_s *c = H->ctx;
-  imsrg_op_s *T = tmp_op(c, 5, H->herm);
-  if (!T) return IMSRG_ENOMEM;
   const ActSet all = all_set(c);
-  op_copy(H, T, all);
-  launch_normal_order(c->stream, c->dl, T->d, H->d, all.d, all.n());
+  launch_normal_order(c->stream, c->dl, H->d, all.d, all.n());
   HIPCHK(hipGetLastError());
   return 0;
 }
 
 // ---------------------------------------------------------------- Hartree-Fock
+static int hf_limits(imsrg_ctx_s *c) {
+  for (int n : c->lay.grp_cnt)
+    if (n > kHFMaxGroup) return fail(IMSRG_EINVAL, "Hartree-Fock: an (l,j,tz) group has more than 16 orbits");
+  return 0;
+}
+// the self-consistency loop on the buffers given; enqueues eight iterations at
+// a time, the device counts them and, once converged, skips the rest
+static int hf_loop(imsrg_ctx_s *c, const double *op, double *D, const double *Tm, double *Vg, double *Fm, double *eig,
+                   double *cp, double *sc, int &it) {
+  const double conv = (double)1e-6f;  // the reference's `crit > 1e-6` compares with a default-real literal
+  for (;;) {
+    for (int k = 0; k < 8; k++)
+      launch_hf_iteration(c->stream, c->dl, op, D, Tm, Vg, Fm, eig, cp, sc, sc + 2, conv, k == 0);
+    launch_hf_test(c->stream, c->dl, cp, sc, sc + 2, conv);
+    HIPCHK(hipMemcpyAsync(c->hscal, sc, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    it = (int)c->hscal[3];
+    if (c->hscal[2] != 0.0) return 0;
+    if (it >= 10000) return fail(IMSRG_ECONV, "Hartree-Fock did not converge in 10000 iterations");
+  }
+}
+// the two-body transform of every block with the weights of D
+static void hf_2b_all(imsrg_ctx_s *c, const double *D, double *op, double *W, int herm) {
+  launch_hf_u(c->stream, c->dl, D, c->hf_U);
+  launch_hf_2b(c->stream, c->dl, c->hf_U, op, W, herm, 0, c->dl.npairs, 0, c->hf_items, c->hf_item0.back(),
+               c->hf_maxdim);
+}
 static int hf_setup(imsrg_ctx_s *c) {
   if (c->hf_D) return 0;
   const Layout &Ly = c->lay;
-  for (int n : Ly.grp_cnt)
-    if (n > kHFMaxGroup) return fail(IMSRG_EINVAL, "Hartree-Fock: an (l,j,tz) group has more than 16 orbits");
+  if (int rc = hf_limits(c)) return rc;
   const size_t n2 = (size_t)Ly.nsp * Ly.nsp;
-  double **mats[5] = {&c->hf_D, &c->hf_rho, &c->hf_Vg, &c->hf_Fm, &c->hf_Tm};
+  double **mats[4] = {&c->hf_D, &c->hf_Vg, &c->hf_Fm, &c->hf_Tm};
   for (double **m : mats) {
     if (int rc = dalloc(c, n2, m)) return rc;
     HIPCHK(hipMemsetAsync(*m, 0, n2 * sizeof(double), c->stream));
@@ -1216,27 +1251,13 @@ int imsrg_hartree_fock(imsrg_op H, double *coefs, int *iterations, double *e_hf)
   if (int rc = hf_setup(c)) return rc;
   const DevLayout &D = c->dl;
   launch_hf_init(c->stream, D, H->d, c->hf_D, c->hf_Tm, c->hf_eig, 1);
-  // the reference's loop test `crit > 1e-6` compares with a default-real
-  // literal.  Iterations are enqueued eight at a time; the device counts them
-  // and, once converged, skips the rest, so the host reads the state once per
-  // eight iterations.
-  const double conv = (double)1e-6f;
   HIPCHK(hipMemsetAsync(c->hf_sc + 2, 0, 2 * sizeof(double), c->stream));
   int it = 0;
-  for (;;) {
-    for (int k = 0; k < 8; k++)
-      launch_hf_iteration(c->stream, D, H->d, c->hf_D, c->hf_rho, c->hf_Tm, c->hf_Vg, c->hf_Fm, c->hf_eig,
-                          c->hf_cp, c->hf_sc, c->hf_sc + 2, conv);
-    HIPCHK(hipMemcpyAsync(c->hscal, c->hf_sc, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    it = (int)c->hscal[3];
-    if (c->hscal[2] != 0.0) break;
-    if (it >= 10000) return fail(IMSRG_ECONV, "Hartree-Fock did not converge in 10000 iterations");
-  }
+  if (int rc = hf_loop(c, H->d, c->hf_D, c->hf_Tm, c->hf_Vg, c->hf_Fm, c->hf_eig, c->hf_cp, c->hf_sc, it)) return rc;
   launch_hf_finish_1b(c->stream, D, c->hf_D, c->hf_Fm, H->d, 1, c->hf_Tm, c->hf_Vg, c->hf_tv, c->hf_sc + 1);
   imsrg_op_s *W = tmp_op(c, 5, 1);
   if (!W) return IMSRG_ENOMEM;
-  launch_hf_2b(c->stream, D, c->hf_D, H->d, W->d, 1);
+  hf_2b_all(c, c->hf_D, H->d, W->d, 1);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(c->hscal, c->hf_sc + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   if (coefs)
@@ -1259,8 +1280,7 @@ int imsrg_hartree_fock_noalloc(imsrg_op H, double *coefs, int *iterations, doubl
   if (H->herm != 1) return fail(IMSRG_EINVAL, "imsrg_hartree_fock_noalloc: H must be hermitian");
   if (!c->hf_scratch) return fail(IMSRG_EDEVICE, "imsrg_hartree_fock_noalloc: scratch not set up");
   const Layout &Ly = c->lay;
-  for (int n : Ly.grp_cnt)
-    if (n > kHFMaxGroup) return fail(IMSRG_EINVAL, "Hartree-Fock: an (l,j,tz) group has more than 16 orbits");
+  if (int rc = hf_limits(c)) return rc;
   auto a32 = [](long long x) { return (x + 31) & ~31LL; };
   const long long n2 = (long long)Ly.nsp * Ly.nsp;
   double *const base = c->hf_scratch;
@@ -1288,22 +1308,14 @@ int imsrg_hartree_fock_noalloc(imsrg_op H, double *coefs, int *iterations, doubl
       return fail(IMSRG_EINVAL, "imsrg_hartree_fock_noalloc: channel block " + std::to_string(q) + " (dim " +
                                     std::to_string(Ly.bdim[q]) + ") exceeds the scratch window of " +
                                     std::to_string(wcap) + " doubles");
-  double *D = m[0], *rho = m[1], *Vg = m[2], *Fm = m[3], *Tm = m[4], *W = base + state;
+  double *D = m[0], *Vg = m[2], *Fm = m[3], *Tm = m[4], *W = base + state;  // (m[1] unused)
   const DevLayout &DL = c->dl;
   launch_fill(c->stream, base, state, 0.0);
   launch_hf_init(c->stream, DL, H->d, D, Tm, eig, 1);
-  const double conv = (double)1e-6f;  // the reference's default-real loop test
   int it = 0;
-  for (;;) {
-    for (int k = 0; k < 8; k++)
-      launch_hf_iteration(c->stream, DL, H->d, D, rho, Tm, Vg, Fm, eig, cp, sc, sc + 2, conv);
-    HIPCHK(hipMemcpyAsync(c->hscal, sc, 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    it = (int)c->hscal[3];
-    if (c->hscal[2] != 0.0) break;
-    if (it >= 10000) return fail(IMSRG_ECONV, "Hartree-Fock did not converge in 10000 iterations");
-  }
+  if (int rc = hf_loop(c, H->d, D, Tm, Vg, Fm, eig, cp, sc, it)) return rc;
   launch_hf_finish_1b(c->stream, DL, D, Fm, H->d, 1, Tm, Vg, tv, sc + 1);
+  launch_hf_u(c->stream, DL, D, c->hf_U);
   // windows of consecutive channel blocks [q0, q1) whose blocks fit wcap
   for (int q0 = 0; q0 < Ly.nblocks;) {
     int q1 = q0 + 1;
@@ -1312,7 +1324,8 @@ int imsrg_hartree_fock_noalloc(imsrg_op H, double *coefs, int *iterations, doubl
       q1++;
     const int r0 = Ly.pbase[q0];
     const int nrows = Ly.pbase[q1 - 1] + Ly.bdim[q1 - 1] - r0;
-    launch_hf_2b_window(c->stream, DL, D, H->d, W, 1, r0, nrows, (long long)Ly.boff[q0]);
+    launch_hf_2b(c->stream, DL, c->hf_U, H->d, W, 1, r0, nrows, (long long)Ly.boff[q0], c->hf_items + c->hf_item0[q0],
+                 c->hf_item0[q1] - c->hf_item0[q0], c->hf_maxdim);
     q0 = q1;
   }
   HIPCHK(hipGetLastError());
@@ -1337,7 +1350,7 @@ int imsrg_observable_to_hf(imsrg_op O, const double *coefs) {
   launch_hf_finish_1b(c->stream, D, c->hf_D, c->hf_Tm, O->d, O->herm, nullptr, nullptr, nullptr, nullptr);
   imsrg_op_s *W = tmp_op(c, 5, O->herm);
   if (!W) return IMSRG_ENOMEM;
-  launch_hf_2b(c->stream, D, c->hf_D, O->d, W->d, O->herm);
+  hf_2b_all(c, c->hf_D, O->d, W->d, O->herm);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->stream));  // the caller's coefs may go away
   return imsrg_normal_order(O);

@@ -130,11 +130,18 @@ struct imsrg_ctx_s {
   int *act_d[kSlots] = {nullptr, nullptr, nullptr, nullptr};
   int *act_h[kSlots] = {nullptr, nullptr, nullptr, nullptr};
   imsrg_op_s *tmp[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  // Hartree-Fock workspace (allocated on first use): D, rho, gamma, Fock and
+  // Hartree-Fock workspace (allocated on first use): D, gamma, Fock and
   // bare one-body matrices (nsp x nsp), eigenvalues, e_HF diagonals,
   // per-group eigenvalue changes, and [crit, e_HF, converged flag, iterations]
-  double *hf_D = nullptr, *hf_rho = nullptr, *hf_Vg = nullptr, *hf_Fm = nullptr, *hf_Tm = nullptr;
+  double *hf_D = nullptr, *hf_Vg = nullptr, *hf_Fm = nullptr, *hf_Tm = nullptr;
   double *hf_eig = nullptr, *hf_tv = nullptr, *hf_cp = nullptr, *hf_sc = nullptr;
+  // two-body transform: weights (one per hf_nb entry) and row runs of the column
+  // pass, made with the context (imsrg_hartree_fock_noalloc allocates nothing);
+  // run k of block q from hf_item0[q]
+  double *hf_U = nullptr;
+  const int2 *hf_items = nullptr;
+  std::vector<int> hf_item0;
+  int hf_maxdim = 0;
   // this device's copy of the static Hartree-Fock scratch array (the
   // allocation-free entry point imsrg_hartree_fock_noalloc)
   double *hf_scratch = nullptr;

@@ -26,41 +26,58 @@ __global__ void k_hf_init(DevLayout L, const double *__restrict__ op, double *__
   }
 }
 
-// density_matrix (HF_mod.f90:346-373) without the (2j+1) that gamma_matrix
-// divides out again: rho(b,d) = sum over hole orbits i of the group of D(b,i) D(d,i)
-// state[0] != 0: the loop has converged and every kernel of a further
-// iteration returns at once (the host enqueues iterations in groups)
-__global__ void k_hf_density(DevLayout L, const double *__restrict__ D, double *__restrict__ rho,
-                             const double *__restrict__ state) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= L.n_hf_bd || state[0] != 0.0) return;
-  const int b = L.hf_b[t], d = L.hf_d[t], N = L.nsp, g = L.grp_of[b];
-  const int *mem = L.grp_list + L.grp_start[g];
+// One iteration is two launches, k_hf_gamma and k_hf_diag.  state = {converged,
+// iterations}: every kernel returns at once when converged (the host enqueues
+// iterations in groups).  The test on the groups' eigenvalue changes, in the
+// reference's block order (crit; `do while (crit > 1e-6)`), is made by every
+// workgroup of the next k_hf_gamma for itself, and noted by the first one.
+__device__ __forceinline__ bool hf_go_on(const DevLayout &L, const double *__restrict__ cpart, double *__restrict__ crit,
+                                         double *__restrict__ state, double conv, bool first, double *sh) {
+  if (state[0] != 0.0) return false;
+  if (first) return true;
   double s = 0.0;
-  for (int k = 0; k < L.grp_cnt[g]; k++) {
-    const int i = mem[k];
-    if (L.con[i]) s += D[b * N + i] * D[d * N + i];
+  for (int k0 = 0; k0 < L.ngrp; k0 += 256) {  // the changes side by side, summed one after another
+    const int k = k0 + (int)threadIdx.x;
+    __syncthreads();
+    sh[threadIdx.x] = k < L.ngrp ? cpart[L.hf_gorder[k]] : 0.0;
+    __syncthreads();
+    for (int i = 0; i < min(256, L.ngrp - k0); i++) s += sh[i];
   }
-  rho[b * N + d] = s;
+  __syncthreads();
+  const bool on = s > conv;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    crit[0] = s;
+    state[1] += 1.0;
+    if (!on) state[0] = 1.0;
+  }
+  return on;
 }
 
 // gamma_matrix (HF_mod.f90:169-232): for a <= c of one group,
 //   gam(a,c) = 1/(ja+1) sum_{groups, b, d} rho(d,b) sum_J (2J+1) v(a,b,c,d;J)
-// one workgroup per (a,c), threads over the (b,d) pairs; the Fock matrix
-// T + gam is written with it (both triangles)
+// with density_matrix (:346-373) formed in place, without the (2j+1) that
+// gamma_matrix divides out again: rho(b,d) = sum over hole orbits i of the
+// group of D(b,i) D(d,i).  One workgroup per (a,c), threads over the (b,d)
+// pairs; the Fock matrix T + gam is written with it (both triangles).
 __global__ __launch_bounds__(256) void k_hf_gamma(DevLayout L, const double *__restrict__ op,
-                                                  const double *__restrict__ rho, const double *__restrict__ Tm,
+                                                  const double *__restrict__ D, const double *__restrict__ Tm,
                                                   double *__restrict__ Vg, double *__restrict__ Fm,
-                                                  const double *__restrict__ state) {
+                                                  const double *__restrict__ cpart, double *__restrict__ crit,
+                                                  double *__restrict__ state, double conv, int first) {
   __shared__ double sh[256];
+  if (!hf_go_on(L, cpart, crit, state, conv, first != 0, sh)) return;
   const int t = blockIdx.x;
-  if (t >= L.n_hf_ac || state[0] != 0.0) return;
   const int a = L.hf_a[t], c = L.hf_c[t], ja = L.jj[a], N = L.nsp;
   const double *V = op + L.v_off;
   double s = 0.0;
   for (int e = threadIdx.x; e < L.n_hf_bd; e += 256) {
-    const int b = L.hf_b[e], d = L.hf_d[e], jr = L.jj[b];
-    const double r = rho[d * N + b];
+    const int b = L.hf_b[e], d = L.hf_d[e], jr = L.jj[b], g = L.grp_of[b];
+    const int *mem = L.grp_list + L.grp_start[g];
+    double r = 0.0;
+    for (int k = 0; k < L.grp_cnt[g]; k++) {
+      const int i = mem[k];
+      if (L.con[i]) r += D[d * N + i] * D[b * N + i];
+    }
     if (r == 0.0) continue;
     double sj = 0.0;
     for (int J = abs(jr - ja); J <= jr + ja; J += 2) sj += (J + 1.0) * dv(L, V, a, b, c, d, J);
@@ -171,17 +188,11 @@ __global__ __launch_bounds__(64) void k_hf_diag(DevLayout L, const double *__res
   cpart[g] = sqrt(cr);
 }
 
-// crit = sum of the groups' eigenvalue changes, in the reference's block
-// order; counts the iteration (state[1]) and ends the loop (state[0] = 1)
-// once crit > conv fails, as the reference's `do while (crit > 1e-6)`
-__global__ void k_hf_crit(DevLayout L, const double *__restrict__ cpart, double *__restrict__ crit,
-                          double *__restrict__ state, double conv) {
-  if (blockIdx.x != 0 || threadIdx.x != 0 || state[0] != 0.0) return;
-  double s = 0.0;
-  for (int k = 0; k < L.ngrp; k++) s += cpart[L.hf_gorder[k]];
-  crit[0] = s;
-  state[1] += 1.0;
-  if (!(s > conv)) state[0] = 1.0;
+// the test after the last iteration of a group of them
+__global__ __launch_bounds__(256) void k_hf_crit(DevLayout L, const double *__restrict__ cpart,
+                                                 double *__restrict__ crit, double *__restrict__ state, double conv) {
+  __shared__ double sh[256];
+  (void)hf_go_on(L, cpart, crit, state, conv, false, sh);
 }
 
 // eigenvectors with a negative diagonal component change sign (HF_mod.f90:84-89)
@@ -199,56 +210,52 @@ __global__ void k_hf_signfix(DevLayout L, double *__restrict__ D) {
 // M'(a,c) in both orders; a particle-hole entry takes M'(particle, hole), its
 // mirror herm times that.  With Tm/Vg, also the diagonals of D^T T D and
 // D^T gam D that e_HF sums (tv[2 i], tv[2 i + 1]).
-__global__ void k_hf_1b(DevLayout L, const double *__restrict__ D, const double *__restrict__ M,
-                        double *__restrict__ op, int herm, const double *__restrict__ Tm,
-                        const double *__restrict__ Vg, double *__restrict__ tv) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= L.n_hf_ac) return;
+// One wavefront per (a,c), lanes over the pairs of the group's orbits.
+__global__ __launch_bounds__(64) void k_hf_1b(DevLayout L, const double *__restrict__ D, const double *__restrict__ M,
+                                              double *__restrict__ op, int herm, const double *__restrict__ Tm,
+                                              const double *__restrict__ Vg, double *__restrict__ tv) {
+  const int t = blockIdx.x, lane = threadIdx.x;
   const int a = L.hf_a[t], c = L.hf_c[t], N = L.nsp, g = L.grp_of[a];
   const int *mem = L.grp_list + L.grp_start[g];
   const int m = L.grp_cnt[g];
   auto tr = [&](const double *X, int i, int k) {  // (D^T X D)(i, k)
     double s = 0.0;
-    for (int u = 0; u < m; u++) {
-      double r = 0.0;
-      for (int w = 0; w < m; w++) r += X[mem[u] * N + mem[w]] * D[mem[w] * N + k];
-      s += D[mem[u] * N + i] * r;
+    for (int e = lane; e < m * m; e += 64) {
+      const int u = mem[e / m], w = mem[e % m];
+      s += D[u * N + i] * (X[u * N + w] * D[w * N + k]);
     }
-    return s;
+    return wave_sum(s);
   };
   double *F = op + L.f_off;
-  if (L.con[a] == L.con[c]) {
-    F[a * N + c] = F[c * N + a] = tr(M, a, c);
-  } else if (L.con[a] == 0) {
-    const double v = tr(M, a, c);
-    F[a * N + c] = v;
-    F[c * N + a] = herm * v;
-  } else {
-    const double v = tr(M, c, a);
-    F[c * N + a] = v;
-    F[a * N + c] = herm * v;
-  }
+  const bool swap = L.con[a] != L.con[c] && L.con[a] != 0;  // the stored entry is (particle, hole)
+  const int i = swap ? c : a, k = swap ? a : c;
+  const double v = tr(M, i, k);
+  double t0 = 0.0, t1 = 0.0;
   if (tv && a == c) {
-    tv[2 * a] = tr(Tm, a, a);
-    tv[2 * a + 1] = tr(Vg, a, a);
+    t0 = tr(Tm, a, a);
+    t1 = tr(Vg, a, a);
+  }
+  if (lane != 0) return;
+  F[i * N + k] = v;
+  if (i != k) F[k * N + i] = L.con[a] == L.con[c] ? v : herm * v;
+  if (tv && a == c) {
+    tv[2 * a] = t0;
+    tv[2 * a + 1] = t1;
   }
 }
 
-// e_HF (HF_mod.f90:376-405): sum over hole orbits of (2j+1)(t + v/2), groups in
-// the reference's order, written as E0
-__global__ void k_hf_ehf(DevLayout L, const double *__restrict__ tv, double *__restrict__ op,
-                         double *__restrict__ out) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// e_HF (HF_mod.f90:376-405): sum over hole orbits of (2j+1)(t + v/2), written as E0
+__global__ __launch_bounds__(256) void k_hf_ehf(DevLayout L, const double *__restrict__ tv, double *__restrict__ op,
+                                                double *__restrict__ out) {
+  __shared__ double sh[256];
   double s = 0.0;
-  for (int k = 0; k < L.ngrp; k++) {
-    const int g = L.hf_gorder[k];
-    for (int x = 0; x < L.grp_cnt[g]; x++) {
-      const int i = L.grp_list[L.grp_start[g] + x];
-      if (L.con[i]) s += (tv[2 * i] + 0.5 * tv[2 * i + 1]) * (L.jj[i] + 1.0);
-    }
+  for (int i = threadIdx.x; i < L.nsp; i += 256)
+    if (L.con[i]) s += (tv[2 * i] + 0.5 * tv[2 * i + 1]) * (L.jj[i] + 1.0);
+  s = block_sum256(s, sh);
+  if (threadIdx.x == 0) {
+    op[0] = s;
+    out[0] = s;
   }
-  op[0] = s;
-  out[0] = s;
 }
 
 // Element (ab, ij) of the pair-basis transform U = C - (-1)^J Crev of
@@ -265,29 +272,48 @@ __device__ __forceinline__ double hf_u(const DevLayout &L, const double *D, int 
   return (i == j) ? u * .70710678118654752 : u;
 }
 
+// U(ab, ij) for every pair row (ij) and the rows (ab) it couples to, once per
+// transform; both passes read it (formed on the fly, its six dependent reads a
+// term were most of either pass)
+__global__ __launch_bounds__(64) void k_hf_u(DevLayout L, const double *__restrict__ D, double *__restrict__ U) {
+  const int r = blockIdx.x, q = L.pair_q[r], base = L.pbase[q], J = L.bJ[q];
+  const int i = L.pair_a[r], j = L.pair_b[r];
+  for (int e = L.hf_nb_start[r] + (int)threadIdx.x; e < L.hf_nb_start[r + 1]; e += 64) {
+    const int p = L.hf_nb[e];
+    U[e] = hf_u(L, D, L.pair_a[base + p], L.pair_b[base + p], i, j, J);
+  }
+}
+
 // pass 1: W = U^T V, row by row: W(ij, s) = sum over the rows (ab) that U
-// couples to (ij) of U(ab,ij) V(ab, s); one wavefront per pair row
-__global__ __launch_bounds__(64) void k_hf_rows(DevLayout L, const double *__restrict__ D,
+// couples to (ij) of U(ab,ij) V(ab, s); one wavefront per pair row and 256
+// columns, four of the rows read at a time.  L2-bound: every row of V is read
+// once per row it couples to.  emax 8: 100 -> 56 us.
+__global__ __launch_bounds__(64) void k_hf_rows(DevLayout L, const double *__restrict__ U,
                                                 const double *__restrict__ op, double *__restrict__ W, int r0,
                                                 long long wofs) {
   const int r = r0 + (int)blockIdx.x;
-  if (r >= L.npairs) return;
-  const int q = L.pair_q[r], base = L.pbase[q], rl = r - base, dim = L.bdim[q], J = L.bJ[q];
-  const int i = L.pair_a[r], j = L.pair_b[r];
+  const int q = L.pair_q[r], base = L.pbase[q], rl = r - base, dim = L.bdim[q];
   const double *VB = op + L.v_off + L.boff[q];
   double *WR = W + (L.v_off + L.boff[q] - wofs) + (long long)rl * dim;
   const int e0 = L.hf_nb_start[r], e1 = L.hf_nb_start[r + 1];
   for (int s0 = 0; s0 < dim; s0 += 256) {
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int e = e0; e < e1; e++) {
-      const int p = L.hf_nb[e];
-      const double u = hf_u(L, D, L.pair_a[base + p], L.pair_b[base + p], i, j, J);
-      const double *row = VB + (long long)p * dim;
+    for (int e = e0; e < e1; e += 4) {
+      double u[4], v[4][4];
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const int s = s0 + 64 * k + (int)threadIdx.x;
-        if (s < dim) acc[k] += u * row[s];
+      for (int x = 0; x < 4; x++) {
+        const int ex = min(e + x, e1 - 1);
+        const double *row = VB + (long long)L.hf_nb[ex] * dim;
+        u[x] = U[ex];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[x][k] = row[min(s0 + 64 * k + (int)threadIdx.x, dim - 1)];
       }
+#pragma unroll
+      for (int x = 0; x < 4; x++)
+        if (e + x < e1) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) acc[k] += u[x] * v[x][k];
+        }
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
@@ -299,27 +325,46 @@ __global__ __launch_bounds__(64) void k_hf_rows(DevLayout L, const double *__res
 
 // pass 2: V' = W U on the upper triangle, V'(ij, kl) = sum over the rows (ab)
 // U couples to (kl) of W(ij, ab) U(ab, kl); the lower triangle is herm times
-// the upper (diagonal zero for herm = -1); one wavefront per pair row (ij)
-__global__ __launch_bounds__(64) void k_hf_cols(DevLayout L, const double *__restrict__ D,
-                                                const double *__restrict__ W, double *__restrict__ op, int herm,
-                                                int r0, long long wofs) {
-  const int r = r0 + (int)blockIdx.x;
-  if (r >= L.npairs) return;
-  const int q = L.pair_q[r], base = L.pbase[q], rl = r - base, dim = L.bdim[q], J = L.bJ[q];
+// the upper (diagonal zero for herm = -1).  A workgroup takes up to R rows
+// (ij), staged in LDS, so that a column's weights are read once for all of
+// them and its mirror elements are written R together.  emax 8: 365 -> 60 us.
+// (Blocks past 8192 pairs: one row a workgroup, read where it lies.)
+template <int R, bool STAGE = true>
+__global__ __launch_bounds__(256) void k_hf_cols(DevLayout L, const double *__restrict__ U,
+                                                 const double *__restrict__ W, double *__restrict__ op, int herm,
+                                                 const int2 *__restrict__ items, long long wofs) {
+  extern __shared__ double WS[];
+  const int2 it = items[blockIdx.x];
+  const int r = it.x, n = it.y;  // first row, rows (of one block)
+  const int q = L.pair_q[r], base = L.pbase[q], rl = r - base, dim = L.bdim[q];
   const double *WR = W + (L.v_off + L.boff[q] - wofs) + (long long)rl * dim;
   double *VB = op + L.v_off + L.boff[q];
-  for (int s = rl + (int)threadIdx.x; s < dim; s += 64) {
-    const int k = L.pair_a[base + s], l = L.pair_b[base + s];
-    double acc = 0.0;
-    for (int e = L.hf_nb_start[base + s]; e < L.hf_nb_start[base + s + 1]; e++) {
+  if (STAGE) {
+    for (int e = threadIdx.x; e < R * dim; e += 256) WS[e] = e < n * dim ? WR[e] : 0.0;
+    __syncthreads();
+  }
+  const double *S = STAGE ? WS : WR;
+  for (int s = rl + (int)threadIdx.x; s < dim; s += 256) {
+    double acc[R];
+#pragma unroll
+    for (int k = 0; k < R; k++) acc[k] = 0.0;
+    const int e1 = L.hf_nb_start[base + s + 1];
+    for (int e = L.hf_nb_start[base + s]; e < e1; e++) {
       const int p = L.hf_nb[e];
-      acc += WR[p] * hf_u(L, D, L.pair_a[base + p], L.pair_b[base + p], k, l, J);
+      const double u = U[e];
+#pragma unroll
+      for (int k = 0; k < R; k++) acc[k] += S[k * dim + p] * u;
     }
-    if (s == rl) {
-      VB[(long long)rl * dim + s] = (herm == 1) ? acc : 0.0;
-    } else {
-      VB[(long long)rl * dim + s] = acc;
-      VB[(long long)s * dim + rl] = herm * acc;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+      const int row = rl + k;
+      if (k >= n || s < row) continue;
+      if (s == row) {
+        VB[(long long)row * dim + s] = (herm == 1) ? acc[k] : 0.0;
+      } else {
+        VB[(long long)row * dim + s] = acc[k];
+        VB[(long long)s * dim + row] = herm * acc[k];
+      }
     }
   }
 }
@@ -330,30 +375,40 @@ void launch_hf_init(hipStream_t s, const DevLayout &L, const double *op, double 
                     int reset) {
   hipLaunchKernelGGL(k_hf_init, dim3(nblk(L.n_hf_bd, 256)), dim3(256), 0, s, L, op, D, Tm, eig, reset);
 }
-void launch_hf_iteration(hipStream_t s, const DevLayout &L, const double *op, double *D, double *rho,
-                         const double *Tm, double *Vg, double *Fm, double *eig, double *cpart, double *crit,
-                         double *state, double conv) {
-  hipLaunchKernelGGL(k_hf_density, dim3(nblk(L.n_hf_bd, 256)), dim3(256), 0, s, L, D, rho, state);
-  hipLaunchKernelGGL(k_hf_gamma, dim3(L.n_hf_ac), dim3(256), 0, s, L, op, rho, Tm, Vg, Fm, state);
+void launch_hf_iteration(hipStream_t s, const DevLayout &L, const double *op, double *D, const double *Tm, double *Vg,
+                         double *Fm, double *eig, double *cpart, double *crit, double *state, double conv, int first) {
+  hipLaunchKernelGGL(k_hf_gamma, dim3(L.n_hf_ac), dim3(256), 0, s, L, op, (const double *)D, Tm, Vg, Fm,
+                     (const double *)cpart, crit, state, conv, first);
   hipLaunchKernelGGL(k_hf_diag, dim3(L.ngrp), dim3(64), 0, s, L, Fm, D, eig, cpart, state);
-  hipLaunchKernelGGL(k_hf_crit, dim3(1), dim3(64), 0, s, L, cpart, crit, state, conv);
+}
+void launch_hf_test(hipStream_t s, const DevLayout &L, const double *cpart, double *crit, double *state, double conv) {
+  hipLaunchKernelGGL(k_hf_crit, dim3(1), dim3(256), 0, s, L, cpart, crit, state, conv);
 }
 void launch_hf_finish_1b(hipStream_t s, const DevLayout &L, double *D, const double *M, double *op, int herm,
                          const double *Tm, const double *Vg, double *tv, double *ehf) {
   if (tv) hipLaunchKernelGGL(k_hf_signfix, dim3(nblk(L.nsp, 64)), dim3(64), 0, s, L, D);
-  hipLaunchKernelGGL(k_hf_1b, dim3(nblk(L.n_hf_ac, 64)), dim3(64), 0, s, L, D, M, op, herm, Tm, Vg, tv);
-  if (tv) hipLaunchKernelGGL(k_hf_ehf, dim3(1), dim3(64), 0, s, L, tv, op, ehf);
+  hipLaunchKernelGGL(k_hf_1b, dim3(L.n_hf_ac), dim3(64), 0, s, L, D, M, op, herm, Tm, Vg, tv);
+  if (tv) hipLaunchKernelGGL(k_hf_ehf, dim3(1), dim3(256), 0, s, L, tv, op, ehf);
 }
-void launch_hf_2b(hipStream_t s, const DevLayout &L, const double *D, double *op, double *W, int herm) {
-  if (L.npairs <= 0) return;
-  hipLaunchKernelGGL(k_hf_rows, dim3(L.npairs), dim3(64), 0, s, L, D, op, W, 0, 0LL);
-  hipLaunchKernelGGL(k_hf_cols, dim3(L.npairs), dim3(64), 0, s, L, D, W, op, herm, 0, 0LL);
+int hf_col_rows(int maxdim) {  // rows staged per workgroup: at most 64 KiB of LDS
+  return maxdim <= 1024 ? 8 : maxdim <= 2048 ? 4 : 1;
 }
-void launch_hf_2b_window(hipStream_t s, const DevLayout &L, const double *D, double *op, double *W, int herm,
-                         int r0, int nrows, long long wofs) {
+void launch_hf_u(hipStream_t s, const DevLayout &L, const double *D, double *U) {
+  if (L.npairs > 0) hipLaunchKernelGGL(k_hf_u, dim3(L.npairs), dim3(64), 0, s, L, D, U);
+}
+void launch_hf_2b(hipStream_t s, const DevLayout &L, const double *U, double *op, double *W, int herm, int r0,
+                  int nrows, long long wofs, const int2 *items, int nitems, int maxdim) {
   if (nrows <= 0) return;
-  hipLaunchKernelGGL(k_hf_rows, dim3(nrows), dim3(64), 0, s, L, D, op, W, r0, wofs);
-  hipLaunchKernelGGL(k_hf_cols, dim3(nrows), dim3(64), 0, s, L, D, W, op, herm, r0, wofs);
+  hipLaunchKernelGGL(k_hf_rows, dim3(nrows), dim3(64), 0, s, L, U, op, W, r0, wofs);
+  const int R = hf_col_rows(maxdim);
+  const size_t lds = sizeof(double) * R * maxdim;
+  if (maxdim > 8192) {
+    hipLaunchKernelGGL((k_hf_cols<1, false>), dim3(nitems), dim3(256), 0, s, L, U, W, op, herm, items, wofs);
+    return;
+  }
+  if (R == 8) hipLaunchKernelGGL(k_hf_cols<8>, dim3(nitems), dim3(256), lds, s, L, U, W, op, herm, items, wofs);
+  else if (R == 4) hipLaunchKernelGGL(k_hf_cols<4>, dim3(nitems), dim3(256), lds, s, L, U, W, op, herm, items, wofs);
+  else hipLaunchKernelGGL(k_hf_cols<1>, dim3(nitems), dim3(256), lds, s, L, U, W, op, herm, items, wofs);
 }
 
 }  // namespace imsrg

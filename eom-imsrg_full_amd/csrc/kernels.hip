@@ -1937,59 +1937,54 @@ void launch_generator(hipStream_t s, const DevLayout &L, const double *Hden, con
 }
 
 // ------------------------------------------------------------------ normal ordering
-// normal_order (basic_IMSRG.f90:2375-2506); T is an unmodified copy of H
-__global__ __launch_bounds__(256) void k_no_e0(DevLayout L, const double *T, double *H, const int *act) {
+// normal_order (basic_IMSRG.f90:2375-2506) in place: E0 from the one-body
+// diagonal and the two-body part, then the one-body part, each entry from
+// itself and the two-body part (which stays as it is).  The (hole, J) terms of
+// a sum lie side by side over the lanes.
+__global__ __launch_bounds__(256) void k_no_e0(DevLayout L, double *H, const int *act) {
   __shared__ double sh[256];
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    const long long o = inst * L.op_size;
-    T += o;
-    H += o;
-  }
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  H += inst * L.op_size;
   const int N = L.nsp;
-  const double *F = T + L.f_off, *V = T + L.v_off;
+  const double *F = H + L.f_off, *V = H + L.v_off;
   double s1 = 0.0;
   for (int i = threadIdx.x; i < N; i += 256) s1 += F[i * N + i] * L.con[i] * (L.jj[i] + 1);
   s1 = block_sum256(s1, sh);
   double s2 = 0.0;
-  for (int e = threadIdx.x; e < N * N; e += 256) {
-    const int i = e / N, j = e % N;
-    if (L.con[i] * L.con[j] == 0) continue;
-    for (int JT = abs(L.jj[i] - L.jj[j]); JT <= L.jj[i] + L.jj[j]; JT += 2)
-      s2 = s2 + dv(L, V, i, j, i, j, JT) * (JT + 1);
+  const int A = L.nhole, MJ = L.nJ;
+  for (int e = threadIdx.x; e < A * A * MJ; e += 256) {
+    // the first A (A + 1) / 2 one-body outputs are the hole pairs; entry (k, k) of row k names hole k
+    const int x = e / (A * MJ), y = (e / MJ) % A;
+    const int i = L.ob_p[x * A - x * (x - 1) / 2], j = L.ob_p[y * A - y * (y - 1) / 2];
+    const int JT = abs(L.jj[i] - L.jj[j]) + 2 * (e % MJ);
+    if (JT <= L.jj[i] + L.jj[j]) s2 = s2 + dv(L, V, i, j, i, j, JT) * (JT + 1);
   }
   s2 = block_sum256(s2, sh);
   if (threadIdx.x == 0) H[0] = (s1 * 2.0 + s2) * 0.5;
 }
-__global__ void k_no_f(DevLayout L, const double *T, double *H, int herm, const int *act) {
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    const long long o = inst * L.op_size;
-    T += o;
-    H += o;
-  }
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= L.nob) return;
-  const int a = L.ob_p[t], b = L.ob_q[t], N = L.nsp;
-  if (!same_ljt(L, a, b)) return;
-  const double *V = T + L.v_off;
+__global__ __launch_bounds__(64) void k_no_f(DevLayout L, double *H, int herm, const int *act) {
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  H += inst * L.op_size;
+  const int t = L.same_ob[blockIdx.x], a = L.ob_p[t], b = L.ob_q[t], N = L.nsp, A = L.nhole, MJ = L.nJ;
+  const double *V = H + L.v_off;
   double s2 = 0.0;
-  for (int ii = 0; ii < N; ii++) {
-    if (L.con[ii] != 1) continue;
-    for (int JT = abs(L.jj[ii] - L.jj[a]); JT <= L.jj[ii] + L.jj[a]; JT += 2)
-      s2 = s2 + (JT + 1.0) / (L.jj[a] + 1) * dv(L, V, a, ii, b, ii, JT);
+  for (int e = threadIdx.x; e < A * MJ; e += 64) {
+    const int x = e / MJ, ii = L.ob_p[x * A - x * (x - 1) / 2];
+    const int JT = abs(L.jj[ii] - L.jj[a]) + 2 * (e % MJ);
+    if (JT <= L.jj[ii] + L.jj[a]) s2 = s2 + (JT + 1.0) / (L.jj[a] + 1) * dv(L, V, a, ii, b, ii, JT);
   }
-  const double val = T[L.f_off + a * N + b] + s2;
+  s2 = wave_sum(s2);
+  if (threadIdx.x != 0) return;
+  const double val = H[L.f_off + a * N + b] + s2;
   H[L.f_off + a * N + b] = val;
   if (a != b) H[L.f_off + b * N + a] = herm * val;
 }
-void launch_normal_order(hipStream_t s, const DevLayout &L, const double *T, double *H, const int *act,
-                         int nact) {
+void launch_normal_order(hipStream_t s, const DevLayout &L, double *H, const int *act, int nact) {
   if (nact <= 0) return;
-  hipLaunchKernelGGL(k_no_e0, dim3(1, nact), dim3(256), 0, s, L, T, H, act);
-  if (L.nob > 0) hipLaunchKernelGGL(k_no_f, dim3((L.nob + 63) / 64, nact), dim3(64), 0, s, L, T, H, 1, act);
+  hipLaunchKernelGGL(k_no_e0, dim3(1, nact), dim3(256), 0, s, L, H, act);
+  if (L.nsame > 0) hipLaunchKernelGGL(k_no_f, dim3(L.nsame, nact), dim3(64), 0, s, L, H, 1, act);
 }
 
 // E0 of every active instance of an operator into out[inst * kScal]

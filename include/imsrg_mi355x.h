@@ -154,7 +154,8 @@ int imsrg_hartree_fock(imsrg_op H, double *coefs, int *iterations, double *e_hf)
  * results and errors as imsrg_hartree_fock (bit for bit), but every work
  * buffer lives in one static 16 MiB device array per GPU (held until the
  * process ends): the self-consistency state (5 nsp^2 + 3 nsp doubles and a
- * few more) and windows of whole channel blocks for the two-body transform.
+ * few more) and windows of whole channel blocks for the two-body transform (whose
+ * pair weights are made with the context).
  * Returns IMSRG_EINVAL when the state or one channel block does not fit.
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * (two host threads, two contexts on one device) race. */
