@@ -45,27 +45,33 @@ struct DevTensor {
   const int *bidx;                // [((J1/2)*nJ + J2/2)*6 + (Tz+1)*2 + P1] -> block (J1 <= J2) or -1
   const int *cJ3, *cJ4, *cq3, *cq4;
   const long long *xoff, *roff, *woff, *xstart, *rstart;
-  const int *cidx;                // [((J3/2)*nJ + J4/2)*4 + Tz*2 + P] -> cross-coupled block or -1
   const int *ccol;                // [(scalar Pandya block * nsp + p) * nsp + h] -> column of (p,h)
   const double *x6, *s6;
   const double *n9;               // 9j table of the ph recoupling and the tensor Pandya (k_fill9j)
   int nd;                         // rank/2 + 1: J4 - J3 and J2 - J1 steps the table holds
-  const unsigned *quads;          // orbit quadruples x0|x1<<8|x2<<16|x3<<24 (x0 <= x1, x2 <= x3) with outputs
-  long long nquad;
-  int nslotmax;                   // most gather slots of any quadruple (k_t222ph_q's LDS list)
-  // the quadruples in four runs by slot count (at most 256, 384, 512,
-  // nslotmax), one launch each with an LDS list of that size: run k starts
-  // at qrun[k]
-  long long qrun[5];
-  int qcap[4];
+  // the ph recoupling's orbit quadruples x0|x1<<8|x2<<16|x3<<24 (x0 <= x1,
+  // x2 <= x3, with stored outputs), class by class (the (l,j,tz) groups of the
+  // four orbits), and its work items (first quadruple, 1..kPhQ quadruples of
+  // one class)
+  const unsigned *quads;
+  const struct PhChunkT *qchunk;
+  int nqchunk, nqpad;             // items; rounded up to whole runs of 64 on 8 XCDs
+  // [(p * nsp + h) * nJ + J/2]: row of the ordered pair in its Pandya block and
+  // the row's place in group order, or -1
+  const int *crow, *cpos;
+  const int *prow;                // [(a * nsp + b) * nJ + J/2], a <= b: row of the pair in its channel, or -1
+  const struct OutBlk *oblk;      // [(J1/2 * nd + (J2-J1)/2) * 6 + (Tz+1)*2 + P1]: tensor blocks
+  const struct CcBlk *cblk;       // [((Tz + 2*P) * nJ + J3/2) * nd + (J4-J3)/2]: cross-coupled product blocks
   // the orbits i the tensor's one-body part couples to orbit x (same tz, l + dpar/2
   // of the same parity, triangle (ji, jx, R)): part[pstart[x] .. pstart[x+1]),
   // each i | ji << 8
   const int *pstart, *part;
-  // thread orders of k_tpandya inside each scalar Pandya block: columns by
-  // (2j of p, 2j of h), rows by the 2j of their two orbits (zero rows last),
-  // so that the lanes of a wavefront sum (J3', J4') runs of equal length;
-  // entry i is the block-local column / row thread i computes
+  // orders inside each scalar Pandya block: columns by (2j of p, 2j of h), rows
+  // by the (l,j,tz) groups of their two orbits (zero rows last); entry i is
+  // the block-local column / row in place i.  k_tpandya's threads take them
+  // so, so that the lanes of a wavefront sum (J3', J4') runs of equal length,
+  // and CCR, Wx and Wy keep their columns in the rows' order: the entries that
+  // quadruples of one class read then share cache lines
   const int *cperm, *rperm;
   // thread order of the 122 and 212 gathers inside each tensor block's rows:
   // the ket pairs of every scalar block by the (l,j,tz) groups of their two
@@ -73,6 +79,25 @@ struct DevTensor {
   // column thread i of a row computes
   const int *sperm;
   long long f_off, v_off;
+};
+
+// a cross-coupled product block: offset of W (negative: none) and its row length
+struct alignas(16) CcBlk {
+  long long wo;
+  int rl4, pad;
+};
+
+// a tensor block: offset in V (negative: none) and its columns
+struct alignas(16) OutBlk {
+  long long off;
+  int n2, pad;
+};
+
+// up to kPhQ quadruples of one class: the first's position, the four orbits'
+// 2j a byte each, their parities of l (bits 0-3) and tz > 0 (bits 4-7), count
+struct alignas(16) PhChunkT {
+  unsigned first, jv, lt;
+  int n;
 };
 
 // A product C (M x N, row-major, ldc) = sum of nseg segments alpha * A * B
@@ -128,6 +153,9 @@ __device__ __forceinline__ double t9j_cc(const DevTensor &T, int a, int b, int J
   const double v = T.n9[n9_index(T, b, a, d, c, J3, J4, J4p, J3p)];
   return ((a + b + J3 + c + d + J4 + J3p + J4p + T.rank) >> 1) & 1 ? -v : v;
 }
+// zeros past the table: a lane's pair of outputs may start up to a wavefront's
+// width of pairs past its row
+constexpr int kN9Pad = 256;
 __global__ void k_fill9j(DevTensor T, double *__restrict__ n9, long long n) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
@@ -553,7 +581,7 @@ __global__ void k_t212(DevLayout L, DevTensor T, const double *__restrict__ GV, 
 // Tensor Pandya matrices of one cross-coupled block (calculate_single_pandya,
 // cross_coupled.f90:1416-1634).  mode 0: CCX (r3 x nb4, rows = ordered pairs at
 // J3 in the scalar Pandya row order, columns = (p,h) at J4); mode 1: CCR
-// (nb3 x r4, rows = (p,h) at J3, columns = ordered pairs (b,a) at J4).
+// (nb3 x r4, rows = (p,h) at J3, columns = ordered pairs (b,a) at J4 in group order).
 __global__ void k_tpandya(DevLayout L, DevTensor T, int mode, const double *__restrict__ RV, double *__restrict__ out,
                           int hR) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -576,7 +604,7 @@ __global__ void k_tpandya(DevLayout L, DevTensor T, int mode, const double *__re
   } else {
     const int r4 = L.ccrlen[q4];
     const int k = (int)(u / r4), G = T.rperm[L.ccrbase[q4] + (int)(u % r4)];
-    o = (long long)k * r4 + G;
+    o = u;
     p = L.cccol_p[L.cccbase[q3] + k];
     h = L.cccol_h[L.cccbase[q3] + k];
     b = L.ccrow_a[L.ccrbase[q4] + G];  // the row pair is (b, a)
@@ -622,19 +650,26 @@ __global__ void k_tpandya(DevLayout L, DevTensor T, int mode, const double *__re
   out[(mode == 0 ? T.xoff[x] : T.roff[x]) + o] = v;
 }
 
+// The scalar Pandya matrices with each column's rows in group order: the right
+// operand of Wy
+__global__ void k_gcc_order(DevLayout L, DevTensor T, const double *__restrict__ gcc, double *__restrict__ out) {
+  const int col = blockIdx.x, q = L.cccol_q[col], rl = L.ccrlen[q];
+  const long long o = L.ccoff[q] + (long long)(col - L.cccbase[q]) * rl;
+  const int *ix = T.rperm + L.ccrbase[q];
+  for (int i = threadIdx.x; i < rl; i += 256) out[o + i] = gcc[o + ix[i]];
+}
+
 // The ph recoupling of TS_commutator_222_ph (TS_commutators.f90:1459-1849) as
-// a gather by orbit quadruple (x0 <= x1 | x2 <= x3), one wavefront each.  The
-// reference adds every product entry W(IX = (d,a) at J3, JX = (c,b) at J4)
-// (Wx or Wy) into up to 16 x (J1, J2) outputs; read backwards, an output
-// (x0 x1 | x2 x3; J1 J2) receives entries through sixteen patterns: the source
-// orbits (a,b,c,d) as a permutation of x, the orbit-order condition of the
-// reference's branch, one of four 9j argument orders, a phase and a herm
-// factor.  The entries a quadruple's outputs read do not depend on the
-// outputs' (J1, J2): they are gathered once, over (pattern, J3, J4), with the
-// parts of their weights that do not depend on (J1, J2) (sign, herm, (J3,J4)
-// phase and norm, the |W| test) and the (J1, J2)-independent part of their 9j
-// table index, into a compacted LDS list; each output (J1, J2) of the
-// quadruple then sums the list across the lanes.
+// a gather by orbit quadruple (x0 <= x1 | x2 <= x3).  The reference adds every
+// product entry W(IX = (d,a) at J3, JX = (c,b) at J4) (Wx or Wy) into up to
+// 16 x (J1, J2) outputs; read backwards, an output (x0 x1 | x2 x3; J1 J2)
+// receives entries through sixteen patterns: the source orbits (a,b,c,d) as a
+// permutation of x, the orbit-order condition of the reference's branch, one
+// of four 9j argument orders, a phase and a herm factor.  The entries a
+// quadruple's outputs read, over the slots (pattern, J3, J4), do not depend on
+// the outputs' (J1, J2), and the weights do not depend on the orbits' radial
+// numbers: quadruples of the same four (l,j,tz) groups share slots, weights
+// and outputs' (J1, J2).  See k_t222ph.
 //
 // The sixteen patterns (TS_commutators.f90:1562-1849): the output receives
 // W(d,a;c,b) times P * 9j * sign * herm, P = sqrt((2J1+1)(2J2+1)(2J3+1)(2J4+1)),
@@ -664,37 +699,77 @@ __global__ void k_tpandya(DevLayout L, DevTensor T, int mode, const double *__re
 // 2: x2 < x3, 3: both)
 constexpr unsigned kPhIa = 0x2727DD88u, kPhIb = 0x88DD88DDu, kPhIc = 0x72727272u, kPhId = 0xDD882727u;
 constexpr unsigned kPhCond = 0xF960F960u;
-struct PhSlot {
-  double c;      // sign * herm * phase(J3,J4) * sqrt((2J3+1)(2J4+1)) * W
-  unsigned b9;   // 9j table index without the (J1, J2) part
-  int ab;        // bit 0: (-1)^(J1/2) applies, bit 1: (-1)^(J2/2) applies
+constexpr int kPhQ = 8;    // quadruples of one class per workgroup
+constexpr int kPhU = 2;    // slots whose 9j a lane reads together
+struct PhPat {
+  double cs;     // sign * herm
+  unsigned b9;   // 9j table index of the four orbits' 2j
+  int start;     // first slot
+  int j3;        // first J3 of its run
+  int flags;     // Tz | parity of the J3 pairs << 1 | ab << 3 | ph34 << 5 | lowest J4 << 6 | highest << 18
 };
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void k_t222ph_q(
-    DevLayout L, DevTensor T, const double *__restrict__ Wx, const double *__restrict__ Wy, double *__restrict__ OV,
-    int hL, int hR, int run) {
-  extern __shared__ double ph_lds[];
-  PhSlot *slot = reinterpret_cast<PhSlot *>(ph_lds);
-  __shared__ int pa[16], pb[16], pc[16], pd[16], pok[16], pab[16], pph[16], pj[16][4], pj3[16], pstart[17];
-  __shared__ double pcs[16];
-  const long long qd = T.qrun[run] + blockIdx.x;
-  const int lane = threadIdx.x, cap = T.qcap[run];
-  if (qd >= T.qrun[run + 1]) return;
-  const unsigned code = T.quads[qd];
-  const int x0 = code & 255, x1 = (code >> 8) & 255, x2 = (code >> 16) & 255, x3 = (int)(code >> 24);
-  const int R = T.rank, n = L.nsp, JM = L.jtot_max, nd = T.nd, nJ = T.nJ, h = T.nh, dpb = (T.dpar >> 1) & 1;
-  if (lane < 16) {
-    const int k = lane;
-    auto pick = [&](unsigned tbl) {
-      const int i = (tbl >> (2 * k)) & 3;
-      return i == 0 ? x0 : i == 1 ? x1 : i == 2 ? x2 : x3;
-    };
-    const int a = pick(kPhIa), b = pick(kPhIb), c = pick(kPhIc), d = pick(kPhId);
-    // the branch condition of the reference
-    const unsigned cond = (kPhCond >> (2 * k)) & 3;
-    bool ok = (!(cond & 1) || x0 < x1) && (!(cond & 2) || x2 < x3);
-    const int ja = L.jj[a], jb = L.jj[b], jc = L.jj[c], jd = L.jj[d];
-    const int Tz = abs(L.tz[d] - L.tz[a]) >> 1, PAR = (L.l[d] + L.l[a]) & 1, PAR2 = PAR ^ ((T.dpar >> 1) & 1);
-    if (((L.l[c] + L.l[b]) & 1) != PAR2 || (abs(L.tz[c] - L.tz[b]) >> 1) != Tz) ok = false;
+struct PhSeg {
+  double c;       // sign * herm * phase(J3,J4) * sqrt((2J3+1)(2J4+1))
+  long long w;    // offset of the slot's product block << 24 | its row length
+  unsigned b9;    // 9j table row without the (J1, J2) part | ab << 30
+  unsigned code;  // pattern | J3/2 << 4 | J4/2 << 12
+};
+// One wavefront takes up to kPhQ quadruples of one class, 32 slots at a time:
+//   1. one lane per slot finds the slots that exist (J4's triangle, no Wy at
+//      J3 = J4), their (J3, J4) weights and product blocks;
+//   2. lanes (slot, quadruple) read the product entries, rows and columns from
+//      per-pair tables (a quadruple's run over J3 is contiguous there); the
+//      entries that pass the reference's |W| > 1e-6 test go weighted to LDS,
+//      slots with no entry left are dropped;
+//   3. groups of lanes as wide as half the outputs take a slot each: a lane
+//      reads the 9j of its two neighbouring outputs (the (J1, J2) part is the
+//      table's fastest index, so a group reads one contiguous run) and adds
+//      slot x output into all kPhQ quadruples from LDS.
+// What bounds it: the entries' reads (W is 1 GB at 90 orbits, rank 4) and the
+// index arithmetic around them.  One wavefront per quadruple with a lane per
+// slot read a 9j cache line per (slot, output): 7.7 ms there (2.6 M
+// quadruples, 256 M slots, 3 G slot-outputs); this form 2.8 ms, 5.3 before
+// the columns of W went into class order.
+// W: Wx, then Wy wsize doubles on
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_t222ph(DevLayout L, DevTensor T, const double *__restrict__ W,
+    long long wsize, double *__restrict__ OV, int hL, int hR) {
+  __shared__ PhPat pat[16];
+  __shared__ PhSeg seg[32 + 64];
+  __shared__ ushort2 base[16][kPhQ];  // per pattern and quadruple: the orbit pairs (d,a) and (c,b)
+  __shared__ alignas(16) double cs[32 + 1][kPhQ];
+  __shared__ unsigned sb9[32 + 1];
+  // runs of 64 class-ordered items per XCD, in turn: its L2 keeps the 9j rows
+  // and product entries that neighbouring items share, and the classes of
+  // high j, with the most slots, spread over all XCDs
+  const int bid = T.nqpad - 1 - (int)blockIdx.x, i8 = bid >> 3;  // the heavy classes come first
+  const int item = ((i8 >> 6) << 9) + ((bid & 7) << 6) + (i8 & 63);
+  if (item >= T.nqchunk) return;
+  const int lane = threadIdx.x;
+  const PhChunkT ch = T.qchunk[item];
+  const int nq = ch.n, R = T.rank, n = L.nsp, JM = L.jtot_max, nd = T.nd, nJ = T.nJ, h = T.nh;
+  const int quad = lane & (kPhQ - 1);
+  const unsigned code = T.quads[ch.first + min(quad, nq - 1)];  // the lane's quadruple
+  // the pattern conditions the lane's quadruple fails (1: x0 < x1, 2: x2 < x3)
+  const unsigned drop = ((code & 255) == ((code >> 8) & 255) ? 1u : 0u) |
+                        (((code >> 16) & 255) == code >> 24 ? 2u : 0u);
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int k = 8 * u + (lane >> 3);
+    auto orb = [&](unsigned tbl) { return (int)((code >> (8 * ((tbl >> (2 * k)) & 3))) & 255); };
+    base[k][quad] = make_ushort2((unsigned short)(orb(kPhId) * n + orb(kPhIa)),
+                                 (unsigned short)(orb(kPhIc) * n + orb(kPhIb)));
+  }
+  const int j0 = ch.jv & 255, j1 = (ch.jv >> 8) & 255, j2 = (ch.jv >> 16) & 255, j3 = (int)(ch.jv >> 24);
+  int nslot;
+  {
+    const int k = lane & 15;
+    auto orb = [&](unsigned tbl) { return (int)((tbl >> (2 * k)) & 3); };
+    const int oa = orb(kPhIa), ob = orb(kPhIb), oc = orb(kPhIc), od = orb(kPhId);
+    const int ja = (ch.jv >> (8 * oa)) & 255, jb = (ch.jv >> (8 * ob)) & 255;
+    const int jc = (ch.jv >> (8 * oc)) & 255, jd = (ch.jv >> (8 * od)) & 255;
+    const unsigned lt = ch.lt, ad_ = (lt >> oa) ^ (lt >> od), bc_ = (lt >> ob) ^ (lt >> oc);  // l, tz differences
+    const int Tz = (ad_ >> 4) & 1, PAR = ad_ & 1, PAR2 = PAR ^ ((T.dpar >> 1) & 1);
+    const bool ok = (int)(bc_ & 1) == PAR2 && (int)((bc_ >> 4) & 1) == Tz;
     // constant sign exponent (halves), J1/J2 flags and the (J3,J4) phase of each pattern
     // (TS_commutators.f90:1562-1849)
     int e = 0, ab = 0;
@@ -721,140 +796,213 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void k_
     const bool ph34 = (k < 8) ? !(k & 1) : (k & 1);
     // the 9j argument order of the pattern: (ja,jd | jb,jc), (jd,ja | jc,jb), (jd,ja | jb,jc), (ja,jd | jc,jb)
     const int var = (k < 8) ? (k & 1) : 2 + (k & 1);
-    pa[k] = a; pb[k] = b; pc[k] = c; pd[k] = d;
-    pok[k] = ok ? (Tz | (PAR << 1) | 4) : 0;
-    pj3[k] = abs(jd - ja);                                   // the pattern's J3 run: |jd-ja| .. jd+ja
-    pstart[k + 1] = ok ? (((jd + ja - abs(jd - ja)) >> 1) + 1) * nd : 0;  // its slots (J3, J4 - J3)
-    pab[k] = ab;
-    pph[k] = ph34;
-    pcs[k] = sg * sgnp(e) * ((k & 1) ? hR : hL);
-    pj[k][0] = (var == 0 || var == 3) ? ja : jd;
-    pj[k][1] = (var == 0 || var == 3) ? jd : ja;
-    pj[k][2] = (var == 0 || var == 2) ? jb : jc;
-    pj[k][3] = (var == 0 || var == 2) ? jc : jb;
-  }
-  __syncthreads();
-  if (lane == 0) {
-    pstart[0] = 0;
-    for (int k = 0; k < 16; k++) pstart[k + 1] += pstart[k];
-  }
-  __syncthreads();
-  // gather: slots (pattern, J3 of its run, J4 - J3), compacted to the entries that pass
-  const int nslot = pstart[16];
-  const double thr = (double)1e-6f;
-  int count = 0, k = 0;  // a lane's pattern: its slot only grows, so k carries over
-  for (int s0 = 0; s0 < nslot; s0 += 64) {
-    const int s = s0 + lane;
-    bool live = false;
-    double cval = 0.0;
-    unsigned b9 = 0;
-    int abk = 0;
-    {
-      // every table read is made for every lane, with indices in range
-      // whatever the tests say, so that they are in flight together: the
-      // entry's row IX = (d,a) in the J3 Pandya block, its column JX = (c,b)
-      // in the J4 one (the block index is arithmetic: J4, Tz and the parity of
-      // the J3 pairs with the tensor's), the product's block, then W
-      const int sc = min(s, nslot - 1);
-      while (pstart[k + 1] <= sc) k++;
-      const int r = sc - pstart[k], J3 = pj3[k] + 2 * (r / nd), J4 = J3 + 2 * (r % nd);
-      const int okc = pok[k];
-      const int a = pa[k], b = pb[k], c = pc[k], d = pd[k], Tz = okc & 1, PAR = (okc >> 1) & 1;
-      const int ja = L.jj[a], jb = L.jj[b], jc = L.jj[c], jd = L.jj[d];
-      const bool isx = k < 8;
-      const bool tri = s < nslot && okc && dtri(jd, ja, J3) && J4 <= 2 * JM && dtri(J3, J4, R) &&
-                       dtri(jc, jb, J4) && (isx || J4 != J3);
-      const int J4c = min(J4, 2 * JM);
-      const int q3 = (J3 >> 1) + Tz * (JM + 1) + 2 * PAR * (JM + 1);
-      const int q4 = (J4c >> 1) + Tz * (JM + 1) + 2 * (PAR ^ dpb) * (JM + 1);
-      const int IX = L.ccrow[((size_t)q3 * n + d) * n + a];
-      const int JX = L.ccrow[((size_t)q4 * n + c) * n + b];
-      const int qx = T.cidx[((J3 >> 1) * nJ + (J4c >> 1)) * 4 + Tz * 2 + PAR];
-      const int rl4 = L.ccrlen[q4];
-      const long long wo = T.woff[max(qx, 0)];
-      const bool ok = tri && IX >= 0 && JX >= 0 && qx >= 0;
-      const long long wi = ok ? wo + (long long)IX * rl4 + JX : 0;
-      const double wv = (isx ? Wx : Wy)[wi];
-      const double w = ok ? (isx ? hL * wv : wv) : 0.0;  // Wx carries LCC%herm (TS_commutators.f90:1506)
-      if (fabs(w) > thr) {
-        live = true;
-        cval = pcs[k] * (pph[k] ? (double)sgnp((J3 + J4) >> 1) : 1.0) * sqrt((J3 + 1.0) * (J4 + 1.0)) * w;
-        b9 = (unsigned)((((((pj[k][0] >> 1) * h + (pj[k][1] >> 1)) * h + (pj[k][2] >> 1)) * h +
-                          (pj[k][3] >> 1)) * nJ + (J3 >> 1)) * nd + ((J4 - J3) >> 1)) * (unsigned)(nJ * nd);
-        abk = pab[k];
-      }
+    const bool ad = var == 0 || var == 3, bc = var == 0 || var == 2;
+    const int len = ok ? (((jd + ja - abs(jd - ja)) >> 1) + 1) * nd : 0;  // slots (J3 of |jd-ja| .. jd+ja, J4 - J3)
+    int end = len;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      const int v = __shfl_up(end, o, 16);
+      if (k >= o) end += v;
     }
-    const unsigned long long m = __ballot(live);
-    if (live) {
-      // pos < this quadruple's slot count <= its run's cap (the host counts the same slots)
-      const int pos = min(count + __popcll(m & ((1ull << lane) - 1ull)), cap - 1);
-      slot[pos].c = cval;
-      slot[pos].b9 = b9;
-      slot[pos].ab = abk;
+    nslot = __shfl(end, 15, 64);
+    if (lane < 16) {
+      PhPat p;
+      p.cs = sg * sgnp(e) * ((k & 1) ? hR : hL);
+      p.b9 = (unsigned)(((((ad ? ja : jd) >> 1) * h + ((ad ? jd : ja) >> 1)) * h + ((bc ? jb : jc) >> 1)) * h +
+                        ((bc ? jc : jb) >> 1));
+      p.start = end - len;
+      p.j3 = abs(jd - ja);
+      p.flags = Tz | PAR << 1 | ab << 3 | (ph34 ? 32 : 0) | abs(jc - jb) << 6 | (jc + jb) << 18;
+      pat[k] = p;
     }
-    count += __popcll(m);
   }
-  __syncthreads();
-  if (count == 0) return;
-  // outputs (x0 x1 | x2 x3; J1 <= J2) of the quadruple, 64 at a time: lane o
-  // takes J1 = |j0 - j1| + 2 (o / nd), J2 = J1 + 2 (o % nd), finds its element
-  // and reads its old value (every table read off any branch, for all the
-  // outputs at once); the outputs' sums over the slots then go four at a time
-  // (their 9j reads in flight together), each lane keeps its own output's sum,
-  // and the lanes write their elements together.
-  const int j0 = L.jj[x0], j1 = L.jj[x1], j2 = L.jj[x2], j3 = L.jj[x3];
-  const int Tzq = (L.tz[x0] + L.tz[x1]) / 2 + 1, P1 = (L.l[x0] + L.l[x1]) & 1;
-  const double pre = (x0 == x1 ? M_SQRT2 : 1.0) * (x2 == x3 ? M_SQRT2 : 1.0);
+  // outputs (x0 x1 | x2 x3; J1 <= J2): o = (J1 - |j0-j1|)/2 * nd + (J2 - J1)/2
   const int Jlo = abs(j0 - j1), nout = (min(j0, j1) + 1) * nd;
-  for (int o0 = 0; o0 < nout; o0 += 64) {
-    const int o = o0 + lane;
-    const int J1 = Jlo + 2 * (o / nd), J2 = J1 + 2 * (o % nd);
-    bool val = o < nout && J1 <= j0 + j1 && J2 >= abs(j2 - j3) && J2 <= j2 + j3 && J1 + J2 >= R &&
-               !(x0 == x1 && ((J1 >> 1) & 1)) && !(x2 == x3 && ((J2 >> 1) & 1));
-    const int J1c = val ? J1 : Jlo, J2c = val ? J2 : Jlo;  // in the tables' range
-    const int q = T.bidx[((J1c >> 1) * nJ + (J2c >> 1)) * 6 + Tzq * 2 + P1];
-    const int r = dpos(L, J1c, x0, x1), sc = dpos(L, J2c, x2, x3);
-    const int qc = max(q, 0);
-    val = val && q >= 0 && (r | sc) >= 0;
-    const long long po = val ? T.off[qc] + (long long)r * T.n2[qc] + sc : 0;
-    const double old = OV[po];
-    unsigned long long vm = __ballot(val);
-    double res = 0.0;
-    while (vm) {
-      int ok_[4];
-      unsigned offk[4];
-      int ek[4][2];
+  const int Tzq = ((ch.lt >> 4) & 1) + ((ch.lt >> 5) & 1), P1 = (ch.lt ^ (ch.lt >> 1)) & 1;
+  const double thr = (double)1e-6f;
+  const int ndinv = 65536 / nd + 1;  // x / nd, exact for x <= 32 nd + 128, nd <= 50
+  auto div = [&](int x) { return (x * ndinv) >> 16; };
+  __syncthreads();
+  for (int o0 = 0; o0 < nout; o0 += 128) {
+    const int nh2 = (min(nout - o0, 128) + 1) >> 1;  // lanes a group needs, two outputs each
+    const int wsh = nh2 <= 4 ? 2 : nh2 <= 8 ? 3 : nh2 <= 16 ? 4 : nh2 <= 32 ? 5 : 6;
+    const int G = 64 >> wsh, grp = lane >> wsh, ol = o0 + 2 * (lane & ((1 << wsh) - 1));
+    unsigned flip = 0;  // bit 4u + ab: the sign of output u's (J1, J2) phase
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        ok_[k] = vm != 0;
-        const int ol = vm ? __ffsll((long long)vm) - 1 : 0;
-        vm &= vm - 1;
-        const int J1k = __shfl(J1, ol, 64), J2k = __shfl(J2, ol, 64);
-        offk[k] = (unsigned)((J1k >> 1) * nd + ((J2k - J1k) >> 1));
-        ek[k][0] = (J1k >> 1) & 1;
-        ek[k][1] = (J2k >> 1) & 1;
-        ok_[k] = ok_[k] ? ol : -1;
+    for (int u = 0; u < 2; u++) {
+      const int oq = div(ol + u);
+      const unsigned e1 = ((Jlo >> 1) + oq) & 1, e2 = (e1 + (ol + u - oq * nd)) & 1;
+      flip |= (e1 << 1 | e2 << 2 | (e1 ^ e2) << 3) << (4 * u);
+    }
+    const double *n9 = T.n9 + (size_t)(Jlo >> 1) * nd + ol;
+    double acc[kPhQ][2];
+#pragma unroll
+    for (int q = 0; q < kPhQ; q++) acc[q][0] = acc[q][1] = 0.0;
+    int k = 0, nseg = 0;  // a lane's pattern: its slot only grows, so k carries over
+    for (int s0 = 0; s0 < nslot || nseg > 0;) {
+      // 1: the slots that exist, until 32 wait or none is left
+      while (nseg < 32 && s0 < nslot) {
+        const int s = min(s0 + lane, nslot - 1);
+        while (k < 15 && pat[k + 1].start <= s) k++;
+        const PhPat p = pat[k];
+        const int r = s - p.start, rq = div(r), J3 = p.j3 + 2 * rq, J4 = J3 + 2 * (r - rq * nd);
+        bool ok = s0 + lane < nslot && J4 <= 2 * JM && J3 + J4 >= R && J4 >= ((p.flags >> 6) & 4095) &&
+                  J4 <= (p.flags >> 18) && (k < 8 || J4 != J3);
+        CcBlk bk{-1, 0, 0};
+        if (ok) bk = T.cblk[((p.flags & 3) * nJ + (J3 >> 1)) * nd + ((J4 - J3) >> 1)];
+        ok = ok && bk.wo >= 0;
+        const unsigned long long m = __ballot(ok);
+        if (ok) {
+          PhSeg g;
+          // Wx carries LCC%herm (TS_commutators.f90:1506)
+          g.c = (k < 8 ? p.cs * hL : p.cs) * ((p.flags & 32) ? (double)sgnp((J3 + J4) >> 1) : 1.0) *
+                sqrt((J3 + 1.0) * (J4 + 1.0));
+          g.w = (bk.wo + (k < 8 ? 0 : wsize)) << 24 | bk.rl4;
+          g.b9 = ((p.b9 * nJ + (J3 >> 1)) * nd + ((J4 - J3) >> 1)) * (unsigned)(nJ * nd) |
+                 (unsigned)((p.flags >> 3) & 3) << 30;
+          g.code = (unsigned)k | (unsigned)(J3 >> 1) << 4 | (unsigned)(J4 >> 1) << 12;
+          seg[nseg + __popcll(m & ((1ull << lane) - 1ull))] = g;
+        }
+        nseg += __popcll(m);
+        s0 += 64;
       }
-      double acc[4] = {0.0, 0.0, 0.0, 0.0};
-      for (int t = lane; t < count; t += 64) {
-        const PhSlot sl = slot[t];
-        double v[4];
+      __syncthreads();
+      // 2: the entries of the first 32
+      const int nb = min(nseg, 32);
+      int count = 0;
+      {
+        double w[4];
+        int ix[4], jx[4];
+        auto slot = [&](int u) -> const PhSeg & { return seg[min(8 * u + (lane >> 3), nb - 1)]; };
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] = T.n9[sl.b9 + offk[k]];
+        for (int u = 0; u < 4; u++) {
+          const unsigned gc = slot(u).code;
+          const int kk = gc & 15;
+          const ushort2 bs = base[kk][quad];
+          ix[u] = T.crow[bs.x * nJ + (int)((gc >> 4) & 255)];
+          jx[u] = T.cpos[bs.y * nJ + (int)(gc >> 12)];
+          // the branch condition of the reference
+          if (8 * u + (lane >> 3) >= nb || quad >= nq || ((kPhCond >> (2 * kk)) & drop)) jx[u] = -1;
+        }
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const int e = ((sl.ab & 1) ? ek[k][0] : 0) + ((sl.ab & 2) ? ek[k][1] : 0);
-          const double x = sl.c * v[k];
-          acc[k] += (e & 1) ? -x : x;
+        for (int u = 0; u < 4; u++) {
+          w[u] = 0.0;
+          const long long gw = slot(u).w;
+          if ((ix[u] | jx[u]) >= 0) w[u] = W[(gw >> 24) + (long long)ix[u] * (int)(gw & 0xffffff) + jx[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const bool live = fabs(w[u]) > thr;
+          // one bit per slot of 8 lanes: some quadruple's entry passes
+          unsigned long long m = __ballot(live);
+          m |= m >> 4;
+          m |= m >> 2;
+          m |= m >> 1;
+          m &= 0x0101010101010101ull;
+          const int sub8 = lane & 56;
+          if ((m >> sub8) & 1) {
+            const int pos = count + __popcll(m & ((1ull << sub8) - 1ull));
+            cs[pos][quad] = live ? slot(u).c * w[u] : 0.0;
+            if (quad == 0) sb9[pos] = slot(u).b9;
+          }
+          count += __popcll(m);
         }
       }
+      if (lane < kPhQ) cs[count][lane] = 0.0;  // what the last round reads past the end
+      if (lane == kPhQ) sb9[count] = 0;
+      // the slots that wait move to the front
+      nseg -= nb;
+      const double mc = seg[32 + lane].c;
+      const long long mw = seg[32 + lane].w;
+      const unsigned mb = seg[32 + lane].b9, mo = seg[32 + lane].code;
+      __syncthreads();
+      if (lane < nseg) {
+        seg[lane].c = mc;
+        seg[lane].w = mw;
+        seg[lane].b9 = mb;
+        seg[lane].code = mo;
+      }
+      // 3: slots times 9j
+      for (int t0 = grp; t0 < count; t0 += kPhU * G) {
+        dpair_t v[kPhU];
+        unsigned ab[kPhU];
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const double a = wave_sum(acc[k]);
-        if (lane == ok_[k]) res = a;
+        for (int u = 0; u < kPhU; u++) {
+          const unsigned b = sb9[min(t0 + u * G, count)];
+          v[u] = *reinterpret_cast<const dpair_t *>(n9 + (b & 0x3fffffffu));
+          ab[u] = b >> 30;
+        }
+#pragma unroll
+        for (int u = 0; u < kPhU; u++) {
+          __builtin_amdgcn_sched_barrier(0);  // one slot's row from LDS at a time: registers
+          const double f0 = ((flip >> ab[u]) & 1) ? -v[u].x : v[u].x;
+          const double f1 = ((flip >> (4 + ab[u])) & 1) ? -v[u].y : v[u].y;
+          const double *cq = cs[min(t0 + u * G, count)];
+#pragma unroll
+          for (int q = 0; q < kPhQ; q++) {
+            const double c = cq[q];
+            acc[q][0] = fma(f0, c, acc[q][0]);
+            acc[q][1] = fma(f1, c, acc[q][1]);
+          }
+        }
+      }
+      __syncthreads();
+    }
+    // the groups' sums, each group left with its share of the quadruples (q0
+    // on), which it writes with one add per element and no wait for the old
+    // value
+    int q0 = 0, nown = kPhQ;
+#pragma unroll
+    for (int st = 0; st < 3; st++) {
+      if (wsh > 5 - st) break;
+      const int half = kPhQ >> (st + 1);
+      const bool up = (lane >> (5 - st)) & 1;
+#pragma unroll
+      for (int i = 0; i < half; i++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const double give = up ? acc[i][u] : acc[i + half][u], keep = up ? acc[i + half][u] : acc[i][u];
+          acc[i][u] = keep + __shfl_xor(give, 32 >> st);
+        }
+      if (up) q0 += half;
+      nown = half;
+    }
+    bool mine = true;
+    if (wsh == 2) {  // 16 groups for 8 quadruples
+#pragma unroll
+      for (int u = 0; u < 2; u++) acc[0][u] += __shfl_xor(acc[0][u], 4);
+      mine = !(lane & 4);
+    }
+    const int oq0 = div(ol), oq1 = div(ol + 1);
+    const int J1o[2] = {Jlo + 2 * oq0, Jlo + 2 * oq1};
+    const int J2o[2] = {J1o[0] + 2 * (ol - oq0 * nd), J1o[1] + 2 * (ol + 1 - oq1 * nd)};
+    OutBlk ob[2];
+    double nrm[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int J1 = J1o[u], J2 = J2o[u];
+      const bool val = mine && ol + u < nout && ol + u < o0 + 128 && J2 >= abs(j2 - j3) && J2 <= j2 + j3 && J1 + J2 >= R;
+      ob[u] = T.oblk[val ? (((J1 >> 1) * nd + ((J2 - J1) >> 1)) * 6 + Tzq * 2 + P1) : 0];
+      if (!val) ob[u].off = -1;
+      nrm[u] = sqrt((J1 + 1.0) * (J2 + 1.0));
+    }
+#pragma unroll
+    for (int i = 0; i < kPhQ; i++) {
+      if (i >= nown) break;
+      const unsigned cd = (unsigned)__shfl((int)code, q0 + i);
+      const int x0 = cd & 255, x1 = (cd >> 8) & 255, x2 = (cd >> 16) & 255, x3 = (int)(cd >> 24);
+      const int *p1 = T.prow + (x0 * n + x1) * nJ, *p2 = T.prow + (x2 * n + x3) * nJ;
+      const double f = (x0 == x1 ? M_SQRT2 : 1.0) * (x2 == x3 ? M_SQRT2 : 1.0);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int e1 = J1o[u] >> 1, e2 = J2o[u] >> 1;
+        if (q0 + i < nq && ob[u].off >= 0 && !(x0 == x1 && (e1 & 1)) && !(x2 == x3 && (e2 & 1))) {
+          const int r = p1[e1], sc = p2[e2];
+          if ((r | sc) >= 0)
+            unsafeAtomicAdd(OV + ob[u].off + (long long)r * ob[u].n2 + sc, acc[i][u] * nrm[u] * f);
+        }
       }
     }
-    if (val) OV[po] = old + res * sqrt((J1 + 1.0) * (J2 + 1.0)) * pre;
   }
 }
 
@@ -968,7 +1116,7 @@ struct TensorSpace {
   std::vector<int> J1, J2, q1, q2, n1, n2, bidx;
   std::vector<long long> off, tstart;
   long long vsize = 0, v_off = 0, op_size = 0, neq = 0, nelem = 0;
-  std::vector<int> cJ3, cJ4, cq3, cq4, cidx, ccol;
+  std::vector<int> cJ3, cJ4, cq3, cq4, ccol;
   std::vector<long long> xoff, roff, woff, xstart, rstart;
   long long xsize = 0, rsize = 0, wsize = 0;
   std::vector<double> x6, s6;
@@ -976,7 +1124,7 @@ struct TensorSpace {
   PackTables pack{};
   double *pack_d = nullptr;
   DevTensor dt{};
-  double *gcc = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
+  double *gcc = nullptr, *gccp = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
   double *w1 = nullptr, *w2 = nullptr, *part = nullptr, *hpart = nullptr;
   const TProb *pp_probs[2] = {nullptr, nullptr}, *cc_probs[2] = {nullptr, nullptr};
   const int4 *pp_tiles = nullptr, *cc_tiles[2] = {nullptr, nullptr};
@@ -1039,20 +1187,17 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   S.neq = 1 + (long long)Ly.nhole * Ly.nhole + (long long)Ly.npart * Ly.npart + (long long)Ly.npart * Ly.nhole + el;
   // cross-coupled tensor blocks (allocate_small_tensor_CCMAT, cross_coupled.f90:498-700):
   // J3, J4 >= J3 within rank, |Tz|, parity of the J3 pairs
-  S.cidx.assign((size_t)nJ * nJ * 4, -1);
   long long xo = 0, ro = 0, wo = 0, xe = 0, re = 0;
   for (int J3 = 0; J3 <= 2 * JM; J3 += 2)
     for (int J4 = std::max(std::abs(J3 - rank), J3); J4 <= std::min(J3 + rank, 2 * JM); J4 += 2)
       for (int Tz = 0; Tz <= 1; Tz++)
         for (int P = 0; P <= 1; P++) {
-          const int x = (int)S.cJ3.size();
           const int q3 = (J3 >> 1) + Tz * (JM + 1) + 2 * P * (JM + 1);
           const int q4 = (J4 >> 1) + Tz * (JM + 1) + 2 * (P ^ dp) * (JM + 1);
           S.cJ3.push_back(J3);
           S.cJ4.push_back(J4);
           S.cq3.push_back(q3);
           S.cq4.push_back(q4);
-          S.cidx[((size_t)(J3 >> 1) * nJ + (J4 >> 1)) * 4 + Tz * 2 + P] = x;
           const long long r3 = Ly.ccrlen[q3], r4 = Ly.ccrlen[q4], nb3 = Ly.ccnph[q3], nb4 = Ly.ccnph[q4];
           S.xoff.push_back(xo);
           S.roff.push_back(ro);
@@ -1112,9 +1257,12 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   TUP(S.off, off); TUP(S.tstart, tstart); TUP(S.bidx, bidx);
   TUP(S.cJ3, cJ3); TUP(S.cJ4, cJ4); TUP(S.cq3, cq3); TUP(S.cq4, cq4);
   TUP(S.xoff, xoff); TUP(S.roff, roff); TUP(S.woff, woff); TUP(S.xstart, xstart); TUP(S.rstart, rstart);
-  TUP(S.cidx, cidx); TUP(S.ccol, ccol); TUP(S.x6, x6); TUP(S.s6, s6);
+  TUP(S.ccol, ccol); TUP(S.x6, x6); TUP(S.s6, s6);
+  std::vector<int> rperm, rpos;  // Pandya rows in group order, and each row's place in it
   {
-    std::vector<int> cperm(Ly.cccbase[Ly.ncc]), rperm(Ly.ccrbase[Ly.ncc]);
+    std::vector<int> cperm(Ly.cccbase[Ly.ncc]);
+    rperm.resize(Ly.ccrbase[Ly.ncc]);
+    rpos.resize(Ly.ccrbase[Ly.ncc]);
     for (int q = 0; q < Ly.ncc; q++) {
       const int c0 = Ly.cccbase[q], nc = Ly.cccbase[q + 1] - c0, r0 = Ly.ccrbase[q], nr = Ly.ccrlen[q];
       std::vector<int> ix(nc);
@@ -1126,12 +1274,18 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       std::copy(ix.begin(), ix.end(), cperm.begin() + c0);
       auto rkey = [&](int g) {
         const int a = Ly.ccrow_a[r0 + g], b = Ly.ccrow_b[r0 + g];
-        return a < 0 ? std::make_pair(1 << 20, 0) : std::make_pair(Ly.jj[a], Ly.jj[b]);
+        return a < 0 ? std::make_pair(1 << 20, 0) : std::make_pair(Ly.grp_of[a], Ly.grp_of[b]);
       };
       ix.resize(nr);
       for (int g = 0; g < nr; g++) ix[g] = g;
-      std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) { return rkey(x) < rkey(y); });
+      std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) {
+        const auto kx = rkey(x), ky = rkey(y);
+        if (kx != ky) return kx < ky;
+        return std::make_pair(Ly.ccrow_a[r0 + x], Ly.ccrow_b[r0 + x]) <
+               std::make_pair(Ly.ccrow_a[r0 + y], Ly.ccrow_b[r0 + y]);
+      });
       std::copy(ix.begin(), ix.end(), rperm.begin() + r0);
+      for (int i = 0; i < nr; i++) rpos[r0 + ix[i]] = i;
     }
     TUP(cperm, cperm); TUP(rperm, rperm);
     std::vector<int> sperm(Ly.npairs);
@@ -1169,70 +1323,94 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
     const long long n9 = (long long)nh * nh * nh * nh * nJ * nJ * D.nd * D.nd;
     if (n9 > (1LL << 29)) return fail(IMSRG_EINVAL, "tensor rank too large for the 9j table at this basis");
     double *t9 = nullptr;
-    if (dalloc(c, n9, &t9)) return IMSRG_ENOMEM;
+    if (dalloc(c, n9 + kN9Pad, &t9)) return IMSRG_ENOMEM;
+    launch_fill(c->stream, t9 + n9, kN9Pad, 0.0);
     hipLaunchKernelGGL(k_fill9j, dim3((unsigned)((n9 + 255) / 256)), dim3(256), 0, c->stream, D, t9, n9);
     D.n9 = t9;
     S.n9size = n9;
   }
-  // orbit quadruples of the recoupling gather (k_t222ph_q): row pair x0 <= x1,
-  // column pair x2 <= x3, with at least one stored output (orbits packed in 8 bits)
+  // orbit quadruples of the recoupling gather (k_t222ph): row pair x0 <= x1,
+  // column pair x2 <= x3, with at least one stored output (orbits packed in 8
+  // bits), by the (l,j,tz) groups of the four orbits
   if (nsp > 256) return fail(IMSRG_EINVAL, "tensor operators need at most 256 orbits");
   {
-    std::vector<unsigned> qrun[4];  // by slot count: at most 256, 384, 512, more
-    std::vector<int> pa_, pb_;
-    int nslotmax = 1;
-    for (int a = 0; a < nsp; a++)
-      for (int b = a; b < nsp; b++) { pa_.push_back(a); pb_.push_back(b); }
-    for (size_t u = 0; u < pa_.size(); u++) {
-      const int x0 = pa_[u], x1 = pb_[u], j0 = Ly.jj[x0], j1 = Ly.jj[x1];
-      const int t1 = Ly.tz[x0] + Ly.tz[x1], p1 = (Ly.l[x0] + Ly.l[x1]) & 1;
-      for (size_t v = 0; v < pa_.size(); v++) {
-        const int x2 = pa_[v], x3 = pb_[v];
-        if (Ly.tz[x2] + Ly.tz[x3] != t1 || ((Ly.l[x2] + Ly.l[x3]) & 1) != (p1 ^ dp)) continue;
-        const int j2 = Ly.jj[x2], j3 = Ly.jj[x3];
-        bool any = false;
-        for (int J1 = std::abs(j0 - j1); J1 <= j0 + j1 && !any; J1 += 2) {
-          if (x0 == x1 && ((J1 >> 1) & 1)) continue;
-          for (int J2 = std::max(J1, std::abs(j2 - j3)); J2 <= std::min(j2 + j3, J1 + rank); J2 += 2) {
-            if (x2 == x3 && ((J2 >> 1) & 1)) continue;
-            if (J1 + J2 < rank) continue;
-            any = true;
-            break;
-          }
-        }
-        if (!any) continue;
-        const unsigned code = (unsigned)x0 | (unsigned)x1 << 8 | (unsigned)x2 << 16 | (unsigned)x3 << 24;
-        // the quadruple's gather slots (k_t222ph_q): a run of J3 times the
-        // J4 - J3 steps per pattern that passes the branch, parity and Tz tests
-        const int xs[4] = {x0, x1, x2, x3};
-        int ns = 0;
-        for (int k = 0; k < 16; k++) {
-          const int a = xs[(kPhIa >> (2 * k)) & 3], b = xs[(kPhIb >> (2 * k)) & 3];
-          const int cc = xs[(kPhIc >> (2 * k)) & 3], dd = xs[(kPhId >> (2 * k)) & 3];
-          const unsigned cond = (kPhCond >> (2 * k)) & 3;
-          if (((cond & 1) && !(x0 < x1)) || ((cond & 2) && !(x2 < x3))) continue;
-          const int Tz = std::abs(Ly.tz[dd] - Ly.tz[a]) >> 1, PAR2 = ((Ly.l[dd] + Ly.l[a]) & 1) ^ dp;
-          if (((Ly.l[cc] + Ly.l[b]) & 1) != PAR2 || (std::abs(Ly.tz[cc] - Ly.tz[b]) >> 1) != Tz) continue;
-          const int jd = Ly.jj[dd], ja = Ly.jj[a];
-          ns += ((jd + ja - std::abs(jd - ja)) / 2 + 1) * (rank / 2 + 1);
-        }
-        nslotmax = std::max(nslotmax, ns);
-        qrun[ns <= 256 ? 0 : ns <= 384 ? 1 : ns <= 512 ? 2 : 3].push_back(code);
-      }
-    }
     std::vector<unsigned> quads;
-    D.qrun[0] = 0;
-    for (int k = 0; k < 4; k++) {
-      quads.insert(quads.end(), qrun[k].begin(), qrun[k].end());
-      D.qrun[k + 1] = (long long)quads.size();
+    std::vector<PhChunkT> chunks;
+    const int ng = (int)Ly.grp_start.size();
+    auto orbits = [&](int g, int &cnt) {
+      cnt = Ly.grp_cnt[g];
+      return Ly.grp_list.data() + Ly.grp_start[g];
+    };
+    for (int g0 = 0; g0 < ng; g0++)
+      for (int g1 = 0; g1 < ng; g1++) {
+        int c0, c1;
+        const int *o0 = orbits(g0, c0), *o1 = orbits(g1, c1);
+        std::vector<std::pair<int, int>> bra;
+        for (int i = 0; i < c0; i++)
+          for (int j = 0; j < c1; j++)
+            if (o0[i] <= o1[j]) bra.push_back({o0[i], o1[j]});
+        if (bra.empty()) continue;
+        const int y0 = o0[0], y1 = o1[0], j0 = Ly.jj[y0], j1 = Ly.jj[y1];
+        const int t1 = Ly.tz[y0] + Ly.tz[y1], p1 = (Ly.l[y0] + Ly.l[y1]) & 1;
+        for (int g2 = 0; g2 < ng; g2++)
+          for (int g3 = 0; g3 < ng; g3++) {
+            int c2, c3;
+            const int *o2 = orbits(g2, c2), *o3 = orbits(g3, c3);
+            if (Ly.tz[o2[0]] + Ly.tz[o3[0]] != t1 || ((Ly.l[o2[0]] + Ly.l[o3[0]]) & 1) != (p1 ^ dp)) continue;
+            const int j2 = Ly.jj[o2[0]], j3 = Ly.jj[o3[0]];
+            bool any[4] = {false, false, false, false};  // [x0 == x1][x2 == x3]
+            for (int J1 = std::abs(j0 - j1); J1 <= j0 + j1; J1 += 2)
+              for (int J2 = std::max(J1, std::abs(j2 - j3)); J2 <= std::min(j2 + j3, J1 + rank); J2 += 2)
+                if (J1 + J2 >= rank)
+                  for (int k = 0; k < 4; k++)
+                    any[k] |= !((k & 2) && ((J1 >> 1) & 1)) && !((k & 1) && ((J2 >> 1) & 1));
+            if (!any[0]) continue;
+            const size_t first = quads.size();
+            for (const auto &x : bra)
+              for (int i = 0; i < c2; i++)
+                for (int j = 0; j < c3; j++)
+                  if (o2[i] <= o3[j] && any[(x.first == x.second) * 2 + (o2[i] == o3[j])])
+                    quads.push_back((unsigned)x.first | (unsigned)x.second << 8 | (unsigned)o2[i] << 16 |
+                                    (unsigned)o3[j] << 24);
+            unsigned lt = 0;
+            const int ys[4] = {y0, y1, o2[0], o3[0]};
+            for (int i = 0; i < 4; i++) lt |= (unsigned)(Ly.l[ys[i]] & 1) << i | (unsigned)(Ly.tz[ys[i]] > 0) << (4 + i);
+            const unsigned jv = (unsigned)j0 | (unsigned)j1 << 8 | (unsigned)j2 << 16 | (unsigned)j3 << 24;
+            for (size_t k = first; k < quads.size(); k += kPhQ)
+              chunks.push_back(PhChunkT{(unsigned)k, jv, lt, (int)std::min<size_t>(kPhQ, quads.size() - k)});
+          }
+      }
+    if (quads.empty()) quads.push_back(0);
+    D.nqchunk = (int)chunks.size();
+    D.nqpad = (D.nqchunk + 511) & ~511;
+    if (chunks.empty()) chunks.push_back(PhChunkT{0, 0, 0, 1});
+    if (upload_table(c, quads, &D.quads) != 0 || upload_table(c, chunks, &D.qchunk) != 0) return IMSRG_ENOMEM;
+    // rows by pair, J fastest
+    std::vector<int> crow((size_t)nsp * nsp * nJ, -1), cpos(crow), prow(crow);
+    for (int a = 0; a < nsp; a++)
+      for (int b = 0; b < nsp; b++)
+        for (int J = 0; J < nJ; J++) {
+          const int Tz = std::abs(Ly.tz[a] - Ly.tz[b]) >> 1, P = (Ly.l[a] + Ly.l[b]) & 1;
+          const int q = J + Tz * (JM + 1) + 2 * P * (JM + 1);
+          const int r = Ly.ccrow[((size_t)q * nsp + a) * nsp + b];
+          crow[((size_t)a * nsp + b) * nJ + J] = r;
+          if (r >= 0) cpos[((size_t)a * nsp + b) * nJ + J] = rpos[Ly.ccrbase[q] + r];
+          prow[((size_t)a * nsp + b) * nJ + J] = Ly.pidx[((size_t)J * nsp + a) * nsp + b];
+        }
+    std::vector<CcBlk> cblk((size_t)4 * nJ * D.nd, CcBlk{-1, 0, 0});
+    for (int x = 0; x < S.ncc; x++) {
+      const int q3 = S.cq3[x], Tz = (q3 / (JM + 1)) & 1, P = q3 / (2 * (JM + 1));
+      cblk[((size_t)(Tz + 2 * P) * nJ + (S.cJ3[x] >> 1)) * D.nd + ((S.cJ4[x] - S.cJ3[x]) >> 1)] =
+          CcBlk{S.woff[x], Ly.ccrlen[S.cq4[x]], 0};
     }
-    if (upload_table(c, quads, &D.quads) != 0) return IMSRG_ENOMEM;
-    D.nquad = (long long)quads.size();
-    D.nslotmax = nslotmax;
-    D.qcap[0] = std::min(256, nslotmax);
-    D.qcap[1] = std::min(384, nslotmax);
-    D.qcap[2] = std::min(512, nslotmax);
-    D.qcap[3] = nslotmax;
+    std::vector<OutBlk> oblk((size_t)6 * nJ * D.nd, OutBlk{-1, 0, 0});
+    for (int q = 0; q < S.nblk; q++)
+      if (S.q1[q] >= 0)
+        oblk[((size_t)(S.J1[q] >> 1) * D.nd + ((S.J2[q] - S.J1[q]) >> 1)) * 6 + S.q1[q] % 6] = OutBlk{S.off[q], S.n2[q], 0};
+    if (upload_table(c, oblk, &D.oblk) != 0) return IMSRG_ENOMEM;
+    if (upload_table(c, crow, &D.crow) != 0 || upload_table(c, cpos, &D.cpos) != 0 || upload_table(c, prow, &D.prow) != 0 ||
+        upload_table(c, cblk, &D.cblk) != 0)
+      return IMSRG_ENOMEM;
   }
   // products: the pp and hh ladders per tensor block (W1, W2)
   {
@@ -1263,7 +1441,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   }
   // the two Pandya products per cross-coupled block (TS_commutator_222_ph, TS_commutators.f90:1496-1521):
   // alpha carries 1/sqrt(J3+1) and 1/sqrt(J4+1); the herm of G that the reference also folds into Wx
-  // is applied where k_t222ph_q reads Wx, so these tables serve every G
+  // is applied where k_t222ph reads Wx, so these tables serve every G
   {
     std::vector<TProb> pr[2];
     std::vector<int4> tiles[2];
@@ -1291,14 +1469,14 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
     }
   }
   // workspaces
-  if (dalloc(c, Ly.ccsize, &S.gcc) || dalloc(c, S.xsize, &S.ccx) || dalloc(c, S.rsize, &S.ccr) ||
-      dalloc(c, S.wsize, &S.wx) || dalloc(c, S.wsize, &S.wy) || dalloc(c, S.vsize, &S.w1) ||
+  if (dalloc(c, Ly.ccsize, &S.gcc) || dalloc(c, Ly.ccsize, &S.gccp) || dalloc(c, S.xsize, &S.ccx) || dalloc(c, S.rsize, &S.ccr) ||
+      dalloc(c, 2 * S.wsize, &S.wx) || dalloc(c, S.vsize, &S.w1) ||
       dalloc(c, S.vsize, &S.w2) || dalloc(c, kNormParts, &S.part))
     return IMSRG_ENOMEM;
   launch_fill(c->stream, S.w1, S.vsize, 0.0);
   launch_fill(c->stream, S.w2, S.vsize, 0.0);
-  launch_fill(c->stream, S.wx, S.wsize, 0.0);
-  launch_fill(c->stream, S.wy, S.wsize, 0.0);
+  S.wy = S.wx + S.wsize;
+  launch_fill(c->stream, S.wx, 2 * S.wsize, 0.0);
   HIPCHK(hipHostMalloc((void **)&S.hpart, kNormParts * sizeof(double)));
   return 0;
 }
@@ -1514,6 +1692,8 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
     hipLaunchKernelGGL(k_t_onebody, dim3(L.nob), dim3(64), 0, s, L, D, 1, GF, RF, RV, (const double *)S.gcc,
                        (const double *)S.w1, (const double *)S.w2, OF, hL, hR, hres);
   if ((mask & IMSRG_TS222PH) && S.nelem > 0) {
+    if (L.nccol > 0)
+      hipLaunchKernelGGL(k_gcc_order, dim3(L.nccol), dim3(256), 0, s, L, D, (const double *)S.gcc, S.gccp);
     if (D.nx > 0) hipLaunchKernelGGL(k_tpandya, dim3(nblk(D.nx)), dim3(256), 0, s, L, D, 0, RV, S.ccx, hR);
     if (D.nr > 0) hipLaunchKernelGGL(k_tpandya, dim3(nblk(D.nr)), dim3(256), 0, s, L, D, 1, RV, S.ccr, hR);
     if (S.n_cc_tiles[0] > 0)
@@ -1521,12 +1701,9 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
                          S.n_cc_tiles[0], (const double *)S.gcc, (const double *)S.ccr, S.wx);
     if (S.n_cc_tiles[1] > 0)
       hipLaunchKernelGGL(k_tgemm, dim3(S.n_cc_tiles[1]), dim3(256), 0, s, S.cc_probs[1], S.cc_tiles[1],
-                         S.n_cc_tiles[1], (const double *)S.ccx, (const double *)S.gcc, S.wy);
-    for (int k = 0; k < 4; k++)
-      if (D.qrun[k + 1] > D.qrun[k])
-        hipLaunchKernelGGL(k_t222ph_q, dim3((unsigned)(D.qrun[k + 1] - D.qrun[k])), dim3(64),
-                           (unsigned)(sizeof(PhSlot) * D.qcap[k]), s, L, D, (const double *)S.wx,
-                           (const double *)S.wy, OV, hL, hR, k);
+                         S.n_cc_tiles[1], (const double *)S.ccx, (const double *)S.gccp, S.wy);
+    if (D.nqchunk > 0)
+      hipLaunchKernelGGL(k_t222ph, dim3(D.nqpad), dim3(64), 0, s, L, D, (const double *)S.wx, S.wsize, OV, hL, hR);
   }
   HIPCHK(hipGetLastError());
   return 0;
