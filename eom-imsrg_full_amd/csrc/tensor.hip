@@ -73,11 +73,6 @@ struct DevTensor {
   // and CCR, Wx and Wy keep their columns in the rows' order: the entries that
   // quadruples of one class read then share cache lines
   const int *cperm, *rperm;
-  // thread order of the 122 and 212 gathers inside each tensor block's rows:
-  // the ket pairs of every scalar block by the (l,j,tz) groups of their two
-  // orbits (the lengths of their partner loops); entry pbase[q] + i is the
-  // column thread i of a row computes
-  const int *sperm;
   long long f_off, v_off;
 };
 
@@ -426,156 +421,197 @@ __global__ __launch_bounds__(64) void k_t_onebody(DevLayout L, DevTensor T, int 
 }
 
 // ---------------------------------------------------------------- two-body gathers
-// flat element e -> block q, orbits, position; with perm, the columns of a
-// row in the sperm order (r, s: row and column in the block)
-__device__ __forceinline__ bool elem_of(const DevLayout &L, const DevTensor &T, long long e, int &q, int &a, int &b,
-                                        int &c, int &d, long long &vpos, bool perm = false, int *rs = nullptr) {
-  if (e >= T.nelem) return false;
-  q = find_item(T.tstart, T.nblk, e);
-  const long long u = e - T.tstart[q];
-  const int n2 = T.n2[q];
-  const int r = (int)(u / n2), s0 = (int)(u % n2), s = perm ? T.sperm[L.pbase[T.q2[q]] + s0] : s0;
-  if (rs) {
-    rs[0] = r;
-    rs[1] = s;
-  }
-  const int g1 = L.pbase[T.q1[q]] + r, g2 = L.pbase[T.q2[q]] + s;
-  a = L.pair_a[g1]; b = L.pair_b[g1]; c = L.pair_a[g2]; d = L.pair_b[g2];
-  vpos = T.off[q] + (long long)r * n2 + s;
-  return true;
-}
-
-// TS_commutator_122 (TS_commutators.f90:555-663): overwrites every element.
-// Per output (ab|cd; J1 J2) four sums over the orbits i of the (l,j,tz) group
-// of a, b, c, d: +LF(a,i) T(ib,cd), +LF(b,i) T(ai,cd), -LF(i,c) T(ab,id),
-// -LF(i,d) T(ab,ci).  Each T element lies in the output's own tensor block
-// with its column (kinds 0, 1) or row (kinds 2, 3) fixed, so it costs one
-// pair lookup and one load; the partners go four at a time with every load
-// off any branch (clamped to a valid entry, weight 0 past the group), as in
-// k_t212.
-__global__ void k_t122(DevLayout L, DevTensor T, const double *__restrict__ LF, const double *__restrict__ RV,
-                       double *__restrict__ OV, int hR) {
-  (void)hR;  // every element read lies in the output's block (J1 <= J2): no hermitian swap
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  int q, a, b, c, d, rs[2];
-  long long vp;
-  if (!elem_of(L, T, e, q, a, b, c, d, vp, true, rs)) return;
-  const int J1 = T.J1[q], J2 = T.J2[q], n = L.nsp, n2 = T.n2[q];
-  const int r1 = rs[0], s2 = rs[1];  // row of (ab), column of (cd) in the block
-  const double *Tq = RV + T.off[q];
-  const int *P1 = L.pidx + (size_t)(J1 >> 1) * n * n, *P2 = L.pidx + (size_t)(J2 >> 1) * n * n;
-  const double rab = a == b ? M_SQRT2 : 1.0, rcd = c == d ? M_SQRT2 : 1.0;
-  double sm = 0.0;
-  // kind 0: x = a, pair (i,b) at J1; 1: x = b, pair (a,i); 2: x = c, pair (i,d) at J2; 3: x = d, pair (c,i)
-#pragma unroll
-  for (int kind = 0; kind < 4; kind++) {
-    const int x = kind == 0 ? a : kind == 1 ? b : kind == 2 ? c : d;
-    const int o = kind == 0 ? b : kind == 1 ? a : kind == 2 ? d : c;  // the pair's other orbit
-    const int jo = L.jj[o], J = kind < 2 ? J1 : J2, g = L.grp_of[x];
-    const int k0 = L.grp_start[g], cnt = L.grp_cnt[g], ji = L.jj[x];  // the group shares x's 2j
-    for (int k = 0; k < cnt; k += 4) {
-      int pi[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) pi[v] = L.grp_list[k0 + min(k + v, cnt - 1)];
-      long long pos[4];
-      double w[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int i = pi[v], lo = min(i, o), hi = max(i, o);
-        const int rr = (kind < 2 ? P1 : P2)[lo * n + hi];
-        // i first in kinds 0 and 2, second in 1 and 3: the stored pair is (lo, hi)
-        const bool swp = (kind == 0 || kind == 2) ? i > o : o > i;
-        const double f = swp ? (double)sgnp(1 + ((ji + jo - J) >> 1)) : (i == o ? M_SQRT2 : 1.0);
-        const double lf = kind == 0 ? LF[(size_t)a * n + i] : kind == 1 ? LF[(size_t)b * n + i]
-                        : kind == 2 ? LF[(size_t)i * n + c] : LF[(size_t)i * n + d];
-        const bool ok = k + v < cnt && rr >= 0 && dtri(ji, jo, J);
-        pos[v] = !ok ? 0 : kind < 2 ? (long long)rr * n2 + s2 : (long long)r1 * n2 + rr;
-        w[v] = ok ? f * lf * (kind < 2 ? rcd : rab) : 0.0;
-      }
-      double t[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) t[v] = Tq[pos[v]];
-#pragma unroll
-      for (int v = 0; v < 4; v++) sm += (kind < 2 ? w[v] : -w[v]) * t[v];
-    }
-  }
-  sm = sm / sqrt(1.0 + (a == b)) / sqrt(1.0 + (c == d));
-  OV[vp] = sm;
-}
-
-// TS_commutator_212 (TS_commutators.f90:666-806): accumulates into every element.
-// GV: the scalar operator's V region (v_elem), RF: the tensor's one-body matrix.
-// Per output (ab|cd; J1 J2) four sums over the orbits i the tensor's one-body
-// part couples to a, b, d, c (the partner lists):
+// TS_commutator_122 (TS_commutators.f90:555-663; overwrites every element) and
+// _212 (:666-806; accumulates).  Per output (ab|cd; J1 J2) of a block q, over
+// the orbits i of the (l,j,tz) group of a, b, c, d:
+//   +LF(a,i) T(ib,cd)  +LF(b,i) T(ai,cd)  -LF(i,c) T(ab,id)  -LF(i,d) T(ab,ci)
+// and over the orbits i the tensor's one-body part couples to a, b, d, c:
 //   -{J1 J2 R; ji ja jb} RF(a,i) v(ib,cd;J2) (-1)^((ja+jb-J2)/2)
 //   +{J1 J2 R; ji jb ja} RF(b,i) v(ia,cd;J2) (-1)^((J1+J2)/2)
 //   +{J1 J2 R; jd ji jc} RF(i,d) v(ab,ci;J1) (-1)^((jc+jd-J1)/2)
 //   -{J1 J2 R; jc ji jd} RF(i,c) v(ab,di;J1) (-1)^((J1+J2)/2)
-// Each v is an element of the scalar channel block of (cd) at J2 or of (ab) at
-// J1 whose fixed pair is the output's own column or row, so it costs one pair
-// lookup and one load; the partners go four at a time with every load off any
-// branch (clamped to a valid entry, weight 0 past the list), so a batch makes
-// three dependent round trips instead of three per partner.
-__global__ void k_t212(DevLayout L, DevTensor T, const double *__restrict__ GV, const double *__restrict__ RF,
-                       double *__restrict__ OV) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  int q, a, b, c, d, rs[2];
-  long long vp;
-  if (!elem_of(L, T, e, q, a, b, c, d, vp, true, rs)) return;
-  const int J1 = T.J1[q], J2 = T.J2[q], n = L.nsp, R = T.rank;
-  const int ja = L.jj[a], jb = L.jj[b], jc = L.jj[c], jd = L.jj[d];
-  const int q1 = T.q1[q], q2 = T.q2[q];
-  const int r1 = rs[0], s2 = rs[1];  // row of (ab) in block q1, column of (cd) in q2
-  const double *V1 = GV + L.boff[q1], *V2 = GV + L.boff[q2];
-  const int d1 = L.bdim[q1], d2 = L.bdim[q2];
-  const int *P1 = L.pidx + (size_t)(J1 >> 1) * n * n, *P2 = L.pidx + (size_t)(J2 >> 1) * n * n;
-  const double rab = a == b ? M_SQRT2 : 1.0, rcd = c == d ? M_SQRT2 : 1.0;
+// (times sqrt((J1+1)(J2+1)) (-1)^(R/2)): a sparse matrix over (ab) times rows
+// of T's block and of G's block at J2, plus rows of T's block and of G's block
+// at J1 times a sparse matrix over (cd).  Which entries exist is fixed with the
+// tensor space; k_t_lists writes their weights once per commutator (every
+// phase, 6j and pair norm; two lists per pair and block, against pair squared
+// outputs), k_t_1body then does one multiply-add per entry and output.
+//
+// Rows go in groups of up to eight of the same or neighbouring (l,j,tz)
+// classes: the rows of one class name the same partner rows of T and two
+// thirds the same of G, so a group keeps one list of partner rows, each with
+// the eight rows' weights.
+struct TList {
+  long long base;  // columns: weight of entry e at base + 64 e; rows: destination of entry e in rdst[base + e]
+  int q, idx, side, n;
+};
+// ng row groups from g0 of block q
+struct TItem {
+  int q, g0, ng, pad;
+};
+// a row group's partner list (n entries from base), or the lists of 64
+// columns (n entries each, entry e of column c at base + 64 e + c)
+struct TSlice {
+  long long base, n;
+};
+struct TLists {
+  const TList *lists;
+  const TItem *items;
+  const TSlice *groups, *cols;
+  const int *cbase;            // first entry of cols of a block
+  const int *grow;             // rows of a group, eight entries, the last ones repeated
+  const int *rsrc;             // partner row of T's block (>= 0) or of G's block at J2 (~row)
+  const int *rdst;             // where a row's entry lies in rw, or -1
+  const unsigned short *cp;    // column lists: position in [T's row | G's row at J1]
+  double *rw, *cw;             // weights: rw[8 * entry + row of the group], cw by columns
+  int nlist, nitem;
+  unsigned lds;                // of k_t_1body
+};
+constexpr int kT1Threads = 768;
+
+// one wavefront per list, a lane per entry
+__global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists W, const double *__restrict__ LF,
+                                                const double *__restrict__ RF, int do122, int do212) {
+  const TList li = W.lists[blockIdx.x];
+  const int q = li.q, n = L.nsp, R = T.rank, J1 = T.J1[q], J2 = T.J2[q];
+  const int pr = L.pbase[li.side ? T.q2[q] : T.q1[q]] + li.idx;
+  const int a = L.pair_a[pr], b = L.pair_b[pr], ja = L.jj[a], jb = L.jj[b];
+  const double dab = a == b ? M_SQRT1_2 : 1.0;
   const double *x6 = T.x6 + (((size_t)(J1 >> 1) * T.nJ + (J2 >> 1)) * T.hx) * T.nh * T.nh;  // {J1 J2 R; . . .}
   auto six = [&](int j4, int j5, int j6) { return x6[((size_t)(j4 >> 1) * T.nh + (j5 >> 1)) * T.nh + (j6 >> 1)]; };
-  double sm = 0.0;
-  // kind 0: x = a, pair (i,b) at J2; 1: x = b, pair (i,a) at J2; 2: x = d, pair (c,i) at J1; 3: x = c, pair (d,i) at J1
-#pragma unroll
-  for (int kind = 0; kind < 4; kind++) {
-    const int x = kind == 0 ? a : kind == 1 ? b : kind == 2 ? d : c;
-    const int o = kind == 0 ? b : kind == 1 ? a : kind == 2 ? c : d;  // the pair's other orbit
-    const int jo = L.jj[o], J = kind < 2 ? J2 : J1;
-    const int k0 = T.pstart[x], k1 = T.pstart[x + 1];
-    const double sg = kind == 0 ? -(double)sgnp((ja + jb - J2) >> 1)
-                      : kind == 1 ? (double)sgnp((J1 + J2) >> 1)
-                      : kind == 2 ? (double)sgnp((jc + jd - J1) >> 1)
-                                  : -(double)sgnp((J1 + J2) >> 1);
-    for (int k = k0; k < k1; k += 4) {
-      int pi[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) pi[v] = T.part[min(k + v, k1 - 1)];
-      long long pos[4];
-      double w[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int i = pi[v] & 255, ji = pi[v] >> 8;
-        // the pair's position in its block and v_elem's factor: kinds 0, 1 put i
-        // first (bra (i,o) against the fixed ket (cd)), kinds 2, 3 second (ket (o,i))
-        const int lo = min(i, o), hi = max(i, o);
-        const int rr = (kind < 2 ? P2 : P1)[lo * n + hi];
-        const bool swp = kind < 2 ? i > o : o > i;
-        double f = swp ? (double)sgnp(1 + ((ji + jo - J) >> 1)) : (i == o ? M_SQRT2 : 1.0);
-        const double rf = kind == 0 ? RF[(size_t)a * n + i] : kind == 1 ? RF[(size_t)b * n + i]
-                        : kind == 2 ? RF[(size_t)i * n + d] : RF[(size_t)i * n + c];
-        const double sx = kind == 0 ? six(ji, ja, jb) : kind == 1 ? six(ji, jb, ja)
-                        : kind == 2 ? six(jd, ji, jc) : six(jc, ji, jd);
-        const bool ok = k + v < k1 && rr >= 0;
-        pos[v] = !ok ? 0 : kind < 2 ? (long long)rr * d2 + s2 : (long long)r1 * d1 + rr;
-        w[v] = ok ? f * rf * sx : 0.0;
+  const int g1 = L.grp_of[a], g2 = L.grp_of[b], c1 = L.grp_cnt[g1], c2 = L.grp_cnt[g2];
+  const int p1 = T.pstart[a], m1 = T.pstart[a + 1] - p1, p2 = T.pstart[b], m2 = T.pstart[b + 1] - p2;
+  const double n212 = sqrt((J1 + 1.0) * (J2 + 1.0)) * sgnp(R >> 1);
+  for (int e = threadIdx.x; e < li.n; e += 64) {
+    double w = 0.0;
+    if (e < c1 + c2) {
+      // i for a (with o = b) or for b (o = a)
+      const bool fa = e < c1;
+      const int i = L.grp_list[fa ? L.grp_start[g1] + e : L.grp_start[g2] + e - c1];
+      const int x = fa ? a : b, o = fa ? b : a, ji = L.jj[i], jo = L.jj[o], J = li.side ? J2 : J1;
+      // the pair is (i,o) when i stands for a, (o,i) when for b
+      const bool swp = fa ? i > o : o > i;
+      const double f = swp ? (double)sgnp(1 + ((ji + jo - J) >> 1)) : (i == o ? M_SQRT2 : 1.0);
+      if (do122) w = li.side ? -f * LF[(size_t)i * n + x] * dab : f * LF[(size_t)x * n + i] * dab;
+    } else if (e < c1 + c2 + m1 + m2) {
+      const int k = e - c1 - c2;
+      const bool fa = k < m1;
+      const int pi = T.part[fa ? p1 + k : p2 + k - m1], i = pi & 255, ji = pi >> 8;
+      const int x = fa ? a : b, o = fa ? b : a, jo = L.jj[o], J = li.side ? J1 : J2;
+      // rows: v(i o, cd; J2); columns: v(ab, o i; J1)
+      const bool swp = li.side ? o > i : i > o;
+      const double f = swp ? (double)sgnp(1 + ((ji + jo - J) >> 1)) : (i == o ? M_SQRT2 : 1.0);
+      if (do212) {
+        double sx, sg;
+        if (!li.side) {
+          sx = fa ? six(ji, ja, jb) : six(ji, jb, ja);
+          sg = fa ? -(double)sgnp((ja + jb - J2) >> 1) : (double)sgnp((J1 + J2) >> 1);
+        } else {  // (a, b) are the reference's (c, d)
+          sx = fa ? six(ja, ji, jb) : six(jb, ji, ja);
+          sg = fa ? -(double)sgnp((J1 + J2) >> 1) : (double)sgnp((ja + jb - J1) >> 1);
+        }
+        w = sg * sx * f * (li.side ? RF[(size_t)i * n + x] : RF[(size_t)x * n + i]) * n212 * dab;
       }
-      double g[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) g[v] = (kind < 2 ? V2 : V1)[pos[v]];
-#pragma unroll
-      for (int v = 0; v < 4; v++) sm += sg * w[v] * g[v] * (kind < 2 ? rcd : rab);
+    }
+    if (li.side) {
+      W.cw[li.base + 64LL * e] = W.cp[li.base + 64LL * e] == 0xffff ? 0.0 : w;
+    } else {
+      const int d = W.rdst[li.base + e];
+      if (d >= 0) W.rw[d] = w;
     }
   }
-  sm *= sqrt((J1 + 1.0) * (J2 + 1.0) / (1.0 + (a == b)) / (1.0 + (c == d))) * sgnp(R >> 1);
-  OV[vp] += sm;
+}
+
+// A workgroup takes row groups of a block and stages T's and G's rows in LDS,
+// where the column lists gather from them, with the groups' partner lists; a
+// wavefront computes a group x 64 columns, so that a column list's entry and a
+// partner row, read once, serve eight outputs.  Eight partner rows' reads are
+// in flight.  Bound by those reads (L2-resident blocks) and the LDS gathers.  A
+// thread per output with a pair lookup, an F entry and a 6j per term took
+// 0.95 + 3.1 ms for the two commutators at 90 orbits, rank 4 (20 M outputs);
+// this kernel 1.0 ms with a partner list per row, 0.66 ms with one per
+// group (and a block on one XCD), k_t_lists 0.09 ms.
+__global__ __launch_bounds__(kT1Threads, 6) void k_t_1body(DevLayout L, DevTensor T, TLists W,
+                                                        const double *__restrict__ GV, const double *__restrict__ RV,
+                                                        double *__restrict__ OV, int add) {
+  extern __shared__ double rows[];
+  const TItem it = W.items[blockIdx.x];
+  if (it.ng == 0) return;
+  const int q = it.q, n2 = T.n2[q], q1 = T.q1[q], q2 = T.q2[q], d1 = L.bdim[q1], ld = (n2 + d1) | 1;
+  const double *Tq = RV + T.off[q], *V1 = GV + L.boff[q1], *V2 = GV + L.boff[q2];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const TSlice *gs = W.groups + it.g0;
+  const int *grow = W.grow + 8 * it.g0;
+  // LDS: 8 rows a group (a repeated row is staged once), the weights, the partner rows
+  const long long b0 = gs[0].base;
+  const int len = (int)(gs[it.ng - 1].base - b0 + gs[it.ng - 1].n);
+  int nst = 0;  // rows before the group's
+  for (int g = 0; g < it.ng; g++) {
+    const int gn = grow[8 * g + 7] >> 24;  // the group's rows, kept with its last entry
+    for (int j = wave; j < gn; j += kT1Threads / 64) {
+      const int r = grow[8 * g + j] & 0xffffff;
+      const double *t = Tq + (long long)r * n2, *v = V1 + (long long)r * d1;
+      double *d = rows + (nst + j) * ld;
+      for (int k = lane; k < n2; k += 64) d[k] = t[k];
+      for (int k = lane; k < d1; k += 64) d[n2 + k] = v[k];
+    }
+    nst += gn;
+  }
+  double *lw = rows + ((nst * ld + 1) & ~1);
+  int *lr = reinterpret_cast<int *>(lw + 8 * len);
+  for (int k = threadIdx.x; k < 8 * len; k += kT1Threads) lw[k] = W.rw[8 * b0 + k];
+  for (int k = threadIdx.x; k < len; k += kT1Threads) lr[k] = W.rsrc[b0 + k];
+  __syncthreads();
+  const int nch = (n2 + 63) >> 6, nu = nch * it.ng;
+  for (int u = wave; u < nu; u += kT1Threads / 64) {
+    const int ch = u % nch, g = u / nch;
+    const int s = ch * 64 + lane, sc = min(s, n2 - 1);
+    double acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[j] = 0.0;
+    const int l0 = (int)(gs[g].base - b0), l1 = l0 + (int)gs[g].n;
+    for (int e = l0; e < l1; e += 8) {  // the list's length is a multiple of 8
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int r = __builtin_amdgcn_readfirstlane(lr[e + k]);
+        v[k] = (r >= 0 ? Tq + (long long)r * n2 : V2 + (long long)~r * n2)[sc];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[j] = fma(lw[8 * (e + k) + j], v[k], acc[j]);
+    }
+    int st = 0;
+    for (int k = 0; k < g; k++) st += grow[8 * k + 7] >> 24;
+    const int gn = grow[8 * g + 7] >> 24;
+    const double *row0 = rows + st * ld;
+    const TSlice sl = W.cols[W.cbase[q] + ch];
+    // four entries of a column list in flight (their number is a multiple of 4)
+    for (int e = 0; e < (int)sl.n; e += 4) {
+      double w[4];
+      int p[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const long long o = sl.base + (long long)(e + v) * 64 + lane;
+        w[v] = W.cw[o];
+        p[v] = W.cp[o];
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int pv = p[v] == 0xffff ? 0 : p[v];
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[j] = fma(w[v], row0[min(j, gn - 1) * ld + pv], acc[j]);
+      }
+    }
+    if (s < n2)
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        if (j < gn) {
+          double *o = OV + T.off[q] + (long long)(grow[8 * g + j] & 0xffffff) * n2 + s;
+          *o = add ? *o + acc[j] : acc[j];
+        }
+  }
 }
 
 // Tensor Pandya matrices of one cross-coupled block (calculate_single_pandya,
@@ -1095,9 +1131,8 @@ __global__ void k_tnorm(DevLayout L, DevTensor T, const double *__restrict__ op,
       if (L.con[a] == L.con[b]) s += v * v;
       else if (L.con[a] == 0) s += 2.0 * v * v;  // (particle, hole); (hole, particle) is derived
     } else {
-      int q, a, b, c, d;
-      long long vp;
-      elem_of(L, T, e - nf, q, a, b, c, d, vp);
+      const int q = find_item(T.tstart, T.nblk, e - nf);
+      const long long vp = T.off[q] + e - nf - T.tstart[q];
       const double v = op[T.v_off + vp];
       s += (T.J1[q] == T.J2[q] ? 1.0 : 2.0) * v * v;
     }
@@ -1124,6 +1159,7 @@ struct TensorSpace {
   PackTables pack{};
   double *pack_d = nullptr;
   DevTensor dt{};
+  TLists lists{};
   double *gcc = nullptr, *gccp = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
   double *w1 = nullptr, *w2 = nullptr, *part = nullptr, *hpart = nullptr;
   const TProb *pp_probs[2] = {nullptr, nullptr}, *cc_probs[2] = {nullptr, nullptr};
@@ -1288,21 +1324,11 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       for (int i = 0; i < nr; i++) rpos[r0 + ix[i]] = i;
     }
     TUP(cperm, cperm); TUP(rperm, rperm);
-    std::vector<int> sperm(Ly.npairs);
-    for (int q = 0; q < Ly.nblocks; q++) {
-      const int p0 = Ly.pbase[q], np = Ly.pbase[q + 1] - p0;
-      std::vector<int> ix(np);
-      for (int k = 0; k < np; k++) ix[k] = k;
-      std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) {
-        return std::make_pair(Ly.grp_of[Ly.pair_a[p0 + x]], Ly.grp_of[Ly.pair_b[p0 + x]]) <
-               std::make_pair(Ly.grp_of[Ly.pair_a[p0 + y]], Ly.grp_of[Ly.pair_b[p0 + y]]);
-      });
-      std::copy(ix.begin(), ix.end(), sperm.begin() + p0);
-    }
-    TUP(sperm, sperm);
   }
+  std::vector<int> pstart_h, part_h;  // the orbits the tensor's one-body part couples
   {
-    std::vector<int> ps(nsp + 1, 0), pl;
+    std::vector<int> &ps = pstart_h, &pl = part_h;
+    ps.assign(nsp + 1, 0);
     for (int x = 0; x < nsp; x++) {
       ps[x] = (int)pl.size();
       for (int i = 0; i < nsp; i++)
@@ -1411,6 +1437,163 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
     if (upload_table(c, crow, &D.crow) != 0 || upload_table(c, cpos, &D.cpos) != 0 || upload_table(c, prow, &D.prow) != 0 ||
         upload_table(c, cblk, &D.cblk) != 0)
       return IMSRG_ENOMEM;
+  }
+  // lists and work items of k_t_lists, k_t_1body
+  {
+    std::vector<TList> lists;
+    std::vector<TItem> items;
+    std::vector<TSlice> groups, cols;
+    std::vector<int> cbase(S.nblk, 0), grow, rsrc, rdst;
+    std::vector<unsigned short> cp;
+    std::vector<long long> cost(S.nblk, 0);
+    unsigned lds = 0;
+    int maxdim = 1;
+    for (int q = 0; q < Ly.nblocks; q++) maxdim = std::max(maxdim, Ly.bdim[q]);
+    // the partner pairs of pair p (block of J1 for side 0, of J2 for side 1), in
+    // k_t_lists' order: its position in T's block or (g) in G's, or -1
+    auto partners = [&](int p, int side, int J1, int J2, auto &&put) {
+      const int a = Ly.pair_a[p], b = Ly.pair_b[p];
+      auto pos = [&](int i, int o, int J) {
+        return Ly.pidx[((size_t)(J >> 1) * nsp + std::min(i, o)) * nsp + std::max(i, o)];
+      };
+      int e = 0;
+      for (int w = 0; w < 2; w++) {
+        const int x = w ? b : a, o = w ? a : b, g = Ly.grp_of[x], J = side ? J2 : J1;
+        const bool tri = J <= Ly.jj[x] + Ly.jj[o] && J >= std::abs(Ly.jj[x] - Ly.jj[o]);
+        for (int k = 0; k < Ly.grp_cnt[g]; k++)
+          put(e++, w, false, tri ? pos(Ly.grp_list[Ly.grp_start[g] + k], o, J) : -1);
+      }
+      for (int w = 0; w < 2; w++) {
+        const int x = w ? b : a, o = w ? a : b;
+        for (int k = pstart_h[x]; k < pstart_h[x + 1]; k++) put(e++, w, true, pos(part_h[k] & 255, o, side ? J1 : J2));
+      }
+      return e;
+    };
+    std::vector<int> seen(4 * (size_t)maxdim, -1), slot(4 * (size_t)maxdim), ix;
+    for (int q = 0; q < S.nblk; q++) {
+      const int m1 = S.n1[q], m2 = S.n2[q];
+      if (m1 == 0 || m2 == 0) continue;
+      const int b1 = S.q1[q], p1 = Ly.pbase[b1], p2 = Ly.pbase[S.q2[q]], J1 = S.J1[q], J2 = S.J2[q];
+      const long long ld = (m2 + Ly.bdim[b1]) | 1;
+      // rows in class order, in groups of up to eight (fewer where eight rows
+      // take more than half of the LDS): whole classes, or parts of one
+      const int cap = (int)std::max<long long>(1, std::min<long long>(8, 9000 / ld));
+      auto key = [&](int r) { return std::make_pair(Ly.grp_of[Ly.pair_a[p1 + r]], Ly.grp_of[Ly.pair_b[p1 + r]]); };
+      ix.resize(m1);
+      for (int r = 0; r < m1; r++) ix[r] = r;
+      std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) { return key(x) < key(y); });
+      const int gfirst = (int)groups.size();
+      std::vector<int> gsize;
+      for (int r = 0; r < m1;) {
+        int n = 0;
+        while (r + n < m1 && n < cap) {
+          int m = 1;  // the next class
+          while (r + n + m < m1 && key(ix[r + n + m]) == key(ix[r + n])) m++;
+          if (n > 0 && n + m > cap) break;
+          n += std::min(m, cap - n);
+        }
+        const int gid = (int)groups.size();
+        const long long base = (long long)rsrc.size();
+        for (int j = 0; j < 8; j++) grow.push_back(ix[r + std::min(j, n - 1)]);
+        grow.back() |= n << 24;
+        for (int j = 0; j < n; j++) {
+          lists.push_back(TList{(long long)rdst.size(), q, ix[r + j], 0, 0});
+          lists.back().n = partners(p1 + ix[r + j], 0, J1, J2, [&](int, int w, bool g, int t) {
+            if (t < 0) {
+              rdst.push_back(-1);
+              return;
+            }
+            const size_t k = ((size_t)(g ? 2 : 0) + w) * maxdim + t;
+            if (seen[k] != gid) {
+              seen[k] = gid;
+              slot[k] = (int)rsrc.size();
+              rsrc.push_back(g ? ~t : t);
+            }
+            rdst.push_back(8 * slot[k] + j);
+          });
+        }
+        while (((long long)rsrc.size() - base) % 8 != 0) rsrc.push_back(0);  // of weight 0
+        groups.push_back(TSlice{base, (long long)rsrc.size() - base});
+        gsize.push_back(n);
+        r += n;
+      }
+      if (rsrc.size() >= (1u << 28)) return fail(IMSRG_EINVAL, "tensor blocks too many for the one-body terms' lists");
+      cbase[q] = (int)cols.size();
+      for (int c0 = 0; c0 < m2; c0 += 64) {
+        const long long base = (long long)cp.size();
+        int n = 0;
+        for (int k = c0; k < std::min(m2, c0 + 64); k++) n = std::max(n, partners(p2 + k, 1, J1, J2, [](int, int, bool, int) {}));
+        n = (n + 3) & ~3;
+        cp.resize(base + 64LL * n, 0xffff);
+        for (int k = c0; k < std::min(m2, c0 + 64); k++) {
+          lists.push_back(TList{base + k - c0, q, k, 1, 0});
+          lists.back().n = partners(p2 + k, 1, J1, J2, [&](int e, int, bool g, int t) {
+            if (t >= 0) cp[base + 64LL * e + k - c0] = (unsigned short)(g ? m2 + t : t);
+          });
+        }
+        cols.push_back(TSlice{base, n});
+      }
+      // groups per workgroup: at least eight units of work (a group x 64
+      // columns) for its wavefronts, in half of the LDS
+      const int ng = m2 > 384 ? 1 : m2 > 192 ? 2 : 4;
+      for (int g = gfirst; g < (int)groups.size();) {
+        long long e = 0, nr = 0, bytes = 0;
+        int k = 0;
+        while (k < ng && g + k < (int)groups.size()) {
+          const long long e1 = e + groups[g + k].n, nr1 = nr + gsize[g + k - gfirst];
+          const long long by = 8 * ((nr1 * ld + 1) & ~1LL) + 68 * e1;
+          if (k > 0 && by > 81920) break;
+          e = e1;
+          nr = nr1;
+          bytes = by;
+          k++;
+        }
+        items.push_back(TItem{q, g, k, 0});
+        cost[q] += nr * m2;
+        lds = (unsigned)std::max<long long>(lds, bytes);
+        g += k;
+      }
+    }
+    if (lds > 163840) return fail(IMSRG_EINVAL, "tensor blocks too wide for the one-body terms' workgroups");
+    // a block's workgroups on one XCD (workgroup i runs on XCD i % 8), whose L2
+    // keeps its rows: blocks in order of size, each to the least loaded XCD
+    {
+      std::vector<int> order;
+      std::vector<std::vector<TItem>> of(S.nblk), queue(8);
+      for (const TItem &it : items) of[it.q].push_back(it);
+      for (int q = 0; q < S.nblk; q++)
+        if (cost[q] > 0) order.push_back(q);
+      std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+      long long load[8] = {0};
+      size_t n = 0;
+      for (int q : order) {
+        const int x = (int)(std::min_element(load, load + 8) - load);
+        load[x] += cost[q];
+        queue[x].insert(queue[x].end(), of[q].begin(), of[q].end());
+        n = std::max(n, queue[x].size());
+      }
+      items.assign(8 * n, TItem{0, 0, 0, 0});
+      for (int x = 0; x < 8; x++)
+        for (size_t i = 0; i < queue[x].size(); i++) items[8 * i + x] = queue[x][i];
+    }
+    TLists &W = S.lists;
+    W.nlist = (int)lists.size();
+    W.nitem = (int)items.size();
+    W.lds = lds;
+    if (W.nlist > 0) {
+      if (upload_table(c, lists, &W.lists) != 0 || upload_table(c, items, &W.items) != 0 ||
+          upload_table(c, groups, &W.groups) != 0 || upload_table(c, cols, &W.cols) != 0 ||
+          upload_table(c, cbase, &W.cbase) != 0 || upload_table(c, grow, &W.grow) != 0 ||
+          upload_table(c, rsrc, &W.rsrc) != 0 || upload_table(c, rdst, &W.rdst) != 0 ||
+          upload_table(c, cp, &W.cp) != 0)
+        return IMSRG_ENOMEM;
+      const long long nr = 8LL * rsrc.size(), nc = (long long)cp.size();
+      if (dalloc(c, nr, &W.rw) || dalloc(c, nc, &W.cw)) return IMSRG_ENOMEM;
+      launch_fill(c->stream, W.rw, nr, 0.0);  // the weights no list writes stay 0
+      launch_fill(c->stream, W.cw, nc, 0.0);
+      if (lds > 65536)
+        HIPCHK(hipFuncSetAttribute((const void *)k_t_1body, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    }
   }
   // products: the pp and hh ladders per tensor block (W1, W2)
   {
@@ -1670,10 +1853,12 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
   if (mask & IMSRG_TS121)
     hipLaunchKernelGGL(k_t_onebody, dim3(L.nob), dim3(64), 0, s, L, D, 0, GF, RF, RV, (const double *)S.gcc,
                        (const double *)S.w1, (const double *)S.w2, OF, hL, hR, hres);
-  if (S.nelem > 0 && (mask & IMSRG_TS122))
-    hipLaunchKernelGGL(k_t122, dim3(nblk(S.nelem)), dim3(256), 0, s, L, D, GF, RV, OV, hR);
-  if (S.nelem > 0 && (mask & IMSRG_TS212))
-    hipLaunchKernelGGL(k_t212, dim3(nblk(S.nelem)), dim3(256), 0, s, L, D, GV, RF, OV);
+  if (S.lists.nlist > 0 && (mask & (IMSRG_TS122 | IMSRG_TS212))) {
+    hipLaunchKernelGGL(k_t_lists, dim3(S.lists.nlist), dim3(64), 0, s, L, D, S.lists, GF, RF,
+                       (mask & IMSRG_TS122) != 0, (mask & IMSRG_TS212) != 0);
+    hipLaunchKernelGGL(k_t_1body, dim3(S.lists.nitem), dim3(kT1Threads), S.lists.lds, s, L, D, S.lists, GV, RV, OV,
+                       !(mask & IMSRG_TS122));
+  }
   if ((mask & (IMSRG_TS222PPHH | IMSRG_TS221)) && S.n_pp_tiles > 0) {
     hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs[0], S.pp_tiles, S.n_pp_tiles, GV, RV,
                        S.w1);
