@@ -15,8 +15,9 @@
 // reference sub-blocks tgam(1..9) tile it and every 222_pp_hh product is a
 // plain GEMM against the scalar full channel blocks of G.
 //
-// Kernels.  One thread per output element for the gathers (111, 121, 211, 221,
-// 122, 212, tensor Pandya, ph recoupling), FP64 MFMA for the products (the
+// Kernels.  Lists of weights for 122 and 212, gathers by classes of orbit
+// quadruples for the tensor Pandya matrices and the ph recoupling, one wavefront
+// per output for the other one-body terms, FP64 MFMA for the products (the
 // pp/hh ladders and the two Pandya products of each cross-coupled block).  The
 // ph recoupling is a gather: every stored output element sums, over the
 // sixteen index patterns through which TS_commutator_222_ph scatters into it
@@ -38,13 +39,11 @@ namespace {
 // ---------------------------------------------------------------- device view
 struct DevTensor {
   int rank, dpar, nblk, ncc, nJ, nh, hx, nhole, npart;
-  long long nelem, nx, nr;      // tensor V elements; CCX / CCR elements
+  long long nelem;              // tensor V elements
   const int *holes, *parts;
   const int *J1, *J2, *q1, *q2, *n1, *n2;
   const long long *off, *tstart;  // per tensor block: V offset; first flat element
   const int *bidx;                // [((J1/2)*nJ + J2/2)*6 + (Tz+1)*2 + P1] -> block (J1 <= J2) or -1
-  const int *cJ3, *cJ4, *cq3, *cq4;
-  const long long *xoff, *roff, *woff, *xstart, *rstart;
   const int *ccol;                // [(scalar Pandya block * nsp + p) * nsp + h] -> column of (p,h)
   const double *x6, *s6;
   const double *n9;               // 9j table of the ph recoupling and the tensor Pandya (k_fill9j)
@@ -66,13 +65,11 @@ struct DevTensor {
   // of the same parity, triangle (ji, jx, R)): part[pstart[x] .. pstart[x+1]),
   // each i | ji << 8
   const int *pstart, *part;
-  // orders inside each scalar Pandya block: columns by (2j of p, 2j of h), rows
-  // by the (l,j,tz) groups of their two orbits (zero rows last); entry i is
-  // the block-local column / row in place i.  k_tpandya's threads take them
-  // so, so that the lanes of a wavefront sum (J3', J4') runs of equal length,
-  // and CCR, Wx and Wy keep their columns in the rows' order: the entries that
+  // group order of the rows inside each scalar Pandya block, by the (l,j,tz)
+  // groups of their two orbits (zero rows last): entry i is the block-local row
+  // in place i.  CCR, Wx and Wy keep their columns so: the entries that
   // quadruples of one class read then share cache lines
-  const int *cperm, *rperm;
+  const int *rperm;
   long long f_off, v_off;
 };
 
@@ -129,25 +126,9 @@ __device__ inline double t9j(const DevTensor &T, int a, int b, int J1, int c, in
   return sm;
 }
 
-// The 9j symbols of the ph recoupling, {j1 j2 J3; j3 j4 J4; J1 J2 R} with
-// J3 <= J4 <= J3 + R and J1 <= J2 <= J1 + R, tabulated once per tensor space:
-// index (((((((k1*nh + k2)*nh + k3)*nh + k4)*nJ + J3/2)*nd + (J4-J3)/2)*nJ + J1/2)*nd + (J2-J1)/2
-__device__ __forceinline__ long long n9_index(const DevTensor &T, int j1, int j2, int j3, int j4, int J3, int J4,
-                                              int J1, int J2) {
-  const int h = T.nh;
-  return ((((((((long long)(j1 >> 1) * h + (j2 >> 1)) * h + (j3 >> 1)) * h + (j4 >> 1)) * T.nJ + (J3 >> 1)) * T.nd +
-            ((J4 - J3) >> 1)) * T.nJ + (J1 >> 1)) * T.nd + ((J2 - J1) >> 1));
-}
-// {a b J3; c d J4; J3p J4p R} with J3 <= J4 <= J3 + R (a cross-coupled block) and any (J3p, J4p):
-// from the table, through the exchange of the first two columns (a factor (-1)^(sum of all nine))
-// when J4p < J3p
-__device__ __forceinline__ double t9j_cc(const DevTensor &T, int a, int b, int J3, int c, int d, int J4, int J3p,
-                                         int J4p) {
-  if (J4p - J3p > T.rank || J3p - J4p > T.rank) return 0.0;  // no triangle (J3p, J4p, R)
-  if (J3p <= J4p) return T.n9[n9_index(T, a, b, c, d, J3, J4, J3p, J4p)];
-  const double v = T.n9[n9_index(T, b, a, d, c, J3, J4, J4p, J3p)];
-  return ((a + b + J3 + c + d + J4 + J3p + J4p + T.rank) >> 1) & 1 ? -v : v;
-}
+// The 9j symbols of the ph recoupling and the tensor Pandya transform, {j1 j2 J3;
+// j3 j4 J4; J1 J2 R} with J3 <= J4 <= J3 + R and J1 <= J2 <= J1 + R, tabulated
+// once per tensor space: index (((((((k1*nh + k2)*nh + k3)*nh + k4)*nJ + J3/2)*nd + (J4-J3)/2)*nJ + J1/2)*nd + (J2-J1)/2
 // zeros past the table: a lane's pair of outputs may start up to a wavefront's
 // width of pairs past its row
 constexpr int kN9Pad = 256;
@@ -614,78 +595,6 @@ __global__ __launch_bounds__(kT1Threads, 6) void k_t_1body(DevLayout L, DevTenso
   }
 }
 
-// Tensor Pandya matrices of one cross-coupled block (calculate_single_pandya,
-// cross_coupled.f90:1416-1634).  mode 0: CCX (r3 x nb4, rows = ordered pairs at
-// J3 in the scalar Pandya row order, columns = (p,h) at J4); mode 1: CCR
-// (nb3 x r4, rows = (p,h) at J3, columns = ordered pairs (b,a) at J4 in group order).
-__global__ void k_tpandya(DevLayout L, DevTensor T, int mode, const double *__restrict__ RV, double *__restrict__ out,
-                          int hR) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long ntot = mode == 0 ? T.nx : T.nr;
-  if (e >= ntot) return;
-  const long long *st = mode == 0 ? T.xstart : T.rstart;
-  const int x = find_item(st, T.ncc, e);
-  const long long u = e - st[x];
-  const int J3 = T.cJ3[x], J4 = T.cJ4[x], q3 = T.cq3[x], q4 = T.cq4[x];
-  int a, b, p, h;
-  long long o;  // the entry's position in its matrix
-  if (mode == 0) {
-    const int nb4 = L.ccnph[q4];
-    const int R1 = (int)(u / nb4), k = T.cperm[L.cccbase[q4] + (int)(u % nb4)];
-    o = (long long)R1 * nb4 + k;
-    a = L.ccrow_a[L.ccrbase[q3] + R1];
-    b = L.ccrow_b[L.ccrbase[q3] + R1];
-    p = L.cccol_p[L.cccbase[q4] + k];
-    h = L.cccol_h[L.cccbase[q4] + k];
-  } else {
-    const int r4 = L.ccrlen[q4];
-    const int k = (int)(u / r4), G = T.rperm[L.ccrbase[q4] + (int)(u % r4)];
-    o = u;
-    p = L.cccol_p[L.cccbase[q3] + k];
-    h = L.cccol_h[L.cccbase[q3] + k];
-    b = L.ccrow_a[L.ccrbase[q4] + G];  // the row pair is (b, a)
-    a = L.ccrow_b[L.ccrbase[q4] + G];
-  }
-  double v = 0.0;
-  if (a >= 0) {
-    const int ja = L.jj[a], jb = L.jj[b], jp = L.jj[p], jh = L.jj[h];
-    if (((L.l[a] + L.l[h]) & 1) == ((L.l[b] + L.l[p] + (T.dpar >> 1)) & 1) && L.tz[a] + L.tz[h] == L.tz[b] + L.tz[p]) {
-      // the (J3', J4') terms four at a time: positions, factors and 9j of a
-      // batch first (every table read off any branch), then its four tensor
-      // reads, so a batch makes three dependent round trips instead of one
-      // chain per term.  The channel test is the same for every term.
-      const int a3 = abs(ja - jh), n3 = (ja + jh - a3) / 2 + 1;
-      const int a4 = abs(jp - jb), n4 = (jp + jb - a4) / 2 + 1, nt = n3 * n4;
-      const bool chan = true;  // the parity and Tz tests above hold for both pairs of every term
-      double sm = 0.0;
-      for (int t0 = 0; t0 < nt; t0 += 4) {
-        long long pos[4];
-        double w[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          const int t = min(t0 + k, nt - 1);
-          const int J3p = a3 + 2 * (t / n4), J4p = a4 + 2 * (t % n4);
-          double f;
-          pos[k] = mode == 0 ? t_pos_all(L, T, hR, a, h, p, b, ja, jh, jp, jb, J3p, J4p, chan, f)
-                             : t_pos_all(L, T, hR, h, a, b, p, jh, ja, jb, jp, J3p, J4p, chan, f);
-          const double nj = mode == 0 ? t9j_cc(T, ja, jb, J3, jh, jp, J4, J3p, J4p)
-                                      : t9j_cc(T, jh, jp, J3, ja, jb, J4, J3p, J4p);
-          w[k] = t0 + k < nt ? -sgnp(J4p >> 1) * sqrt((J3p + 1.0) * (J4p + 1.0)) * nj * f : 0.0;
-        }
-        double g[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) g[k] = RV[pos[k]];
-#pragma unroll
-        for (int k = 0; k < 4; k++) sm += w[k] * g[k];
-      }
-      const double s34 = sqrt((J3 + 1.0) * (J4 + 1.0));
-      v = mode == 0 ? sm * sgnp((jh + jb + J4) >> 1) * s34
-                    : sm * sgnp((jp + ja + J4) >> 1) * s34 * sgnp((jp + jh) >> 1);
-    }
-  }
-  out[(mode == 0 ? T.xoff[x] : T.roff[x]) + o] = v;
-}
-
 // The scalar Pandya matrices with each column's rows in group order: the right
 // operand of Wy
 __global__ void k_gcc_order(DevLayout L, DevTensor T, const double *__restrict__ gcc, double *__restrict__ out) {
@@ -737,6 +646,273 @@ constexpr unsigned kPhIa = 0x2727DD88u, kPhIb = 0x88DD88DDu, kPhIc = 0x72727272u
 constexpr unsigned kPhCond = 0xF960F960u;
 constexpr int kPhQ = 8;    // quadruples of one class per workgroup
 constexpr int kPhU = 2;    // slots whose 9j a lane reads together
+constexpr int kPhB = 32;   // slots a workgroup weights at a time
+
+// The sums of the recoupling and the tensor Pandya transform: a quadruple's
+// outputs o = (J - Jlo)/2 * nd + (J' - J)/2 over up to 128 consecutive o, each
+// the sum over slots of weight[slot][quadruple] * 9j[slot][o], for kPhQ
+// quadruples of one class at once.  The table's fastest indices are the
+// outputs' (J, J'), so a slot's 9j are one contiguous run: groups of lanes as
+// wide as half the outputs take a slot each, a lane two neighbouring outputs.
+struct Recouple {
+  int wsh, G, grp, ol;
+  unsigned flip;  // bit 4u + ab: the sign of output u's phase, ab a slot's flags (J/2, J'/2)
+  double acc[kPhQ][2];
+
+  // outputs from o0 on, nout of them in all; x / nd = x * ndinv >> 16
+  __device__ __forceinline__ void begin(int lane, int o0, int nout, int Jlo, int nd, int ndinv) {
+    const int nh2 = (min(nout - o0, 128) + 1) >> 1;  // lanes a group needs
+    wsh = nh2 <= 4 ? 2 : nh2 <= 8 ? 3 : nh2 <= 16 ? 4 : nh2 <= 32 ? 5 : 6;
+    G = 64 >> wsh;
+    grp = lane >> wsh;
+    ol = o0 + 2 * (lane & ((1 << wsh) - 1));
+    flip = 0;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int oq = ((ol + u) * ndinv) >> 16;
+      const unsigned e1 = ((Jlo >> 1) + oq) & 1, e2 = (e1 + (ol + u - oq * nd)) & 1;
+      flip |= (e1 << 1 | e2 << 2 | (e1 ^ e2) << 3) << (4 * u);
+    }
+#pragma unroll
+    for (int q = 0; q < kPhQ; q++) acc[q][0] = acc[q][1] = 0.0;
+  }
+  // count slots: weights cs (row count: zeros), 9j rows sb9 (flags in the top two bits) from n9
+  __device__ __forceinline__ void add(const double *__restrict__ n9, const double (*cs)[kPhQ], const unsigned *sb9,
+                                      int count) {
+    for (int t0 = grp; t0 < count; t0 += kPhU * G) {
+      dpair_t v[kPhU];
+      unsigned ab[kPhU];
+#pragma unroll
+      for (int u = 0; u < kPhU; u++) {
+        const unsigned b = sb9[min(t0 + u * G, count)];
+        v[u] = *reinterpret_cast<const dpair_t *>(n9 + (b & 0x3fffffffu));
+        ab[u] = b >> 30;
+      }
+#pragma unroll
+      for (int u = 0; u < kPhU; u++) {
+        __builtin_amdgcn_sched_barrier(0);  // one slot's row from LDS at a time: registers
+        const double f0 = ((flip >> ab[u]) & 1) ? -v[u].x : v[u].x;
+        const double f1 = ((flip >> (4 + ab[u])) & 1) ? -v[u].y : v[u].y;
+        const double *cq = cs[min(t0 + u * G, count)];
+#pragma unroll
+        for (int q = 0; q < kPhQ; q++) {
+          const double c = cq[q];
+          acc[q][0] = fma(f0, c, acc[q][0]);
+          acc[q][1] = fma(f1, c, acc[q][1]);
+        }
+      }
+    }
+  }
+  // the groups' sums; each group is left with nown quadruples from q0 (mine
+  // false: another group holds the same one)
+  __device__ __forceinline__ void reduce(int lane, int &q0, int &nown, bool &mine) {
+    q0 = 0;
+    nown = kPhQ;
+#pragma unroll
+    for (int st = 0; st < 3; st++) {
+      if (wsh > 5 - st) break;
+      const int half = kPhQ >> (st + 1);
+      const bool up = (lane >> (5 - st)) & 1;
+#pragma unroll
+      for (int i = 0; i < half; i++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const double give = up ? acc[i][u] : acc[i + half][u], keep = up ? acc[i + half][u] : acc[i][u];
+          acc[i][u] = keep + __shfl_xor(give, 32 >> st);
+        }
+      if (up) q0 += half;
+      nown = half;
+    }
+    mine = true;
+    if (wsh == 2) {  // 16 groups for 8 quadruples
+#pragma unroll
+      for (int u = 0; u < 2; u++) acc[0][u] += __shfl_xor(acc[0][u], 4);
+      mine = !(lane & 4);
+    }
+  }
+};
+// Runs of 64 class-ordered items per XCD, in turn: its L2 keeps the 9j rows
+// and entries that neighbouring items share, and the classes of high j, with
+// the most slots, spread over all XCDs.  bid of npad (a multiple of 512), the
+// heavy classes first
+__device__ __forceinline__ int class_item(int bid, int npad) {
+  const int b = npad - 1 - bid, i8 = b >> 3;
+  return ((i8 >> 6) << 9) + ((b & 7) << 6) + (i8 & 63);
+}
+
+// The tensor Pandya matrices of the cross-coupled blocks (calculate_single_pandya,
+// cross_coupled.f90:1416-1634): CCX (rows: ordered pairs (a,b) at J3 in the
+// scalar Pandya row order, columns: (p,h) at J4) and CCR (rows: (p,h) at J3,
+// columns: ordered pairs (b,a) at J4 in group order).  Both are, for orbits
+// (u,v,x,y) = (a,h,b,p) or (h,a,p,b), the sum over (J', J'') of
+//   -(-1)^(J''/2) sqrt((J'+1)(J''+1)(J3+1)(J4+1)) {u v J'; x y J''; J3 J4 R}
+//   T^{J' J''}(u v, y x) (-1)^((jv+jx+J4)/2), times (-1)^((jp+jh)/2) in CCR
+// in row (u,x) at J3 and column (y,v) at J4.  The entries T that a quadruple
+// reads do not depend on (J3, J4): gathered once, as in the recoupling, by
+// classes of quadruples.  (J', J'') with J' > J'' exchanges the first two
+// rows of the 9j, which the table holds for J' <= J'' only.
+//
+// One thread per element, with a 9j and five table reads per term, took
+// 3.8 ms for both matrices at 90 orbits, rank 4 (16 M elements), 100 us at 30
+// orbits, rank 2; this kernel 0.55 ms and 20 us.
+struct TPan {
+  const unsigned *quads;  // u | v<<8 | x<<16 | y<<24
+  const PhChunkT *chunks;
+  int nchunk, npad;
+  const int *rtab, *ctab;     // row of the pair (u,x) or (x,u), column of (y,v), by pair, J fastest
+  const struct CcBlk *blk;    // the matrices, as DevTensor::cblk
+  double *out;
+};
+struct PanSeg {
+  double c;
+  long long off;  // of the tensor block
+  unsigned b9;    // 9j table row | 3 << 30 where (-1)^((J3+J4)/2) applies
+  int n2;         // its row length
+  unsigned code;  // J'/2 | J''/2 << 8 | (J' > J'') << 16
+};
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_t_pandya(
+    DevLayout L, DevTensor T, TPan P0, TPan P1, const double *__restrict__ RV, int hR) {
+  __shared__ PanSeg seg[kPhB + 64];
+  __shared__ alignas(16) double cs[kPhB + 1][kPhQ];
+  __shared__ unsigned sb9[kPhB + 1];
+  const int mode = (int)blockIdx.x >= P0.npad;
+  const TPan P = mode ? P1 : P0;
+  const int item = class_item((int)blockIdx.x - (mode ? P0.npad : 0), P.npad);
+  if (item >= P.nchunk) return;
+  const int lane = threadIdx.x, quad = lane & (kPhQ - 1);
+  const PhChunkT ch = P.chunks[item];
+  const int nq = ch.n, R = T.rank, n = L.nsp, nd = T.nd, nJ = T.nJ, h = T.nh, nd2 = 2 * nd - 1;
+  const unsigned code = P.quads[ch.first + min(quad, nq - 1)];  // the lane's quadruple
+  const int u = code & 255, v = (code >> 8) & 255, x = (code >> 16) & 255, y = (int)(code >> 24);
+  const int ju = ch.jv & 255, jv = (ch.jv >> 8) & 255, jx = (ch.jv >> 16) & 255, jy = (int)(ch.jv >> 24);
+  const unsigned lt = ch.lt;  // bits 0-3: l of u, v, x, y; 4-7: tz
+  const int Tzq = (int)((lt >> 4) & 1) + (int)((lt >> 5) & 1);
+  const int Puv = (lt ^ (lt >> 1)) & 1, Pyx = ((lt >> 2) ^ (lt >> 3)) & 1;
+  const int ndinv = 65536 / nd + 1, nd2inv = 65536 / nd2 + 1;  // exact for x <= 32 nd2 + 128, nd2 <= 50
+  // the lane's pairs in the channels' order, and what an exchange does
+  const int puv = (min(u, v) * n + max(u, v)) * nJ, pyx = (min(x, y) * n + max(x, y)) * nJ;
+  const double fq = (u == v ? M_SQRT2 : 1.0) * (x == y ? M_SQRT2 : 1.0);
+  const unsigned b9a = (unsigned)((((ju >> 1) * h + (jv >> 1)) * h + (jx >> 1)) * h + (jy >> 1));
+  const unsigned b9b = (unsigned)((((jx >> 1) * h + (jy >> 1)) * h + (ju >> 1)) * h + (jv >> 1));
+  const int Jlo = abs(ju - jx), nout = (min(ju, jx) + 1) * nd;  // J3 of the row pair
+  const int J1lo = abs(ju - jv), nslot = (min(ju, jv) + 1) * nd2;
+  Recouple rc;
+  for (int o0 = 0; o0 < nout; o0 += 128) {
+    rc.begin(lane, o0, nout, Jlo, nd, ndinv);
+    const double *n9 = T.n9 + (size_t)(Jlo >> 1) * nd + rc.ol;
+    int nseg = 0;
+    for (int s0 = 0; s0 < nslot || nseg > 0;) {
+      // the slots (J', J'') that exist, until kPhB wait or none is left
+      while (nseg < kPhB && s0 < nslot) {
+        const int s = s0 + lane, r = min(s, nslot - 1), rq = (r * nd2inv) >> 16;
+        const int Ja = J1lo + 2 * rq, Jb = Ja + 2 * (r - rq * nd2 - (nd - 1));
+        bool ok = s < nslot && Jb >= abs(jx - jy) && Jb <= jx + jy && Ja + Jb >= R;
+        const bool sw = Ja > Jb;
+        const int lo = sw ? Jb : Ja, dJ = abs(Jb - Ja);
+        OutBlk ob{-1, 0, 0};
+        if (ok) ob = T.oblk[((lo >> 1) * nd + (dJ >> 1)) * 6 + Tzq * 2 + (sw ? Pyx : Puv)];
+        ok = ok && ob.off >= 0;
+        const unsigned long long m = __ballot(ok);
+        if (ok) {
+          PanSeg g;
+          g.c = -sgnp(Jb >> 1) * sqrt((Ja + 1.0) * (Jb + 1.0));
+          if (sw) g.c *= sgnp((dJ >> 1) + ((ju + jv + Ja + jx + jy + Jb + R) >> 1)) * hR;
+          g.off = ob.off;
+          g.n2 = ob.n2;
+          g.b9 = (((sw ? b9b : b9a) * nJ + (lo >> 1)) * nd + (dJ >> 1)) * (unsigned)(nJ * nd) | (sw ? 3u << 30 : 0u);
+          g.code = (unsigned)(Ja >> 1) | (unsigned)(Jb >> 1) << 8 | (sw ? 1u << 16 : 0u);
+          seg[nseg + __popcll(m & ((1ull << lane) - 1ull))] = g;
+        }
+        nseg += __popcll(m);
+        s0 += 64;
+      }
+      __syncthreads();
+      const int nb = min(nseg, kPhB);
+      {
+        int ix[4], jx_[4];
+        double w[4];
+        auto slot = [&](int k) -> const PanSeg & { return seg[min(8 * k + (lane >> 3), max(nb - 1, 0))]; };
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const unsigned gc = slot(k).code;
+          ix[k] = T.prow[puv + (int)(gc & 31)];
+          jx_[k] = T.prow[pyx + (int)((gc >> 8) & 31)];
+          if (8 * k + (lane >> 3) >= nb || quad >= nq) ix[k] = -1;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const bool sw = (slot(k).code >> 16) & 1;
+          w[k] = 0.0;
+          if ((ix[k] | jx_[k]) >= 0)
+            w[k] = RV[slot(k).off + (long long)(sw ? jx_[k] : ix[k]) * slot(k).n2 + (sw ? ix[k] : jx_[k])];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          const int pos = 8 * k + (lane >> 3);
+          if (pos < nb) {
+            const unsigned gc = slot(k).code;
+            // a pair read against its order: (-1)^(1 + (j + j' - J)/2)
+            int e = 0;
+            if (u > v) e += 1 + ((ju + jv) >> 1) - (int)(gc & 31);
+            if (y > x) e += 1 + ((jx + jy) >> 1) - (int)((gc >> 8) & 31);
+            const double c = slot(k).c * w[k] * fq;
+            cs[pos][quad] = (e & 1) ? -c : c;
+            if (quad == 0) sb9[pos] = slot(k).b9;
+          }
+        }
+      }
+      if (lane < kPhQ) cs[nb][lane] = 0.0;  // what the last round reads past the end
+      if (lane == kPhQ) sb9[nb] = 0;
+      // the slots that wait move to the front
+      nseg -= nb;
+      const double mc = seg[kPhB + lane].c;
+      const long long mw = seg[kPhB + lane].off;
+      const unsigned mb = seg[kPhB + lane].b9, mo = seg[kPhB + lane].code;
+      const int mn = seg[kPhB + lane].n2;
+      __syncthreads();
+      if (lane < nseg) {
+        seg[lane].c = mc;
+        seg[lane].off = mw;
+        seg[lane].b9 = mb;
+        seg[lane].code = mo;
+        seg[lane].n2 = mn;
+      }
+      rc.add(n9, cs, sb9, nb);
+      __syncthreads();
+    }
+    int q0, nown;
+    bool mine;
+    rc.reduce(lane, q0, nown, mine);
+    const int ol = rc.ol, oq0 = (ol * ndinv) >> 16, oq1 = ((ol + 1) * ndinv) >> 16;
+    const int J3o[2] = {Jlo + 2 * oq0, Jlo + 2 * oq1};
+    const int J4o[2] = {J3o[0] + 2 * (ol - oq0 * nd), J3o[1] + 2 * (ol + 1 - oq1 * nd)};
+    CcBlk ob[2];
+    double nrm[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int J3 = J3o[k], J4 = J4o[k];
+      const bool val = mine && ol + k < nout && ol + k < o0 + 128 && J4 >= abs(jy - jv) && J4 <= jy + jv;
+      const unsigned dl = lt ^ (lt >> 2);  // l and tz of u against x
+      ob[k] = P.blk[val ? ((int)(((dl >> 4) & 1) + 2 * (dl & 1)) * nJ + (J3 >> 1)) * nd + ((J4 - J3) >> 1) : 0];
+      if (!val) ob[k].wo = -1;
+      nrm[k] = sqrt((J3 + 1.0) * (J4 + 1.0)) * sgnp(((jv + jx + J4) >> 1) + (mode ? (ju + jx) >> 1 : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < kPhQ; i++) {
+      if (i >= nown) break;
+      const unsigned cd = (unsigned)__shfl((int)code, q0 + i);
+      const int cu = cd & 255, cv = (cd >> 8) & 255, cx = (cd >> 16) & 255, cy = (int)(cd >> 24);
+      const int *p1 = P.rtab + (mode ? cx * n + cu : cu * n + cx) * nJ, *p2 = P.ctab + (cy * n + cv) * nJ;
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+        if (q0 + i < nq && ob[k].wo >= 0) {
+          const int r = p1[J3o[k] >> 1], c = p2[J4o[k] >> 1];
+          if ((r | c) >= 0) P.out[ob[k].wo + (long long)r * ob[k].rl4 + c] = rc.acc[i][k] * nrm[k];
+        }
+    }
+  }
+}
+
 struct PhPat {
   double cs;     // sign * herm
   unsigned b9;   // 9j table index of the four orbits' 2j
@@ -750,35 +926,28 @@ struct PhSeg {
   unsigned b9;    // 9j table row without the (J1, J2) part | ab << 30
   unsigned code;  // pattern | J3/2 << 4 | J4/2 << 12
 };
-// One wavefront takes up to kPhQ quadruples of one class, 32 slots at a time:
+// One wavefront takes up to kPhQ quadruples of one class, kPhB slots at a time:
 //   1. one lane per slot finds the slots that exist (J4's triangle, no Wy at
 //      J3 = J4), their (J3, J4) weights and product blocks;
 //   2. lanes (slot, quadruple) read the product entries, rows and columns from
 //      per-pair tables (a quadruple's run over J3 is contiguous there); the
 //      entries that pass the reference's |W| > 1e-6 test go weighted to LDS,
 //      slots with no entry left are dropped;
-//   3. groups of lanes as wide as half the outputs take a slot each: a lane
-//      reads the 9j of its two neighbouring outputs (the (J1, J2) part is the
-//      table's fastest index, so a group reads one contiguous run) and adds
-//      slot x output into all kPhQ quadruples from LDS.
+//   3. the slots are summed into the outputs (Recouple).
 // What bounds it: the entries' reads (W is 1 GB at 90 orbits, rank 4) and the
 // index arithmetic around them.  One wavefront per quadruple with a lane per
 // slot read a 9j cache line per (slot, output): 7.7 ms there (2.6 M
 // quadruples, 256 M slots, 3 G slot-outputs); this form 2.8 ms, 5.3 before
 // the columns of W went into class order.
 // W: Wx, then Wy wsize doubles on
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_t222ph(DevLayout L, DevTensor T, const double *__restrict__ W,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_t222ph(DevLayout L, DevTensor T, const double *__restrict__ W,
     long long wsize, double *__restrict__ OV, int hL, int hR) {
   __shared__ PhPat pat[16];
-  __shared__ PhSeg seg[32 + 64];
+  __shared__ PhSeg seg[kPhB + 64];
   __shared__ ushort2 base[16][kPhQ];  // per pattern and quadruple: the orbit pairs (d,a) and (c,b)
-  __shared__ alignas(16) double cs[32 + 1][kPhQ];
-  __shared__ unsigned sb9[32 + 1];
-  // runs of 64 class-ordered items per XCD, in turn: its L2 keeps the 9j rows
-  // and product entries that neighbouring items share, and the classes of
-  // high j, with the most slots, spread over all XCDs
-  const int bid = T.nqpad - 1 - (int)blockIdx.x, i8 = bid >> 3;  // the heavy classes come first
-  const int item = ((i8 >> 6) << 9) + ((bid & 7) << 6) + (i8 & 63);
+  __shared__ alignas(16) double cs[kPhB + 1][kPhQ];
+  __shared__ unsigned sb9[kPhB + 1];
+  const int item = class_item(blockIdx.x, T.nqpad);
   if (item >= T.nqchunk) return;
   const int lane = threadIdx.x;
   const PhChunkT ch = T.qchunk[item];
@@ -859,25 +1028,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
   const int ndinv = 65536 / nd + 1;  // x / nd, exact for x <= 32 nd + 128, nd <= 50
   auto div = [&](int x) { return (x * ndinv) >> 16; };
   __syncthreads();
+  Recouple rc;
   for (int o0 = 0; o0 < nout; o0 += 128) {
-    const int nh2 = (min(nout - o0, 128) + 1) >> 1;  // lanes a group needs, two outputs each
-    const int wsh = nh2 <= 4 ? 2 : nh2 <= 8 ? 3 : nh2 <= 16 ? 4 : nh2 <= 32 ? 5 : 6;
-    const int G = 64 >> wsh, grp = lane >> wsh, ol = o0 + 2 * (lane & ((1 << wsh) - 1));
-    unsigned flip = 0;  // bit 4u + ab: the sign of output u's (J1, J2) phase
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int oq = div(ol + u);
-      const unsigned e1 = ((Jlo >> 1) + oq) & 1, e2 = (e1 + (ol + u - oq * nd)) & 1;
-      flip |= (e1 << 1 | e2 << 2 | (e1 ^ e2) << 3) << (4 * u);
-    }
+    rc.begin(lane, o0, nout, Jlo, nd, ndinv);
+    const int ol = rc.ol;
     const double *n9 = T.n9 + (size_t)(Jlo >> 1) * nd + ol;
-    double acc[kPhQ][2];
-#pragma unroll
-    for (int q = 0; q < kPhQ; q++) acc[q][0] = acc[q][1] = 0.0;
     int k = 0, nseg = 0;  // a lane's pattern: its slot only grows, so k carries over
     for (int s0 = 0; s0 < nslot || nseg > 0;) {
-      // 1: the slots that exist, until 32 wait or none is left
-      while (nseg < 32 && s0 < nslot) {
+      // 1: the slots that exist, until kPhB wait or none is left
+      while (nseg < kPhB && s0 < nslot) {
         const int s = min(s0 + lane, nslot - 1);
         while (k < 15 && pat[k + 1].start <= s) k++;
         const PhPat p = pat[k];
@@ -903,8 +1062,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
         s0 += 64;
       }
       __syncthreads();
-      // 2: the entries of the first 32
-      const int nb = min(nseg, 32);
+      // 2: the entries of the first kPhB
+      const int nb = min(nseg, kPhB);
       int count = 0;
       {
         double w[4];
@@ -948,9 +1107,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
       if (lane == kPhQ) sb9[count] = 0;
       // the slots that wait move to the front
       nseg -= nb;
-      const double mc = seg[32 + lane].c;
-      const long long mw = seg[32 + lane].w;
-      const unsigned mb = seg[32 + lane].b9, mo = seg[32 + lane].code;
+      const double mc = seg[kPhB + lane].c;
+      const long long mw = seg[kPhB + lane].w;
+      const unsigned mb = seg[kPhB + lane].b9, mo = seg[kPhB + lane].code;
       __syncthreads();
       if (lane < nseg) {
         seg[lane].c = mc;
@@ -958,57 +1117,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
         seg[lane].b9 = mb;
         seg[lane].code = mo;
       }
-      // 3: slots times 9j
-      for (int t0 = grp; t0 < count; t0 += kPhU * G) {
-        dpair_t v[kPhU];
-        unsigned ab[kPhU];
-#pragma unroll
-        for (int u = 0; u < kPhU; u++) {
-          const unsigned b = sb9[min(t0 + u * G, count)];
-          v[u] = *reinterpret_cast<const dpair_t *>(n9 + (b & 0x3fffffffu));
-          ab[u] = b >> 30;
-        }
-#pragma unroll
-        for (int u = 0; u < kPhU; u++) {
-          __builtin_amdgcn_sched_barrier(0);  // one slot's row from LDS at a time: registers
-          const double f0 = ((flip >> ab[u]) & 1) ? -v[u].x : v[u].x;
-          const double f1 = ((flip >> (4 + ab[u])) & 1) ? -v[u].y : v[u].y;
-          const double *cq = cs[min(t0 + u * G, count)];
-#pragma unroll
-          for (int q = 0; q < kPhQ; q++) {
-            const double c = cq[q];
-            acc[q][0] = fma(f0, c, acc[q][0]);
-            acc[q][1] = fma(f1, c, acc[q][1]);
-          }
-        }
-      }
+      rc.add(n9, cs, sb9, count);  // 3
       __syncthreads();
     }
-    // the groups' sums, each group left with its share of the quadruples (q0
-    // on), which it writes with one add per element and no wait for the old
-    // value
-    int q0 = 0, nown = kPhQ;
-#pragma unroll
-    for (int st = 0; st < 3; st++) {
-      if (wsh > 5 - st) break;
-      const int half = kPhQ >> (st + 1);
-      const bool up = (lane >> (5 - st)) & 1;
-#pragma unroll
-      for (int i = 0; i < half; i++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-          const double give = up ? acc[i][u] : acc[i + half][u], keep = up ? acc[i + half][u] : acc[i][u];
-          acc[i][u] = keep + __shfl_xor(give, 32 >> st);
-        }
-      if (up) q0 += half;
-      nown = half;
-    }
-    bool mine = true;
-    if (wsh == 2) {  // 16 groups for 8 quadruples
-#pragma unroll
-      for (int u = 0; u < 2; u++) acc[0][u] += __shfl_xor(acc[0][u], 4);
-      mine = !(lane & 4);
-    }
+    // each group writes its share of the quadruples, with one add per element
+    // and no wait for the old value
+    int q0, nown;
+    bool mine;
+    rc.reduce(lane, q0, nown, mine);
     const int oq0 = div(ol), oq1 = div(ol + 1);
     const int J1o[2] = {Jlo + 2 * oq0, Jlo + 2 * oq1};
     const int J2o[2] = {J1o[0] + 2 * (ol - oq0 * nd), J1o[1] + 2 * (ol + 1 - oq1 * nd)};
@@ -1035,7 +1151,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
         if (q0 + i < nq && ob[u].off >= 0 && !(x0 == x1 && (e1 & 1)) && !(x2 == x3 && (e2 & 1))) {
           const int r = p1[e1], sc = p2[e2];
           if ((r | sc) >= 0)
-            unsafeAtomicAdd(OV + ob[u].off + (long long)r * ob[u].n2 + sc, acc[i][u] * nrm[u] * f);
+            unsafeAtomicAdd(OV + ob[u].off + (long long)r * ob[u].n2 + sc, rc.acc[i][u] * nrm[u] * f);
         }
       }
     }
@@ -1152,7 +1268,7 @@ struct TensorSpace {
   std::vector<long long> off, tstart;
   long long vsize = 0, v_off = 0, op_size = 0, neq = 0, nelem = 0;
   std::vector<int> cJ3, cJ4, cq3, cq4, ccol;
-  std::vector<long long> xoff, roff, woff, xstart, rstart;
+  std::vector<long long> xoff, roff, woff;
   long long xsize = 0, rsize = 0, wsize = 0;
   std::vector<double> x6, s6;
   long long n9size = 0;
@@ -1160,6 +1276,7 @@ struct TensorSpace {
   double *pack_d = nullptr;
   DevTensor dt{};
   TLists lists{};
+  TPan pan[2]{};  // CCX, CCR
   double *gcc = nullptr, *gccp = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
   double *w1 = nullptr, *w2 = nullptr, *part = nullptr, *hpart = nullptr;
   const TProb *pp_probs[2] = {nullptr, nullptr}, *cc_probs[2] = {nullptr, nullptr};
@@ -1223,7 +1340,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   S.neq = 1 + (long long)Ly.nhole * Ly.nhole + (long long)Ly.npart * Ly.npart + (long long)Ly.npart * Ly.nhole + el;
   // cross-coupled tensor blocks (allocate_small_tensor_CCMAT, cross_coupled.f90:498-700):
   // J3, J4 >= J3 within rank, |Tz|, parity of the J3 pairs
-  long long xo = 0, ro = 0, wo = 0, xe = 0, re = 0;
+  long long xo = 0, ro = 0, wo = 0;
   for (int J3 = 0; J3 <= 2 * JM; J3 += 2)
     for (int J4 = std::max(std::abs(J3 - rank), J3); J4 <= std::min(J3 + rank, 2 * JM); J4 += 2)
       for (int Tz = 0; Tz <= 1; Tz++)
@@ -1238,17 +1355,11 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
           S.xoff.push_back(xo);
           S.roff.push_back(ro);
           S.woff.push_back(wo);
-          S.xstart.push_back(xe);
-          S.rstart.push_back(re);
           xo = align32(xo + r3 * nb4);
           ro = align32(ro + nb3 * r4);
           wo = align32(wo + r3 * r4);
-          xe += r3 * nb4;
-          re += nb3 * r4;
         }
   S.ncc = (int)S.cJ3.size();
-  S.xstart.push_back(xe);
-  S.rstart.push_back(re);
   S.xsize = xo;
   S.rsize = ro;
   S.wsize = wo;
@@ -1284,35 +1395,25 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   // device tables
   DevTensor &D = S.dt;
   D.rank = rank; D.dpar = dpar; D.nblk = S.nblk; D.ncc = S.ncc; D.nJ = nJ; D.nh = nh; D.hx = hx;
-  D.nhole = Ly.nhole; D.npart = Ly.npart; D.nelem = S.nelem; D.nx = xe; D.nr = re;
+  D.nhole = Ly.nhole; D.npart = Ly.npart; D.nelem = S.nelem;
   D.f_off = Ly.f_off; D.v_off = S.v_off;
 #define TUP(vec, field) \
   if (upload_table(c, vec, &D.field) != 0) return IMSRG_ENOMEM
   TUP(Ly.holes, holes); TUP(Ly.parts, parts);
   TUP(S.J1, J1); TUP(S.J2, J2); TUP(S.q1, q1); TUP(S.q2, q2); TUP(S.n1, n1); TUP(S.n2, n2);
   TUP(S.off, off); TUP(S.tstart, tstart); TUP(S.bidx, bidx);
-  TUP(S.cJ3, cJ3); TUP(S.cJ4, cJ4); TUP(S.cq3, cq3); TUP(S.cq4, cq4);
-  TUP(S.xoff, xoff); TUP(S.roff, roff); TUP(S.woff, woff); TUP(S.xstart, xstart); TUP(S.rstart, rstart);
   TUP(S.ccol, ccol); TUP(S.x6, x6); TUP(S.s6, s6);
   std::vector<int> rperm, rpos;  // Pandya rows in group order, and each row's place in it
   {
-    std::vector<int> cperm(Ly.cccbase[Ly.ncc]);
     rperm.resize(Ly.ccrbase[Ly.ncc]);
     rpos.resize(Ly.ccrbase[Ly.ncc]);
     for (int q = 0; q < Ly.ncc; q++) {
-      const int c0 = Ly.cccbase[q], nc = Ly.cccbase[q + 1] - c0, r0 = Ly.ccrbase[q], nr = Ly.ccrlen[q];
-      std::vector<int> ix(nc);
-      for (int k = 0; k < nc; k++) ix[k] = k;
-      std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) {
-        return std::make_pair(Ly.jj[Ly.cccol_p[c0 + x]], Ly.jj[Ly.cccol_h[c0 + x]]) <
-               std::make_pair(Ly.jj[Ly.cccol_p[c0 + y]], Ly.jj[Ly.cccol_h[c0 + y]]);
-      });
-      std::copy(ix.begin(), ix.end(), cperm.begin() + c0);
+      const int r0 = Ly.ccrbase[q], nr = Ly.ccrlen[q];
+      std::vector<int> ix(nr);
       auto rkey = [&](int g) {
         const int a = Ly.ccrow_a[r0 + g], b = Ly.ccrow_b[r0 + g];
         return a < 0 ? std::make_pair(1 << 20, 0) : std::make_pair(Ly.grp_of[a], Ly.grp_of[b]);
       };
-      ix.resize(nr);
       for (int g = 0; g < nr; g++) ix[g] = g;
       std::stable_sort(ix.begin(), ix.end(), [&](int x, int y) {
         const auto kx = rkey(x), ky = rkey(y);
@@ -1323,7 +1424,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       std::copy(ix.begin(), ix.end(), rperm.begin() + r0);
       for (int i = 0; i < nr; i++) rpos[r0 + ix[i]] = i;
     }
-    TUP(cperm, cperm); TUP(rperm, rperm);
+    TUP(rperm, rperm);
   }
   std::vector<int> pstart_h, part_h;  // the orbits the tensor's one-body part couples
   {
@@ -1437,6 +1538,75 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
     if (upload_table(c, crow, &D.crow) != 0 || upload_table(c, cpos, &D.cpos) != 0 || upload_table(c, prow, &D.prow) != 0 ||
         upload_table(c, cblk, &D.cblk) != 0)
       return IMSRG_ENOMEM;
+  }
+  // quadruples of the tensor Pandya matrices, by class: (u,v,x,y) = (a,h,b,p)
+  // of CCX, (h,a,p,b) of CCR, h a hole, p a particle, a and b any
+  {
+    const int ng = (int)Ly.grp_start.size();
+    std::vector<std::vector<int>> of[3];  // a group's orbits, holes, particles
+    for (auto &o : of) o.resize(ng);
+    for (int g = 0; g < ng; g++)
+      for (int k = 0; k < Ly.grp_cnt[g]; k++) {
+        const int x = Ly.grp_list[Ly.grp_start[g] + k];
+        of[0][g].push_back(x);
+        of[Ly.con[x] ? 1 : 2][g].push_back(x);
+      }
+    auto gj = [&](int g) { return Ly.jj[Ly.grp_list[Ly.grp_start[g]]]; };
+    auto gl = [&](int g) { return Ly.l[Ly.grp_list[Ly.grp_start[g]]] & 1; };
+    auto gt = [&](int g) { return Ly.tz[Ly.grp_list[Ly.grp_start[g]]] > 0 ? 1 : 0; };
+    std::vector<int> pcol((size_t)nsp * nsp * nJ, -1);
+    for (int q = 0; q < Ly.ncc; q++)
+      for (int k = Ly.cccbase[q]; k < Ly.cccbase[q + 1]; k++)
+        pcol[((size_t)Ly.cccol_p[k] * nsp + Ly.cccol_h[k]) * nJ + Ly.ccJ[q] / 2] = k - Ly.cccbase[q];
+    const int *dpcol = nullptr;
+    if (upload_table(c, pcol, &dpcol) != 0) return IMSRG_ENOMEM;
+    for (int mode = 0; mode < 2; mode++) {
+      TPan &P = S.pan[mode];
+      const auto &fu = of[mode ? 1 : 0], &fv = of[mode ? 0 : 1], &fx = of[mode ? 2 : 0], &fy = of[mode ? 0 : 2];
+      std::vector<unsigned> quads;
+      std::vector<PhChunkT> chunks;
+      for (int u = 0; u < ng; u++)
+        for (int v = 0; v < ng; v++) {
+          if (fu[u].empty() || fv[v].empty()) continue;
+          for (int x = 0; x < ng; x++)
+            for (int y = 0; y < ng; y++) {
+              if (fx[x].empty() || fy[y].empty()) continue;
+              if ((gl(u) ^ gl(v)) != (gl(x) ^ gl(y) ^ dp) || gt(u) + gt(v) != gt(x) + gt(y)) continue;
+              const int ju = gj(u), jv = gj(v), jx = gj(x), jy = gj(y);
+              bool any = false;  // some (J3 of (u,x), J4 of (v,y)) with a block
+              for (int J3 = std::abs(ju - jx); J3 <= ju + jx && !any; J3 += 2)
+                for (int J4 = std::max(J3, std::abs(jv - jy)); J4 <= std::min(jv + jy, J3 + rank); J4 += 2)
+                  any |= J3 + J4 >= rank;
+              if (!any) continue;
+              const size_t first = quads.size();
+              for (int a : fu[u])
+                for (int b : fv[v])
+                  for (int e : fx[x])
+                    for (int f : fy[y])
+                      quads.push_back((unsigned)a | (unsigned)b << 8 | (unsigned)e << 16 | (unsigned)f << 24);
+              const unsigned jc = (unsigned)ju | (unsigned)jv << 8 | (unsigned)jx << 16 | (unsigned)jy << 24;
+              const unsigned lt = (unsigned)(gl(u) | gl(v) << 1 | gl(x) << 2 | gl(y) << 3 | gt(u) << 4 | gt(v) << 5 |
+                                             gt(x) << 6 | gt(y) << 7);
+              for (size_t k = first; k < quads.size(); k += kPhQ)
+                chunks.push_back(PhChunkT{(unsigned)k, jc, lt, (int)std::min<size_t>(kPhQ, quads.size() - k)});
+            }
+        }
+      P.nchunk = (int)chunks.size();
+      P.npad = (P.nchunk + 511) & ~511;
+      if (chunks.empty()) continue;
+      // the matrices by (Tz, parity) of the J3 pair and (J3, J4)
+      std::vector<CcBlk> blk((size_t)4 * nJ * D.nd, CcBlk{-1, 0, 0});
+      for (int i = 0; i < S.ncc; i++) {
+        const int q3 = S.cq3[i], Tz = (q3 / (JM + 1)) & 1, Pr = q3 / (2 * (JM + 1));
+        blk[((size_t)(Tz + 2 * Pr) * nJ + (S.cJ3[i] >> 1)) * D.nd + ((S.cJ4[i] - S.cJ3[i]) >> 1)] =
+            mode ? CcBlk{S.roff[i], Ly.ccrlen[S.cq4[i]], 0} : CcBlk{S.xoff[i], Ly.ccnph[S.cq4[i]], 0};
+      }
+      if (upload_table(c, quads, &P.quads) != 0 || upload_table(c, chunks, &P.chunks) != 0 ||
+          upload_table(c, blk, &P.blk) != 0)
+        return IMSRG_ENOMEM;
+      P.rtab = mode ? dpcol : D.crow;
+      P.ctab = mode ? D.cpos : dpcol;
+    }
   }
   // lists and work items of k_t_lists, k_t_1body
   {
@@ -1656,6 +1826,11 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       dalloc(c, 2 * S.wsize, &S.wx) || dalloc(c, S.vsize, &S.w1) ||
       dalloc(c, S.vsize, &S.w2) || dalloc(c, kNormParts, &S.part))
     return IMSRG_ENOMEM;
+  // entries that the selection rules exclude are never written
+  launch_fill(c->stream, S.ccx, S.xsize, 0.0);
+  launch_fill(c->stream, S.ccr, S.rsize, 0.0);
+  S.pan[0].out = S.ccx;
+  S.pan[1].out = S.ccr;
   launch_fill(c->stream, S.w1, S.vsize, 0.0);
   launch_fill(c->stream, S.w2, S.vsize, 0.0);
   S.wy = S.wx + S.wsize;
@@ -1879,8 +2054,9 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
   if ((mask & IMSRG_TS222PH) && S.nelem > 0) {
     if (L.nccol > 0)
       hipLaunchKernelGGL(k_gcc_order, dim3(L.nccol), dim3(256), 0, s, L, D, (const double *)S.gcc, S.gccp);
-    if (D.nx > 0) hipLaunchKernelGGL(k_tpandya, dim3(nblk(D.nx)), dim3(256), 0, s, L, D, 0, RV, S.ccx, hR);
-    if (D.nr > 0) hipLaunchKernelGGL(k_tpandya, dim3(nblk(D.nr)), dim3(256), 0, s, L, D, 1, RV, S.ccr, hR);
+    if (S.pan[0].npad + S.pan[1].npad > 0)
+      hipLaunchKernelGGL(k_t_pandya, dim3(S.pan[0].npad + S.pan[1].npad), dim3(64), 0, s, L, D, S.pan[0], S.pan[1],
+                         RV, hR);
     if (S.n_cc_tiles[0] > 0)
       hipLaunchKernelGGL(k_tgemm, dim3(S.n_cc_tiles[0]), dim3(256), 0, s, S.cc_probs[0], S.cc_tiles[0],
                          S.n_cc_tiles[0], (const double *)S.gcc, (const double *)S.ccr, S.wx);
