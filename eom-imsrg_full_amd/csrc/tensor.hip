@@ -25,6 +25,7 @@
 // that pass the reference's |W| > 1e-6 test.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -42,7 +43,7 @@ struct DevTensor {
   long long nelem;              // tensor V elements
   const int *holes, *parts;
   const int *J1, *J2, *q1, *q2, *n1, *n2;
-  const long long *off, *tstart;  // per tensor block: V offset; first flat element
+  const long long *off;           // per tensor block: V offset
   const int *bidx;                // [((J1/2)*nJ + J2/2)*6 + (Tz+1)*2 + P1] -> block (J1 <= J2) or -1
   const int *ccol;                // [(scalar Pandya block * nsp + p) * nsp + h] -> column of (p,h)
   const double *x6, *s6;
@@ -93,18 +94,23 @@ struct alignas(16) PhChunkT {
 };
 
 // A product C (M x N, row-major, ldc) = sum of nseg segments alpha * A * B
-// with A(m,k) = X[asrc][a_off + m*a_rs + k*a_cs], B(k,n) = X[bsrc][b_off + k*b_rs + n*b_cs].
+// with A(m,k) = X[asrc][a_off + m*a_rs + k*a_cs], B(k,n) = X[bsrc][b_off + k*b_rs + n*b_cs];
+// with nseg2 a second one, into C2, from the segments after them.
 struct TSeg {
   long long a_off, b_off;
   int K, a_rs, a_cs, b_rs, b_cs, asrc, bsrc;
   double alpha;
 };
 struct TProb {
-  int M, N, ldc, nseg;
+  int M, N, ldc, nseg, nseg2, c;
   long long c_off;
-  TSeg seg[2];
+  TSeg seg[4];
 };
-
+struct TGemm {
+  const double *x[4];  // operands
+  double *c[2];        // C by the problem's c; C2 is c[1]
+  double *res;         // += C - C2 (null: not)
+};
 
 // {J1 J2 R; j4 j5 j6} with J1, J2 integer (doubled), j4 up to jmax + R, j5, j6 of the basis
 __device__ __forceinline__ double tx6(const DevTensor &T, int J1, int J2, int j4, int j5, int j6) {
@@ -148,48 +154,10 @@ __global__ void k_fill9j(DevTensor T, double *__restrict__ n9, long long n) {
   n9[e] = (J4 <= JM2 && J2 <= JM2) ? t9j(T, 2 * k1 + 1, 2 * k2 + 1, J3, 2 * k3 + 1, 2 * k4 + 1, J4, J1, J2) : 0.0;
 }
 
-// tensor_elem (basic_IMSRG.f90:1504-1641): position in V of T^{J1x J2x}_{ax bx, cx dx}
-// and the factor applied to the stored value (switch phase, exchange phase, sqrt 2)
-__device__ inline long long t_pos(const DevLayout &L, const DevTensor &T, int herm, int ax, int bx, int cx, int dx,
-                                  int J1x, int J2x, double &pre) {
-  pre = 0.0;
-  int a = ax, b = bx, c = cx, d = dx, J1 = J1x, J2 = J2x;
-  bool sw = false;
-  if (J1x > J2x) {
-    a = cx; b = dx; c = ax; d = bx; J1 = J2x; J2 = J1x;
-    sw = true;
-  }
-  if (!dtri(J1, J2, T.rank)) return -1;
-  const int ja = L.jj[a], jb = L.jj[b], jc = L.jj[c], jd = L.jj[d];
-  if (!(dtri(ja, jb, J1) && dtri(jc, jd, J2))) return -1;
-  const int P = (L.l[a] + L.l[b]) & 1;
-  if (((L.l[c] + L.l[d]) & 1) != (P ^ ((T.dpar >> 1) & 1))) return -1;
-  const int T2 = L.tz[a] + L.tz[b];
-  if (L.tz[c] + L.tz[d] != T2) return -1;
-  const int q = T.bidx[((J1 >> 1) * T.nJ + (J2 >> 1)) * 6 + (T2 / 2 + 1) * 2 + P];
-  if (q < 0) return -1;
-  double f = sw ? (double)(sgnp((J2 - J1) >> 1) * herm) : 1.0;
-  int r, s;
-  if (a > b) {
-    r = dpos(L, J1, b, a);
-    f *= sgnp(1 + ((ja + jb - J1) >> 1));
-  } else {
-    if (a == b) f *= M_SQRT2;
-    r = dpos(L, J1, a, b);
-  }
-  if (c > d) {
-    s = dpos(L, J2, d, c);
-    f *= sgnp(1 + ((jc + jd - J2) >> 1));
-  } else {
-    if (c == d) f *= M_SQRT2;
-    s = dpos(L, J2, c, d);
-  }
-  if ((r | s) < 0) return -1;
-  pre = f;
-  return T.off[q] + (long long)r * T.n2[q] + s;
-}
-// t_pos with every table read made (indices in range whatever the tests
-// say) and no early return: an element the tensor does not hold gets
+// tensor_elem (basic_IMSRG.f90:1504-1641): position in V of T^{J1x J2x}_{ax bx,
+// cx dx} and the factor applied to the stored value (switch phase, exchange
+// phase, sqrt 2), with every table read made (indices in range whatever the
+// tests say) and no early return: an element the tensor does not hold gets
 // position 0 and factor 0.  For batches whose loads should be in flight
 // together.  chan: the caller's test that the pairs' parities (with the
 // tensor's) and Tz match; j*x the orbits' 2j.
@@ -212,129 +180,96 @@ __device__ inline long long t_pos_all(const DevLayout &L, const DevTensor &T, in
   pre = ok ? f : 0.0;
   return ok ? o + (long long)r * n2 + s : 0;
 }
-__device__ __forceinline__ double t_elem(const DevLayout &L, const DevTensor &T, const double *V, int herm, int a,
-                                         int b, int c, int d, int J1, int J2) {
-  double f;
-  const long long p = t_pos(L, T, herm, a, b, c, d, J1, J2, f);
-  return p < 0 ? 0.0 : V[p] * f;
-}
-
-// flat element e of a prefix table (n + 1 entries) -> item
-__device__ __forceinline__ int find_item(const long long *start, int n, long long e) {
-  int lo = 0, hi = n;  // start[lo] <= e < start[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (start[mid] <= e) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
 // ---------------------------------------------------------------- one-body terms
-// TS_commutator_111 (TS_commutators.f90:10-55): overwrites fhh, fph, fpp of RES.
-// LF: the scalar operator's full one-body matrix, RF the tensor's.
-__global__ void k_t111(DevLayout L, DevTensor T, const double *__restrict__ LF, const double *__restrict__ RF,
-                       double *__restrict__ F, int hL, int hR, int hres) {
-  const int A = T.nhole, P = T.npart, n = L.nsp;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)A * A + (long long)P * A + (long long)P * P) return;
-  auto lf = [&](int a, int b) { return LF[(size_t)a * n + b]; };
-  auto rf = [&](int a, int b) { return RF[(size_t)a * n + b]; };
-  if (t < (long long)A * A) {
-    const int i = T.holes[t / A], j = T.holes[t % A];
-    // th1 = Lhh Rhh, th2 = Lph^T Rph at (i,j) and (j,i)
-    double th1 = 0, th2 = 0, th1t = 0, th2t = 0;
-    for (int k = 0; k < A; k++) {
-      const int hk = T.holes[k];
-      th1 += lf(i, hk) * rf(hk, j);
-      th1t += lf(j, hk) * rf(hk, i);
-    }
-    for (int k = 0; k < P; k++) {
-      const int p = T.parts[k];
-      th2 += lf(p, i) * rf(p, j);
-      th2t += lf(p, j) * rf(p, i);
-    }
-    const double ph = sgnp((L.jj[i] - L.jj[j]) >> 1);
-    F[(size_t)i * n + j] = th1 + th2 * hL - (th1t * hL + th2t) * hR * ph;
-  } else if (t < (long long)A * A + (long long)P * A) {
-    const long long u = t - (long long)A * A;
-    const int p = T.parts[u / A], h = T.holes[u % A];
-    double sm = 0;
-    for (int k = 0; k < A; k++) {
-      const int hk = T.holes[k];
-      sm += lf(p, hk) * rf(hk, h);
-    }
-    for (int k = 0; k < P; k++) {
-      const int q = T.parts[k];
-      sm += lf(p, q) * rf(q, h);
-    }
-    double sm2 = 0;
-    for (int k = 0; k < A; k++) {
-      const int hk = T.holes[k];
-      sm2 += rf(p, hk) * lf(hk, h);
-    }
-    for (int k = 0; k < P; k++) {
-      const int q = T.parts[k];
-      sm2 += rf(p, q) * lf(q, h);
-    }
-    const double v = sm - sm2;
-    F[(size_t)p * n + h] = v;
-    F[(size_t)h * n + p] = v * hres * sgnp((L.jj[h] - L.jj[p]) >> 1);
-  } else {
-    const long long u = t - (long long)A * A - (long long)P * A;
-    const int p = T.parts[u / P], q = T.parts[u % P];
-    // tp1 = Lph Rph^T, tp2 = Lpp Rpp at (p,q) and (q,p)
-    double tp1 = 0, tp1t = 0, tp2 = 0, tp2t = 0;
-    for (int k = 0; k < A; k++) {
-      const int h = T.holes[k];
-      tp1 += lf(p, h) * rf(q, h);
-      tp1t += lf(q, h) * rf(p, h);
-    }
-    for (int k = 0; k < P; k++) {
-      const int r = T.parts[k];
-      tp2 += lf(p, r) * rf(r, q);
-      tp2t += lf(q, r) * rf(r, p);
-    }
-    const double ph = sgnp((L.jj[p] - L.jj[q]) >> 1);
-    F[(size_t)p * n + q] = tp1 * hR * ph + tp2 - (tp1t + tp2t * hR * ph) * hL;
-  }
-}
-
-// TS_commutator_121 (kind 0, :58-303), _211 (kind 1, :307-552) and _221
-// (kind 2, :809-1067): per upper output (p,q) allowed by the tensor's
-// selection rules, F(p,q) += sum, then the lower entry becomes
-// herm * (-1)^((jp-jq)/2) F(p,q) (diagonal included), exactly as each
-// reference routine leaves it; (particle, hole) outputs also refresh the
-// derived (hole, particle) entry.  One wavefront per output: the lanes split
-// the intermediate orbits and reduce.
-__global__ __launch_bounds__(64) void k_t_onebody(DevLayout L, DevTensor T, int kind, const double *__restrict__ LF,
-                                                  const double *__restrict__ RF, const double *__restrict__ RV,
-                                                  const double *__restrict__ gcc, const double *__restrict__ W1,
-                                                  const double *__restrict__ W2, double *__restrict__ F, int hL,
-                                                  int hR, int hres) {
-  const int t = blockIdx.x, lane = threadIdx.x;
-  if (t >= L.nob) return;
-  const int p = L.ob_p[t], q = L.ob_q[t], n = L.nsp, R = T.rank;
+// TS_commutator_111 (TS_commutators.f90:10-55; overwrites the one-body part), _121
+// (:58-303), _211 (:307-552) and _221 (:809-1067; these add to it).  LF: the
+// scalar operator's one-body matrix, RF the tensor's.  One workgroup per
+// upper output (p,q): (hole, hole), (particle, particle), (particle, hole).
+// 111 is the matrix commutator, each class in the stored entries the reference
+// reads; the other three, for outputs that the tensor's selection rules allow,
+// add to the upper entry, and the lower one becomes herm (-1)^((jp-jq)/2) times
+// it (diagonal included, after each term), as each reference routine leaves it;
+// (hole, particle) entries are derived.  The terms, flattened over the intermediate
+// orbits and the first angular momentum with the 2 rank + 1 second ones the
+// tensor couples to it, are spread over the threads.
+//
+// What bounds it: the latency of a term's dependent lookups.  A wavefront per
+// output with a lane per intermediate orbit, a launch per term, took 0.07 +
+// 0.40 ms at 90 orbits, rank 4, 20 + 89 us at 30 orbits, rank 2; this kernel
+// 0.12 ms and 11 us.
+constexpr int kTfThreads = 512;
+enum { kTf111 = 1, kTf121 = 2, kTf221 = 4, kTf211 = 8 };
+__global__ __launch_bounds__(kTfThreads) void k_t_f(DevLayout L, DevTensor T, int terms, const double *__restrict__ LF,
+                                                    const double *__restrict__ RF, const double *__restrict__ RV,
+                                                    const double *__restrict__ gcc, const double *__restrict__ W1,
+                                                    const double *__restrict__ W2, double *__restrict__ F, int hL,
+                                                    int hR, int hres) {
+  __shared__ double sh[5][kTfThreads / 64];
+  const int tid = threadIdx.x, p = L.ob_p[blockIdx.x], q = L.ob_q[blockIdx.x], n = L.nsp, R = T.rank;
   const int jp = L.jj[p], jq = L.jj[q], lp = L.l[p], lq = L.l[q];
-  if ((lq & 1) != ((lp + (T.dpar >> 1)) & 1)) return;
-  if (L.tz[q] != L.tz[p]) return;
-  if (!dtri(jq, jp, R)) return;
-  double sm = 0.0;
-  if (kind == 0) {
-    for (int u = lane; u < L.nphp; u += 64) {
-      const int a = L.php_a[u], i = L.php_i[u];
-      const int ja = L.jj[a], ji = L.jj[i];
-      double smx = 0.0, smy = 0.0;
-      for (int J2 = abs(ji - jq); J2 <= ji + jq; J2 += 2)
-        for (int J1 = abs(ja - jp); J1 <= ja + jp; J1 += 2)
-          smx += t_elem(L, T, RV, hR, a, p, i, q, J1, J2) * sqrt((J1 + 1.0) * (J2 + 1.0)) * sgnp(J1 >> 1) *
-                 tx6(T, J1, J2, jq, jp, ji);
-      for (int J1 = abs(ji - jp); J1 <= ji + jp; J1 += 2)
-        for (int J2 = abs(ja - jq); J2 <= ja + jq; J2 += 2)
-          smy += t_elem(L, T, RV, hR, i, p, a, q, J1, J2) * sqrt((J1 + 1.0) * (J2 + 1.0)) * sgnp(J1 >> 1) *
-                 tx6(T, J1, J2, jq, jp, ji);
-      sm += LF[(size_t)a * n + i] * (hL * smx - smy) * sgnp((R + jq + ji) >> 1);
+  const bool allowed = (lq & 1) == ((lp + (T.dpar >> 1)) & 1) && L.tz[q] == L.tz[p] && dtri(jq, jp, R);
+  const int cp = L.con[p], cq = L.con[q];
+  if (!(terms & kTf111) && !allowed) return;
+  // 111's upper entry, and the lower one where 111 alone sets it; 121, 221, 211
+  double up = 0.0, dn = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  if (terms & kTf111) {
+    const double ph = sgnp((jp - jq) >> 1);
+    auto lf = [&](int a, int b) { return LF[(size_t)a * n + b]; };
+    auto rf = [&](int a, int b) { return RF[(size_t)a * n + b]; };
+    for (int k = tid; k < n; k += kTfThreads) {
+      const bool hole = L.con[k] != 0;
+      if (cp != cq) {
+        up += lf(p, k) * rf(k, q) - rf(p, k) * lf(k, q);
+      } else if (cp) {
+        // hh: Lhh Rhh + hL Lph^T Rph - (hL hR ph) (Lhh Rhh)^T - (hR ph) (Lph^T Rph)^T
+        const double x = hole ? lf(p, k) * rf(k, q) : lf(k, p) * rf(k, q) * hL;
+        const double y = hole ? lf(q, k) * rf(k, p) : lf(k, q) * rf(k, p) * hL;
+        const double f = hL * hR * ph;
+        up += x - y * f;
+        dn += y - x * f;
+      } else {
+        // pp: (hR ph) Lph Rph^T + Lpp Rpp - hL (Lph Rph^T)^T - (hL hR ph) (Lpp Rpp)^T
+        const double f = hR * ph;
+        const double x = hole ? lf(p, k) * rf(q, k) * f : lf(p, k) * rf(k, q);
+        const double y = hole ? lf(q, k) * rf(p, k) * f : lf(q, k) * rf(k, p);
+        up += x - y * (hL * f);
+        dn += y - x * (hL * f);
+      }
     }
-  } else if (kind == 1) {
+  }
+  const int nd2 = 2 * T.nd - 1;
+  if (allowed && (terms & kTf121)) {
+    const int K = jp + 1;  // J1 values of (a,p), at most
+    for (int t = tid; t < L.nphp * K * nd2; t += kTfThreads) {
+      const int d = t % nd2, v = t / nd2, k = v % K, u = v / K;
+      const int a = L.php_a[u], i = L.php_i[u], ji = L.jj[i];  // ja = ji
+      const int J1 = abs(ji - jp) + 2 * k, J2 = J1 + 2 * (d - (T.nd - 1));
+      if (J1 > ji + jp || J2 < abs(ji - jq) || J2 > ji + jq || J1 + J2 < R) continue;
+      double f1, f2;
+      const long long p1 = t_pos_all(L, T, hR, a, p, i, q, ji, jp, ji, jq, J1, J2, true, f1);
+      const long long p2 = t_pos_all(L, T, hR, i, p, a, q, ji, jp, ji, jq, J1, J2, true, f2);
+      s1 += LF[(size_t)a * n + i] * (hL * f1 * RV[p1] - f2 * RV[p2]) * sqrt((J1 + 1.0) * (J2 + 1.0)) *
+            sgnp((J1 >> 1) + ((R + jq + ji) >> 1)) * tx6(T, J1, J2, jq, jp, ji);
+    }
+  }
+  if (allowed && (terms & kTf221)) {
+    // over every orbit c, holes with W1 and particles with W2: J2 < J1 reads
+    // W(cq, cp; J2 J1) (the lower half, by herm), J2 >= J1 W(cp, cq; J1 J2).
+    // The pairs' channel matches the output's, which passed the tensor's tests.
+    const int K = jp + 1;
+    for (int t = tid; t < n * K * nd2; t += kTfThreads) {
+      const int d = t % nd2, v = t / nd2, k = v % K, c = v / K, jc = L.jj[c];
+      const int J1 = abs(jc - jp) + 2 * k, J2 = J1 + 2 * (d - (T.nd - 1));
+      if (J1 > jc + jp || J2 < abs(jc - jq) || J2 > jc + jq || J1 + J2 < R) continue;
+      const bool lo = J2 < J1;
+      double f;
+      const long long pos = lo ? t_pos_all(L, T, hR, c, q, c, p, jc, jq, jc, jp, J2, J1, true, f)
+                               : t_pos_all(L, T, hR, c, p, c, q, jc, jp, jc, jq, J1, J2, true, f);
+      const double co = sqrt((J1 + 1.0) * (J2 + 1.0)) * tx6(T, J1, J2, jq, jp, jc) * sgnp((jc + jq + R) >> 1);
+      s2 += (lo ? -co * sgnp(J2 >> 1) * (hL * hR) : co * sgnp(J1 >> 1)) * f * (L.con[c] ? W1 : W2)[pos];
+    }
+  }
+  if (allowed && (terms & kTf211)) {
     const int PAR = (lp + lq) & 1;
     const int qx = (R >> 1) + 2 * PAR * (L.jtot_max + 1);  // Pandya block (J = R, Tz = 0, PAR)
     const int rpq = L.ccrow[((size_t)qx * n + p) * n + q], rqp = L.ccrow[((size_t)qx * n + q) * n + p];
@@ -342,63 +277,40 @@ __global__ __launch_bounds__(64) void k_t_onebody(DevLayout L, DevTensor T, int 
     const int rlen = L.ccrlen[qx];
     const double inv = 1.0 / sqrt(R + 1.0);
     const double c1 = sgnp((jp - jq + R) >> 1), c2 = (double)(hR * hL * sgnp(R >> 1));
-    for (int u = lane; u < T.npart * T.nhole; u += 64) {
-      const int a = T.parts[u / T.nhole], i = T.holes[u % T.nhole];
-      const int ja = L.jj[a], la = L.l[a], ji = L.jj[i], li = L.l[i];
-      if ((li & 1) != ((la + (T.dpar >> 1)) & 1)) continue;
-      if (L.tz[i] != L.tz[a]) continue;
-      if (!dtri(ja, ji, R)) continue;
-      if (((la + li) & 1) != PAR) continue;
-      const int col = T.ccol[((size_t)qx * n + a) * n + i];
-      if (col < 0 || rpq < 0 || rqp < 0) continue;  // unreachable for allowed outputs
-      sm += RF[(size_t)a * n + i] *
-            (c1 * gcc[base + (long long)col * rlen + rpq] - c2 * gcc[base + (long long)col * rlen + rqp]) * inv;
-    }
-  } else {
-    const int pm = hL * hR, i = p, j = q, ji = jp, jj = jq;
-    for (int u = lane; u < n; u += 64) {  // c over holes with W1, over particles with W2
-      const int c = u < T.nhole ? T.holes[u] : T.parts[u - T.nhole], jc = L.jj[c];
-      const double *W = u < T.nhole ? W1 : W2;
-      double s1 = 0.0;
-      // J2 over its whole range, four at a time with every load off any
-      // branch: J2 < J1 reads W(cj, ci; J2 J1) (the lower half, by herm), J2 >= J1
-      // W(ci, cj; J1 J2).  The pairs' channel matches the output's, which
-      // passed the tensor's parity and Tz tests.
-      const int J2lo = abs(jc - jj), n2 = (jc + jj - J2lo) / 2 + 1;
-      for (int J1 = abs(jc - ji); J1 <= jc + ji; J1 += 2) {
-        for (int k0 = 0; k0 < n2; k0 += 4) {
-          long long pos[4];
-          double w[4];
-#pragma unroll
-          for (int v = 0; v < 4; v++) {
-            const int J2 = J2lo + 2 * min(k0 + v, n2 - 1);
-            const bool lo = J2 < J1;
-            double f;
-            pos[v] = lo ? t_pos_all(L, T, hR, c, j, c, i, jc, jj, jc, ji, J2, J1, true, f)
-                        : t_pos_all(L, T, hR, c, i, c, j, jc, ji, jc, jj, J1, J2, true, f);
-            const double co = sqrt((J1 + 1.0) * (J2 + 1.0)) * tx6(T, J1, J2, jj, ji, jc);
-            w[v] = k0 + v < n2 ? (lo ? -co * sgnp(J2 >> 1) * pm : co * sgnp(J1 >> 1)) * f : 0.0;
-          }
-          double g[4];
-#pragma unroll
-          for (int v = 0; v < 4; v++) g[v] = W[pos[v]];
-#pragma unroll
-          for (int v = 0; v < 4; v++) s1 += w[v] * g[v];
-        }
+    if (rpq >= 0 && rqp >= 0)
+      for (int u = tid; u < T.npart * T.nhole; u += kTfThreads) {
+        const int a = T.parts[u / T.nhole], i = T.holes[u % T.nhole];
+        if (((L.l[a] + L.l[i]) & 1) != ((T.dpar >> 1) & 1) || L.tz[i] != L.tz[a] || !dtri(L.jj[a], L.jj[i], R)) continue;
+        const int col = T.ccol[((size_t)qx * n + a) * n + i];
+        if (col < 0) continue;
+        s3 += RF[(size_t)a * n + i] *
+              (c1 * gcc[base + (long long)col * rlen + rpq] - c2 * gcc[base + (long long)col * rlen + rqp]) * inv;
       }
-      sm += s1 * sgnp((jc + jj) >> 1);
-    }
-    sm *= sgnp(R >> 1);
   }
-  sm = wave_sum(sm);
-  if (lane != 0) return;
+  const double part[5] = {wave_sum(up), wave_sum(dn), wave_sum(s1), wave_sum(s2), wave_sum(s3)};
+  if ((tid & 63) == 0)
+    for (int v = 0; v < 5; v++) sh[v][tid >> 6] = part[v];
+  __syncthreads();
+  if (tid) return;
+  double sum[5];
+  for (int v = 0; v < 5; v++) {
+    sum[v] = 0.0;
+    for (int k = 0; k < kTfThreads / 64; k++) sum[v] += sh[v][k];
+  }
   const size_t pq = (size_t)p * n + q, qp = (size_t)q * n + p;
-  const double v = F[pq] + sm;
+  double v = (terms & kTf111) ? sum[0] : F[pq];
+  const bool others = allowed && (terms & ~kTf111);
+  if (others)
+    for (int k = 0; k < 3; k++)
+      if (terms & (kTf121 << k)) {
+        v += sum[2 + k];
+        if (p == q) v *= hres;
+      }
   F[pq] = v;
-  if (L.con[p] == L.con[q])
-    F[qp] = v * hres * sgnp((jp - jq) >> 1);
-  else
+  if (cp != cq)
     F[qp] = v * hres * sgnp((jq - jp) >> 1);  // (hole, particle): f_tensor_elem's phase
+  else if (p != q)
+    F[qp] = others ? v * hres * sgnp((jp - jq) >> 1) : sum[1];
 }
 
 // ---------------------------------------------------------------- two-body gathers
@@ -1159,10 +1071,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 }
 
 // ---------------------------------------------------------------- products
-// 64 x 64 tiles, 4 waves of 32 x 32 on v_mfma_f64_16x16x4; tiles (problem, tile row, tile column)
+// 64 x 64 tiles, 4 waves of 32 x 32 on v_mfma_f64_16x16x4; tiles (problem, tile row, tile column).
+// Matrix-core bound in large bases (59 TF/s over a commutator's products at 90
+// orbits, rank 4).  The pp and hh ladders of a tile in one workgroup: the hh
+// product's short K follows the pp product's without a launch, and RES takes
+// their difference here, not in two more passes over three operators.
 __global__ __launch_bounds__(256) void k_tgemm(const TProb *__restrict__ probs, const int4 *__restrict__ tiles,
-                                               int ntiles, const double *__restrict__ X0,
-                                               const double *__restrict__ X1, double *__restrict__ C) {
+                                               int ntiles, TGemm X) {
   const int t = blockIdx.x;
   if (t >= ntiles) return;
   const int4 tl = tiles[t];
@@ -1177,10 +1092,25 @@ __global__ __launch_bounds__(256) void k_tgemm(const TProb *__restrict__ probs, 
   // step's elements are loaded into registers (clamped to the operand, so
   // every load is unconditional and the eight stay in flight together) while
   // the current step runs on the matrix cores
-  for (int sgi = 0; sgi < p.nseg; sgi++) {
+  // v_mfma_f64_16x16x4: row lane/16 + 4v, column lane%16; W2 - W1 needs W1 again, which
+  // this thread wrote
+  auto store = [&](double *C, bool diff) {
+    for (int ti = 0; ti < 2; ti++)
+      for (int tj = 0; tj < 2; tj++)
+        for (int v = 0; v < 4; v++) {
+          const int row = m0 + wm * 32 + ti * 16 + (lane >> 4) + 4 * v, col = n0 + wn * 32 + tj * 16 + (lane & 15);
+          if (row >= p.M || col >= p.N) continue;
+          const long long o = p.c_off + (long long)row * p.ldc + col;
+          C[o] = acc[ti][tj][v];
+          if (diff) X.res[o] += X.c[p.c][o] - acc[ti][tj][v];
+          acc[ti][tj][v] = 0.0;
+        }
+  };
+  for (int sgi = 0; sgi < p.nseg + p.nseg2; sgi++) {
+    if (sgi == p.nseg) store(X.c[p.c], false);
     const TSeg sg = p.seg[sgi];
     if (sg.K <= 0) continue;
-    const double *Ap = (sg.asrc ? X1 : X0) + sg.a_off, *Bp = (sg.bsrc ? X1 : X0) + sg.b_off;
+    const double *Ap = X.x[sg.asrc] + sg.a_off, *Bp = X.x[sg.bsrc] + sg.b_off;
     const bool arow = sg.a_cs == 1, brow = sg.b_cs == 1;
     int am[4], ak[4], bn[4], bk[4];  // element (row/column, k) of each staged value in the tile
 #pragma unroll
@@ -1223,41 +1153,59 @@ __global__ __launch_bounds__(256) void k_tgemm(const TProb *__restrict__ probs, 
       __syncthreads();
     }
   }
-  double *Cp = C + p.c_off;
-  const int g = lane >> 4;
-  for (int ti = 0; ti < 2; ti++)
-    for (int tj = 0; tj < 2; tj++)
-      for (int v = 0; v < 4; v++) {  // v_mfma_f64_16x16x4: row lane/16 + 4v, column lane%16
-        const int row = m0 + wm * 32 + ti * 16 + g + 4 * v, col = n0 + wn * 32 + tj * 16 + (lane & 15);
-        if (row < p.M && col < p.N) Cp[(long long)row * p.ldc + col] = acc[ti][tj][v];
-      }
+  store(p.nseg2 ? X.c[1] : X.c[p.c], p.nseg2 && X.res);
 }
 
-// mat_frob_norm of a tensor (basic_IMSRG.f90:3921-3952): fhh^2 + 2 fph^2 + fpp^2
-// + sum over blocks (1 if J1 = J2, else 2) x block^2; one partial per workgroup
-__global__ void k_tnorm(DevLayout L, DevTensor T, const double *__restrict__ op, double *__restrict__ part) {
+// One term of BCH_TENSOR's series and its norm: HS += coef X (HS null: the norm
+// only), and mat_frob_norm of X (basic_IMSRG.f90:3921-3952): fhh^2 + 2 fph^2 +
+// fpp^2 + sum over blocks (1 if J1 = J2, else 2) x block^2.  A workgroup per
+// run of one block's elements; k_t_norm adds the runs' sums and writes the result
+// to host memory, where the host waits for it.
+struct TRun {
+  long long off;  // into the operator
+  int n, w;       // elements, weight; w 0: the one-body matrix
+};
+struct TNorm {
+  double v;
+  int seq;
+};
+__global__ __launch_bounds__(256) void k_t_step(DevLayout L, const TRun *__restrict__ runs,
+                                                const double *__restrict__ X, double *__restrict__ HS, double coef,
+                                                double *__restrict__ part) {
   __shared__ double sh[256];
-  const int n = L.nsp;
-  const long long nf = (long long)n * n, ntot = nf + T.nelem;
+  const TRun r = runs[blockIdx.x];
   double s = 0.0;
-  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < ntot; e += (long long)gridDim.x * blockDim.x) {
-    if (e < nf) {
-      const int a = (int)(e / n), b = (int)(e % n);
-      const double v = op[T.f_off + e];
+  if (r.w) {
+#pragma unroll 4
+    for (int e = threadIdx.x; e < r.n; e += 256) {
+      const double v = X[r.off + e];
+      if (HS) HS[r.off + e] += coef * v;
+      s += v * v;
+    }
+    s *= r.w;
+  } else {
+    for (int e = threadIdx.x; e < r.n; e += 256) {
+      const double v = X[r.off + e];
+      const int a = e / L.nsp, b = e % L.nsp;
+      if (HS) HS[r.off + e] += coef * v;
       if (L.con[a] == L.con[b]) s += v * v;
       else if (L.con[a] == 0) s += 2.0 * v * v;  // (particle, hole); (hole, particle) is derived
-    } else {
-      const int q = find_item(T.tstart, T.nblk, e - nf);
-      const long long vp = T.off[q] + e - nf - T.tstart[q];
-      const double v = op[T.v_off + vp];
-      s += (T.J1[q] == T.J2[q] ? 1.0 : 2.0) * v * v;
     }
   }
-  const double r = block_sum256(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = r;
+  s = block_sum256(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
-
-constexpr int kNormParts = 512;
+__global__ __launch_bounds__(256) void k_t_norm(const double *__restrict__ part, int n, TNorm *out, int seq) {
+  __shared__ double sh[256];
+  double s = 0.0;
+  for (int k = threadIdx.x; k < n; k += 256) s += part[k];
+  s = block_sum256(s, sh);
+  if (threadIdx.x == 0) {
+    out->v = s;
+    __threadfence_system();
+    __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
 
 }  // namespace
 
@@ -1265,7 +1213,7 @@ constexpr int kNormParts = 512;
 struct TensorSpace {
   int rank = 0, dpar = 0, nblk = 0, ncc = 0, hx = 0;
   std::vector<int> J1, J2, q1, q2, n1, n2, bidx;
-  std::vector<long long> off, tstart;
+  std::vector<long long> off;
   long long vsize = 0, v_off = 0, op_size = 0, neq = 0, nelem = 0;
   std::vector<int> cJ3, cJ4, cq3, cq4, ccol;
   std::vector<long long> xoff, roff, woff;
@@ -1278,12 +1226,17 @@ struct TensorSpace {
   TLists lists{};
   TPan pan[2]{};  // CCX, CCR
   double *gcc = nullptr, *gccp = nullptr, *ccx = nullptr, *ccr = nullptr, *wx = nullptr, *wy = nullptr;
-  double *w1 = nullptr, *w2 = nullptr, *part = nullptr, *hpart = nullptr;
-  const TProb *pp_probs[2] = {nullptr, nullptr}, *cc_probs[2] = {nullptr, nullptr};
-  const int4 *pp_tiles = nullptr, *cc_tiles[2] = {nullptr, nullptr};
-  int n_pp_tiles = 0, n_cc_tiles[2] = {0, 0};
+  double *w1 = nullptr, *w2 = nullptr, *part = nullptr;
+  const TRun *runs = nullptr;
+  int nrun = 0, seq = 0;
+  TNorm *norm = nullptr;   // host memory
+  double *bch = nullptr;   // BCH_TENSOR's two work operators, kept up to kBchKeep bytes
+  const TProb *pp_probs = nullptr, *cc_probs = nullptr;
+  const int4 *pp_tiles = nullptr, *cc_tiles = nullptr;
+  int n_pp_tiles = 0, n_cc_tiles = 0;
   ~TensorSpace() {
-    if (hpart) (void)hipHostFree(hpart);
+    if (norm) (void)hipHostFree(norm);
+    if (bch) (void)hipFree(bch);
   }
 };
 
@@ -1326,13 +1279,11 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
           S.n1.push_back(m1);
           S.n2.push_back(m2);
           S.off.push_back(off);
-          S.tstart.push_back(el);
           off = align32(off + (long long)m1 * m2);
           el += (long long)m1 * m2;
           if (live) S.bidx[((size_t)(J1 >> 1) * nJ + (J2 >> 1)) * 6 + (Tz + 1) * 2 + P1] = q;
         }
   S.nblk = (int)S.J1.size();
-  S.tstart.push_back(el);
   S.nelem = el;
   S.vsize = off;
   S.v_off = align32(Ly.f_off + (long long)nsp * nsp);
@@ -1401,7 +1352,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   if (upload_table(c, vec, &D.field) != 0) return IMSRG_ENOMEM
   TUP(Ly.holes, holes); TUP(Ly.parts, parts);
   TUP(S.J1, J1); TUP(S.J2, J2); TUP(S.q1, q1); TUP(S.q2, q2); TUP(S.n1, n1); TUP(S.n2, n2);
-  TUP(S.off, off); TUP(S.tstart, tstart); TUP(S.bidx, bidx);
+  TUP(S.off, off); TUP(S.bidx, bidx);
   TUP(S.ccol, ccol); TUP(S.x6, x6); TUP(S.s6, s6);
   std::vector<int> rperm, rpos;  // Pandya rows in group order, and each row's place in it
   {
@@ -1765,9 +1716,9 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
         HIPCHK(hipFuncSetAttribute((const void *)k_t_1body, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     }
   }
-  // products: the pp and hh ladders per tensor block (W1, W2)
+  // products: the pp and hh ladders per tensor block (W1, W2); operand 0: G's V, 1: T's V
   {
-    std::vector<TProb> pr[2];
+    std::vector<TProb> pr;
     std::vector<int4> tiles;
     for (int q = 0; q < S.nblk; q++) {
       const int m1 = S.n1[q], m2 = S.n2[q];
@@ -1775,56 +1726,50 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       const int b1 = S.q1[q], b2 = S.q2[q];
       const int np1 = Ly.bnp[b1], nb1 = Ly.bnb[b1], nh1 = Ly.bnh[b1];
       const int np2 = Ly.bnp[b2], nb2 = Ly.bnb[b2], nh2 = Ly.bnh[b2];
+      TProb p{};
+      p.M = m1; p.N = m2; p.ldc = m2; p.nseg = p.nseg2 = 2; p.c_off = S.off[q];
       for (int w = 0; w < 2; w++) {  // w 0: pp intermediate, 1: hh
         const int k1 = w ? np1 + nb1 : 0, K1 = w ? nh1 : np1, k2 = w ? np2 + nb2 : 0, K2 = w ? nh2 : np2;
-        TProb p{};
-        p.M = m1; p.N = m2; p.ldc = m2; p.nseg = 2; p.c_off = S.off[q];
-        // G(J1)[:, k] T[k, :]  (operand 0: G's V, 1: T's V)
-        p.seg[0] = TSeg{Ly.boff[b1] + k1, S.off[q] + (long long)k1 * m2, K1, m1, 1, m2, 1, 0, 1, 1.0};
-        // - T[:, k] G(J2)[k, :]
-        p.seg[1] = TSeg{S.off[q] + k2, Ly.boff[b2] + (long long)k2 * m2, K2, m2, 1, m2, 1, 1, 0, -1.0};
-        pr[w].push_back(p);
+        // G(J1)[:, k] T[k, :] - T[:, k] G(J2)[k, :]
+        p.seg[2 * w] = TSeg{Ly.boff[b1] + k1, S.off[q] + (long long)k1 * m2, K1, m1, 1, m2, 1, 0, 1, 1.0};
+        p.seg[2 * w + 1] = TSeg{S.off[q] + k2, Ly.boff[b2] + (long long)k2 * m2, K2, m2, 1, m2, 1, 1, 0, -1.0};
       }
-      add_tiles((int)pr[0].size() - 1, m1, m2, tiles);
+      pr.push_back(p);
+      add_tiles((int)pr.size() - 1, m1, m2, tiles);
     }
-    for (int w = 0; w < 2; w++)
-      if (upload_table(c, pr[w], &S.pp_probs[w]) != 0) return IMSRG_ENOMEM;
-    if (upload_table(c, tiles, &S.pp_tiles) != 0) return IMSRG_ENOMEM;
+    if (upload_table(c, pr, &S.pp_probs) != 0 || upload_table(c, tiles, &S.pp_tiles) != 0) return IMSRG_ENOMEM;
     S.n_pp_tiles = (int)tiles.size();
   }
   // the two Pandya products per cross-coupled block (TS_commutator_222_ph, TS_commutators.f90:1496-1521):
   // alpha carries 1/sqrt(J3+1) and 1/sqrt(J4+1); the herm of G that the reference also folds into Wx
   // is applied where k_t222ph reads Wx, so these tables serve every G
   {
-    std::vector<TProb> pr[2];
-    std::vector<int4> tiles[2];
+    std::vector<TProb> pr;
+    std::vector<int4> tiles;
     for (int x = 0; x < S.ncc; x++) {
       const int q3 = S.cq3[x], q4 = S.cq4[x];
       const int r3 = Ly.ccrlen[q3], r4 = Ly.ccrlen[q4], nb3 = Ly.ccnph[q3], nb4 = Ly.ccnph[q4];
       if (r3 == 0 || r4 == 0) continue;
-      TProb px{};  // Wx = LCC(J3) CCR / sqrt(J3+1): operand 0 the Pandya matrices of G, 1 CCR
+      TProb px{};  // Wx = LCC(J3) CCR / sqrt(J3+1): operand 0 the Pandya matrices of G, 1 CCR (2 CCX, 3 G's in group order)
       px.M = r3; px.N = r4; px.ldc = r4; px.c_off = S.woff[x];
       px.nseg = nb3 > 0 ? 1 : 0;
       px.seg[0] = TSeg{Ly.ccoff[q3], S.roff[x], nb3, 1, r3, r4, 1, 0, 1, 1.0 / std::sqrt(S.cJ3[x] + 1.0)};
-      pr[0].push_back(px);
-      add_tiles((int)pr[0].size() - 1, r3, r4, tiles[0]);
-      TProb py{};  // Wy = CCX LCC(J4)^T / sqrt(J4+1): operand 0 CCX, 1 the Pandya matrices of G
-      py.M = r3; py.N = r4; py.ldc = r4; py.c_off = S.woff[x];
+      pr.push_back(px);
+      add_tiles((int)pr.size() - 1, r3, r4, tiles);
+      TProb py{};  // Wy = CCX LCC(J4)^T / sqrt(J4+1)
+      py.M = r3; py.N = r4; py.ldc = r4; py.c_off = S.woff[x]; py.c = 1;
       py.nseg = (nb4 > 0 && S.cJ3[x] != S.cJ4[x]) ? 1 : 0;
-      py.seg[0] = TSeg{S.xoff[x], Ly.ccoff[q4], nb4, nb4, 1, r4, 1, 0, 1, 1.0 / std::sqrt(S.cJ4[x] + 1.0)};
-      pr[1].push_back(py);
-      add_tiles((int)pr[1].size() - 1, r3, r4, tiles[1]);
+      py.seg[0] = TSeg{S.xoff[x], Ly.ccoff[q4], nb4, nb4, 1, r4, 1, 2, 3, 1.0 / std::sqrt(S.cJ4[x] + 1.0)};
+      pr.push_back(py);
+      add_tiles((int)pr.size() - 1, r3, r4, tiles);
     }
-    for (int w = 0; w < 2; w++) {
-      if (upload_table(c, pr[w], &S.cc_probs[w]) != 0) return IMSRG_ENOMEM;
-      if (upload_table(c, tiles[w], &S.cc_tiles[w]) != 0) return IMSRG_ENOMEM;
-      S.n_cc_tiles[w] = (int)tiles[w].size();
-    }
+    if (upload_table(c, pr, &S.cc_probs) != 0 || upload_table(c, tiles, &S.cc_tiles) != 0) return IMSRG_ENOMEM;
+    S.n_cc_tiles = (int)tiles.size();
   }
   // workspaces
   if (dalloc(c, Ly.ccsize, &S.gcc) || dalloc(c, Ly.ccsize, &S.gccp) || dalloc(c, S.xsize, &S.ccx) || dalloc(c, S.rsize, &S.ccr) ||
       dalloc(c, 2 * S.wsize, &S.wx) || dalloc(c, S.vsize, &S.w1) ||
-      dalloc(c, S.vsize, &S.w2) || dalloc(c, kNormParts, &S.part))
+      dalloc(c, S.vsize, &S.w2))
     return IMSRG_ENOMEM;
   // entries that the selection rules exclude are never written
   launch_fill(c->stream, S.ccx, S.xsize, 0.0);
@@ -1835,7 +1780,19 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
   launch_fill(c->stream, S.w2, S.vsize, 0.0);
   S.wy = S.wx + S.wsize;
   launch_fill(c->stream, S.wx, 2 * S.wsize, 0.0);
-  HIPCHK(hipHostMalloc((void **)&S.hpart, kNormParts * sizeof(double)));
+  {
+    std::vector<TRun> runs(1, TRun{Ly.f_off, nsp * nsp, 0});
+    constexpr int run = 2048;
+    for (int q = 0; q < S.nblk; q++) {
+      const long long m = (long long)S.n1[q] * S.n2[q];
+      for (long long k = 0; k < m; k += run)
+        runs.push_back(TRun{S.v_off + S.off[q] + k, (int)std::min<long long>(run, m - k), S.J1[q] == S.J2[q] ? 1 : 2});
+    }
+    S.nrun = (int)runs.size();
+    if (upload_table(c, runs, &S.runs) != 0 || dalloc(c, S.nrun, &S.part)) return IMSRG_ENOMEM;
+  }
+  HIPCHK(hipHostMalloc((void **)&S.norm, sizeof(TNorm)));
+  S.norm->seq = 0;
   return 0;
 }
 
@@ -1855,7 +1812,6 @@ static int tspace_get(imsrg_ctx_s *c, int rank, int dpar, TensorSpace **out) {
 }
 
 // ---------------------------------------------------------------- C ABI
-static unsigned nblk(long long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
 int imsrg_tensor_create(imsrg_ctx c, int rank, int dpar, int herm, imsrg_tensor *out) {
   if (!c || !out) return fail(IMSRG_EINVAL, "null argument");
@@ -1988,27 +1944,35 @@ int imsrg_tensor_add(imsrg_tensor A, double ax, imsrg_tensor B, double bx, imsrg
   return 0;
 }
 
-static int tnorm(imsrg_tensor t, double *out) {
-  imsrg_ctx_s *c = t->ctx;
-  TensorSpace &S = *t->ts;
-  hipLaunchKernelGGL(k_tnorm, dim3(kNormParts), dim3(256), 0, c->stream, c->dl, S.dt, (const double *)t->d, S.part);
-  HIPCHK(hipMemcpyAsync(S.hpart, S.part, kNormParts * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  double s = 0.0;
-  for (int k = 0; k < kNormParts; k++) s += S.hpart[k];
-  *out = std::sqrt(s);
+// ||X|| (and HS += coef X first), read from host memory as the kernel writes it
+static int tstep(imsrg_ctx_s *c, TensorSpace &S, const double *X, double *HS, double coef, double *out) {
+  S.seq = S.seq == (1 << 30) ? 1 : S.seq + 1;
+  hipLaunchKernelGGL(k_t_step, dim3(S.nrun), dim3(256), 0, c->stream, c->dl, S.runs, X, HS, coef, S.part);
+  hipLaunchKernelGGL(k_t_norm, dim3(1), dim3(256), 0, c->stream, (const double *)S.part, S.nrun, S.norm, S.seq);
+  HIPCHK(hipGetLastError());
+  const volatile int *seq = &S.norm->seq;
+  for (long long spin = 1; *seq != S.seq; spin++) {
+    if (spin % 4096) continue;
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e == hipErrorNotReady || (e == hipSuccess && *seq == S.seq)) continue;
+    return fail(IMSRG_EDEVICE, std::string("tensor norm: ") + hipGetErrorString(e));
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  *out = std::sqrt(*(const volatile double *)&S.norm->v);
   return 0;
 }
 
 int imsrg_tensor_norm(imsrg_tensor t, double *out) {
   if (!t || !out) return fail(IMSRG_EINVAL, "null argument");
-  return tnorm(t, out);
+  return tstep(t->ctx, *t->ts, t->d, nullptr, 0.0, out);
 }
 
 // [G, T] into RES in BCH_TENSOR's call order (IMSRG_MAGNUS.f90:427-446):
 // 111 (overwrites the one-body part), 121, 122 (overwrites the two-body
-// part), 212, 222_pp_hh, 221, 211, 222_ph; the others accumulate.  221 reads
-// the pp/hh ladder products, computed here whenever 221 is asked for.  Gd:
+// part), 212, 222_pp_hh, 221, 211, 222_ph; the others accumulate, so the
+// one-body terms run together once the ladder products and G's Pandya matrices
+// are there.  221 reads the ladder products, computed here whenever it is
+// asked for.  Gd:
 // the scalar operator's buffer (may be null when only 211 / 222_ph run on
 // Pandya matrices already in S.gcc, gcc_ready).
 static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, imsrg_tensor RES, unsigned mask,
@@ -2022,34 +1986,20 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
   const double *RF = T->d + c->lay.f_off, *RV = T->d + S.v_off;
   double *OF = RES->d + c->lay.f_off, *OV = RES->d + S.v_off;
   if (!Gd && (mask & ~(IMSRG_TS211 | IMSRG_TS222PH))) return fail(IMSRG_EINVAL, "terms need the scalar operator");
-  const long long nf = (long long)D.nhole * D.nhole + (long long)D.npart * D.nhole + (long long)D.npart * D.npart;
-  if (mask & IMSRG_TS111)
-    hipLaunchKernelGGL(k_t111, dim3(nblk(nf)), dim3(256), 0, s, L, D, GF, RF, OF, hL, hR, hres);
-  if (mask & IMSRG_TS121)
-    hipLaunchKernelGGL(k_t_onebody, dim3(L.nob), dim3(64), 0, s, L, D, 0, GF, RF, RV, (const double *)S.gcc,
-                       (const double *)S.w1, (const double *)S.w2, OF, hL, hR, hres);
   if (S.lists.nlist > 0 && (mask & (IMSRG_TS122 | IMSRG_TS212))) {
     hipLaunchKernelGGL(k_t_lists, dim3(S.lists.nlist), dim3(64), 0, s, L, D, S.lists, GF, RF,
                        (mask & IMSRG_TS122) != 0, (mask & IMSRG_TS212) != 0);
     hipLaunchKernelGGL(k_t_1body, dim3(S.lists.nitem), dim3(kT1Threads), S.lists.lds, s, L, D, S.lists, GV, RV, OV,
                        !(mask & IMSRG_TS122));
   }
-  if ((mask & (IMSRG_TS222PPHH | IMSRG_TS221)) && S.n_pp_tiles > 0) {
-    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs[0], S.pp_tiles, S.n_pp_tiles, GV, RV,
-                       S.w1);
-    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs[1], S.pp_tiles, S.n_pp_tiles, GV, RV,
-                       S.w2);
-  }
-  if (mask & IMSRG_TS222PPHH) {
-    launch_axpby(s, S.vsize, 1.0, OV, 1.0, S.w1, OV, nullptr, 1, 0);
-    launch_axpby(s, S.vsize, 1.0, OV, -1.0, S.w2, OV, nullptr, 1, 0);
-  }
-  if (mask & IMSRG_TS221)
-    hipLaunchKernelGGL(k_t_onebody, dim3(L.nob), dim3(64), 0, s, L, D, 2, GF, RF, RV, (const double *)S.gcc,
-                       (const double *)S.w1, (const double *)S.w2, OF, hL, hR, hres);
+  if ((mask & (IMSRG_TS222PPHH | IMSRG_TS221)) && S.n_pp_tiles > 0)
+    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs, S.pp_tiles, S.n_pp_tiles,
+                       TGemm{{GV, RV, nullptr, nullptr}, {S.w1, S.w2}, (mask & IMSRG_TS222PPHH) ? OV : nullptr});
   if ((mask & (IMSRG_TS211 | IMSRG_TS222PH)) && !gcc_ready) launch_pandya(s, L, Gd, S.gcc, nullptr, 1);
-  if (mask & IMSRG_TS211)
-    hipLaunchKernelGGL(k_t_onebody, dim3(L.nob), dim3(64), 0, s, L, D, 1, GF, RF, RV, (const double *)S.gcc,
+  const int one = ((mask & IMSRG_TS111) ? kTf111 : 0) | ((mask & IMSRG_TS121) ? kTf121 : 0) |
+                  ((mask & IMSRG_TS221) ? kTf221 : 0) | ((mask & IMSRG_TS211) ? kTf211 : 0);
+  if (one)
+    hipLaunchKernelGGL(k_t_f, dim3(L.nob), dim3(kTfThreads), 0, s, L, D, one, GF, RF, RV, (const double *)S.gcc,
                        (const double *)S.w1, (const double *)S.w2, OF, hL, hR, hres);
   if ((mask & IMSRG_TS222PH) && S.nelem > 0) {
     if (L.nccol > 0)
@@ -2057,12 +2007,9 @@ static int ts_comm(imsrg_ctx_s *c, const double *Gd, int hG, imsrg_tensor T, ims
     if (S.pan[0].npad + S.pan[1].npad > 0)
       hipLaunchKernelGGL(k_t_pandya, dim3(S.pan[0].npad + S.pan[1].npad), dim3(64), 0, s, L, D, S.pan[0], S.pan[1],
                          RV, hR);
-    if (S.n_cc_tiles[0] > 0)
-      hipLaunchKernelGGL(k_tgemm, dim3(S.n_cc_tiles[0]), dim3(256), 0, s, S.cc_probs[0], S.cc_tiles[0],
-                         S.n_cc_tiles[0], (const double *)S.gcc, (const double *)S.ccr, S.wx);
-    if (S.n_cc_tiles[1] > 0)
-      hipLaunchKernelGGL(k_tgemm, dim3(S.n_cc_tiles[1]), dim3(256), 0, s, S.cc_probs[1], S.cc_tiles[1],
-                         S.n_cc_tiles[1], (const double *)S.ccx, (const double *)S.gccp, S.wy);
+    if (S.n_cc_tiles > 0)
+      hipLaunchKernelGGL(k_tgemm, dim3(S.n_cc_tiles), dim3(256), 0, s, S.cc_probs, S.cc_tiles, S.n_cc_tiles,
+                         TGemm{{S.gcc, S.ccr, S.ccx, S.gccp}, {S.wx, S.wy}, nullptr});
     if (D.nqchunk > 0)
       hipLaunchKernelGGL(k_t222ph, dim3(D.nqpad), dim3(64), 0, s, L, D, (const double *)S.wx, S.wsize, OV, hL, hR);
   }
@@ -2115,12 +2062,9 @@ int imsrg_tensor_ladders(imsrg_op G, imsrg_tensor T, imsrg_tensor W1, imsrg_tens
   const double *GV = G->d + c->lay.v_off, *RV = T->d + S.v_off;
   launch_fill(s, W1->d, S.op_size, 0.0);
   launch_fill(s, W2->d, S.op_size, 0.0);
-  if (S.n_pp_tiles > 0) {
-    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs[0], S.pp_tiles, S.n_pp_tiles, GV, RV,
-                       W1->d + S.v_off);
-    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs[1], S.pp_tiles, S.n_pp_tiles, GV, RV,
-                       W2->d + S.v_off);
-  }
+  if (S.n_pp_tiles > 0)
+    hipLaunchKernelGGL(k_tgemm, dim3(S.n_pp_tiles), dim3(256), 0, s, S.pp_probs, S.pp_tiles, S.n_pp_tiles,
+                       TGemm{{GV, RV, nullptr, nullptr}, {W1->d + S.v_off, W2->d + S.v_off}, nullptr});
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -2133,45 +2077,58 @@ int imsrg_tensor_commutator_221(imsrg_tensor W1, imsrg_tensor W2, int pm, imsrg_
   imsrg_ctx_s *c = RES->ctx;
   TensorSpace &S = *RES->ts;
   double *OF = RES->d + c->lay.f_off;
-  const double *RV = RES->d + S.v_off;  // not read by the 221 kernel
-  hipLaunchKernelGGL(k_t_onebody, dim3(c->dl.nob), dim3(64), 0, c->stream, c->dl, S.dt, 2, (const double *)OF,
-                     (const double *)OF, RV, (const double *)S.gcc, (const double *)(W1->d + S.v_off),
-                     (const double *)(W2->d + S.v_off), OF, pm, 1, RES->herm);
+  hipLaunchKernelGGL(k_t_f, dim3(c->dl.nob), dim3(kTfThreads), 0, c->stream, c->dl, S.dt, (int)kTf221,
+                     (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, (const double *)nullptr,
+                     (const double *)(W1->d + S.v_off), (const double *)(W2->d + S.v_off), OF, pm, 1, RES->herm);
   HIPCHK(hipGetLastError());
   return 0;
 }
 
+// BCH_TENSOR: HS += sum of the nested commutators [G, .. [G, HS]] / n! until
+// ||ad^n|| / n! < conv.  The nested commutators alternate between two work
+// operators; the first reads HS itself, which only changes after it.  All of a
+// work operator's one- and two-body elements are overwritten by 111 and 122.
+static constexpr long long kBchKeep = 1LL << 30;
 int imsrg_bch_tensor(imsrg_op G, imsrg_tensor HS, int *nterms) {
   if (!G || !HS) return fail(IMSRG_EINVAL, "null argument");
   imsrg_ctx_s *c = HS->ctx;
   if (G->ctx != c) return fail(IMSRG_EINVAL, "G and HS belong to different contexts");
   TensorSpace &S = *HS->ts;
-  imsrg_tensor_s INT2, AD;
-  INT2.ctx = AD.ctx = c;
-  INT2.ts = AD.ts = &S;
-  double *buf = nullptr;
-  if (hipMalloc(&buf, sizeof(double) * S.op_size * 2) != hipSuccess)
-    return fail(IMSRG_ENOMEM, "hipMalloc BCH_TENSOR workspace failed");
-  INT2.d = buf;
-  AD.d = buf + S.op_size;
-  // INT2 = HS (copy_sq_op keeps HS's herm, IMSRG_MAGNUS.f90:419-422)
-  int rc = imsrg_tensor_copy(HS, &INT2);
+  const long long bytes = 2LL * (long long)sizeof(double) * S.op_size;
+  double *buf = S.bch;
+  if (!buf) {
+    if (hipMalloc(&buf, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc BCH_TENSOR workspace failed");
+    launch_fill(c->stream, buf, 2 * S.op_size, 0.0);
+  }
+  imsrg_tensor_s W[2];
+  for (int k = 0; k < 2; k++) {
+    W[k].ctx = c;
+    W[k].ts = &S;
+    W[k].d = buf + k * S.op_size;
+    W[k].herm = HS->herm;  // copy_sq_op keeps HS's herm (IMSRG_MAGNUS.f90:419-422)
+  }
   const double conv = (double)1e-6f;  // real(8), parameter :: conv = 1e-6
   double coef = 1.0;
-  int n = 0;
-  for (int iw = 2; iw <= 30 && rc == 0; iw++) {
+  int n = 0, rc = 0;
+  imsrg_tensor AD = HS;
+  for (int iw = 2; iw <= 30; iw++) {
     coef = coef / (iw - 1.0);
-    if ((rc = imsrg_tensor_copy(&INT2, &AD))) break;
-    launch_fill(c->stream, INT2.d, S.op_size, 0.0);
-    if ((rc = ts_comm(c, G->d, G->herm, &AD, &INT2, IMSRG_TSALL, false))) break;
+    imsrg_tensor INT2 = &W[iw & 1];
+    if ((rc = ts_comm(c, G->d, G->herm, AD, INT2, IMSRG_TSALL, false))) break;
     n++;
-    launch_axpby(c->stream, S.op_size, 1.0, HS->d, coef, INT2.d, HS->d, nullptr, 1, 0);
     double nrm = 0.0;
-    if ((rc = tnorm(&INT2, &nrm))) break;
+    if ((rc = tstep(c, S, INT2->d, HS->d, coef, &nrm))) break;
     if (nrm * coef < conv) break;
+    AD = INT2;
   }
-  (void)hipStreamSynchronize(c->stream);
-  (void)hipFree(buf);
+  if (bytes <= kBchKeep && rc == 0) {
+    S.bch = buf;
+  } else {
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(buf);
+    S.bch = nullptr;
+  }
   if (nterms) *nterms = n;
   return rc;
 }
+
