@@ -35,10 +35,11 @@ __device__ __forceinline__ long long zidx(int R, int C, int M) {
 // row, before any barrier.
 __device__ __forceinline__ long long inst_id(const int *act) { return act ? act[blockIdx.y] : 0; }
 
-__device__ __forceinline__ int xcd_item(const XcdSplit &x) {
-  const int xcd = blockIdx.x & 7, it = x.start[xcd] + (int)(blockIdx.x >> 3);
+__device__ __forceinline__ int xcd_item(const XcdSplit &x, int b) {
+  const int xcd = b & 7, it = x.start[xcd] + (b >> 3);
   return it < x.start[xcd + 1] ? it : -1;
 }
+__device__ __forceinline__ int xcd_item(const XcdSplit &x) { return xcd_item(x, blockIdx.x); }
 
 __device__ __forceinline__ int sgnp(int e) { return (e & 1) ? -1 : 1; }  // (-1)^e
 __device__ __forceinline__ bool dtri(int a, int b, int J) { return J <= a + b && J >= abs(a - b); }

@@ -336,13 +336,15 @@ struct SmallArgs {
   const double *Lop, *Rop;
   double *RES, *acc;
   double *ccL, *ccR, *Z, *wpp, *partials, *npart;
+  double *w122;             // the 122 weight table, where the first launch is its parts' own kernels (else null)
+  double *T, *obpart;       // J' terms and one-body partial sums, made by a launch of their own (T null: in the last)
   int hL, hR, hres, prepL;  // prepL: ccL is still to be made from L
   unsigned mask;
   double coef;
   const double *coefp;
   const SegProb *pp_probs, *ph_probs;
   const int4 *pp_tiles, *ph_tiles, *tiles16;
-  int n_pp, n_ph, n16, n_diff, nsplit, split;
+  int n_pp, n_ph, ntile, n_diff, nsplit, split;  // ntile: of the last launch, 16 x 16 (T null) or 32 x 32
   const int *diff_ob;       // one-body outputs whose orbits differ in (l, j, tz)
   const PhRow *phrow;
   const int *act;

@@ -280,12 +280,13 @@ static int scratch_setup(imsrg_ctx_s *c) {
 // ---------------------------------------------------------------- context
 // Tables of the three-launch commutator (launch_small), for bases that may use it.
 static constexpr long long kSplitElems = 300000;  // two-body elements (the rule at wave_pair)
-static constexpr long long kSmallElems = 1000000;  // two-body elements times instances (the rule at use_small)
+// two-body elements times instances (the rules at comm_form)
+static constexpr long long kFusedElems = 200000, kMergedElems = 4000000, kTuneElems = 1000000;
 static int small_setup(imsrg_ctx_s *c, const std::vector<int> &same_ob) {
   const Layout &Ly = c->lay;
   const DevLayout &D = c->dl;
-  if (Ly.vsize > kSmallElems || D.n122_frows > 0 || D.n122_items == 0 || D.nccol == 0 || D.nphterm == 0 || D.nob == 0)
-    return 0;
+  c->mergeable = D.n122_frows == 0 && D.n122_items > 0 && D.nccol > 0 && D.nphterm > 0 && D.nob > 0;
+  if (!c->mergeable || Ly.vsize > kFusedElems) return 0;
   std::vector<int4> t16;
   for (int q = 0; q < Ly.nblocks; q++) {
     const int nt = (Ly.bdim[q] + 15) / 16;
@@ -670,7 +671,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
     if (!rc) rc = upload_table(c, ph, (const GemmProb **)&c->adj_ph_probs);
     if (!rc) rc = upload_table(c, th, (const int4 **)&c->adj_ph_tiles);
   }
-  if (!rc && c->small) {
+  if (!rc && c->mergeable) {
     const std::vector<DevLayout> dl(1, c->dl);
     rc = upload_table(c, dl, &c->dl_d);
   }
@@ -1378,19 +1379,31 @@ enum { kLPrepped = 1, kLPandya = 2, kRPandya = 4 };
 static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                          int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi());
 
-// The three-launch form (launch_small) of a whole FP64 commutator: while the
-// two-body part of all instances holds at most 10^6 elements, issuing the
-// separate kernels costs more than they run.  Per commutator of a BCH series,
-// separate / three launches, in us: emax 2 82 / 39, emax 4 91 / 52, emax 5
-// 124 / 83, emax 6 (9.6e5 elements) 151 / 146, 4 x emax 5 (1.15e6) 163 / 175,
-// 16 x emax 4 (1.16e6) 187 / 222, emax 7 323 / 349, emax 8 640 / 912: past the
-// line the ph sums straight from Z cost more than the J' terms made once.
-// Masks with terms left out, profiling, tile shapes set to 128 x 64 and bases
-// with 122 sets past 32 rows keep the separate kernels.
-static bool use_small(imsrg_ctx_s *c, unsigned mask, int cc_ready, int na) {
+// The form of a commutator (launch_small; all forms give the same bits).  Per
+// commutator of a BCH series, in us, separate kernels on two streams / merged
+// (five launches) / fused (three), by two-body elements times instances:
+//   emax 4 (7.1e4)      74 / 44 / 42     4 x emax 4 (2.9e5)  103 / 80 / 80
+//   emax 5 (2.9e5)     103 / 61 / 67     emax 6 (9.6e5)      142 / 101 / 125
+//   4 x emax 5 (1.1e6) 145 / 139         emax 7 (2.8e6)      248 / 207
+//   4 x emax 6 (3.8e6) 321 / 294         16 x emax 5 (4.6e6) 407 / 428
+//   emax 8 (7.2e6)     637 / 613         2 x emax 8 (1.4e7)  1100 / 1088
+//   16 x emax 6 (1.5e7) 1114 / 1133
+// Fused pays while launches are what a commutator costs; past 2e5 the ph sums
+// straight from Z, made anew for every J, cost more than a launch for the J'
+// terms.  Merged pays while a kernel's last workgroups leave much of the chip
+// idle: up to 4e6 elements, and for one or two instances in any basis; with
+// many instances the separate kernels fill the chip and overlap on two streams.
+// Masks with terms left out, profiling, tile shapes set to 128 x 64, other
+// precisions and bases with 122 sets past 32 rows keep the separate kernels.
+enum CommForm { kSeparate, kMerged, kFused };
+static CommForm comm_form(const imsrg_ctx_s *c, unsigned mask, int cc_ready, int na) {
   const unsigned all = T111 | T121 | T122 | T221 | T222PPHH | T222PH;
-  return c->small && c->prec == IMSRG_PREC_FP64 && !c->prof_on && (mask & all) == all &&
-         !(cc_ready & (kLPandya | kRPandya)) && c->shape_pp != 1 && c->shape_ph != 1 && c->lay.vsize * na <= kSmallElems;
+  if (!c->mergeable || c->prec != IMSRG_PREC_FP64 || c->prof_on || (mask & all) != all ||
+      (cc_ready & (kLPandya | kRPandya)) || c->shape_pp == 1 || c->shape_ph == 1)
+    return kSeparate;
+  const long long n = (long long)c->lay.vsize * na;
+  if (c->small && n <= kFusedElems) return kFused;
+  return n <= kMergedElems || na <= 2 ? kMerged : kSeparate;
 }
 
 // Tile-shape autotuner: on the first FP64 commutator of a context, each 222
@@ -1455,7 +1468,7 @@ static int autotune(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R) {
 static int comm_impl(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                      int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi()) {
   if (c->prec == IMSRG_PREC_FP64 && c->shape_pp < 0 && a.n() > 0 && (mask & (T222PPHH | T221 | T222PH)) &&
-      !use_small(c, mask, cc_ready, a.g())) {
+      (comm_form(c, mask, cc_ready, a.g()) == kSeparate || c->lay.vsize * a.g() > kTuneElems)) {
     c->fork_mark = nullptr;  // the tuning launches follow the mark on the stream
     int rc = autotune(c, L, R);
     if (rc) return rc;
@@ -1512,7 +1525,7 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     c->fork_mark = nullptr;
     return 0;
   }
-  if (use_small(c, mask, cc_ready, na)) {
+  if (const CommForm form = comm_form(c, mask, cc_ready, na); form != kSeparate) {
     SmallArgs A{};
     A.Lop = L->d; A.Rop = R->d; A.RES = RES->d; A.acc = epi.acc;
     A.ccL = c->cc[0]; A.ccR = c->cc[1]; A.Z = c->wph; A.wpp = c->wpp; A.partials = c->partials;
@@ -1523,12 +1536,19 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     A.split = c->split;
     A.pp_tiles = c->pp_tiles_s; A.ph_tiles = c->split ? c->ph_tiles_s : c->ph_tiles;
     A.n_pp = c->n_pp_tiles_s; A.n_ph = c->split ? c->n_ph_tiles_s : c->n_ph_tiles;
-    A.tiles16 = c->tiles16; A.n16 = c->n_tiles16; A.n_diff = c->n_diff_ob;
+    A.tiles16 = c->tiles16; A.n_diff = c->n_diff_ob;
+    A.ntile = form == kFused ? c->n_tiles16 : D.nmirror;
+    A.T = form == kFused ? nullptr : c->tph;
+    A.obpart = c->obpart;
+    // the first launch's parts as kernels of their own, the 122 weights from a
+    // table, where they are long: emax 8 613 us a commutator against 624, 16 x
+    // emax 4 177 / 196, but emax 7 215 / 207, emax 6 110 / 101
+    A.w122 = form == kMerged && D.vsize * na > (na == 1 ? 3000000 : 1000000) ? c->w122 : nullptr;
     A.diff_ob = c->diff_ob; A.phrow = c->phrow; A.act = ad;
     launch_small(s, D, c->dl_d, A, na);
     c->fork_mark = nullptr;
-    if (epi.gate_act) launch_norm_gate(s, c->npart, c->n_tiles16 + D.nob, epi.gate_act, na, c->scal, epi.gate);
-    else if (epi.norm) launch_norm_from_parts(s, c->n_tiles16 + D.nob, c->npart, c->scal, ad, na);
+    if (epi.gate_act) launch_norm_gate(s, c->npart, A.ntile + D.nob, epi.gate_act, na, c->scal, epi.gate);
+    else if (epi.norm) launch_norm_from_parts(s, A.ntile + D.nob, c->npart, c->scal, ad, na);
     HIPCHK(hipGetLastError());
     return 0;
   }
@@ -1828,7 +1848,7 @@ static GateArgs gate_args(imsrg_ctx_s *c, int n, int mode, double coef, int stor
 // marks gate n on the stream: the second stream of the next commutator forks
 // from there (nullptr when that commutator runs on one stream)
 static hipEvent_t gate_mark(imsrg_ctx_s *c, int n, const ActSet &set) {
-  if (!c->dual || c->graphs || use_small(c, IMSRG_TALL, kLPrepped, set.g())) return nullptr;
+  if (!c->dual || c->graphs || comm_form(c, IMSRG_TALL, kLPrepped, set.g()) != kSeparate) return nullptr;
   hipEvent_t e = c->ev_gate[n % imsrg_ctx_s::kGateRing];
   return hipEventRecord(e, c->stream) == hipSuccess ? e : nullptr;
 }

@@ -98,9 +98,10 @@ struct imsrg_ctx_s {
   int n_pp_tiles = 0, n_ph_tiles = 0;
   int4 *pp_tiles_w = nullptr, *ph_tiles_w = nullptr;    // 128 x 64 tiles (FP64 path)
   int n_pp_tiles_w = 0, n_ph_tiles_w = 0;
-  // the three-launch commutator of small bases (launch_small): tables, and the
-  // layout's view in device memory; small = false when the basis is not taken
-  bool small = false;
+  // commutators in few launches (launch_small): whether the basis may take the
+  // merged form, whether it has the fused form's tables; these, and the layout's
+  // view in device memory
+  bool mergeable = false, small = false;
   const DevLayout *dl_d = nullptr;
   const int4 *tiles16 = nullptr;
   const PhRow *phrow = nullptr;

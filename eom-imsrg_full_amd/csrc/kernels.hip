@@ -1215,24 +1215,18 @@ __device__ __forceinline__ double ph_term(unsigned sel, double2 b, double2 c, do
 // Work items past the XCD split's are the (a,a) terms, one per thread; the
 // chunks skip them.  Every load is unconditional (past the end: the last
 // term; invalid terms: half 0), so the four terms' loads stay in flight together.
-__global__ __launch_bounds__(256) void k_ph_terms(DevLayout L, const double *__restrict__ Z,
-                                                  double *__restrict__ Tbuf, double sigma, const int *act) {
-  {
-    const long long inst = inst_id(act);
-    if (inst < 0) return;
-    Z += inst * L.cwsize;
-    Tbuf += inst * L.nphterm;
-  }
+__device__ __forceinline__ void ph_terms_item(const DevLayout &L, const double *__restrict__ Z,
+                                              double *__restrict__ Tbuf, double sigma, int b0) {
   const double2 *Z2 = reinterpret_cast<const double2 *>(Z);
   const int nchunk = 8 * L.xs_terms.len;
-  if ((int)blockIdx.x >= nchunk) {
-    const long long k = (long long)(blockIdx.x - nchunk) * 256 + threadIdx.x;
+  if (b0 >= nchunk) {
+    const long long k = (long long)(b0 - nchunk) * 256 + threadIdx.x;
     if (k >= L.nphtwo) return;
     const unsigned t = L.ph_two[k], sel = L.ph_zsel[t], blk = L.ph_zblk[t];
     Tbuf[t] = ph_term(sel, Z2[blk], Z2[blk ^ 1u], sigma);
     return;
   }
-  const int chunk = xcd_item(L.xs_terms);
+  const int chunk = xcd_item(L.xs_terms, b0);
   if (chunk < 0) return;
   const long long t0 = (long long)chunk * 1024 + threadIdx.x;
   unsigned sel[4], blk[4];
@@ -1254,6 +1248,12 @@ __global__ __launch_bounds__(256) void k_ph_terms(DevLayout L, const double *__r
     const long long t = t0 + 256 * u;
     if (t < L.nphterm && (sel[u] & 130) != 130) Tbuf[t] = ph_term(sel[u], b[u], b[u], sigma);
   }
+}
+__global__ __launch_bounds__(256) void k_ph_terms(DevLayout L, const double *__restrict__ Z,
+                                                  double *__restrict__ Tbuf, double sigma, const int *act) {
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  ph_terms_item(L, Z + inst * L.cwsize, Tbuf + inst * L.nphterm, sigma, blockIdx.x);
 }
 void launch_ph_terms(hipStream_t s, const DevLayout &L, const double *Z, double *Tbuf, double hL, double hR,
                      const int *act, int nact) {
@@ -1372,18 +1372,13 @@ void launch_ph_apply(hipStream_t s, const DevLayout &L, const double *Tbuf, doub
 // reference's "upper triangle then mirror x herm" contract (commutators.f90
 // 388-395, 915-923).  32x32 tile pairs go through LDS so all reads and
 // writes are row-contiguous.
-__global__ __launch_bounds__(256) void k_sym_mirror(DevLayout L, const int4 *__restrict__ tiles, double *RES,
-                                                    int herm, const int *act, double *acc, double coef,
-                                                    const double *coefp, double *npart, long long nstride) {
-  __shared__ double sh[256];
-  const long long inst = inst_id(act);
-  if (inst < 0) return;
-  if (coefp) coef = *coefp;
-  RES += inst * L.op_size;
-  const int4 t = tiles[blockIdx.x];  // x = block, y = tile row, z = tile col (y <= z)
+// tile pair t of one instance (RES, acc at its start; acc null: none); returns the
+// thread's sum of squares
+__device__ __forceinline__ double mirror_tile(const DevLayout &L, const int4 t, double *RES, int herm, double *acc,
+                                              double coef) {
   const int q = t.x, dim = L.bdim[q];
   double *OV = RES + L.v_off + L.boff[q];
-  double *AV = acc ? acc + inst * L.op_size + L.v_off + L.boff[q] : nullptr;
+  double *AV = acc ? acc + L.v_off + L.boff[q] : nullptr;
   __shared__ double U[32][33], W[32][33];
   const int r0 = t.y * 32, c0 = t.z * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
@@ -1443,6 +1438,17 @@ __global__ __launch_bounds__(256) void k_sym_mirror(DevLayout L, const int4 *__r
       if (AV) AV[o] = al[m] + coef * v;
     }
   }
+  return sq;
+}
+__global__ __launch_bounds__(256) void k_sym_mirror(DevLayout L, const int4 *__restrict__ tiles, double *RES,
+                                                    int herm, const int *act, double *acc, double coef,
+                                                    const double *coefp, double *npart, long long nstride) {
+  __shared__ double sh[256];
+  const long long inst = inst_id(act);
+  if (inst < 0) return;
+  if (coefp) coef = *coefp;
+  const long long o = inst * L.op_size;
+  double sq = mirror_tile(L, tiles[blockIdx.x], RES + o, herm, acc ? acc + o : nullptr, coef);
   if (npart) {
     sq = block_sum256(sq, sh);
     if (threadIdx.x == 0) npart[inst * nstride + blockIdx.x] = sq;
@@ -1548,22 +1554,27 @@ __device__ __forceinline__ double ob_term(const DevLayout &L, const double *__re
   }
   return v;
 }
+// chunk b % ob_nchunk of same-group output b / ob_nchunk
+__device__ __forceinline__ void ob_partial_item(const DevLayout &L, const double *__restrict__ Lop,
+                                                const double *__restrict__ Rop, const double *__restrict__ Wpp,
+                                                double *__restrict__ part, int hL, int hR, unsigned mask, int b) {
+  __shared__ double red[4];
+  const int sp = b / L.ob_nchunk, ch = b - sp * L.ob_nchunk;
+  if (sp >= L.nsame) return;
+  const int tid = threadIdx.x;
+  const double v = wave_sum(ob_term(L, Lop, Rop, Wpp, L.same_ob[sp], ch * 256 + tid, hL, hR, mask));
+  if ((tid & 63) == 0) red[tid >> 6] = v;
+  __syncthreads();
+  if (tid == 0) part[b] = red[0] + red[1] + red[2] + red[3];
+}
 __global__ __launch_bounds__(256) void k_ob_partial(DevLayout L, const double *__restrict__ Lop,
                                                     const double *__restrict__ Rop,
                                                     const double *__restrict__ Wpp, double *__restrict__ part,
                                                     int hL, int hR, unsigned mask, const int *act) {
-  __shared__ double red[4];
-  const int sp = blockIdx.x / L.ob_nchunk, ch = blockIdx.x - sp * L.ob_nchunk;
-  if (sp >= L.nsame) return;
   const long long inst = inst_id(act);
   if (inst < 0) return;
-  const int tid = threadIdx.x;
-  double v = ob_term(L, Lop + inst * L.op_size, Rop + inst * L.op_size, Wpp + inst * L.vsize, L.same_ob[sp],
-                     ch * 256 + tid, hL, hR, mask);
-  v = wave_sum(v);
-  if ((tid & 63) == 0) red[tid >> 6] = v;
-  __syncthreads();
-  if (tid == 0) part[inst * (long long)L.nsame * L.ob_nchunk + blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  ob_partial_item(L, Lop + inst * L.op_size, Rop + inst * L.op_size, Wpp + inst * L.vsize,
+                  part + inst * (long long)L.nsame * L.ob_nchunk, hL, hR, mask, blockIdx.x);
 }
 // writes one-body output (p,q) and its mirror, adds coef times both to AF when
 // there is one, and returns the output's sum of squares
@@ -2081,19 +2092,23 @@ void launch_magnus_gate(hipStream_t s, const DevLayout &L, const double *DG, con
   hipLaunchKernelGGL(k_magnus_gate, dim3(1, nact), dim3(256), 0, s, partials, ps, act, scal, G);
 }
 
-// ------------------------------------------------------------------ small bases: a commutator in three launches
+// ------------------------------------------------------------------ a commutator in few launches
 // In bases up to about emax = 5 a commutator's thirteen kernels run 2-8 us
 // each and issuing them costs the host more (5 us a launch, and as much for
-// each event between the two streams).  The same work in three launches: every
-// kernel below is a list of workgroups of different kinds that only need what
-// the launch before left behind.
+// each event between the two streams); up to emax = 8 most of them end in a tail
+// that leaves the chip idle.  The same work in three launches (fused) or five
+// (merged): every kernel below is a list of workgroups of different kinds that
+// only need what the launch before left behind.
 //   k_small_a  Pandya columns, 122 sets (weights formed in place), E0 partials
 //   k_small_b  the pp/hh product (onto the 122 rows) and the Pandya product
-//   k_small_c  per 16 x 16 tile pair: the ph terms and their 6j-weighted sums
-//              straight from Z, then symmetrise + mirror; one-body outputs; E0
+//   fused: k_small_c<true>, per 16 x 16 tile pair the ph terms and their
+//              6j-weighted sums straight from Z, then symmetrise + mirror;
+//              one-body outputs; E0
+//   merged: k_small_t, the J' terms and the one-body partial sums; k_ph_apply;
+//              k_small_c<false>, symmetrise + mirror, one-body outputs, E0
 // The arithmetic and its order are those of the separate kernels, so results
-// are the same bits (the norm's partial sums are per 16 x 16 tile here).
-// Measured, whole flows (per commutator): see the rule in comm_launches.
+// are the same bits (the norm's partial sums are per tile).  Measured: see the
+// rule at comm_form.
 __global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ Lp, SmallArgs A) {
   extern __shared__ double lds[];
   const DevLayout &L = *Lp;
@@ -2144,6 +2159,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double hL = A.hL, hR = A.hR;
     gemm_tile<true, SPLIT>(A.ph_probs, A.ph_tiles[b - A.n_pp], A.ccL + o, A.ccR + o, hL, -hR, A.Z + inst * L.cwsize,
                            nullptr, -hL * hR, &S);
+  }
+}
+
+// the J' terms, and the 121 + 221 partial sums (first: the long ones)
+__global__ __launch_bounds__(256) void k_small_t(const DevLayout *__restrict__ Lp, SmallArgs A, int nob) {
+  const DevLayout &L = *Lp;
+  const long long inst = inst_id(A.act);
+  if (inst < 0) return;
+  const int b = blockIdx.x;
+  if (b < nob) {
+    const long long o = inst * L.op_size;
+    ob_partial_item(L, A.Lop + o, A.Rop + o, A.wpp + inst * L.vsize, A.obpart + inst * (long long)L.nsame * L.ob_nchunk,
+                    A.hL, A.hR, A.mask, b);
+  } else {
+    ph_terms_item(L, A.Z + inst * L.cwsize, A.T + inst * L.nphterm, -(double)A.hL * (double)A.hR, b - nob);
   }
 }
 
@@ -2265,9 +2295,12 @@ __device__ __forceinline__ void small_tile(const DevLayout &L, const SmallArgs &
   }
   if (A.npart) {
     sq = block_sum256(sq, sh);
-    if (tid == 0) A.npart[inst * (A.n16 + L.nob) + bt] = sq;
+    if (tid == 0) A.npart[inst * (A.ntile + L.nob) + bt] = sq;
   }
 }
+// FUSED: with the ph sums, on 16 x 16 tiles; else they are there already and the
+// 32 x 32 tiles are only mirrored
+template <bool FUSED>
 __global__ __launch_bounds__(256) void k_small_c(const DevLayout *__restrict__ Lp, SmallArgs A) {
   __shared__ double sh[256];
   const DevLayout &L = *Lp;
@@ -2275,11 +2308,20 @@ __global__ __launch_bounds__(256) void k_small_c(const DevLayout *__restrict__ L
   if (inst < 0) return;
   if (A.coefp) A.coef = *A.coefp;
   int b = blockIdx.x;
-  if (b < A.n16) {
-    small_tile(L, A, inst, b, sh);
+  if (b < A.ntile) {
+    if constexpr (!FUSED) {
+      const long long o = inst * L.op_size;
+      double sq = mirror_tile(L, L.mirror_tiles[b], A.RES + o, A.hres, A.acc ? A.acc + o : nullptr, A.coef);
+      if (A.npart) {
+        sq = block_sum256(sq, sh);
+        if (threadIdx.x == 0) A.npart[inst * (A.ntile + L.nob) + b] = sq;
+      }
+    } else {
+      small_tile(L, A, inst, b, sh);
+    }
     return;
   }
-  b -= A.n16;
+  b -= A.ntile;
   const long long o = inst * L.op_size;
   const double *Lop = A.Lop + o, *Rop = A.Rop + o;
   double *RES = A.RES + o, *acc = A.acc ? A.acc + o : nullptr;
@@ -2292,31 +2334,50 @@ __global__ __launch_bounds__(256) void k_small_c(const DevLayout *__restrict__ L
   };
   auto put = [&](int t, int p, int qo, double val) {
     const double sq = ob_write(L, RES + L.f_off, acc ? acc + L.f_off : nullptr, p, qo, val, A.hres, A.coef);
-    if (A.npart) A.npart[inst * (A.n16 + L.nob) + A.n16 + t] = sq;
+    if (A.npart) A.npart[inst * (A.ntile + L.nob) + A.ntile + t] = sq;
   };
-  if (b < L.nsame) {  // 111 + 121 + 221 of one output, the chunks of k_ob_partial one after another
-    const int t = L.same_ob[b], p = L.ob_p[t], qo = L.ob_q[t];
-    double val = f111(p, qo), sm = 0.0;
-    for (int ch = 0; ch < L.ob_nchunk; ch++) {
-      const double v = wave_sum(ob_term(L, Lop, Rop, A.wpp + inst * L.vsize, t, ch * 256 + tid, A.hL, A.hR, A.mask));
-      __syncthreads();
-      if (lane == 0) sh[wave] = v;
-      __syncthreads();
-      sm += sh[0] + sh[1] + sh[2] + sh[3];
+  if constexpr (!FUSED) {  // every output, one wavefront each, as k_ob_final
+    const int nw = (L.nob + 3) / 4, t = 4 * b + wave;
+    if (b < nw) {
+      if (t >= L.nob) return;
+      const int p = L.ob_p[t], qo = L.ob_q[t], sp = L.ob_same[t];
+      double val = f111(p, qo);
+      if (lane == 0) {
+        if (sp >= 0) {
+          const double *part = A.obpart + (inst * L.nsame + sp) * L.ob_nchunk;
+          double sm = 0.0;
+          for (int c = 0; c < L.ob_nchunk; c++) sm += part[c];
+          val += sm / (L.jj[p] + 1.0);
+        }
+        put(t, p, qo, val);
+      }
+      return;
     }
-    val += sm / (L.jj[p] + 1.0);
-    if (tid == 0) put(t, p, qo, val);
-    return;
-  }
-  b -= L.nsame;
-  const int nd = (A.n_diff + 3) / 4;
-  if (b < nd) {  // the other outputs: 111 alone, one wavefront each
-    const int i = 4 * b + wave;
-    if (i >= A.n_diff) return;
-    const int t = A.diff_ob[i], p = L.ob_p[t], qo = L.ob_q[t];
-    const double val = f111(p, qo);
-    if (lane == 0) put(t, p, qo, val);
-    return;
+  } else {
+    if (b < L.nsame) {  // 111 + 121 + 221 of one output, the chunks of k_ob_partial one after another
+      const int t = L.same_ob[b], p = L.ob_p[t], qo = L.ob_q[t];
+      double val = f111(p, qo), sm = 0.0;
+      for (int ch = 0; ch < L.ob_nchunk; ch++) {
+        const double v = wave_sum(ob_term(L, Lop, Rop, A.wpp + inst * L.vsize, t, ch * 256 + tid, A.hL, A.hR, A.mask));
+        __syncthreads();
+        if (lane == 0) sh[wave] = v;
+        __syncthreads();
+        sm += sh[0] + sh[1] + sh[2] + sh[3];
+      }
+      val += sm / (L.jj[p] + 1.0);
+      if (tid == 0) put(t, p, qo, val);
+      return;
+    }
+    b -= L.nsame;
+    const int nd = (A.n_diff + 3) / 4;
+    if (b < nd) {  // the other outputs: 111 alone, one wavefront each
+      const int i = 4 * b + wave;
+      if (i >= A.n_diff) return;
+      const int t = A.diff_ob[i], p = L.ob_p[t], qo = L.ob_q[t];
+      const double val = f111(p, qo);
+      if (lane == 0) put(t, p, qo, val);
+      return;
+    }
   }
   // E0: k_e0_final's sum, and its share of the series accumulator
   if (A.mask & (T110 | T220)) {
@@ -2340,9 +2401,26 @@ void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallA
   const int ne0 = (A.mask & (T110 | T220)) ? L.nblocks * A.nsplit + 1 : 0;
   const int na = L.nccol * (A.prepL ? 2 : 1) + (L.n122_items + 3) / 4 + ne0;
   const size_t lds = std::max(pandya_lds_bytes(L), 256 * sizeof(double));
-  hipLaunchKernelGGL(k_small_a, dim3(na, nact), dim3(256), lds, s, Ld, A);
+  if (A.w122) {
+    if (A.prepL) launch_pandya(s, L, A.Lop, A.ccL, A.act, nact);
+    launch_pandya(s, L, A.Rop, A.ccR, A.act, nact);
+    launch_122(s, L, A.Lop, A.Rop, A.RES, A.hres, A.act, nact, A.w122);
+    if (ne0)
+      hipLaunchKernelGGL(k_e0_partial, dim3(ne0, nact), dim3(256), 0, s, L, A.Lop, A.Rop, A.hL, A.hR, A.partials, A.act,
+                         A.nsplit);
+  } else {
+    hipLaunchKernelGGL(k_small_a, dim3(na, nact), dim3(256), lds, s, Ld, A);
+  }
   if (A.split) hipLaunchKernelGGL(k_small_b<true>, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
   else hipLaunchKernelGGL(k_small_b<false>, dim3(A.n_pp + A.n_ph, nact), dim3(256), 0, s, Ld, A);
-  hipLaunchKernelGGL(k_small_c, dim3(A.n16 + L.nsame + (A.n_diff + 3) / 4 + 1, nact), dim3(256), 0, s, Ld, A);
+  if (A.T) {
+    const int nob = (L.nsame * L.ob_nchunk + 7) & ~7;  // (a multiple of 8: the terms' XCDs)
+    const int nt = 8 * L.xs_terms.len + (int)((L.nphtwo + 255) / 256);
+    hipLaunchKernelGGL(k_small_t, dim3(nob + nt, nact), dim3(256), 0, s, Ld, A, nob);
+    launch_ph_apply(s, L, A.T, A.RES, A.act, nact);
+    hipLaunchKernelGGL(k_small_c<false>, dim3(A.ntile + (L.nob + 3) / 4 + 1, nact), dim3(256), 0, s, Ld, A);
+  } else {
+    hipLaunchKernelGGL(k_small_c<true>, dim3(A.ntile + L.nsame + (A.n_diff + 3) / 4 + 1, nact), dim3(256), 0, s, Ld, A);
+  }
 }
 }  // namespace imsrg
