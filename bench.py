@@ -230,7 +230,7 @@ def basis_tag(basis):
 
 # kernel class -> kernel symbol of the FP64 path (rocprofv3 names)
 KERNEL_NAME = {
-    "gemm_pphh": "k_seg_gemm<false, 0, 0>", "gemm_ph": "k_seg_gemm<true, 0, 1>", "pandya": "k_pandya(",
+    "gemm_pphh": "k_wave_gemm<false, true>", "gemm_ph": "k_wave_gemm<true, false>", "pandya": "k_pandya(",
     "k122": "k_122s(", "ph_terms": "k_ph_terms(", "ph_apply": "k_ph_apply(", "sym_mirror": "k_sym_mirror(",
     "onebody": "k_ob_partial(",
     # int8 products and slicing, five slices (int8x5) and four (int8x4)
