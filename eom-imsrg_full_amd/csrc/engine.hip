@@ -85,7 +85,7 @@ static XcdSplit make_split(const std::vector<double> &w) {
   return x;
 }
 
-// Upper-triangle 64x64 tile schedule (tm <= tn) of one segmented-GEMM launch.
+// Upper-triangle tile schedule (TM x TN tiles, tm <= tn) of one segmented-GEMM launch.
 // Workgroup i is dispatched to XCD i % 8, so problems are spread over the 8
 // XCDs by flop weight (heaviest first onto the least-loaded XCD): every tile
 // of one channel block then runs on one XCD and shares its L2, and each XCD's

@@ -846,7 +846,7 @@ struct PhSeg {
 //      entries that pass the reference's |W| > 1e-6 test go weighted to LDS,
 //      slots with no entry left are dropped;
 //   3. the slots are summed into the outputs (Recouple).
-// What bounds it: the entries' reads (W is 1 GB at 90 orbits, rank 4) and the
+// What bounds it: the entries' reads (W is two products of 0.85 GB at 90 orbits, rank 2) and the
 // index arithmetic around them.  One wavefront per quadruple with a lane per
 // slot read a 9j cache line per (slot, output): 7.7 ms there (2.6 M
 // quadruples, 256 M slots, 3 G slot-outputs); this form 2.8 ms, 5.3 before

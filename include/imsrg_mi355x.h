@@ -90,7 +90,7 @@ int64_t imsrg_ctx_neq(imsrg_ctx ctx);
  * device bytes per operator, vsize, ccsize, cwsize, flop_pphh, flop_ph
  * (as doubles: algorithmic GEMM flop per commutator), ph recoupling J' terms,
  * upper-triangle two-body elements, FP64 tile shapes chosen by the autotuner
- * (4*(pp+1) + (ph+1), shapes -1 untuned, 0 64x64, 1 128x64) */
+ * (4*(pp+1) + (ph+1), shapes -1 untuned, 0 wavefront tiles, 1 128x64 workgroup tiles) */
 int imsrg_ctx_info(imsrg_ctx ctx, double *info16);
 int imsrg_ctx_set_precision(imsrg_ctx ctx, int prec);
 int imsrg_ctx_synchronize(imsrg_ctx ctx);
@@ -100,8 +100,9 @@ int imsrg_ctx_synchronize(imsrg_ctx ctx);
  * precision) into a hipGraph and replayed.  Off while profiling is on. */
 int imsrg_ctx_set_graphs(imsrg_ctx ctx, int enable);
 /* FP64 tile shapes the autotuner chose on the context's first FP64 commutator
- * (-1 not yet, 0 64x64, 1 128x64) and the four timings (ms: pp/hh 64x64,
- * pp/hh 128x64, Pandya product 64x64, 128x64) */
+ * (-1 not yet or a basis below the tuner's size, 0 32x32 wavefront tiles, 1
+ * 128x64 workgroup tiles) and the four timings (ms: pp/hh shape 0, pp/hh 1,
+ * Pandya product 0, 1) */
 int imsrg_ctx_tuning(imsrg_ctx ctx, int *shape_pp, int *shape_ph, float *ms4);
 /* fix the FP64 tile shapes (0 or 1 each), or -1 to tune again on the next commutator */
 int imsrg_ctx_set_tile_shapes(imsrg_ctx ctx, int shape_pp, int shape_ph);
