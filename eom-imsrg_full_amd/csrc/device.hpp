@@ -315,6 +315,14 @@ struct GateArgs {
   int seq;           // this gate's number: live[k] = seq << 1 | goes on
   int *live;         // host memory, one entry per position
 };
+// a series gate not yet made: its table, and the partial sums of the norm it tests
+struct PendingGate {
+  int *act;
+  const double *npart;
+  int n, na;         // partial sums per instance; positions
+  double *scal;
+  GateArgs G;
+};
 void launch_series_gate(hipStream_t s, int *act, int nact, double *scal, const GateArgs &G);
 // launch_norm_from_parts (n partials per instance) and the gate after it in one launch
 void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
@@ -348,6 +356,7 @@ struct SmallArgs {
   const int *diff_ob;       // one-body outputs whose orbits differ in (l, j, tz)
   const PhRow *phrow;
   const int *act;
+  PendingGate gate;         // of the commutator before, to be made by the first launch (act null: none)
 };
 void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallArgs A, int nact);
 

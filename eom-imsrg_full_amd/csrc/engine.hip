@@ -1382,7 +1382,7 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
 // The form of a commutator (launch_small; all forms give the same bits).  Per
 // commutator of a BCH series, in us, separate kernels on two streams / merged
 // (five launches) / fused (three), by two-body elements times instances:
-//   emax 4 (7.1e4)      74 / 44 / 42     4 x emax 4 (2.9e5)  103 / 80 / 80
+//   emax 4 (7.1e4)      74 / 44 / 39     4 x emax 4 (2.9e5)  103 / 80 / 80
 //   emax 5 (2.9e5)     103 / 61 / 67     emax 6 (9.6e5)      142 / 101 / 125
 //   4 x emax 5 (1.1e6) 145 / 139         emax 7 (2.8e6)      248 / 207
 //   4 x emax 6 (3.8e6) 321 / 294         16 x emax 5 (4.6e6) 407 / 428
@@ -1405,6 +1405,19 @@ static CommForm comm_form(const imsrg_ctx_s *c, unsigned mask, int cc_ready, int
   if (c->small && n <= kFusedElems) return kFused;
   return n <= kMergedElems || na <= 2 ? kMerged : kSeparate;
 }
+
+// The pending gate in a launch of its own.
+static void flush_gate(imsrg_ctx_s *c) {
+  const PendingGate &p = c->gate_pend;
+  if (p.act) launch_norm_gate(c->stream, p.npart, p.n, p.act, p.na, p.scal, p.G);
+  c->gate_pend.act = nullptr;
+}
+// Whether a series gate waits for the next commutator's first launch, which
+// then sums the norm in every workgroup.  That saves a launch of 4-6 us where
+// the sum is over a few hundred numbers: fused, emax 4, 41.6 -> 39.2 us a
+// commutator.  Merged it is over thousands and there are more workgroups to make
+// it: emax 6 100.8 -> 102.6 us, emax 7 205 -> 215, so the gate keeps its launch.
+static bool defer_gate(const imsrg_ctx_s *c, CommForm form, int na) { return !c->graphs && form == kFused; }
 
 // Tile-shape autotuner: on the first FP64 commutator of a context, each 222
 // GEMM is timed (HIP events, best of 3) in both FP64 tile shapes on the
@@ -1525,7 +1538,9 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     c->fork_mark = nullptr;
     return 0;
   }
-  if (const CommForm form = comm_form(c, mask, cc_ready, na); form != kSeparate) {
+  const CommForm form = comm_form(c, mask, cc_ready, na);
+  if (form == kSeparate) flush_gate(c);
+  if (form != kSeparate) {
     SmallArgs A{};
     A.Lop = L->d; A.Rop = R->d; A.RES = RES->d; A.acc = epi.acc;
     A.ccL = c->cc[0]; A.ccR = c->cc[1]; A.Z = c->wph; A.wpp = c->wpp; A.partials = c->partials;
@@ -1545,10 +1560,15 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     // emax 4 177 / 196, but emax 7 215 / 207, emax 6 110 / 101
     A.w122 = form == kMerged && D.vsize * na > (na == 1 ? 3000000 : 1000000) ? c->w122 : nullptr;
     A.diff_ob = c->diff_ob; A.phrow = c->phrow; A.act = ad;
+    if (c->gate_pend.act && (c->gate_pend.act != ad || A.w122)) flush_gate(c);
+    A.gate = c->gate_pend;
+    c->gate_pend.act = nullptr;
     launch_small(s, D, c->dl_d, A, na);
     c->fork_mark = nullptr;
-    if (epi.gate_act) launch_norm_gate(s, c->npart, A.ntile + D.nob, epi.gate_act, na, c->scal, epi.gate);
-    else if (epi.norm) launch_norm_from_parts(s, A.ntile + D.nob, c->npart, c->scal, ad, na);
+    if (epi.gate_act) {
+      c->gate_pend = PendingGate{epi.gate_act, c->npart, A.ntile + D.nob, na, c->scal, epi.gate};
+      if (!defer_gate(c, form, na)) flush_gate(c);
+    } else if (epi.norm) launch_norm_from_parts(s, A.ntile + D.nob, c->npart, c->scal, ad, na);
     HIPCHK(hipGetLastError());
     return 0;
   }
@@ -1830,13 +1850,16 @@ static ActSet series_begin(imsrg_ctx_s *c, int slot, const ActSet &a, imsrg_op_s
 }
 // The operand L = Omega of every nested commutator of a series, prepared once:
 // its Pandya matrices and, with int8 slices, the slices of its V rows and of
-// those matrices.
-static void prep_L(imsrg_ctx_s *c, imsrg_op_s *G, const ActSet &set) {
+// those matrices.  Returns the cc_ready bits of the first commutator: in the
+// forms of few launches its first launch makes the matrices.
+static int prep_L(imsrg_ctx_s *c, imsrg_op_s *G, const ActSet &set) {
+  if (!c->graphs && comm_form(c, IMSRG_TALL, 0, set.g()) != kSeparate) return 0;
   launch_pandya(c->stream, c->dl, G->d, c->cc[0], set.d, set.n());
   if (const int ns = i8_planes(c->prec)) {
     launch_slice_v(c->stream, c->dl, c->i8, ns, G->d, c->i8v[0], c->i8vs[0], set.d, set.n());
     launch_slice_cc(c->stream, c->dl, c->i8, ns, c->cc[0], c->i8pm, c->i8c[0], c->i8cs[0], set.d, set.n());
   }
+  return kLPrepped;
 }
 // The series gate after nested commutator n: the test on the device, its live
 // flags into ring slot n % kGateRing under the gate's sequence number.
@@ -1856,6 +1879,7 @@ static hipEvent_t gate_mark(imsrg_ctx_s *c, int n, const ActSet &set) {
 // pinned ring as the kernel writes them (an event costs a record and a wake-up
 // per commutator); live[k] = 1 for positions that go on.
 static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, int seq, std::vector<int> &live, int &nlive) {
+  if (c->gate_pend.act && c->gate_pend.G.seq == seq) flush_gate(c);
   const volatile int *f = c->live_h + (size_t)(n % imsrg_ctx_s::kGateRing) * c->nbatch;
   live.assign(set.n(), 0);
   nlive = 0;
@@ -1866,6 +1890,13 @@ static int series_live(imsrg_ctx_s *c, const ActSet &set, int n, int seq, std::v
   }
   return 0;
 }
+
+// A series leaves no gate behind, however it ends: one still pending belongs to
+// a commutator that every instance skips.
+struct SeriesEnd {
+  imsrg_ctx_s *c;
+  ~SeriesEnd() { c->gate_pend.act = nullptr; }
+};
 
 // BCH_EXPAND (IMSRG_MAGNUS.f90:149-234) on the instances of `a`.  Every
 // instance keeps its own truncation: after each nested commutator the gate
@@ -1886,7 +1917,8 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
   // AD_1 = H itself; [G, X] with G anti-hermitian keeps the hermiticity of X
   imsrg_op_s *AD = H, *INT2 = T[0];
   T[0]->herm = T[1]->herm = H->herm;
-  prep_L(c, G, cur);
+  const SeriesEnd end{c};
+  int prepped = prep_L(c, G, cur);
   std::vector<int> live(a.n(), 1);  // positions in the series for nested commutator iw
   int nlive = a.n(), seq = 0;
   hipEvent_t mark = nullptr;
@@ -1902,7 +1934,8 @@ static int bch_impl(imsrg_ctx_s *c, imsrg_op_s *HS, imsrg_op_s *G, imsrg_op_s *H
     epi.gate = gate_args(c, iw, 0, coef, -1, 0);
     // nothing was enqueued since the last gate: the second stream can fork from its event
     c->fork_mark = mark;
-    int rc = comm_impl(c, G, AD, INT2, IMSRG_TALL, kLPrepped, cur, epi);
+    int rc = comm_impl(c, G, AD, INT2, IMSRG_TALL, prepped, cur, epi);
+    prepped = kLPrepped;
     mark = gate_mark(c, iw, cur);
     if (!rc && iw > 2) rc = series_live(c, cur, iw - 1, seq, live, nlive);
     seq = epi.gate.seq;
@@ -1972,7 +2005,8 @@ static int magexp_impl(imsrg_ctx_s *c, imsrg_op_s *DG, imsrg_op_s *G, const ActS
   const GateArgs g = gate_args(c, 1, 1, 0.0, -1, 0);
   PROF(c, IMSRG_PROF_NORM,
        launch_magnus_gate(c->stream, c->dl, DG->d, G->d, c->partials, c->nbatch, c->act_d[2], set.g(), c->scal, g));
-  prep_L(c, G, set);
+  const SeriesEnd end{c};
+  int prepped = prep_L(c, G, set);
   std::vector<int> live;
   int nlive = 0, seq = g.seq, rc = 0;
   hipEvent_t mark = nullptr;  // prep_L follows the first gate on the stream
@@ -1989,7 +2023,8 @@ static int magexp_impl(imsrg_ctx_s *c, imsrg_op_s *DG, imsrg_op_s *G, const ActS
       epi.gate = gate_args(c, i, 1, std::fabs(cof[i - 1]), i - 1, i - q);
     }
     c->fork_mark = mark;
-    rc = comm_impl(c, G, cur, oth, IMSRG_TALL & ~(T110 | T220), kLPrepped, set, epi);
+    rc = comm_impl(c, G, cur, oth, IMSRG_TALL & ~(T110 | T220), prepped, set, epi);
+    prepped = kLPrepped;
     mark = i < 7 ? gate_mark(c, i, set) : nullptr;
     if (!rc) rc = series_live(c, set, i - 1, seq, live, nlive);
     seq = epi.gate.seq;
@@ -2290,11 +2325,12 @@ static int nested_chain(imsrg_ctx_s *c, imsrg_op_s *Om, imsrg_op_s *X0, int K, u
                         std::vector<imsrg_op_s *> &A) {
   const ActSet all = all_set(c);
   op_copy(X0, A[0], all);
-  prep_L(c, Om, all);
+  int prepped = prep_L(c, Om, all);
   for (int k = 1; k <= K; k++) {
     A[k]->herm = -Om->herm * A[k - 1]->herm;
-    int rc = comm_impl(c, Om, A[k - 1], A[k], mask, kLPrepped, all);
+    int rc = comm_impl(c, Om, A[k - 1], A[k], mask, prepped, all);
     if (rc) return rc;
+    prepped = kLPrepped;
   }
   return 0;
 }

@@ -46,6 +46,8 @@ struct imsrg_ctx_s {
   // the next commutator's fork waits on instead of recording ev_fork; cleared
   // by that commutator
   hipEvent_t fork_mark = nullptr;
+  // the gate of a series' last enqueued commutator, left to the next one's first launch (act null: none)
+  PendingGate gate_pend{};
   bool dual = true;        // use stream2 (imsrg_ctx_set_concurrency)
   // BCH / Magnus series: the gate kernel after nested commutator n writes one
   // live flag per series position, under the gate's sequence number, into ring

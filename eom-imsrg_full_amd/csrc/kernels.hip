@@ -2024,18 +2024,18 @@ void launch_gather_e0(hipStream_t s, const double *op, long long stride, double 
 // ||ad^n|| is scalar slot 0.  live[k] (host memory) gets 1 or 0 per position.
 // live[k] carries the gate's sequence number above its flag, so that the host
 // can wait for this gate's answer by reading the flag itself.
+__device__ __forceinline__ bool gate_test(const double *sc, double norm, const GateArgs &G) {
+  if (G.mode == 0) return !(norm * G.coef < G.conv);
+  const double full = sc[kFullSlot], adv = G.test == G.store ? norm * G.coef : sc[kAdvSlot + G.test];
+  return !(full < G.tiny) && !(fabs(adv / full) < G.conv);
+}
 __device__ __forceinline__ void gate_position(int *act, int k, double *scal, const GateArgs &G) {
   const int inst = act[k];
   int on = 0;
   if (inst >= 0) {
     double *sc = scal + (long long)inst * kScal;
-    if (G.mode == 0) {
-      on = !(sc[0] * G.coef < G.conv);
-    } else {
-      if (G.store >= 0) sc[kAdvSlot + G.store] = sc[0] * G.coef;
-      const double full = sc[kFullSlot];
-      on = !(full < G.tiny) && !(fabs(sc[kAdvSlot + G.test] / full) < G.conv);
-    }
+    on = gate_test(sc, sc[0], G);
+    if (G.mode && G.store >= 0) sc[kAdvSlot + G.store] = sc[0] * G.coef;
     if (!on) act[k] = -1;
   }
   G.live[k] = (G.seq << 1) | on;
@@ -2061,6 +2061,20 @@ __global__ __launch_bounds__(256) void k_norm_gate(const double *npart, int n, i
     if (threadIdx.x == 0) scal[(long long)inst * kScal] = sqrt(s);
   }
   if (threadIdx.x == 0) gate_position(act, blockIdx.y, scal, G);
+}
+// The same at the start of the next commutator's first launch: every workgroup
+// of a position sums the norm and makes the test for itself, the first one
+// also writes it down (a workgroup that already reads -1 leaves as well).
+// Returns whether the position goes on.
+__device__ __forceinline__ bool gate_here(const PendingGate &P, long long inst, double *sh) {
+  const double norm = sqrt(sum256(P.npart + inst * P.n, P.n, sh));
+  double *sc = P.scal + inst * kScal;
+  const bool on = gate_test(sc, norm, P.G);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[0] = norm;
+    gate_position(P.act, blockIdx.y, P.scal, P.G);
+  }
+  return on;
 }
 void launch_norm_gate(hipStream_t s, const double *npart, int n, int *act, int nact, double *scal,
                       const GateArgs &G) {
@@ -2099,7 +2113,8 @@ void launch_magnus_gate(hipStream_t s, const DevLayout &L, const double *DG, con
 // that leaves the chip idle.  The same work in three launches (fused) or five
 // (merged): every kernel below is a list of workgroups of different kinds that
 // only need what the launch before left behind.
-//   k_small_a  Pandya columns, 122 sets (weights formed in place), E0 partials
+//   k_small_a  Pandya columns, 122 sets (weights formed in place), E0 partials;
+//              before them the series gate of the commutator before, where it was left
 //   k_small_b  the pp/hh product (onto the 122 rows) and the Pandya product
 //   fused: k_small_c<true>, per 16 x 16 tile pair the ph terms and their
 //              6j-weighted sums straight from Z, then symmetrise + mirror;
@@ -2113,7 +2128,11 @@ __global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ L
   extern __shared__ double lds[];
   const DevLayout &L = *Lp;
   const long long inst = inst_id(A.act);
-  if (inst < 0) return;
+  if (inst < 0) {
+    if (A.gate.act && blockIdx.x == 0 && threadIdx.x == 0) gate_position(A.gate.act, blockIdx.y, A.gate.scal, A.gate.G);
+    return;
+  }
+  if (A.gate.act && !gate_here(A.gate, inst, lds)) return;
   const long long o = inst * L.op_size;
   const double *Lop = A.Lop + o, *Rop = A.Rop + o;
   int b = blockIdx.x;
