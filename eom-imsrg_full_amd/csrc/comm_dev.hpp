@@ -184,8 +184,8 @@ __device__ __forceinline__ double ph_coef(const double *S6, int m, int n, int n1
 // as long, which is the time in small bases and the tail of the schedule in
 // large ones.  Measured alone, in us (64 x 64 tiles of LDS slabs, the form
 // before / a quadrant a wavefront / four wavefronts a tile): pp/hh emax 4 17 / - / 7,
-// emax 6 43 / 25 / 20, 16 x emax 6 233 / 263 / 240, emax 7 73 / 55 / 47, emax 8
-// 168 / 162 / 149 (36 TF/s); Pandya product emax 4 9.6 / 7.5 / 5.0, emax 6
+// emax 6 43 / 25 / 20, 16 x emax 6 233 / 263 / 234, emax 7 73 / 55 / 48, emax 8
+// 168 / 162 / 145 (37 TF/s); Pandya product emax 4 9.6 / 7.5 / 5.0, emax 6
 // 20.5 / 15.9 / 18.0, 16 x emax 6 202 / 162 / 221, emax 8 177 / 147 (44 TF/s) / 165.
 // Hence pp/hh always shares, the Pandya product while the basis' two-body part
 // holds at most 3e5 elements (emax 5); the choice is the basis', so a batch has

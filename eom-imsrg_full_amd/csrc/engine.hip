@@ -1386,7 +1386,7 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
 //   emax 5 (2.9e5)     103 / 61 / 67     emax 6 (9.6e5)      142 / 101 / 125
 //   4 x emax 5 (1.1e6) 145 / 139         emax 7 (2.8e6)      248 / 207
 //   4 x emax 6 (3.8e6) 321 / 294         16 x emax 5 (4.6e6) 407 / 428
-//   emax 8 (7.2e6)     637 / 613         2 x emax 8 (1.4e7)  1100 / 1088
+//   emax 8 (7.2e6)     637 / 601         2 x emax 8 (1.4e7)  1100 / 1088
 //   16 x emax 6 (1.5e7) 1114 / 1133
 // Fused pays while launches are what a commutator costs; past 2e5 the ph sums
 // straight from Z, made anew for every J, cost more than a launch for the J'

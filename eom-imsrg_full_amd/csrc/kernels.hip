@@ -747,8 +747,11 @@ __device__ __forceinline__ void wave_tile_z(const SegProb *__restrict__ probs, c
             acc[1][0][v], acc[1][1][v], sigma);
 }
 // Either product on a 32 x 32 tile list, four wavefronts to a tile (row-major A:
-// element (ti, tj, v) at row 16 ti + lane/16 + 4 v).  The partial sums lie in LDS as [wavefront][row][column]; thread t adds and writes the 2x2
-// block (t/16, t%16).
+// element (ti, tj, v) at row 16 ti + lane/16 + 4 v).  The partial sums lie in LDS
+// as [wavefront][row][column]; thread t adds and writes the 2x2 block (t/16, t%16).
+// The old C values are read after the products, under the reduction: read before
+// them they went to scratch memory, so the K loop waited for them (a commutator
+// at emax 8 610 -> 601 us, pp/hh of 16 x emax 6 240 -> 234).
 template <bool Z>
 __device__ __forceinline__ void split_tile(const SegProb *__restrict__ probs, const int4 tl,
                                            const double *__restrict__ X0, const double *__restrict__ X1, double g0,
@@ -795,14 +798,6 @@ __device__ __forceinline__ void split_tile(const SegProb *__restrict__ probs, co
     z_block(C + p.c_off, M, row >> 1, col >> 1, z[0][0], z[0][1], z[1][0], z[1][1], sigma);
     return;
   }
-  double old[2][2];
-  if (C) {
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        old[i][j] = C[p.c_off + (row + i < M && col + j < M && row + i <= col + j ? (long long)(row + i) * M + col + j : 0)];
-  }
   wave_segments<false, 4>(p, 0, p.nmid, X0, X1, g0, g1, m0, n0, wave, acc);
   if (W) {
     reduce();
@@ -814,6 +809,12 @@ __device__ __forceinline__ void split_tile(const SegProb *__restrict__ probs, co
   }
   wave_segments<false, 4>(p, p.nmid, p.nseg, X0, X1, g0, g1, m0, n0, wave, acc);
   if (C) {
+    double old[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        old[i][j] = C[p.c_off + (row + i < M && col + j < M && row + i <= col + j ? (long long)(row + i) * M + col + j : 0)];
     reduce();
 #pragma unroll
     for (int i = 0; i < 2; i++)
