@@ -423,8 +423,11 @@ __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists
 // thread per output with a pair lookup, an F entry and a 6j per term took
 // 0.95 + 3.1 ms for the two commutators at 90 orbits, rank 4 (20 M outputs);
 // this kernel 1.0 ms with a partner list per row, 0.66 ms with one per
-// group (and a block on one XCD), k_t_lists 0.09 ms.
-__global__ __launch_bounds__(kT1Threads, 6) void k_t_1body(DevLayout L, DevTensor T, TLists W,
+// group (and a block on one XCD), 0.58 without spills: asked for six wavefronts a
+// SIMD the compiler stores 44 bytes a lane, asked for four it needs 80 registers
+// and six fit all the same.  The next batch of either list read ahead: 0.73.
+// k_t_lists 0.09 ms.
+__global__ __launch_bounds__(kT1Threads, 4) void k_t_1body(DevLayout L, DevTensor T, TLists W,
                                                         const double *__restrict__ GV, const double *__restrict__ RV,
                                                         double *__restrict__ OV, int add) {
   extern __shared__ double rows[];
