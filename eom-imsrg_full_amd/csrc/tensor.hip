@@ -743,10 +743,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
       }
       __syncthreads();
       const int nb = min(nseg, kPhB);
+      if (nb == 0) break;  // the scan found no further slot: there is none to read below
       {
         int ix[4], jx_[4];
         double w[4];
-        auto slot = [&](int k) -> const PanSeg & { return seg[min(8 * k + (lane >> 3), max(nb - 1, 0))]; };
+        auto slot = [&](int k) -> const PanSeg & { return seg[min(8 * k + (lane >> 3), nb - 1)]; };
 #pragma unroll
         for (int k = 0; k < 4; k++) {
           const unsigned gc = slot(k).code;
@@ -979,6 +980,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
       __syncthreads();
       // 2: the entries of the first kPhB
       const int nb = min(nseg, kPhB);
+      if (nb == 0) break;  // the scan found no further slot: there is none to read below
       int count = 0;
       {
         double w[4];
