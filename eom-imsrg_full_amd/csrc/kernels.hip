@@ -2037,7 +2037,7 @@ __device__ __forceinline__ void gate_position(int *act, int k, double *scal, con
     double *sc = scal + (long long)inst * kScal;
     on = gate_test(sc, sc[0], G);
     if (G.mode && G.store >= 0) sc[kAdvSlot + G.store] = sc[0] * G.coef;
-    if (!on) act[k] = -1;
+    if (!on) __hip_atomic_store(act + k, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (gate_inst reads it)
   }
   G.live[k] = (G.seq << 1) | on;
   __threadfence_system();
@@ -2065,8 +2065,18 @@ __global__ __launch_bounds__(256) void k_norm_gate(const double *npart, int n, i
 }
 // The same at the start of the next commutator's first launch: every workgroup
 // of a position sums the norm and makes the test for itself, the first one
-// also writes it down (a workgroup that already reads -1 leaves as well).
-// Returns whether the position goes on.
+// also writes it down.  Returns whether the position goes on.
+// gate_inst: the instance, read once for all wavefronts of the workgroup, since
+// the first workgroup may write the table at any moment: one that starts late
+// reads -1 and leaves, all of it.
+__device__ __forceinline__ long long gate_inst(const PendingGate &P, double *sh) {
+  int *const word = reinterpret_cast<int *>(sh);
+  if (threadIdx.x == 0) *word = __hip_atomic_load(P.act + blockIdx.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int inst = *word;
+  __syncthreads();
+  return inst;
+}
 __device__ __forceinline__ bool gate_here(const PendingGate &P, long long inst, double *sh) {
   const double norm = sqrt(sum256(P.npart + inst * P.n, P.n, sh));
   double *sc = P.scal + inst * kScal;
@@ -2128,7 +2138,7 @@ void launch_magnus_gate(hipStream_t s, const DevLayout &L, const double *DG, con
 __global__ __launch_bounds__(256) void k_small_a(const DevLayout *__restrict__ Lp, SmallArgs A) {
   extern __shared__ double lds[];
   const DevLayout &L = *Lp;
-  const long long inst = inst_id(A.act);
+  const long long inst = A.gate.act ? gate_inst(A.gate, lds) : inst_id(A.act);
   if (inst < 0) {
     if (A.gate.act && blockIdx.x == 0 && threadIdx.x == 0) gate_position(A.gate.act, blockIdx.y, A.gate.scal, A.gate.G);
     return;
