@@ -33,7 +33,12 @@ __global__ void k_hf_init(DevLayout L, const double *__restrict__ op, double *__
 // workgroup of the next k_hf_gamma for itself, and noted by the first one.
 __device__ __forceinline__ bool hf_go_on(const DevLayout &L, const double *__restrict__ cpart, double *__restrict__ crit,
                                          double *__restrict__ state, double conv, bool first, double *sh) {
-  if (state[0] != 0.0) return false;
+  // the flag is read once for all wavefronts: the first workgroup may set it meanwhile
+  if (threadIdx.x == 0) sh[0] = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const bool over = sh[0] != 0.0;
+  __syncthreads();
+  if (over) return false;
   if (first) return true;
   double s = 0.0;
   for (int k0 = 0; k0 < L.ngrp; k0 += 256) {  // the changes side by side, summed one after another
@@ -48,7 +53,7 @@ __device__ __forceinline__ bool hf_go_on(const DevLayout &L, const double *__res
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     crit[0] = s;
     state[1] += 1.0;
-    if (!on) state[0] = 1.0;
+    if (!on) __hip_atomic_store(state, 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   return on;
 }

@@ -23,8 +23,8 @@
 #define __HIP_MEMORY_SCOPE_AGENT 0
 #undef __hip_atomic_store
 #undef __hip_atomic_load
-#define __hip_atomic_store(p, v, order, scope) __atomic_store_n(p, v, order)
-#define __hip_atomic_load(p, order, scope) __atomic_load_n(p, order)
+#define __hip_atomic_store(p, v, order, scope) ((void)(*(p) = (v)))
+#define __hip_atomic_load(p, order, scope) (*(p))
 #define __threadfence_system() ((void)0)
 #define __threadfence() ((void)0)
 

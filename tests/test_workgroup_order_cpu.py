@@ -21,3 +21,15 @@ print(n, m, HS.download().tobytes().hex(), DG.download().tobytes().hex())
 @pytest.mark.parametrize("wave", [0, 1, 3])
 def test_series_gates(wave):
     assert run(SERIES, IMSRG_EMU_SPLIT=wave) == run(SERIES)
+
+
+HF = """
+H = E.Context(Basis.ho(2, 1)).op(1, synthetic_hamiltonian(Basis.ho(2, 1), 0))
+D, e, n = H.hartree_fock()
+print(e, n, np.asarray(D).tobytes().hex(), H.download().tobytes().hex())
+"""
+
+
+@pytest.mark.parametrize("wave", [0, 1, 3])
+def test_hartree_fock_convergence(wave):
+    assert run(HF, IMSRG_EMU_SPLIT=wave) == run(HF)
