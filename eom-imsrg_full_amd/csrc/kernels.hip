@@ -909,11 +909,6 @@ size_t pandya_lds_bytes(const DevLayout &L) {
   return sizeof(double) * L.nhalf * L.nhalf * L.nJ + sizeof(long long) * L.nblocks +
          sizeof(int) * (L.nblocks + L.nsp) + sizeof(short) * 2 * L.nJ * L.nsp;
 }
-// lets k_pandya take more than 64 KiB of dynamic LDS (up to the device's per-workgroup limit)
-hipError_t pandya_allow_lds(size_t bytes) {
-  return hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pandya), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)bytes);
-}
 void launch_pandya(hipStream_t s, const DevLayout &L, const double *op, double *cc, const int *act, int nact) {
   if (L.nccol <= 0 || nact <= 0) return;
   hipLaunchKernelGGL(k_pandya, dim3(L.nccol, nact), dim3(256), pandya_lds_bytes(L), s, L, op, cc, act);
@@ -2424,6 +2419,14 @@ __global__ __launch_bounds__(256) void k_small_c(const DevLayout *__restrict__ L
     }
   }
   if (tid == 0 && acc) acc[0] = acc[0] + A.coef * RES[0];
+}
+// lets the kernels that stage Pandya tables take more than 64 KiB of dynamic LDS
+hipError_t pandya_allow_lds(size_t bytes) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_pandya),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  return e != hipSuccess ? e
+                         : hipFuncSetAttribute(reinterpret_cast<const void *>(&k_small_a),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 void launch_small(hipStream_t s, const DevLayout &L, const DevLayout *Ld, SmallArgs A, int nact) {
   if (nact <= 0) return;

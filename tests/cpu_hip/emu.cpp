@@ -8,6 +8,7 @@
 // compiled with bounds checks (SIGILL).  A launch with more dynamic LDS than
 // 64 KiB, or than hipFuncSetAttribute allowed it, fails.
 //
+// IMSRG_EMU_CHECK: launches are checked, kernels not run.
 // IMSRG_EMU_SPLIT=w: wavefront w of workgroup 1 of every launch starts before
 // workgroup 0, which then runs whole before the rest of workgroup 1 (LDS kept
 // apart), as two workgroups on two compute units may.
@@ -195,6 +196,7 @@ void run(const void *kernel, dim3 g, dim3 b, size_t lds, const std::function<voi
     last = hipErrorInvalidValue;
     return;
   }
+  if (std::getenv("IMSRG_EMU_CHECK")) return;
   if (!stacks) stacks = (char *)mmap(nullptr, kStack * kMaxItems, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
   body = &f;
   bdim = Index{b.x, b.y, b.z};

@@ -1,0 +1,19 @@
+"""Dynamic LDS past 64 KiB has to be allowed for a kernel before its launch; on
+the host such a launch fails otherwise (the kernels themselves are not run
+here).  Bases of many orbits of which a few have 2j = 29 stage more than that for
+their Pandya columns, though their two-body part is that of a merged
+commutator."""
+from cpu_library import run
+
+HIGH_J = """
+low = [(0, 1), (1, 1), (1, 3), (2, 3), (2, 5), (3, 5), (3, 7)]
+def basis(nj):
+    orb = [o for tz in (-1, 1) for o in [(k, l, j, tz) for l, j in low for k in range(5)] + [(k, 14, 29, tz) for k in range(nj)]]
+    return Basis.from_orbits(orb, [int(o[0] == 0 and o[1] == 0) for o in orb])
+B = basis(3)
+ctx = E.Context(B)
+"""
+
+
+def test_high_j_commutator():
+    run(HIGH_J + "ctx.commutator(ctx.op(-1), ctx.op(1))", IMSRG_EMU_CHECK=1)
