@@ -384,7 +384,8 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
       return fail(IMSRG_EINVAL, "basis too large: the Pandya kernel stages " + std::to_string(need) +
                                     " bytes of tables per workgroup (device limit " + std::to_string(lds_max) + ")");
     }
-    if (need > 65536 && (pandya_allow_lds(need) != hipSuccess || adjoint_allow_lds(need) != hipSuccess)) {
+    // (the limit is the kernel's, for every context of the process: the device's, not this basis')
+    if (need > 65536 && (pandya_allow_lds(lds_max) != hipSuccess || adjoint_allow_lds(lds_max) != hipSuccess)) {
       imsrg_ctx_destroy(c);
       return fail(IMSRG_EDEVICE, "the Pandya kernel cannot take " + std::to_string(need) + " bytes of LDS");
     }

@@ -17,3 +17,14 @@ ctx = E.Context(B)
 
 def test_high_j_commutator():
     run(HIGH_J + "ctx.commutator(ctx.op(-1), ctx.op(1))", IMSRG_EMU_CHECK=1)
+
+
+def test_second_context_keeps_the_limit():
+    """a later context of a smaller basis, still past 64 KiB, takes nothing back"""
+    run(HIGH_J + """
+B2 = basis(5)
+big = E.Context(B2)
+ctx = E.Context(B)
+big.commutator_adjoint(big.op(-1), big.op(1), 1)
+big.cross_coupled(big.op(1))
+""", IMSRG_EMU_CHECK=1)
