@@ -361,6 +361,7 @@ struct TLists {
   unsigned lds;                // of k_t_1body
 };
 constexpr int kT1Threads = 768;
+constexpr int kT1Lds = 163840;  // LDS of a workgroup at most
 
 // one wavefront per list, a lane per entry
 __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists W, const double *__restrict__ LF,
@@ -1680,7 +1681,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
         g += k;
       }
     }
-    if (lds > 163840) return fail(IMSRG_EINVAL, "tensor blocks too wide for the one-body terms' workgroups");
+    if (lds > kT1Lds) return fail(IMSRG_EINVAL, "tensor blocks too wide for the one-body terms' workgroups");
     // a block's workgroups on one XCD (workgroup i runs on XCD i % 8), whose L2
     // keeps its rows: blocks in order of size, each to the least loaded XCD
     {
@@ -1718,7 +1719,8 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
       launch_fill(c->stream, W.rw, nr, 0.0);  // the weights no list writes stay 0
       launch_fill(c->stream, W.cw, nc, 0.0);
       if (lds > 65536)
-        HIPCHK(hipFuncSetAttribute((const void *)k_t_1body, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        // (the kernel's limit in the whole process: the most any space may take, not this one's)
+        HIPCHK(hipFuncSetAttribute((const void *)k_t_1body, hipFuncAttributeMaxDynamicSharedMemorySize, kT1Lds));
     }
   }
   // products: the pp and hh ladders per tensor block (W1, W2); operand 0: G's V, 1: T's V

@@ -28,3 +28,13 @@ ctx = E.Context(B)
 big.commutator_adjoint(big.op(-1), big.op(1), 1)
 big.cross_coupled(big.op(1))
 """, IMSRG_EMU_CHECK=1)
+
+
+def test_second_tensor_space_keeps_the_limit():
+    """E1, then E2, in one context: the one-body kernel of the first still starts"""
+    run("""
+ctx = E.Context(Basis.ho(5, 1))
+E1, E2, G = ctx.tensor(2, 2), ctx.tensor(4, 0), ctx.op(-1)
+ctx.tensor_commutator(G, E1)
+ctx.tensor_commutator(G, E2)
+""", IMSRG_EMU_CHECK=1)
