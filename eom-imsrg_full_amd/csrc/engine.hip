@@ -195,10 +195,8 @@ static int op_new(imsrg_ctx_s *c, int herm, imsrg_op_s **out) {
   op->herm = herm;
   // (the FP64 products' 16-byte reads may take one element past the last block)
   const size_t bytes = sizeof(double) * (c->lay.op_size * c->nbatch + 8);
-  if (!c->op_pool.empty()) {
-    op->d = c->op_pool.back();
-    c->op_pool.pop_back();
-  } else if (dev_malloc(c, (void **)&op->d, bytes) != hipSuccess) {
+  op->d = c->op_pool.take();
+  if (!op->d && dev_malloc(c, (void **)&op->d, bytes) != hipSuccess) {
     delete op;
     return fail(IMSRG_ENOMEM, "hipMalloc operator failed");
   }
@@ -210,9 +208,7 @@ static int op_new(imsrg_ctx_s *c, int herm, imsrg_op_s **out) {
 static void op_release(imsrg_op_s *op) {
   imsrg_ctx_s *c = op->ctx;
   const size_t bytes = sizeof(double) * c->lay.op_size * c->nbatch;
-  if (c->op_pool.size() < imsrg_ctx_s::kOpPool && (c->op_pool.size() + 1) * bytes <= imsrg_ctx_s::kOpPoolBytes) {
-    c->op_pool.push_back(op->d);
-  } else {
+  if (!c->op_pool.give(op->d, bytes)) {
     (void)hipStreamSynchronize(c->stream);
     (void)hipFree(op->d);
   }
@@ -696,7 +692,6 @@ int imsrg_ctx_destroy(imsrg_ctx c) {
       (void)hipFree(t->d);
       delete t;
     }
-  for (double *p : c->op_pool) (void)hipFree(p);
   for (auto &kv : c->gexec) (void)hipGraphExecDestroy(kv.second);
   for (hipEvent_t e : c->evpool) (void)hipEventDestroy(e);
   for (void *p : c->dallocs) (void)hipFree(p);

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <utility>
@@ -33,6 +34,41 @@ inline int fail(int code, const std::string &msg) {
 
 struct imsrg_op_s;
 
+// Operator buffers a context keeps for its next operator, whose work is ordered
+// behind theirs by the context's streams: at most kMax of them and kMaxBytes.
+// They go back to the device with the context, or when an allocation fails.
+// Operators may be destroyed by another thread than the one that computes.
+struct OpPool {
+  static constexpr size_t kMax = 64, kMaxBytes = (size_t)4 << 30;
+  OpPool() = default;
+  ~OpPool() { (void)drain(); }
+  OpPool(const OpPool &) = delete;
+  OpPool &operator=(const OpPool &) = delete;
+  double *take() {
+    std::lock_guard<std::mutex> lock(mu);
+    if (v.empty()) return nullptr;
+    double *p = v.back();
+    v.pop_back();
+    return p;
+  }
+  bool give(double *p, size_t bytes) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (v.size() >= kMax || (v.size() + 1) * bytes > kMaxBytes) return false;
+    v.push_back(p);
+    return true;
+  }
+  bool drain() {  // (hipFree waits for the work that still reads a buffer)
+    std::lock_guard<std::mutex> lock(mu);
+    const bool any = !v.empty();
+    for (double *p : v) (void)hipFree(p);
+    v.clear();
+    return any;
+  }
+
+ private:
+  std::mutex mu;
+  std::vector<double *> v;
+};
 struct imsrg_ctx_s {
   Layout lay;
   DevLayout dl{};
@@ -57,12 +93,7 @@ struct imsrg_ctx_s {
   int *live_h = nullptr, *live_d = nullptr;  // host and device views, kGateRing * nbatch
   hipEvent_t ev_gate[kGateRing] = {};
   StepReport *rep_h = nullptr, *rep_d = nullptr;  // flow step reports (pinned), one per instance
-  // operator buffers given back (imsrg_op_destroy, drivers' temporaries), reused
-  // by the next op_new of this context: its work is all ordered by its streams.
-  // At most kOpPool of them and kOpPoolBytes; freed with the context, or when
-  // an allocation fails.
-  static constexpr size_t kOpPool = 64, kOpPoolBytes = (size_t)4 << 30;
-  std::vector<double *> op_pool;
+  OpPool op_pool;          // operator buffers given back (imsrg_op_destroy, drivers' temporaries)
   int rep_seq = 0;         // number of the last flow step report
   int gate_seq = 0;        // number of the last series gate (GateArgs::seq)
   bool capturing = false;  // graph capture records one stream only
@@ -193,11 +224,8 @@ int stream_to_dev(imsrg_ctx_s *c, const double *host, int64_t n, double *dev);
 // buffers goes back to the device and the call is made again
 inline hipError_t dev_malloc(imsrg_ctx_s *c, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e == hipSuccess || c->op_pool.empty()) return e;
+  if (e == hipSuccess || !c->op_pool.drain()) return e;
   (void)hipGetLastError();
-  (void)hipStreamSynchronize(c->stream);
-  for (double *q : c->op_pool) (void)hipFree(q);
-  c->op_pool.clear();
   return hipMalloc(p, bytes);
 }
 template <class T>

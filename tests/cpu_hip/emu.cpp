@@ -206,6 +206,8 @@ void run(const void *kernel, dim3 g, dim3 b, size_t lds, const std::function<voi
   const int sw = split_wave();
   Tls tls;
   dl_iterate_phdr(find_tls, &tls);
+  // (the host's own thread-local variables are there too)
+  const std::vector<char> host(tls.p, tls.p + tls.n);
   auto fresh = [&] {
     std::memset(tls.p, 0x7f, tls.n);  // what an LDS word holds before it is written: a large number
     for (int i = 0; i < nitem; i++) start(i);
@@ -238,6 +240,7 @@ void run(const void *kernel, dim3 g, dim3 b, size_t lds, const std::function<voi
         finish();
       }
     }
+  std::memcpy(tls.p, host.data(), tls.n);
 }
 }  // namespace emu
 
