@@ -196,7 +196,7 @@ static int op_new(imsrg_ctx_s *c, int herm, imsrg_op_s **out) {
   // (the FP64 products' 16-byte reads may take one element past the last block)
   const size_t bytes = sizeof(double) * (c->lay.op_size * c->nbatch + 8);
   op->d = c->op_pool.take();
-  if (!op->d && dev_malloc(c, (void **)&op->d, bytes) != hipSuccess) {
+  if (!op->d && dev_malloc((void **)&op->d, bytes) != hipSuccess) {
     delete op;
     return fail(IMSRG_ENOMEM, "hipMalloc operator failed");
   }
@@ -541,7 +541,7 @@ int imsrg_ctx_create_batch(int nsp, const int *n, const int *l, const int *jj, c
   if (!rc) rc = dalloc(c, (size_t)Ly.nsp * Ly.nsp, &c->mbar);
   for (int k = 0; k < imsrg_ctx_s::kSlots && !rc; k++) {
     void *p = nullptr;
-    if (hipMalloc(&p, B * sizeof(int)) != hipSuccess) {
+    if (dev_malloc(&p, B * sizeof(int)) != hipSuccess) {
       rc = fail(IMSRG_ENOMEM, "hipMalloc instance table failed");
       break;
     }
@@ -830,11 +830,11 @@ static int i8_setup(imsrg_ctx_s *c) {
   for (int k = 0; k < 2 && !rc; k++) {
     void *p = nullptr;
     const size_t vb = (size_t)c->i8.v_bytes * B, cb = (size_t)c->i8.c_bytes * B;
-    if (dev_malloc(c, &p, std::max<size_t>(vb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
+    if (dev_malloc(&p, std::max<size_t>(vb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
     c->dallocs.push_back(p);
     c->i8v[k] = (signed char *)p;
     HIPCHK(hipMemset(p, 0, std::max<size_t>(vb, 256)));
-    if (dev_malloc(c, &p, std::max<size_t>(cb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
+    if (dev_malloc(&p, std::max<size_t>(cb, 256)) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc int8 planes failed");
     c->dallocs.push_back(p);
     c->i8c[k] = (signed char *)p;
     HIPCHK(hipMemset(p, 0, std::max<size_t>(cb, 256)));

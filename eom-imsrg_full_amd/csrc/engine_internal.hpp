@@ -36,12 +36,14 @@ struct imsrg_op_s;
 
 // Operator buffers a context keeps for its next operator, whose work is ordered
 // behind theirs by the context's streams: at most kMax of them and kMaxBytes.
-// They go back to the device with the context, or when an allocation fails.
-// Operators may be destroyed by another thread than the one that computes.
+// They go back to the device with the context, or when an allocation of any
+// context fails (a destroyed operator's memory is not the context's alone: it was
+// free for everyone when hipFree took it).  Operators may be destroyed by another
+// thread than the one that computes.
 struct OpPool {
   static constexpr size_t kMax = 64, kMaxBytes = (size_t)4 << 30;
-  OpPool() = default;
-  ~OpPool() { (void)drain(); }
+  OpPool();
+  ~OpPool();
   OpPool(const OpPool &) = delete;
   OpPool &operator=(const OpPool &) = delete;
   double *take() {
@@ -69,6 +71,39 @@ struct OpPool {
   std::mutex mu;
   std::vector<double *> v;
 };
+// the pools of all contexts
+struct OpPools {
+  static bool drain() {
+    OpPools &a = all();
+    std::lock_guard<std::mutex> lock(a.mu);
+    bool any = false;
+    for (OpPool *p : a.v) any |= p->drain();
+    return any;
+  }
+
+ private:
+  friend struct OpPool;
+  static OpPools &all() {
+    static OpPools *const a = new OpPools;  // never destroyed: contexts may outlive statics
+    return *a;
+  }
+  std::mutex mu;
+  std::vector<OpPool *> v;
+};
+inline OpPool::OpPool() {
+  OpPools &a = OpPools::all();
+  std::lock_guard<std::mutex> lock(a.mu);
+  a.v.push_back(this);
+}
+inline OpPool::~OpPool() {
+  OpPools &a = OpPools::all();
+  {
+    std::lock_guard<std::mutex> lock(a.mu);
+    a.v.erase(std::find(a.v.begin(), a.v.end(), this));
+  }
+  (void)drain();
+}
+
 struct imsrg_ctx_s {
   Layout lay;
   DevLayout dl{};
@@ -220,11 +255,11 @@ int pack_tables(imsrg_ctx_s *c, const std::vector<PackSeg> &segs, const std::vec
 // context's stream; the call returns when they are there
 int stream_to_host(imsrg_ctx_s *c, const double *dev, int64_t n, double *host);
 int stream_to_dev(imsrg_ctx_s *c, const double *host, int64_t n, double *dev);
-// hipMalloc for a context; when it fails, the context's pool of operator
+// hipMalloc for a context; when it fails, every context's pool of operator
 // buffers goes back to the device and the call is made again
-inline hipError_t dev_malloc(imsrg_ctx_s *c, void **p, size_t bytes) {
+inline hipError_t dev_malloc(void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
-  if (e == hipSuccess || !c->op_pool.drain()) return e;
+  if (e == hipSuccess || !OpPools::drain()) return e;
   (void)hipGetLastError();
   return hipMalloc(p, bytes);
 }
@@ -232,7 +267,7 @@ template <class T>
 inline int upload_table(imsrg_ctx_s *c, const std::vector<T> &v, const T **out) {
   size_t bytes = std::max<size_t>(v.size(), 1) * sizeof(T);
   void *p = nullptr;
-  if (dev_malloc(c, &p, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc table failed");
+  if (dev_malloc(&p, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc table failed");
   c->dallocs.push_back(p);
   if (!v.empty()) HIPCHK(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
   *out = (const T *)p;
@@ -240,7 +275,7 @@ inline int upload_table(imsrg_ctx_s *c, const std::vector<T> &v, const T **out) 
 }
 inline int dalloc(imsrg_ctx_s *c, size_t ndouble, double **out) {
   void *p = nullptr;
-  if (dev_malloc(c, &p, std::max<size_t>(ndouble, 1) * sizeof(double)) != hipSuccess)
+  if (dev_malloc(&p, std::max<size_t>(ndouble, 1) * sizeof(double)) != hipSuccess)
     return fail(IMSRG_ENOMEM, "hipMalloc workspace failed (" + std::to_string(ndouble * 8) + " bytes)");
   c->dallocs.push_back(p);
   *out = (double *)p;

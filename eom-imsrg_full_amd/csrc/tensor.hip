@@ -1832,7 +1832,7 @@ int imsrg_tensor_create(imsrg_ctx c, int rank, int dpar, int herm, imsrg_tensor 
   t->ctx = c;
   t->ts = S;
   t->herm = herm;
-  if (hipMalloc(&t->d, sizeof(double) * S->op_size) != hipSuccess) {
+  if (dev_malloc((void **)&t->d, sizeof(double) * S->op_size) != hipSuccess) {
     delete t;
     return fail(IMSRG_ENOMEM, "hipMalloc tensor operator failed");
   }
@@ -2104,7 +2104,7 @@ int imsrg_bch_tensor(imsrg_op G, imsrg_tensor HS, int *nterms) {
   const long long bytes = 2LL * (long long)sizeof(double) * S.op_size;
   double *buf = S.bch;
   if (!buf) {
-    if (hipMalloc(&buf, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc BCH_TENSOR workspace failed");
+    if (dev_malloc((void **)&buf, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc BCH_TENSOR workspace failed");
     launch_fill(c->stream, buf, 2 * S.op_size, 0.0);
   }
   imsrg_tensor_s W[2];

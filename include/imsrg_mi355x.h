@@ -118,6 +118,10 @@ void *imsrg_ctx_stream(imsrg_ctx ctx);
 
 /* ---- operators (sq_op, basic_IMSRG.f90:50-76) ---------------------------- */
 int imsrg_op_create(imsrg_ctx ctx, int herm, imsrg_op *out);     /* duplicate_sq_op :2736 */
+/* The context keeps the buffers of up to 64 destroyed operators (4 GiB) for its
+ * next ones.  They go back to the device with the context, or as soon as an
+ * allocation of any context of the process fails; other users of the device see
+ * that memory as taken until then. */
 int imsrg_op_destroy(imsrg_op op);
 int imsrg_op_set_herm(imsrg_op op, int herm);
 int imsrg_op_get_herm(imsrg_op op, int *herm);
