@@ -277,7 +277,7 @@ static int scratch_setup(imsrg_ctx_s *c) {
 // Tables of the three-launch commutator (launch_small), for bases that may use it.
 static constexpr long long kSplitElems = 300000;  // two-body elements (the rule at wave_pair)
 // two-body elements times instances (the rules at comm_form)
-static constexpr long long kFusedElems = 200000, kMergedElems = 4000000, kTuneElems = 1000000;
+static constexpr long long kFusedElems = 200000, kMergedElems = 4000000;
 static int small_setup(imsrg_ctx_s *c, const std::vector<int> &same_ob) {
   const Layout &Ly = c->lay;
   const DevLayout &D = c->dl;
@@ -865,12 +865,12 @@ int imsrg_ctx_tuning(imsrg_ctx c, int *shape_pp, int *shape_ph, float *ms4) {
   if (!c || !shape_pp || !shape_ph) return fail(IMSRG_EINVAL, "null argument");
   *shape_pp = c->shape_pp;
   *shape_ph = c->shape_ph;
-  if (ms4) std::memcpy(ms4, c->tune_ms, sizeof(c->tune_ms));
+  if (ms4) std::fill(ms4, ms4 + 4, 0.f);  // nothing is timed: the shapes go by a rule
   return 0;
 }
 int imsrg_ctx_set_tile_shapes(imsrg_ctx c, int shape_pp, int shape_ph) {
   if (!c || shape_pp < -1 || shape_pp > 1 || shape_ph < -1 || shape_ph > 1)
-    return fail(IMSRG_EINVAL, "shapes: -1 (tune), 0 (64x64) or 1 (128x64)");
+    return fail(IMSRG_EINVAL, "shapes: -1 (by the rule), 0 (wavefront tiles) or 1 (128x64)");
   if (shape_pp < 0 || shape_ph < 0) shape_pp = shape_ph = -1;
   c->shape_pp = shape_pp;
   c->shape_ph = shape_ph;
@@ -1375,6 +1375,19 @@ enum { kLPrepped = 1, kLPandya = 2, kRPandya = 4 };
 static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                          int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi());
 
+// The FP64 tile shapes of a context that has not fixed them: a rule on the basis,
+// so that results do not depend on a stopwatch (the shapes add K in different
+// orders) and a batch has its instances' bits.  pp/hh, us for 32 x 32 wavefront
+// tiles / 128 x 64 workgroup tiles, six holes: emax 8 (7.2e6 elements) 121 / 199,
+// emax 9 (1.7e7) 417 / 551, emax 10 (3.7e7) 1493 / 1645, emax 11 (7.6e7) 4623 /
+// 4264, emax 12 (1.5e8) 13666 / 10937, emax 14 (5.0e8) 87529 / 60970; with 1 and 20
+// holes the line is the same (20 holes: emax 10 1060 / 1141, emax 11 3342 / 3253).
+// The Pandya product: 132 / 179 at emax 8, 835 / 1015 at emax 10, 4008 / 4563 at
+// emax 12, 14770 / 17061 at emax 14 (with 20 holes at emax 12 16918 / 16633): the
+// wavefront tiles.
+static constexpr long long kWideElems = 50000000;
+static int rule_shape_pp(const imsrg_ctx_s *c) { return c->lay.vsize > kWideElems; }
+
 // The form of a commutator (launch_small; all forms give the same bits).  Per
 // commutator of a BCH series, in us, separate kernels on two streams / merged
 // (five launches) / fused (three), by two-body elements times instances:
@@ -1395,7 +1408,7 @@ enum CommForm { kSeparate, kMerged, kFused };
 static CommForm comm_form(const imsrg_ctx_s *c, unsigned mask, int cc_ready, int na) {
   const unsigned all = T111 | T121 | T122 | T221 | T222PPHH | T222PH;
   if (!c->mergeable || c->prec != IMSRG_PREC_FP64 || c->prof_on || (mask & all) != all ||
-      (cc_ready & (kLPandya | kRPandya)) || c->shape_pp == 1 || c->shape_ph == 1)
+      (cc_ready & (kLPandya | kRPandya)) || (c->shape_pp < 0 ? rule_shape_pp(c) : c->shape_pp) == 1 || c->shape_ph == 1)
     return kSeparate;
   const long long n = (long long)c->lay.vsize * na;
   if (c->small && n <= kFusedElems) return kFused;
@@ -1415,72 +1428,15 @@ static void flush_gate(imsrg_ctx_s *c) {
 // it: emax 6 100.8 -> 102.6 us, emax 7 205 -> 215, so the gate keeps its launch.
 static bool defer_gate(const imsrg_ctx_s *c, CommForm form, int na) { return !c->graphs && form == kFused; }
 
-// Tile-shape autotuner: on the first FP64 commutator of a context, each 222
-// GEMM is timed (HIP events, best of 3) in both FP64 tile shapes on the
-// context's real channel/Pandya blocks and the faster one is kept.  The
-// pp/hh timing writes nothing (no C, no W); the Pandya timing writes the Z
-// workspace, which every commutator recomputes before reading.  The timing
-// covers every instance of the context (a series table may already mark
-// instances as stopped, and skipped workgroups would time nothing).
-static int autotune(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R) {
-  const ActSet a = all_set(c);
-  hipStream_t s = c->stream;
-  const DevLayout &D = c->dl;
-  hipEvent_t e0, e1;
-  HIPCHK(hipEventCreate(&e0));
-  HIPCHK(hipEventCreate(&e1));
-  auto timed = [&](auto &&launch) {
-    float best = 1e30f;
-    for (int r = 0; r < 4; r++) {
-      (void)hipEventRecord(e0, s);
-      launch();
-      (void)hipEventRecord(e1, s);
-      (void)hipEventSynchronize(e1);
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      if (r > 0) best = std::min(best, ms);  // first run warms up
-    }
-    return best;
-  };
-  const double *X0 = L->d + D.v_off, *X1 = R->d + D.v_off;
-  const bool sp = c->split;
-  c->tune_ms[0] = timed([&] {
-    launch_seg_gemm_pphh(s, 0, c->pp_probs, c->pp_tiles_s, c->n_pp_tiles_s, X0, X1, nullptr, nullptr, a.d, a.n(), D.op_size,
-                         D.vsize);
-  });
-  c->tune_ms[1] = timed([&] {
-    launch_seg_gemm_pphh(s, 3, c->pp_probs, c->pp_tiles_w, c->n_pp_tiles_w, X0, X1, nullptr, nullptr, a.d, a.n(),
-                         D.op_size, D.vsize);
-  });
-  launch_pandya(s, D, L->d, c->cc[0], a.d, a.n());
-  launch_pandya(s, D, R->d, c->cc[1], a.d, a.n());
-  c->tune_ms[2] = timed([&] {
-    launch_seg_gemm_z(s, sp ? 4 : 0, c->ph_probs, sp ? c->ph_tiles_s : c->ph_tiles,
-                      sp ? c->n_ph_tiles_s : c->n_ph_tiles, c->cc[0], c->cc[1], c->wph, (double)L->herm,
-                      (double)R->herm, a.d, a.n(), D.ccsize, D.cwsize);
-  });
-  c->tune_ms[3] = timed([&] {
-    launch_seg_gemm_z(s, 3, c->ph_probs, c->ph_tiles_w, c->n_ph_tiles_w, c->cc[0], c->cc[1], c->wph, (double)L->herm,
-                      (double)R->herm, a.d, a.n(), D.ccsize, D.cwsize);
-  });
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  c->shape_pp = c->tune_ms[1] < c->tune_ms[0] ? 1 : 0;
-  c->shape_ph = c->tune_ms[3] < c->tune_ms[2] ? 1 : 0;
-  HIPCHK(hipGetLastError());
-  return 0;
-}
 // One commutator: the launch sequence of comm_launches, replayed from a cached
 // hipGraph when graph mode is on (and profiling off).  The graph holds kernel
 // nodes only; operands, workspaces and the instance table are fixed device
 // addresses, so a replay is the same work as the eager sequence.
 static int comm_impl(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_s *RES, unsigned mask,
                      int cc_ready, const ActSet &a, const CommEpi &epi = CommEpi()) {
-  if (c->prec == IMSRG_PREC_FP64 && c->shape_pp < 0 && a.n() > 0 && (mask & (T222PPHH | T221 | T222PH)) &&
-      (comm_form(c, mask, cc_ready, a.g()) == kSeparate || c->lay.vsize * a.g() > kTuneElems)) {
-    c->fork_mark = nullptr;  // the tuning launches follow the mark on the stream
-    int rc = autotune(c, L, R);
-    if (rc) return rc;
+  if (c->prec == IMSRG_PREC_FP64 && c->shape_pp < 0 && a.n() > 0 && (mask & (T222PPHH | T221 | T222PH))) {
+    c->shape_pp = rule_shape_pp(c);
+    c->shape_ph = 0;
   }
   if (!c->graphs || c->prof_on || a.n() == 0) return comm_launches(c, L, R, RES, mask, cc_ready, a, epi);
   // the gate's arguments change with every term: it stays outside the graph

@@ -179,11 +179,10 @@ struct imsrg_ctx_s {
   int4 *pp_tiles_s = nullptr, *ph_tiles_s = nullptr;
   int n_pp_tiles_s = 0, n_ph_tiles_s = 0;
   bool split = false;
-  // FP64 tile shape per GEMM, chosen by timing both on the first FP64
-  // commutator of the context: -1 not yet tuned, 0 the wavefront GEMM (its tiles
-  // by the rule at wave_pair), 1 128x64 workgroup tiles
+  // FP64 tile shape per GEMM: -1 before the first FP64 commutator (then by the rule
+  // at rule_shape_pp), 0 the wavefront GEMM (its tiles by the rule at wave_pair), 1
+  // 128x64 workgroup tiles
   int shape_pp = -1, shape_ph = -1;
-  float tune_ms[4] = {0, 0, 0, 0};                      // pp shape 0, pp 128x64, ph shape 0, ph 128x64
   int prec = IMSRG_PREC_FP64;
   // int8-sliced GEMM operands (IMSRG_PREC_INT8X5 / INT8X4), built on first use:
   // planes and row scales of operand 0 (L) and 1 (R), V rows and Pandya rows

@@ -214,11 +214,11 @@ class Context:
         _chk(_lib.imsrg_ctx_set_concurrency(self.h, 1 if enable else 0))
 
     def tuning(self):
-        """FP64 tile shapes chosen by the autotuner and its four timings (ms)"""
+        """FP64 tile shapes of the context's products (by a rule on its basis, or as set)"""
         a, b = C.c_int(0), C.c_int(0)
         ms = (C.c_float * 4)()
         _chk(_lib.imsrg_ctx_tuning(self.h, C.byref(a), C.byref(b), ms))
-        # the names of the two shapes; "64x64" runs as 32 x 32 tiles a wavefront
+        # the names of the two shapes ("64x64" runs as 32 x 32 tiles a wavefront); the times are zeros
         names = {-1: "untuned", 0: "64x64", 1: "128x64"}
         return dict(pphh=names[a.value], ph=names[b.value], ms_pphh_64=ms[0], ms_pphh_128x64=ms[1],
                     ms_ph_64=ms[2], ms_ph_128x64=ms[3])

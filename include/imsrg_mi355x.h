@@ -89,8 +89,8 @@ int64_t imsrg_ctx_neq(imsrg_ctx ctx);
 /* info[0..15]: nsp, nhole, nblocks, ncc, npairs, max block dim, max CC rows,
  * device bytes per operator, vsize, ccsize, cwsize, flop_pphh, flop_ph
  * (as doubles: algorithmic GEMM flop per commutator), ph recoupling J' terms,
- * upper-triangle two-body elements, FP64 tile shapes chosen by the autotuner
- * (4*(pp+1) + (ph+1), shapes -1 untuned, 0 wavefront tiles, 1 128x64 workgroup tiles) */
+ * upper-triangle two-body elements, FP64 tile shapes
+ * (4*(pp+1) + (ph+1), as imsrg_ctx_tuning reports them) */
 int imsrg_ctx_info(imsrg_ctx ctx, double *info16);
 int imsrg_ctx_set_precision(imsrg_ctx ctx, int prec);
 int imsrg_ctx_synchronize(imsrg_ctx ctx);
@@ -99,12 +99,12 @@ int imsrg_ctx_synchronize(imsrg_ctx ctx);
  * once per distinct (operands, hermiticities, term mask, instance set,
  * precision) into a hipGraph and replayed.  Off while profiling is on. */
 int imsrg_ctx_set_graphs(imsrg_ctx ctx, int enable);
-/* FP64 tile shapes the autotuner chose on the context's first FP64 commutator
- * (-1 not yet or a basis below the tuner's size, 0 32x32 wavefront tiles, 1
- * 128x64 workgroup tiles) and the four timings (ms: pp/hh shape 0, pp/hh 1,
- * Pandya product 0, 1) */
+/* FP64 tile shapes of the pp/hh and the Pandya product: -1 before the context's
+ * first FP64 commutator, then 0 (32x32 wavefront tiles) or 1 (128x64 workgroup
+ * tiles) by a rule on the size of the basis, the same in every run.  ms4: four
+ * zeros (the shapes used to be timed). */
 int imsrg_ctx_tuning(imsrg_ctx ctx, int *shape_pp, int *shape_ph, float *ms4);
-/* fix the FP64 tile shapes (0 or 1 each), or -1 to tune again on the next commutator */
+/* fix the FP64 tile shapes (0 or 1 each; they round differently), or -1 for the rule */
 int imsrg_ctx_set_tile_shapes(imsrg_ctx ctx, int shape_pp, int shape_ph);
 int imsrg_ctx_graph_stats(imsrg_ctx ctx, long long *builds, long long *launches);
 /* Commutator concurrency (no counterpart in the reference): with enable = 1
