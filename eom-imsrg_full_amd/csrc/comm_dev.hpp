@@ -115,6 +115,7 @@ __device__ __forceinline__ void pandya_col(const DevLayout &L, std::conditional_
       for (int J0 = Jmin; J0 <= Jmax; J0 += 16) {
         long long off[8];
         double w[8];
+        unsigned held = 0;  // bit u: the block holds the element
 #pragma unroll
         for (int u = 0; u < 8; u++) {
           const int JT = min(J0 + 2 * u, Jmax);
@@ -127,12 +128,13 @@ __device__ __forceinline__ void pandya_col(const DevLayout &L, std::conditional_
           const bool ok = J0 + 2 * u <= Jmax && (rr | ss) >= 0;
           off[u] = ok ? BO[q] + (long long)rr * BD[q] + ss : 0;
           w[u] = ok ? pre * (double)(sgnp(JT >> 1) * (JT + 1)) * six[JT >> 1] : 0.0;
+          held |= (unsigned)ok << u;
         }
         if constexpr (ADJ) {
           const double g0 = val * sgnp((jh + jb + JC) >> 1) * sq;
 #pragma unroll
           for (int u = 0; u < 8; u++)
-            if (g0 * w[u] != 0.0) atomicAdd(V + off[u], g0 * w[u]);
+            if ((held >> u & 1) && g0 * w[u] != 0.0) atomicAdd(V + off[u], g0 * w[u]);
         } else {
           double vv[8];
 #pragma unroll
