@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <cfloat>
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -363,6 +364,12 @@ struct TLists {
 constexpr int kT1Threads = 768;
 constexpr int kT1Lds = 163840;  // LDS of a workgroup at most
 
+// The weight of an entry that an output does not have: it adds nothing, and no
+// weight of a term is -0.  Where a sum is not finite it is made again without
+// such entries, since 0 times an infinite element is not 0.
+constexpr double kAbsent = -0.0;
+__device__ __forceinline__ bool absent(double w) { return w == 0.0 && std::signbit(w); }
+
 // one wavefront per list, a lane per entry
 __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists W, const double *__restrict__ LF,
                                                 const double *__restrict__ RF, int do122, int do212) {
@@ -377,7 +384,7 @@ __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists
   const int p1 = T.pstart[a], m1 = T.pstart[a + 1] - p1, p2 = T.pstart[b], m2 = T.pstart[b + 1] - p2;
   const double n212 = sqrt((J1 + 1.0) * (J2 + 1.0)) * sgnp(R >> 1);
   for (int e = threadIdx.x; e < li.n; e += 64) {
-    double w = 0.0;
+    double w = kAbsent;
     if (e < c1 + c2) {
       // i for a (with o = b) or for b (o = a)
       const bool fa = e < c1;
@@ -386,7 +393,7 @@ __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists
       // the pair is (i,o) when i stands for a, (o,i) when for b
       const bool swp = fa ? i > o : o > i;
       const double f = swp ? (double)sgnp(1 + ((ji + jo - J) >> 1)) : (i == o ? M_SQRT2 : 1.0);
-      if (do122) w = li.side ? -f * LF[(size_t)i * n + x] * dab : f * LF[(size_t)x * n + i] * dab;
+      if (do122) w = (li.side ? -f * LF[(size_t)i * n + x] * dab : f * LF[(size_t)x * n + i] * dab) + 0.0;
     } else if (e < c1 + c2 + m1 + m2) {
       const int k = e - c1 - c2;
       const bool fa = k < m1;
@@ -404,11 +411,11 @@ __global__ __launch_bounds__(64) void k_t_lists(DevLayout L, DevTensor T, TLists
           sx = fa ? six(ja, ji, jb) : six(jb, ji, ja);
           sg = fa ? -(double)sgnp((J1 + J2) >> 1) : (double)sgnp((ja + jb - J1) >> 1);
         }
-        w = sg * sx * f * (li.side ? RF[(size_t)i * n + x] : RF[(size_t)x * n + i]) * n212 * dab;
+        w = sg * sx * f * (li.side ? RF[(size_t)i * n + x] : RF[(size_t)x * n + i]) * n212 * dab + 0.0;
       }
     }
     if (li.side) {
-      W.cw[li.base + 64LL * e] = W.cp[li.base + 64LL * e] == 0xffff ? 0.0 : w;
+      W.cw[li.base + 64LL * e] = W.cp[li.base + 64LL * e] == 0xffff ? kAbsent : w;
     } else {
       const int d = W.rdst[li.base + e];
       if (d >= 0) W.rw[d] = w;
@@ -501,13 +508,36 @@ __global__ __launch_bounds__(kT1Threads, 4) void k_t_1body(DevLayout L, DevTenso
         for (int j = 0; j < 8; j++) acc[j] = fma(w[v], row0[min(j, gn - 1) * ld + pv], acc[j]);
       }
     }
-    if (s < n2)
+    bool finite = true;
+#pragma unroll
+    for (int j = 0; j < 8; j++) finite = finite && fabs(acc[j]) <= DBL_MAX;
+    if (s < n2 && finite) {
 #pragma unroll
       for (int j = 0; j < 8; j++)
         if (j < gn) {
           double *o = OV + T.off[q] + (long long)(grow[8 * g + j] & 0xffffff) * n2 + s;
           *o = add ? *o + acc[j] : acc[j];
         }
+    } else if (s < n2) {
+      // (everything read again here, so that the loops above keep their registers)
+#pragma unroll 1
+      for (int j = 0; j < grow[8 * g + 7] >> 24; j++) {
+        double sum = 0.0;
+#pragma unroll 1
+        for (int e = (int)(gs[g].base - b0); e < (int)(gs[g].base - b0 + gs[g].n); e++) {
+          const int r = lr[e];
+          if (!absent(lw[8 * e + j]))
+            sum = fma(lw[8 * e + j], (r >= 0 ? Tq + (long long)r * n2 : V2 + (long long)~r * n2)[s], sum);
+        }
+#pragma unroll 1
+        for (int e = 0; e < (int)W.cols[W.cbase[q] + ch].n; e++) {
+          const long long o = W.cols[W.cbase[q] + ch].base + (long long)e * 64 + lane;
+          if (!absent(W.cw[o])) sum = fma(W.cw[o], rows[(st + j) * ld + W.cp[o]], sum);
+        }
+        double *o = OV + T.off[q] + (long long)(grow[8 * g + j] & 0xffffff) * n2 + s;
+        *o = add ? *o + sum : sum;
+      }
+    }
   }
 }
 
@@ -1639,7 +1669,7 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
             rdst.push_back(8 * slot[k] + j);
           });
         }
-        while (((long long)rsrc.size() - base) % 8 != 0) rsrc.push_back(0);  // of weight 0
+        while (((long long)rsrc.size() - base) % 8 != 0) rsrc.push_back(0);  // absent
         groups.push_back(TSlice{base, (long long)rsrc.size() - base});
         gsize.push_back(n);
         r += n;
@@ -1716,8 +1746,8 @@ static int tspace_build(imsrg_ctx_s *c, int rank, int dpar, TensorSpace &S) {
         return IMSRG_ENOMEM;
       const long long nr = 8LL * rsrc.size(), nc = (long long)cp.size();
       if (dalloc(c, nr, &W.rw) || dalloc(c, nc, &W.cw)) return IMSRG_ENOMEM;
-      launch_fill(c->stream, W.rw, nr, 0.0);  // the weights no list writes stay 0
-      launch_fill(c->stream, W.cw, nc, 0.0);
+      launch_fill(c->stream, W.rw, nr, kAbsent);  // the weights no list writes stay so
+      launch_fill(c->stream, W.cw, nc, kAbsent);
       if (lds > 65536)
         // (the kernel's limit in the whole process: the most any space may take, not this one's)
         HIPCHK(hipFuncSetAttribute((const void *)k_t_1body, hipFuncAttributeMaxDynamicSharedMemorySize, kT1Lds));

@@ -26,3 +26,25 @@ call = lambda x: ctx.commutator_adjoint(P, ctx.op(1, x), 1, mask=E.T222PH).downl
 ks = np.flatnonzero(v)[::97][[2, 6, 7, 8, 9]]  # whose terms have no vanishing 6j symbols
 assert [spread(call, v, k) for k in ks] == [0] * 5
 """)
+
+
+@pytest.mark.parametrize("rank,dpar", [(2, 0), (2, 2), (4, 0)])
+def test_tensor_one_body_terms(rank, dpar):
+    """122: at emax 1 every orbit stands alone in its class, so an element of T
+    reaches one output; 212 reads T's one-body part only"""
+    run(f"""
+B = Basis.ho(1, 1)
+ctx = E.Context(B)
+G, T, R = ctx.op(-1, random_operator(B, -1, 7)), ctx.tensor({rank}, {dpar}), ctx.tensor({rank}, {dpar})
+rng = np.random.default_rng(0)
+v0 = 1 + len(B.holes) ** 2 + len(B.parts) ** 2 + len(B.parts) * len(B.holes)
+for k in rng.choice(np.arange(v0, T.neq), 12, replace=False):
+    t = rng.uniform(-1, 1, T.neq)
+    t[k] = np.inf
+    T.upload(t)
+    n = []
+    for mask in (8, 16):
+        R.clear()
+        n.append(int((~np.isfinite(ctx.tensor_commutator(G, T, R, mask=mask).download())).sum()))
+    assert n[0] <= 1 and n[1] == 0, (k, n)
+""")
