@@ -2068,7 +2068,7 @@ __device__ __forceinline__ long long gate_inst(const PendingGate &P, double *sh)
   int *const word = reinterpret_cast<int *>(sh);
   if (threadIdx.x == 0) *word = __hip_atomic_load(P.act + blockIdx.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  const int inst = *word;
+  const int inst = __builtin_amdgcn_readfirstlane(*word);  // (in a scalar register, as one read from the table)
   __syncthreads();
   return inst;
 }
