@@ -772,13 +772,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
         nseg += __popcll(m);
         s0 += 64;
       }
+      // none may be left: the reads below then take this for slot 0 (leaving the
+      // loop here instead costs the compiler 39 more spilled registers)
+      if (lane == 0 && nseg == 0) seg[0].code = 0;
       __syncthreads();
       const int nb = min(nseg, kPhB);
-      if (nb == 0) break;  // the scan found no further slot: there is none to read below
       {
         int ix[4], jx_[4];
         double w[4];
-        auto slot = [&](int k) -> const PanSeg & { return seg[min(8 * k + (lane >> 3), nb - 1)]; };
+        auto slot = [&](int k) -> const PanSeg & { return seg[min(8 * k + (lane >> 3), max(nb - 1, 0))]; };
 #pragma unroll
         for (int k = 0; k < 4; k++) {
           const unsigned gc = slot(k).code;
