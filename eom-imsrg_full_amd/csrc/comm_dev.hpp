@@ -283,7 +283,7 @@ __device__ __forceinline__ void wave_segments(const SegProb &p, int s0, int s1, 
 // wavefronts as above, summed through LDS; reads and writes stay inside
 // M x K, K x N and M x N except the neighbour an odd K's or N's last 16-byte
 // pair takes (in a channel block: its padding or next row).
-struct SplitSmem {
+struct alignas(16) SplitSmem {  // (read and written in pairs)
   double s[4][32][34];
 };
 __device__ __forceinline__ void plain_tile(const GemmProb &p, int m0, int n0, const double *__restrict__ A,
