@@ -170,9 +170,10 @@ static ActSet all_set(imsrg_ctx_s *c) {
   for (int k = 0; k < c->nbatch; k++) a.h[k] = k;
   return a;
 }
-// Writes `list` into table `slot` (an asynchronous copy on the context
-// stream).  Drivers rewrite a slot only after a stream synchronization, so
-// the pinned source is never overwritten while a copy from it is pending.
+// Writes `list` into table `slot` (an asynchronous copy on the context stream).
+// A driver rewrites a slot only after it has waited for something that follows the
+// copy on the stream (a flow step for its step report), so the pinned source is
+// never overwritten while a copy from it is pending.
 // Slots 1 and 2 are the BCH and Magnus series tables (series_begin).
 // With pad > list size the table is padded with -1 entries to pad entries.
 static ActSet make_set(imsrg_ctx_s *c, int slot, const std::vector<int> &list, int pad = 0) {
@@ -1305,7 +1306,8 @@ int imsrg_hartree_fock_noalloc(imsrg_op H, double *coefs, int *iterations, doubl
       return fail(IMSRG_EINVAL, "imsrg_hartree_fock_noalloc: channel block " + std::to_string(q) + " (dim " +
                                     std::to_string(Ly.bdim[q]) + ") exceeds the scratch window of " +
                                     std::to_string(wcap) + " doubles");
-  double *D = m[0], *Vg = m[2], *Fm = m[3], *Tm = m[4], *W = base + state;  // (m[1] unused)
+  double *D = m[0], *Vg = m[2], *Fm = m[3], *Tm = m[4], *W = base + state;
+  // (m[1] is not used any more; its place stays, and with it the bases the call takes)
   const DevLayout &DL = c->dl;
   launch_fill(c->stream, base, state, 0.0);
   launch_hf_init(c->stream, DL, H->d, D, Tm, eig, 1);
@@ -1395,13 +1397,15 @@ static int rule_shape_pp(const imsrg_ctx_s *c) { return c->lay.vsize > kWideElem
 //   emax 5 (2.9e5)     103 / 61 / 67     emax 6 (9.6e5)      142 / 101 / 125
 //   4 x emax 5 (1.1e6) 145 / 139         emax 7 (2.8e6)      248 / 207
 //   4 x emax 6 (3.8e6) 321 / 294         16 x emax 5 (4.6e6) 407 / 428
-//   emax 8 (7.2e6)     637 / 601         2 x emax 8 (1.4e7)  1100 / 1088
+//   emax 8 (7.2e6)     641 / 605         2 x emax 8 (1.4e7)  1227 / 1215
+//   emax 9 (1.7e7)    1595 / 1556        2 x emax 9 (3.4e7)  3184 / 3091
 //   16 x emax 6 (1.5e7) 1114 / 1133
 // Fused pays while launches are what a commutator costs; past 2e5 the ph sums
 // straight from Z, made anew for every J, cost more than a launch for the J'
 // terms.  Merged pays while a kernel's last workgroups leave much of the chip
-// idle: up to 4e6 elements, and for one or two instances in any basis; with
-// many instances the separate kernels fill the chip and overlap on two streams.
+// idle: up to 4e6 elements, and for one or two instances in any basis (full ones
+// past emax 9 have 122 sets past 32 rows); with many instances the separate
+// kernels fill the chip and overlap on two streams.
 // Masks with terms left out, profiling, tile shapes set to 128 x 64, other
 // precisions and bases with 122 sets past 32 rows keep the separate kernels.
 enum CommForm { kSeparate, kMerged, kFused };
@@ -1508,8 +1512,10 @@ static int comm_launches(imsrg_ctx_s *c, imsrg_op_s *L, imsrg_op_s *R, imsrg_op_
     A.T = form == kFused ? nullptr : c->tph;
     A.obpart = c->obpart;
     // the first launch's parts as kernels of their own, the 122 weights from a
-    // table, where they are long: emax 8 613 us a commutator against 624, 16 x
-    // emax 4 177 / 196, but emax 7 215 / 207, emax 6 110 / 101
+    // table, where they are long (us a commutator so / in one launch): emax 8 605 /
+    // 619, 2 x emax 8 1215 / 1258, emax 9 1556 / 1586, 2 x emax 7 400 / 405, 4 x
+    // emax 6 280 / 289, 16 x emax 4 177 / 196, but emax 7 205 / 196, emax 6 105 / 96
+    // (2 x emax 6, at the line, 156 / 153)
     A.w122 = form == kMerged && D.vsize * na > (na == 1 ? 3000000 : 1000000) ? c->w122 : nullptr;
     A.diff_ob = c->diff_ob; A.phrow = c->phrow; A.act = ad;
     if (c->gate_pend.act && (c->gate_pend.act != ad || A.w122)) flush_gate(c);
