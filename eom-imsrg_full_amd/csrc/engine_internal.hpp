@@ -35,7 +35,8 @@ inline int fail(int code, const std::string &msg) {
 struct imsrg_op_s;
 
 // Operator buffers a context keeps for its next operator, whose work is ordered
-// behind theirs by the context's streams: at most kMax of them and kMaxBytes.
+// behind theirs by the context's streams: at most kMax of them and kMaxBytes.  (A
+// tensor space keeps BCH_TENSOR's work operators the same way.)
 // They go back to the device with the context, or when an allocation of any
 // context fails (a destroyed operator's memory is not the context's alone: it was
 // free for everyone when hipFree took it).  Operators may be destroyed by another

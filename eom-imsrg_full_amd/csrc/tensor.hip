@@ -1268,13 +1268,12 @@ struct TensorSpace {
   const TRun *runs = nullptr;
   int nrun = 0, seq = 0;
   TNorm *norm = nullptr;   // host memory
-  double *bch = nullptr;   // BCH_TENSOR's two work operators, kept up to kBchKeep bytes
+  OpPool bch;              // BCH_TENSOR's two work operators, in one buffer, kept up to kBchKeep bytes
   const TProb *pp_probs = nullptr, *cc_probs = nullptr;
   const int4 *pp_tiles = nullptr, *cc_tiles = nullptr;
   int n_pp_tiles = 0, n_cc_tiles = 0;
   ~TensorSpace() {
     if (norm) (void)hipHostFree(norm);
-    if (bch) (void)hipFree(bch);
   }
 };
 
@@ -2134,7 +2133,7 @@ int imsrg_bch_tensor(imsrg_op G, imsrg_tensor HS, int *nterms) {
   if (G->ctx != c) return fail(IMSRG_EINVAL, "G and HS belong to different contexts");
   TensorSpace &S = *HS->ts;
   const long long bytes = 2LL * (long long)sizeof(double) * S.op_size;
-  double *buf = S.bch;
+  double *buf = S.bch.take();
   if (!buf) {
     if (dev_malloc((void **)&buf, bytes) != hipSuccess) return fail(IMSRG_ENOMEM, "hipMalloc BCH_TENSOR workspace failed");
     launch_fill(c->stream, buf, 2 * S.op_size, 0.0);
@@ -2160,12 +2159,9 @@ int imsrg_bch_tensor(imsrg_op G, imsrg_tensor HS, int *nterms) {
     if (nrm * coef < conv) break;
     AD = INT2;
   }
-  if (bytes <= kBchKeep && rc == 0) {
-    S.bch = buf;
-  } else {
+  if (bytes > kBchKeep || rc != 0 || !S.bch.give(buf, bytes)) {
     (void)hipStreamSynchronize(c->stream);
     (void)hipFree(buf);
-    S.bch = nullptr;
   }
   if (nterms) *nterms = n;
   return rc;

@@ -58,3 +58,14 @@ ts = [threading.Thread(target=work) for _ in range(8)]
 [t.join() for t in ts]
 assert not bad
 """, IMSRG_EMU_CHECK=1)
+
+
+def test_tensor_workspace_is_given_back():
+    """BCH_TENSOR's work operators, kept for its next call"""
+    run(HOARD + """
+ctx.bch_tensor(G, T)
+full()
+U = ctx.tensor(2, 0)
+lib.emu_set_limit(2 ** 62)
+assert ctx.bch_tensor(G, T) >= 1
+""")
