@@ -1,6 +1,7 @@
 """The library built for the host: the same sources compiled as C++ against
 cpu_hip/, whose runtime runs a kernel one workgroup at a time with bounds
 checks and guard pages (cpu_hip/emu.cpp).  For what must not be tried on a GPU."""
+import fcntl
 import os
 import subprocess
 import sys
@@ -18,6 +19,12 @@ FLAGS = ["-std=c++17", "-O1", "-g1", "-fPIC", "-fno-strict-aliasing", "-fsanitiz
 def build():
     """path of the host library, built anew where a source is younger"""
     os.makedirs(OUT, exist_ok=True)
+    with open(os.path.join(OUT, "lock"), "w") as lock:  # one builder at a time
+        fcntl.flock(lock, fcntl.LOCK_EX)
+        return _build()
+
+
+def _build():
     lib = os.path.join(OUT, "libimsrg_cpu.so")
     src = [os.path.join(CSRC, f) for f in ("kernels.hip", "ozaki.hip", "adjoint.hip", "hf.hip", "engine.hip", "layout.cpp",
                                            "interaction_io.cpp")]
